@@ -128,6 +128,24 @@ __device__ __forceinline__ float wave_sum_dpp(float v) {
            __builtin_bit_cast(float, __builtin_amdgcn_readlane(iv, 32)) + __builtin_bit_cast(float, __builtin_amdgcn_readlane(iv, 48));
 }
 
+// Lane `src` of a 64-bit / float register as a wave-uniform value (src is wave-uniform).
+__device__ __forceinline__ uint64_t readlane64(uint64_t v, uint32_t src) {
+    const uint32_t lo = __builtin_amdgcn_readlane((int)(uint32_t)v, src), hi = __builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), src);
+    return ((uint64_t)hi << 32) | lo;
+}
+__device__ __forceinline__ float readlane_f32(float v, uint32_t src) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), src));
+}
+
+// Smallest value over the wave, in every lane.
+__device__ __forceinline__ float wave_min_dpp(float v) {
+    v = fminf(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0xB1, 0xF, 0xF, false)));
+    v = fminf(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x4E, 0xF, 0xF, false)));
+    v = fminf(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x141, 0xF, 0xF, false)));
+    v = fminf(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x140, 0xF, 0xF, false)));
+    return fminf(fminf(readlane_f32(v, 0), readlane_f32(v, 16)), fminf(readlane_f32(v, 32), readlane_f32(v, 48)));
+}
+
 // Total order on floats as unsigned integers (negative distances are common: 1 - IP).
 __device__ __forceinline__ uint32_t float_key(float f) {
     uint32_t u = __float_as_uint(f);
@@ -336,15 +354,6 @@ __device__ __forceinline__ void eval_issue_desc(PendingEval& p, const CorpusView
     }
 }
 
-// Lane `src` of a 64-bit / float register as a wave-uniform value (src is wave-uniform).
-__device__ __forceinline__ uint64_t readlane64(uint64_t v, uint32_t src) {
-    const uint32_t lo = __builtin_amdgcn_readlane((int)(uint32_t)v, src), hi = __builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), src);
-    return ((uint64_t)hi << 32) | lo;
-}
-__device__ __forceinline__ float readlane_f32(float v, uint32_t src) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), src));
-}
-
 // ---- query term tables for the search kernels ----
 // One table per path (SPLADE first, BM25 second, each sized for the longest row of its path), two (key, value)
 // entries per 16-byte bucket, so a lookup is ONE ds_read_b128 and no probe loop: every lane can issue
@@ -355,10 +364,15 @@ __device__ __forceinline__ float readlane_f32(float v, uint32_t src) {
 // path. A term whose bucket is already full goes to an overflow list that holds up to every term of
 // the row (with at least twice as many buckets as terms it is empty for most rows); its length is
 // wave-uniform and the list is only walked when it is not zero.
+// Keyword-filter search: bit 31 of a stored BM25 key says that the query requires the term (the path of a key follows
+// from its table there, and keys are compared without that bit), so a match tells a keyword hit by itself; a separate
+// set of the required terms, asked in a divergent probe loop for every BM25 match, cost 0.4 ms of the 2.55 ms of 777
+// queries at cands 128 on 100 k documents.
 struct QueryTabs {
     uint4* b;        // [(mask_s + 1) + (mask_b + 1)] buckets: (key0, value0, key1, value1)
     uint2* ovf;      // overflow entries: (term | path bit, value)
-    uint32_t* n_ovf; // their number
+    uint32_t* n_ovf; // their number; keyword-filter search: required terms are counted in the upper half and fill the list from its end
+    uint32_t ovf_cap;
     uint32_t mask_s, mask_b; // buckets of the SPLADE / BM25 table - 1
 };
 
@@ -375,25 +389,29 @@ __device__ __forceinline__ void query_tabs_clear(const QueryTabs& T, int tid, in
     if (tid == 0) *T.n_ovf = 0;
 }
 
-// key carries the path bit; keys inserted into one table are distinct.
-template <bool NARROW>
-__device__ __forceinline__ void query_tabs_insert(const QueryTabs& T, uint32_t key, float val) {
-    const uint32_t raw = NARROW ? key & ~BM25_BIT : key;
-    const uint32_t h = query_hash<NARROW>(raw);
+// key carries the path bit; keys inserted into one table are distinct. required: keyword-filter search only.
+template <bool NARROW, bool KWD>
+__device__ __forceinline__ void query_tabs_insert(const QueryTabs& T, uint32_t key, float val, bool required) {
+    const uint32_t term = key & ~BM25_BIT;
+    const uint32_t raw = KWD ? term | (required ? BM25_BIT : 0u) : NARROW ? term : key;
+    const uint32_t h = query_hash<NARROW>(term);
     uint4* e = T.b + ((key & BM25_BIT) ? T.mask_s + 1 + (h & T.mask_b) : (h & T.mask_s));
     if (atomicCAS(&e->x, EMPTY, raw) == EMPTY) { e->y = __float_as_uint(val); return; }
     if (atomicCAS(&e->z, EMPTY, raw) == EMPTY) { e->w = __float_as_uint(val); return; }
-    T.ovf[atomicAdd(T.n_ovf, 1u)] = make_uint2(key, __float_as_uint(val));
+    const bool back = KWD && required;
+    const uint32_t before = atomicAdd(T.n_ovf, back ? 0x10000u : 1u);
+    T.ovf[back ? T.ovf_cap - 1 - (before >> 16) : KWD ? before & 0xFFFFu : before] = make_uint2(key, __float_as_uint(val));
 }
 
-template <bool NARROW>
+// Required keywords: BM25 query terms whose id arrives with bit 31 set (query.cu:1828-1843).
+template <bool NARROW, bool KWD>
 __device__ __forceinline__ void query_tabs_fill(const QueryTabs& T, const SetView& Q, uint32_t q, float w_s, float w_b, bool use_s, bool use_b,
                                                 int tid, int nthreads) {
     if (use_s)
-        for (uint32_t j = Q.s_off[q] + tid; j < Q.s_off[q + 1]; j += nthreads) query_tabs_insert<NARROW>(T, Q.s_idx[j], Q.s_val[j] * w_s);
+        for (uint32_t j = Q.s_off[q] + tid; j < Q.s_off[q + 1]; j += nthreads) query_tabs_insert<NARROW, KWD>(T, Q.s_idx[j], Q.s_val[j] * w_s, false);
     if (use_b)
         for (uint32_t j = Q.b_off[q] + tid; j < Q.b_off[q + 1]; j += nthreads)
-            query_tabs_insert<NARROW>(T, Q.b_idx[j] | BM25_BIT, Q.b_val[j] * w_b);
+            query_tabs_insert<NARROW, KWD>(T, Q.b_idx[j] | BM25_BIT, Q.b_val[j] * w_b, Q.b_idx[j] & BM25_BIT);
 }
 
 // The pairs of one candidate row on their way to a probe: three chunks of 64, raw keys and value
@@ -444,29 +462,26 @@ __device__ __forceinline__ void row_issue(RowLoad& r, RowInfo& s, const CorpusVi
 }
 
 template <bool NARROW, bool KWD>
-__device__ __forceinline__ void query_match(const uint4 e, uint32_t raw, uint32_t val_bits, bool valid, bool bm25, float& acc, const uint32_t* kwset,
-                                            uint32_t kwmask, bool& hit) {
-    const bool m0 = e.x == raw, m1 = e.z == raw;
+__device__ __forceinline__ void query_match(const uint4 e, uint32_t raw, uint32_t val_bits, bool valid, bool bm25, float& acc, bool& hit) {
+    constexpr uint32_t cmp = KWD ? ~BM25_BIT : ~0u; // the bits of a key that name its term
+    const bool m0 = ((e.x ^ raw) & cmp) == 0, m1 = ((e.z ^ raw) & cmp) == 0;
     const float v = __uint_as_float(m0 ? e.y : e.w);
     const bool found = valid && (m0 || m1);
     const float next = fmaf(__uint_as_float(val_bits), v, acc);
     acc = found ? next : acc;
-    if (KWD) {
-        if (found && bm25 && id_set_contains(kwset, kwmask, raw | BM25_BIT)) hit = true;
-    }
+    if (KWD) hit |= valid && bm25 && ((m0 && (int)e.x < 0) || (m1 && (int)e.z < 0));
 }
 
 template <bool NARROW, bool KWD>
-__device__ __forceinline__ void query_overflow(const QueryTabs& T, uint32_t n_ovf, uint32_t raw, uint32_t val_bits, bool valid, bool bm25, float& acc,
-                                               const uint32_t* kwset, uint32_t kwmask, bool& hit) {
+__device__ __forceinline__ void query_overflow(const QueryTabs& T, uint32_t n_ovf, uint32_t raw, uint32_t val_bits, bool valid, bool bm25, float& acc, bool& hit) {
     const uint32_t key = NARROW ? raw | (bm25 ? BM25_BIT : 0u) : raw;
-    for (uint32_t i = 0; i < n_ovf; i++) {
-        const uint2 o = T.ovf[i];
+    const uint32_t front = KWD ? n_ovf & 0xFFFFu : n_ovf, all = KWD ? front + (n_ovf >> 16) : n_ovf; // LDS holds a few thousand entries: both counts fit 16 bits
+    for (uint32_t i = 0; i < all; i++) {
+        const bool required = KWD && i >= front;
+        const uint2 o = T.ovf[required ? T.ovf_cap - 1 - (i - front) : i];
         if (valid && o.x == key) {
             acc = fmaf(__uint_as_float(val_bits), __uint_as_float(o.y), acc);
-            if (KWD) {
-                if (bm25 && id_set_contains(kwset, kwmask, key)) hit = true;
-            }
+            if (KWD) hit |= required;
         }
     }
 }
@@ -476,7 +491,7 @@ __device__ __forceinline__ void query_overflow(const QueryTabs& T, uint32_t n_ov
 // n_ovf is the (wave-uniform) overflow count read after the tables were built.
 template <bool NARROW, bool KWD>
 __device__ __forceinline__ float row_probe(const CorpusView& C, const RowLoad& r, const RowInfo& s, const QueryTabs& T, uint32_t n_ovf,
-                                           const uint32_t* kwset, uint32_t kwmask, bool& hit) {
+                                           bool& hit) {
     const int lane = lane_id();
     float acc = 0.f;
     bool in[3], bm[3];
@@ -492,10 +507,10 @@ __device__ __forceinline__ float row_probe(const CorpusView& C, const RowLoad& r
     // keep the three reads together: nothing below may be scheduled between them
     asm volatile("" : "+v"(e[0].x), "+v"(e[1].x), "+v"(e[2].x));
 #pragma unroll
-    for (int c = 0; c < 3; c++) query_match<NARROW, KWD>(e[c], r.k[c], r.v[c], in[c], bm[c], acc, kwset, kwmask, hit);
+    for (int c = 0; c < 3; c++) query_match<NARROW, KWD>(e[c], r.k[c], r.v[c], in[c], bm[c], acc, hit);
     if (n_ovf) {
 #pragma unroll
-        for (int c = 0; c < 3; c++) query_overflow<NARROW, KWD>(T, n_ovf, r.k[c], r.v[c], in[c], bm[c], acc, kwset, kwmask, hit);
+        for (int c = 0; c < 3; c++) query_overflow<NARROW, KWD>(T, n_ovf, r.k[c], r.v[c], in[c], bm[c], acc, hit);
     }
     if (s.n > 3 * WAVE) { // rows with more than 192 pairs
         Pairs sp = record_pairs(C, s.rec, s.ns, s.nb);
@@ -503,9 +518,8 @@ __device__ __forceinline__ float row_probe(const CorpusView& C, const RowLoad& r
         for (uint32_t j = s.begin + 3 * WAVE + lane; j < s.begin + s.n; j += WAVE) {
             const uint2 kv = sp.raw(j);
             const bool b = NARROW ? j >= s.ns : (int)kv.x < 0;
-            query_match<NARROW, KWD>((b ? tab_b : tab_s)[query_hash<NARROW>(kv.x) & (b ? T.mask_b : T.mask_s)], kv.x, kv.y, true, b, acc, kwset, kwmask,
-                                     hit);
-            query_overflow<NARROW, KWD>(T, n_ovf, kv.x, kv.y, true, b, acc, kwset, kwmask, hit);
+            query_match<NARROW, KWD>((b ? tab_b : tab_s)[query_hash<NARROW>(kv.x) & (b ? T.mask_b : T.mask_s)], kv.x, kv.y, true, b, acc, hit);
+            query_overflow<NARROW, KWD>(T, n_ovf, kv.x, kv.y, true, b, acc, hit);
         }
     }
     return acc;

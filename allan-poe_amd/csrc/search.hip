@@ -2,6 +2,7 @@
 // query's dense row, its sparse-term tables and the fresh-neighbour list in LDS; an exact
 // visited bitmap per workgroup in HBM.
 #include <mutex>
+#include <type_traits>
 
 #include "apoe_internal.h"
 
@@ -50,14 +51,13 @@ struct SearchArgs {
     const uint32_t *e2e_off, *e2e_idx, *e2d_off, *e2d_idx;
     uint32_t n_entities;
     float kg_weight;
-    uint32_t kw_slots; // keyword-filter kernels only: slots of the per-query keyword term set
 };
 
 // LDS carve-up shared by host (size) and device (pointers).
 struct SearchLds {
-    uint32_t qd, stat, part, tab, ovf, pool_id, pool_dist, pool_ent, pool_hop, new_lb, new_id, new_dist, new_ent, new_hop, seed_id, seed_ent, seed_dist, link, ring_id,
-        ring_dist, kwset, ctl, total;
-    __host__ __device__ SearchLds(uint32_t slots_s, uint32_t slots_b, uint32_t ovf_cap, uint32_t cands, int mode, uint32_t kw_slots) {
+    uint32_t qd, stat, part, tab, ovf, pool_id, pool_dist, pool_ent, pool_hop, new_desc, new_dn, new_id, new_dist, new_ent, new_hop, seed_id, seed_ent, seed_dist, link, ring_id,
+        ring_dist, ctl, total;
+    __host__ __device__ SearchLds(uint32_t slots_s, uint32_t slots_b, uint32_t ovf_cap, uint32_t cands, int mode) {
         const bool kg = mode == MODE_KG, kwd = mode == MODE_KEYWORD;
         // fixed-size arrays first: their offsets are compile-time constants
         uint32_t o = 0;
@@ -65,7 +65,8 @@ struct SearchLds {
         ctl = o; o += 16 * 4;
         stat = o; o += 8 * 8;           // the workgroup's counters (work[1..7]), sent once when it leaves
         part = o; o += MAX_NEW * 16;    // sparse sum of a fresh candidate as four partial sums (one per 16 lanes)
-        new_lb = o; o += MAX_NEW * 4;
+        new_desc = o; o += MAX_NEW * 8; // descriptors and dense norms of the fresh candidates
+        new_dn = o; o += MAX_NEW * 4;
         new_id = o; o += MAX_NEW * 4;
         new_dist = o; o += MAX_NEW * 4;
         new_ent = o; o += kg || kwd ? MAX_NEW * 4 : 0; // KG: linking entity; keyword search: the hit flag of a fresh candidate
@@ -83,7 +84,6 @@ struct SearchLds {
         seed_id = o; o += kg ? (cands + MAX_NEW) * 4 : 0;
         seed_ent = o; o += kg ? (cands + MAX_NEW) * 4 : 0;
         seed_dist = o; o += kg ? (cands + MAX_NEW) * 4 : 0;
-        kwset = o; o += kwd ? kw_slots * 4 : 0;
         total = o;
     }
 };
@@ -95,7 +95,6 @@ struct Pool {
     float* dist;    // [cands]
     uint32_t* ent;  // KG only
     uint32_t* hop;  // KG only
-    uint32_t* lb;   // [MAX_NEW] scratch of the merge
     uint32_t cands;
 };
 
@@ -114,129 +113,188 @@ __device__ __forceinline__ void wave_fence() {
     __builtin_amdgcn_wave_barrier();
 }
 
-// Wave 0 only. Orders the n (<= 64) new candidates by (distance, id) and merges them into the
-// sorted pool in place: a pool element keeps rank pos + #{new <= it}, a new element takes rank
-// pos + #{pool < it}, so on equal distance the new one goes first (query.cu:181-224); ranks >=
-// cands fall off. With lb_i = #{pool < new_i}: new_i <= pool[p]  <=>  lb_i <= p, so a pool element
-// moves up by the number of new elements whose lb is <= its position, and nothing below lb_0
-// moves at all -- only the 64-element rounds from the top down to lb_0 are touched (each round
-// is read into registers before anything at or above it is written). Returns the lowest rank a
-// new element took (cands if none entered).
-// Keyword-filter search: nent[i] != 0 says that new candidate i holds a required keyword; it
-// enters the pool with KW_HIT set on its id (ordering uses the plain id).
+// Wave 0 only: the new candidates of one expansion, lane l holds the l-th.
+struct Fresh {
+    float d;
+    uint32_t id, ent, hop; // KG: linking entity and hop; keyword-filter search: ent != 0: holds a required keyword
+    uint64_t kept;         // lanes whose candidate can enter the pool: the others (with a full pool that is most of them:
+                           // everything the bound rejected, and more) are dropped
+    uint32_t rank;         // of a kept candidate among the kept ones, by (distance, id); set by fresh_rank
+};
+
 template <int MODE>
-__device__ __forceinline__ uint32_t sort_merge(const Pool& P, uint32_t* nid, float* ndist, uint32_t* nent, uint32_t* nhop, uint32_t n, Ring& R) {
+__device__ __forceinline__ void fresh_load(Fresh& F, const Pool& P, const uint32_t* nid, const float* ndist, const uint32_t* nent, const uint32_t* nhop,
+                                           uint32_t n) {
+    const int lane = lane_id();
+    F.d = INF_DIS;
+    F.id = F.ent = EMPTY;
+    F.hop = F.rank = 0;
+    if (lane < (int)n) {
+        F.d = ndist[lane];
+        F.id = nid[lane];
+        if (MODE == MODE_KG) { F.ent = nent[lane]; F.hop = nhop[lane]; }
+        if (MODE == MODE_KEYWORD) F.ent = nent[lane];
+    }
+    F.kept = __ballot(lane < (int)n && F.d <= P.dist[P.cands - 1]);
+}
+
+// The kept candidate that comes first by (distance, id): its lane. F.kept must not be empty.
+__device__ __forceinline__ uint32_t fresh_first(const Fresh& F) {
+    const bool keep = (F.kept >> lane_id()) & 1;
+    const float low = wave_min_dpp(keep ? F.d : __builtin_inff());
+    uint64_t at = __ballot(keep && F.d == low);
+    uint32_t best = __builtin_ctzll(at);
+    for (at &= at - 1; at; at &= at - 1) { // equal distances: the smallest id
+        const uint32_t i = __builtin_ctzll(at);
+        if ((uint32_t)__builtin_amdgcn_readlane((int)F.id, i) < (uint32_t)__builtin_amdgcn_readlane((int)F.id, best)) best = i;
+    }
+    return best;
+}
+
+__device__ __forceinline__ void fresh_rank(Fresh& F) {
+    for (uint64_t rest = F.kept; rest; rest &= rest - 1) { // ids are distinct
+        const uint32_t i = __builtin_ctzll(rest);
+        const float di = readlane_f32(F.d, i);
+        const uint32_t ii = (uint32_t)__builtin_amdgcn_readlane((int)F.id, i);
+        F.rank += (di < F.d) || (di == F.d && ii < F.id);
+    }
+}
+
+// Wave 0 only: the first unexplored pool entry at or behind `from`.
+struct Front {
+    uint32_t id, slot; // id EMPTY: there is none
+    float dist;
+};
+__device__ __forceinline__ Front pool_front(const Pool& P, uint32_t from) {
+    Front f;
+    f.id = EMPTY;
+    f.slot = P.cands;
+    f.dist = INF_DIS;
+    const uint32_t lane = lane_id();
+    for (uint32_t base = from & ~(uint32_t)(WAVE - 1); base < P.cands; base += WAVE) {
+        const uint32_t p = base + lane;
+        const uint32_t id = p < P.cands && p >= from ? P.id[p] : EMPTY;
+        const float d = p < P.cands ? P.dist[p] : INF_DIS;
+        const uint64_t b = __ballot((id & FLAG) == 0);
+        if (b) {
+            const uint32_t l = __builtin_ctzll(b);
+            f.id = (uint32_t)__builtin_amdgcn_readlane((int)id, l);
+            f.dist = readlane_f32(d, l);
+            f.slot = base + l;
+            break;
+        }
+    }
+    return f;
+}
+
+// Wave 0 only. Merges the kept new candidates (ranked) into the sorted pool in place: a pool element keeps rank
+// pos + #{new <= it}, a new element takes rank #{new before it by (distance, id)} + #{pool < it}, so on equal distance
+// the new one goes first (query.cu:181-224); ranks >= cands fall off. The pool is read in groups of MERGE_ROUNDS x 64
+// entries from its end, coalesced into registers; every new candidate that can enter (wave-uniform loop over the kept
+// lanes) is compared with the whole group at once, which gives the group's shifts (per lane) and the candidate's own
+// count of pool entries at or beyond it (population count of the compare mask). A group only writes at or above its own
+// positions, into rounds that were read before; the first group whose lowest entry does not move is the last.
+// The chain of a merge bounds short batches (one wave works, the others wait): a group costs one LDS round trip plus
+// about twenty instructions per kept candidate. Sorting the new ones through LDS first and finding each rank by a binary
+// search (one dependent LDS read per halving) took 3 900 cycles a merge at cands 128 and 8 600 at cands 1000 (one query
+// per CU); this takes 1 830 and 3 360 (500 queries at cands 1000 on 100 k documents: 10.3 -> 8.0 ms).
+// Returns the lowest rank a new element took (cands if none entered).
+// Keyword-filter search: a candidate that holds a required keyword enters the pool with KW_HIT set on its id (ordering
+// uses the plain id).
+template <int MODE>
+__device__ __forceinline__ uint32_t sort_merge(const Pool& P, const Fresh& F, Ring& R) {
     constexpr bool KG = MODE == MODE_KG, KWD = MODE == MODE_KEYWORD;
     const int lane = lane_id();
     const uint32_t cands = P.cands;
-    if (n == 0) return cands;
-    // a candidate beyond the pool's worst entry cannot enter (with a full pool that is most of them:
-    // everything the bound rejected, and more): only the others are ordered and merged
-    float d = INF_DIS;
-    uint32_t id = EMPTY, ent = EMPTY, hop = 0, rank = 0;
-    if (lane < (int)n) d = ndist[lane];
-    const bool keep = lane < (int)n && d <= P.dist[cands - 1];
-    const uint64_t kept = __ballot(keep);
+    const uint64_t kept = F.kept;
     if (kept == 0) return cands;
-    // order by counting: rank = #{kept (d, id) pairs below mine}; ids are distinct
-    if (keep) {
-        id = nid[lane];
-        if (KG) { ent = nent[lane]; hop = nhop[lane]; }
-        if (KWD) ent = nent[lane];
-    }
-    for (uint64_t rest = kept; rest; rest &= rest - 1) {
-        const uint32_t i = __builtin_ctzll(rest); // wave-uniform
-        const float di = ndist[i];
-        const uint32_t ii = nid[i];
-        rank += (di < d) || (di == d && ii < id);
-    }
-    wave_fence();
-    if (keep) {
-        ndist[rank] = d;
-        nid[rank] = id;
-        if (KG) { nent[rank] = ent; nhop[rank] = hop; }
-        if (KWD) nent[rank] = ent;
-    }
-    n = __popcll(kept);
-    wave_fence();
-    // lane i now takes the i-th smallest
-    uint32_t lb = cands;
-    if (lane < (int)n) {
-        d = ndist[lane];
-        id = nid[lane];
-        if (KG) { ent = nent[lane]; hop = nhop[lane]; }
-        if (KWD) id |= nent[lane] ? KW_HIT : 0u;
-        if (d <= P.dist[cands - 1]) {
-            uint32_t lo = 0, len = cands;
-            while (len > 0) {
-                const uint32_t half = len >> 1;
-                if (P.dist[lo + half] < d) { lo += half + 1; len -= half + 1; } else len = half;
-            }
-            lb = lo;
-        }
-        P.lb[lane] = lb;
-    }
-    const bool enters = lane < (int)n && lb + lane < cands;
-    const uint32_t n_in = __popcll(__ballot(enters)); // ranks grow with the lane: the first n_in enter
-    if (n_in == 0) return cands;
-    wave_fence();
-    if (KWD) {
-        // exactly the last n_in pool entries fall off; lane l looks at the l-th from the end
-        uint32_t eid = EMPTY;
-        float ed = 0.f;
-        if ((uint32_t)lane < n_in) { eid = P.id[cands - 1 - lane]; ed = P.dist[cands - 1 - lane]; }
-        const bool hit = eid != EMPTY && (eid & KW_HIT);
-        const uint64_t hb = __ballot(hit);
-        const uint32_t cnt = __popcll(hb), rank = __popcll(hb & ((1ull << lane) - 1));
-        if (hit && rank + RING >= cnt) {
-            const uint32_t slot = (R.n + rank) % RING;
-            R.id[slot] = eid & ID_MASK;
-            R.dist[slot] = ed;
-        }
-        R.n += cnt;
-        wave_fence();
-    }
-    const uint32_t lo0 = uniform(P.lb[0]);
-    // MERGE_ROUNDS rounds are read before any of them is written: one LDS round trip per group, and a
-    // group only writes at or above its own positions (into rounds that were moved before it)
-    for (int top = (int)((cands - 1) & ~(uint32_t)(WAVE - 1)); top >= 0 && (uint32_t)top + WAVE > lo0; top -= WAVE * MERGE_ROUNDS) {
+    const bool keep = (kept >> lane) & 1;
+    const float d = F.d;
+    uint32_t beyond = 0;   // pool entries at or beyond this lane's candidate
+    uint64_t open = kept;  // candidates whose place is not found yet
+    for (int top = (int)((cands - 1) & ~(uint32_t)(WAVE - 1));; top -= WAVE * MERGE_ROUNDS) {
         float v[MERGE_ROUNDS];
-        uint32_t pid[MERGE_ROUNDS], pent[MERGE_ROUNDS], phop[MERGE_ROUNDS], dst[MERGE_ROUNDS];
+        uint32_t pid[MERGE_ROUNDS], pent[MERGE_ROUNDS], phop[MERGE_ROUNDS], shift[MERGE_ROUNDS];
 #pragma unroll
         for (int r = 0; r < MERGE_ROUNDS; r++) {
             const int base = top - r * WAVE;
             const uint32_t p = (uint32_t)(base + lane);
-            const bool act = base >= 0 && (uint32_t)base + WAVE > lo0 && p >= lo0 && p < cands;
-            dst[r] = cands; // nothing to write
-            v[r] = 0.f;
-            pid[r] = pent[r] = phop[r] = 0;
-            if (act) {
+            v[r] = __builtin_nanf(""); // not there: compares false with everything
+            pid[r] = pent[r] = phop[r] = shift[r] = 0;
+            if (base >= 0 && p < cands) {
                 v[r] = P.dist[p];
                 pid[r] = P.id[p];
                 if (KG) { pent[r] = P.ent[p]; phop[r] = P.hop[p]; }
-                uint32_t shift = 0;
-                for (uint32_t i = 0; i < n_in; i++) shift += (uint32_t)__builtin_amdgcn_readlane((int)lb, i) <= p;
-                dst[r] = p + shift;
             }
+        }
+        auto place = [&](uint32_t i) { // candidate i against every entry of the group
+            const float di = readlane_f32(d, i);
+            uint32_t cnt = 0;
+#pragma unroll
+            for (int r = 0; r < MERGE_ROUNDS; r++) {
+                const bool at_or_beyond = v[r] >= di;
+                cnt += (uint32_t)__popcll(__ballot(at_or_beyond));
+                shift[r] += at_or_beyond ? 1u : 0u;
+            }
+            beyond += (uint32_t)lane == i ? cnt : 0u;
+        };
+        const int next = top - WAVE * MERGE_ROUNDS;
+        uint32_t all = 0; // candidates that go before the whole group
+        if (next >= 0) {
+            const uint64_t before = __ballot(((open >> lane) & 1) && readlane_f32(v[MERGE_ROUNDS - 1], 0) >= d);
+            beyond += (before >> lane) & 1 ? min(cands - (uint32_t)(next + WAVE), (uint32_t)(WAVE * MERGE_ROUNDS)) : 0u;
+            all = (uint32_t)__popcll(before);
+#pragma unroll
+            for (int r = 0; r < MERGE_ROUNDS; r++) shift[r] = all;
+            open &= ~before;
+            for (uint64_t rest = open; rest; rest &= rest - 1) place(__builtin_ctzll(rest));
+            open = before;
+        } else {
+            for (uint64_t rest = open; rest; rest &= rest - 1) place(__builtin_ctzll(rest));
+        }
+        if (KWD && top + WAVE >= (int)cands) {
+            // the pool entries that fall off all sit in the last 64 positions; lane l looks at the l-th from the end
+            uint32_t n_off = 0;
+#pragma unroll
+            for (int r = 0; r < 2; r++) {
+                const uint32_t p = (uint32_t)(top - r * WAVE + lane);
+                n_off += (uint32_t)__popcll(__ballot(shift[r] > 0 && p < cands && p + shift[r] >= cands));
+            }
+            uint32_t eid = EMPTY;
+            float ed = 0.f;
+            if ((uint32_t)lane < n_off) { eid = P.id[cands - 1 - lane]; ed = P.dist[cands - 1 - lane]; }
+            const bool hit = eid != EMPTY && (eid & KW_HIT);
+            const uint64_t hb = __ballot(hit);
+            const uint32_t cnt = __popcll(hb), nth = __popcll(hb & ((1ull << lane) - 1));
+            if (hit && nth + RING >= cnt) {
+                const uint32_t slot = (R.n + nth) % RING;
+                R.id[slot] = eid & ID_MASK;
+                R.dist[slot] = ed;
+            }
+            R.n += cnt;
         }
         wave_fence();
 #pragma unroll
         for (int r = 0; r < MERGE_ROUNDS; r++) {
-            if (dst[r] < cands) {
-                P.dist[dst[r]] = v[r];
-                P.id[dst[r]] = pid[r];
-                if (KG) { P.ent[dst[r]] = pent[r]; P.hop[dst[r]] = phop[r]; }
+            const uint32_t dst = (uint32_t)(top - r * WAVE + lane) + shift[r];
+            if (shift[r] > 0 && dst < cands) {
+                P.dist[dst] = v[r];
+                P.id[dst] = pid[r];
+                if (KG) { P.ent[dst] = pent[r]; P.hop[dst] = phop[r]; }
             }
         }
         wave_fence();
+        if (next < 0 || all == 0) break; // none goes before the group: nothing below it moves
     }
-    if (enters) {
-        P.dist[lb + lane] = d;
-        P.id[lb + lane] = id;
-        if (KG) { P.ent[lb + lane] = ent; P.hop[lb + lane] = hop; }
+    const uint32_t lb = cands - beyond; // #{pool < mine}
+    const uint32_t at = lb + F.rank;
+    if (keep && at < cands) {
+        P.dist[at] = d;
+        P.id[at] = KWD && F.ent ? F.id | KW_HIT : F.id;
+        if (KG) { P.ent[at] = F.ent; P.hop[at] = F.hop; }
     }
     wave_fence();
-    return lo0;
+    return (uint32_t)__builtin_amdgcn_readlane((int)lb, __builtin_ctzll(__ballot(keep && F.rank == 0)));
 }
 
 template <int NW, int MODE, bool NARROW, bool HALF>
@@ -244,13 +302,14 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
     constexpr bool KG = MODE == MODE_KG, KWD = MODE == MODE_KEYWORD;
     a.C.narrow = NARROW ? 1u : 0u; // the pair format as a compile-time constant: no branch at the loads
     extern __shared__ __align__(16) char smem[];
-    const SearchLds L(a.slots_s, a.slots_b, a.ovf_cap, a.cands, MODE, a.kw_slots);
+    const SearchLds L(a.slots_s, a.slots_b, a.ovf_cap, a.cands, MODE);
     volatile uint32_t* ctl = reinterpret_cast<volatile uint32_t*>(smem + L.ctl);
     float4* qd = reinterpret_cast<float4*>(smem + L.qd);
     float* part = reinterpret_cast<float*>(smem + L.part);
     QueryTabs T;
     T.b = reinterpret_cast<uint4*>(smem + L.tab);
     T.ovf = reinterpret_cast<uint2*>(smem + L.ovf);
+    T.ovf_cap = a.ovf_cap;
     T.n_ovf = const_cast<uint32_t*>(&ctl[CTL_NOVF]);
     T.mask_s = a.slots_s - 1;
     T.mask_b = a.slots_b - 1;
@@ -259,8 +318,9 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
     P.dist = reinterpret_cast<float*>(smem + L.pool_dist);
     P.ent = reinterpret_cast<uint32_t*>(smem + L.pool_ent);
     P.hop = reinterpret_cast<uint32_t*>(smem + L.pool_hop);
-    P.lb = reinterpret_cast<uint32_t*>(smem + L.new_lb);
     P.cands = a.cands;
+    uint64_t* new_desc = reinterpret_cast<uint64_t*>(smem + L.new_desc);
+    float* new_dn = reinterpret_cast<float*>(smem + L.new_dn);
     uint32_t* new_id = reinterpret_cast<uint32_t*>(smem + L.new_id);
     float* new_dist = reinterpret_cast<float*>(smem + L.new_dist);
     uint32_t* new_ent = reinterpret_cast<uint32_t*>(smem + L.new_ent);
@@ -269,7 +329,6 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
     uint32_t* seed_ent = reinterpret_cast<uint32_t*>(smem + L.seed_ent);
     float* seed_dist = reinterpret_cast<float*>(smem + L.seed_dist);
     uint32_t* link = reinterpret_cast<uint32_t*>(smem + L.link);
-    uint32_t* kwset = reinterpret_cast<uint32_t*>(smem + L.kwset);
     Ring R;
     R.id = reinterpret_cast<uint32_t*>(smem + L.ring_id);
     R.dist = reinterpret_cast<float*>(smem + L.ring_dist);
@@ -296,10 +355,7 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
             for (uint32_t i = tid; i < a.bitmap_words / 4; i += NW * WAVE) b4[i] = make_uint4(0, 0, 0, 0);
         }
         query_tabs_clear(T, tid, NW * WAVE);
-        if (KWD) {
-            for (uint32_t i = tid; i < a.kw_slots; i += NW * WAVE) kwset[i] = EMPTY;
-            R.n = 0;
-        }
+        R.n = 0;
         for (uint32_t i = tid; i < cands; i += NW * WAVE) {
             P.id[i] = EMPTY;
             P.dist[i] = INF_DIS;
@@ -314,20 +370,15 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
         }
         __threadfence();
         __syncthreads();
-        query_tabs_fill<NARROW>(T, a.cold->Q, q, a.cold->w_s, a.cold->w_b, a.paths & PATH_SPARSE, a.paths & PATH_BM25, tid, NW * WAVE);
-        if (KWD) {
-            // required keywords: BM25 query terms whose id arrives with bit 31 set (query.cu:1828-1843)
-            for (uint32_t j = a.cold->Q.b_off[q] + tid; j < a.cold->Q.b_off[q + 1]; j += NW * WAVE) {
-                const uint32_t t = a.cold->Q.b_idx[j];
-                if (t & BM25_BIT) id_set_insert(kwset, a.kw_slots - 1, t);
-            }
-        }
-
+        query_tabs_fill<NARROW, KWD>(T, a.cold->Q, q, a.cold->w_s, a.cold->w_b, a.paths & PATH_SPARSE, a.paths & PATH_BM25, tid, NW * WAVE);
         __syncthreads();
         const float pv_norm = pivot_dense_norm_lds(qd);
         uint64_t st_exp = 0, st_eval = 0, st_dense = 0, st_again = 0, st_again_pairs = 0; // wave-uniform counters
         uint32_t ln_s = 0, ln_b = 0;                    // pairs read for the candidates this lane decided
-        uint32_t hint = 0;                                       // wave 0: every pool slot below hint is explored
+        Front front; // wave 0: the first unexplored pool entry
+        front.id = EMPTY;
+        front.slot = 0;
+        front.dist = INF_DIS;
 
         // ---- seeds ----
         if (!KG) {
@@ -340,7 +391,12 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
                     fresh = !(atomicOr(&bitmap[c >> 5], bit) & bit);
                 }
                 const uint64_t b = __ballot(fresh);
-                if (fresh) new_id[__popcll(b & lane_lt)] = c;
+                if (fresh) {
+                    const uint32_t pos = __popcll(b & lane_lt);
+                    new_id[pos] = c;
+                    new_desc[pos] = a.C.desc[c];
+                    new_dn[pos] = a.C.dnorm[c];
+                }
                 if (lane == 0) { ctl[CTL_NNEW] = __popcll(b); ctl[CTL_PARENT] = 0; }
             }
             __syncthreads();
@@ -392,7 +448,7 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
                 RowInfo ri;
                 row_issue<NARROW>(rl, ri, a.C, a.C.desc[id], true, a.paths);
                 bool hit = false;
-                const float acc = row_probe<NARROW, false>(a.C, rl, ri, T, n_ovf_seed, nullptr, 0, hit);
+                const float acc = row_probe<NARROW, false>(a.C, rl, ri, T, n_ovf_seed, hit);
                 const float ssum = (a.paths & (PATH_SPARSE | PATH_BM25)) ? wave_sum_dpp(acc) : 0.f;
                 float dist = 1.0f - ssum - bonus;
                 if (a.paths & PATH_DENSE) { // seeds are never dropped by the bound
@@ -419,13 +475,25 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
                         new_hop[lane] = 0;
                     }
                     wave_fence();
-                    sort_merge<MODE>(P, new_id, new_dist, new_ent, new_hop, nb, R);
+                    Fresh F;
+                    fresh_load<MODE>(F, P, new_id, new_dist, new_ent, new_hop, nb);
+                    fresh_rank(F);
+                    sort_merge<MODE>(P, F, R);
                 }
+                front = pool_front(P, 0);
                 if (lane == 0) { ctl[CTL_NNEW] = 0; ctl[CTL_PARENT] = 0; }
             }
             __syncthreads();
         }
 
+        // The next parent is the first unexplored pool entry or a new candidate that goes before it, so it is known BEFORE
+        // the merge: wave 0 starts the parent's three dependent reads (graph row, visited words, descriptors) first and
+        // merges while they are under way; the row of the first unexplored entry is requested while the candidates are
+        // evaluated. At one query per compute unit the three reads were
+        // 2 000 cycles of an iteration after the merge; of them 150 to 280 are left behind it. (Looking one whole expansion ahead,
+        // with the visited marks taken back when a candidate overtakes: it is right for 0.55 to 0.64 of the expansions only, and
+        // the marks and rows of the others cost long batches 5 %.)
+        uint32_t g_c = EMPTY, g_kw = 0; // lane l: neighbour of `front`, later of the parent; (keyword search) word l of the row's tail
         for (uint32_t it = 0; it <= a.max_iter; it++) {
             // ---- evaluate the fresh candidates: one wave per candidate ----
             const uint32_t n_new = uniform(ctl[CTL_NNEW]);
@@ -435,34 +503,39 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
             const float thr = a.full_eval ? __builtin_inff() : P.dist[cands - 1];
             const float thr_eff = thr < INF_DIS ? thr : __builtin_inff();
             const uint32_t n_ovf = uniform(ctl[CTL_NOVF]);
-            // descriptors and dense norms of all fresh candidates in one gather: lane l holds candidate l's
+            // descriptors and dense norms of all fresh candidates: lane l holds candidate l's
             uint64_t my_desc = 0;
             float my_dn = 0.f;
             if ((uint32_t)lane < n_new) {
-                const uint32_t cid = new_id[lane];
-                my_desc = a.C.desc[cid];
-                my_dn = a.C.dnorm[cid];
+                my_desc = new_desc[lane];
+                my_dn = new_dn[lane];
+            }
+            if (wave == 0 && front.id != EMPTY) {
+                const uint32_t* row = a.graph + (size_t)(KWD ? front.id & ID_MASK : front.id) * a.W;
+                g_c = lane < (int)a.degree ? row[lane] : EMPTY;
+                if (KWD) g_kw = lane < APOE_KW_SLOTS ? row[a.degree + lane] : 0u;
             }
             // stage 1: the sparse parts of this wave's candidates (wave + k * NW), EVAL_BATCH of them in flight.
             // No branch on whether a candidate of the batch exists: one that does not is a row of no pairs,
             // so the loads of the whole batch are issued back to back.
-            for (uint32_t j = wave; j < n_new; j += NW * EVAL_BATCH) {
-                RowLoad rl[EVAL_BATCH];
-                RowInfo ri[EVAL_BATCH];
+            auto eval_rows = [&](auto nb, uint32_t j) {
+                constexpr int NB = decltype(nb)::value;
+                RowLoad rl[NB];
+                RowInfo ri[NB];
 #pragma unroll
-                for (int b = 0; b < EVAL_BATCH; b++) {
+                for (int b = 0; b < NB; b++) {
                     const uint32_t jj = j + b * NW;
                     row_issue<NARROW>(rl[b], ri[b], a.C, readlane64(my_desc, jj & (WAVE - 1)), jj < n_new, a.paths);
                 }
-                float acc[EVAL_BATCH];
-                bool hit[EVAL_BATCH];
+                float acc[NB];
+                bool hit[NB];
 #pragma unroll
-                for (int b = 0; b < EVAL_BATCH; b++) {
+                for (int b = 0; b < NB; b++) {
                     hit[b] = false;
-                    acc[b] = row_probe<NARROW, KWD>(a.C, rl[b], ri[b], T, n_ovf, kwset, a.kw_slots - 1, hit[b]);
+                    acc[b] = row_probe<NARROW, KWD>(a.C, rl[b], ri[b], T, n_ovf, hit[b]);
                 }
 #pragma unroll
-                for (int b = 0; b < EVAL_BATCH; b++) {
+                for (int b = 0; b < NB; b++) {
                     const uint32_t jj = j + b * NW;
                     const float rs = row_sum_dpp(acc[b]);
                     if (jj < n_new) {
@@ -473,6 +546,15 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
                         }
                     }
                 }
+            };
+            if (NW >= 8) { // one or two rows a wave at most expansions: a row that is not there would cost issue slots of a SIMD that four to six waves share
+                for (uint32_t j = wave; j < n_new; j += NW * EVAL_BATCH) {
+                    if (j + 2 * NW < n_new) eval_rows(std::integral_constant<int, 3>{}, j);
+                    else if (j + NW < n_new) eval_rows(std::integral_constant<int, 2>{}, j);
+                    else eval_rows(std::integral_constant<int, 1>{}, j);
+                }
+            } else {
+                for (uint32_t j = wave; j < n_new; j += NW * EVAL_BATCH) eval_rows(std::integral_constant<int, EVAL_BATCH>{}, j);
             }
             wave_fence();
             // the decision for all of the wave's candidates at once, lane l for candidate l: a candidate whose
@@ -562,33 +644,46 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
             __syncthreads();
             // ---- wave 0: merge, pick the next parent, fetch its neighbours ----
             if (wave == 0) {
-                hint = min(hint, sort_merge<MODE>(P, new_id, new_dist, new_ent, new_hop, n_new, R));
-                uint32_t parent = EMPTY, slot = 0, n_next = 0;
+                Fresh F;
+                fresh_load<MODE>(F, P, new_id, new_dist, new_ent, new_hop, n_new);
+                uint32_t parent = EMPTY, n_next = 0;
+                bool overtaken = false; // the parent is a new candidate (on equal distance the new one goes first)
                 if (it < a.max_iter) {
-                    for (uint32_t base = hint & ~(uint32_t)(WAVE - 1); base < cands; base += WAVE) {
-                        const uint32_t id = base + lane < cands ? P.id[base + lane] : EMPTY;
-                        const uint64_t b = __ballot((id & FLAG) == 0);
-                        if (b) {
-                            const int l = __ffsll((unsigned long long)b) - 1;
-                            slot = base + l;
-                            parent = __shfl(id, l, WAVE);
-                            break;
+                    parent = front.id;
+                    if (F.kept) {
+                        const uint32_t l = fresh_first(F);
+                        if (parent == EMPTY || readlane_f32(F.d, l) <= front.dist) {
+                            overtaken = true;
+                            parent = (uint32_t)__builtin_amdgcn_readlane((int)F.id, l);
                         }
                     }
-                    hint = parent != EMPTY ? slot + 1 : cands;
+                    if (KWD && parent != EMPTY) parent &= ID_MASK;
                 }
+                if (parent != EMPTY && overtaken) {
+                    const uint32_t* row = a.graph + (size_t)parent * a.W;
+                    g_c = lane < (int)a.degree ? row[lane] : EMPTY;
+                    if (KWD) g_kw = lane < APOE_KW_SLOTS ? row[a.degree + lane] : 0u;
+                }
+                fresh_rank(F);
+                bool fresh = false;
+                uint64_t g_desc = 0;
+                float g_dn = 0.f;
+                if (parent != EMPTY && g_c < a.C.n) {
+                    const uint32_t bit = 1u << (g_c & 31);
+                    fresh = !(atomicOr(&bitmap[g_c >> 5], bit) & bit);
+                    g_desc = a.C.desc[g_c];
+                    g_dn = a.C.dnorm[g_c];
+                }
+                const uint32_t lowest = sort_merge<MODE>(P, F, R);
                 if (parent != EMPTY) {
+                    const uint32_t slot = overtaken ? lowest : front.slot; // nothing new goes before an entry that was not overtaken
                     uint32_t p_ent = EMPTY, p_hop = 0;
                     if (KG) { p_ent = P.ent[slot]; p_hop = P.hop[slot]; }
-                    if (lane == 0) P.id[slot] = parent | FLAG;
-                    if (KWD) parent &= ID_MASK;
+                    if (lane == 0) P.id[slot] |= FLAG;
+                    wave_fence();
+                    front = pool_front(P, slot + 1);
                     st_exp++;
-                    uint32_t c = lane < (int)a.degree ? a.graph[(size_t)parent * a.W + lane] : EMPTY;
-                    bool fresh = false;
-                    if (c < a.C.n) {
-                        const uint32_t bit = 1u << (c & 31);
-                        fresh = !(atomicOr(&bitmap[c >> 5], bit) & bit);
-                    }
+                    uint32_t c = g_c;
                     bool alive = fresh;
                     uint32_t ent = EMPTY;
                     if (KWD) {
@@ -597,9 +692,9 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
                         // (query.cu:1397-1409; which slot gets which edge does not matter)
                         const bool dup = lane < (int)a.degree && !fresh;
                         const uint32_t t = __popcll(__ballot(dup) & lane_lt);
-                        const uint32_t n_kw = min(uniform(a.graph[(size_t)parent * a.W + a.degree]), (uint32_t)APOE_KW_SLOTS - 1u);
+                        const uint32_t n_kw = min(uniform(g_kw), (uint32_t)APOE_KW_SLOTS - 1u);
+                        const uint32_t c2 = __shfl(g_kw, (int)min(t + 1u, (uint32_t)APOE_KW_SLOTS - 1u), WAVE);
                         if (dup && t < n_kw) {
-                            const uint32_t c2 = a.graph[(size_t)parent * a.W + a.degree + 1 + t];
                             if (c2 < a.C.n) {
                                 const uint32_t bit = 1u << (c2 & 31);
                                 if (!(atomicOr(&bitmap[c2 >> 5], bit) & bit)) { c = c2; alive = true; }
@@ -683,6 +778,12 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
                     if (alive) {
                         const uint32_t pos = __popcll(b & lane_lt);
                         new_id[pos] = c;
+                        if ((KG || KWD) && !fresh) { // not a graph neighbour: recycled through a keyword or logical edge
+                            g_desc = a.C.desc[c];
+                            g_dn = a.C.dnorm[c];
+                        }
+                        new_desc[pos] = g_desc;
+                        new_dn[pos] = g_dn;
                         if (KG) { new_ent[pos] = ent; new_hop[pos] = p_hop + 1; }
                     }
                     n_next = __popcll(b);
@@ -702,7 +803,7 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
                 RowInfo ri;
                 row_issue<NARROW>(rl, ri, a.C, a.C.desc[id], true, a.paths);
                 bool hit = false;
-                const float acc = row_probe<NARROW, false>(a.C, rl, ri, T, n_ovf, nullptr, 0, hit);
+                const float acc = row_probe<NARROW, false>(a.C, rl, ri, T, n_ovf, hit);
                 const float ssum = (a.paths & (PATH_SPARSE | PATH_BM25)) ? wave_sum_dpp(acc) : 0.f;
                 // the same expressions as in the walk, so an entry gets the bits the default search gives it
                 float dist = 1.0f - ssum - 0.f;
@@ -920,7 +1021,6 @@ int launch_search(apoe_ctx* ctx, const apoe_corpus* c, const apoe_queries* q, co
     if (use_kw) {
         APOE_REQUIRE(c->n < (1u << 30), "keyword-filter search keeps two flag bits on a document id: %u documents are too many", c->n);
         a.paths = PATH_DENSE | PATH_SPARSE | PATH_BM25; // query.cu:2005-2007: always the three-path loop
-        a.kw_slots = next_pow2(std::max(64u, 2 * q->max_keywords));
     }
     if (use_kg) {
         APOE_REQUIRE(kg->n_queries >= p->q_begin + q_count, "knowledge graph holds entities for %u queries, %u needed", kg->n_queries, p->q_begin + q_count);
@@ -932,7 +1032,7 @@ int launch_search(apoe_ctx* ctx, const apoe_corpus* c, const apoe_queries* q, co
         cold.q2e_idx = kg->q2e_idx.p;
         a.n_entities = kg->n_entities;
     }
-    const SearchLds L(a.slots_s, a.slots_b, a.ovf_cap, a.cands, mode, a.kw_slots);
+    const SearchLds L(a.slots_s, a.slots_b, a.ovf_cap, a.cands, mode);
     APOE_REQUIRE(L.total <= 64 * 1024, "search needs %u bytes of LDS (query rows with up to %u sparse terms)", L.total, q->max_nnz);
 
     a.bitmap_words = ((c->n + 31) / 32 + 3) & ~3u;

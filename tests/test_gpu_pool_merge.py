@@ -1,0 +1,64 @@
+"""The pool merge (groups of 4 x 64 entries read from the pool's end) at pool sizes around its group and round edges, and
+keyword flags that travel in the keys of the query's term table, overflow entries included."""
+import numpy as np
+import pytest
+
+from keyword_worlds import EMPTY_ID, KW
+from parity import assert_dist_close, assert_topk_match
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("variant", [1, 4, 5])
+@pytest.mark.parametrize("cands", [2, 63, 64, 65, 255, 256, 257, 320, 513])
+def test_pool_sizes_around_the_merge_groups(gpu_world, cands, variant):
+    """Whole pools, not only their heads: an entry that a merge loses or doubles shows up behind the top ten."""
+    import apoe
+    import oracle as O
+    w = gpu_world
+    nq = 24
+    ids, dist, _ = apoe.search(w["ctx"], w["gc"], w["gq"], w["gg"], (1, 1, 1), cands, q_count=nq, variant=variant)
+    oid, odist, _ = O.search(w["C"], w["Q"].head(nq), w["rows"], w["entry"], (1, 1, 1), cands)
+    assert_topk_match(ids, dist, oid, odist, cands, f"cands {cands}")
+    assert_dist_close(dist, odist, f"cands {cands}: pool distances") # an order that differs at a tie keeps the sorted distances
+    for row in ids:
+        real = row[row != EMPTY_ID]
+        assert len(set(real.tolist())) == len(real)
+
+
+def colliding_terms(count, buckets):
+    """Term ids below 65 536 whose table bucket is the same: ((term * 0x9E3779) mod 2^32 >> 10) mod buckets."""
+    t = np.arange(1, 65536, dtype=np.uint64)
+    h = ((t * 0x9E3779) & 0xFFFFFFFF) >> 10
+    return t[h % buckets == 5][:count].astype(np.uint32)
+
+
+@pytest.mark.parametrize("n_flagged", [0, 1, 3, 6, 12])
+@pytest.mark.parametrize("wide", [False, True])
+def test_flags_of_overflow_entries(gpu_ctx, wide, n_flagged):
+    """Twelve query terms in one bucket of two entries: ten go to the overflow list, required ones from its end. Every document
+    holds one of the terms, so the hits are exactly the documents of the flagged ones (the walk reaches every document)."""
+    import apoe
+    import oracle as O
+    n, d, nt = 48, 8, 12
+    rng = np.random.default_rng(4)
+    terms = colliding_terms(nt, 32) # 12 terms: next power of two above 24 buckets
+    dense = rng.standard_normal((n + 1, 1024)).astype(np.float32)
+    dense /= np.linalg.norm(dense, axis=1, keepdims=True)
+    none = lambda k: (np.zeros(k + 1, np.uint32), np.zeros(0, np.uint32), np.zeros(0, np.float32))
+    doc_terms = terms[np.arange(n) % nt]
+    extra = np.full(n, 69999 if wide else 9, np.uint32) # one term past 65 535 takes the wide pair format
+    b_idx = np.stack([doc_terms, extra], 1).reshape(-1)
+    C = O.HybridSet(dense[:n], *none(n), np.arange(0, 2 * n + 1, 2, dtype=np.uint32), b_idx, rng.random(2 * n).astype(np.float32))
+    flags = np.zeros(nt, np.uint32)
+    flags[rng.permutation(nt)[:n_flagged]] = KW
+    Q = O.HybridSet(dense[n:], *none(1), np.array([0, nt], np.uint32), terms | flags, rng.random(nt).astype(np.float32))
+    rows = np.zeros((n, d + 8), np.uint32)
+    rows[:, :d] = (np.arange(n)[:, None] + np.arange(1, d + 1)) % n
+    entry = np.arange(d, dtype=np.uint32)
+    gc, gq, gg = apoe.Corpus(gpu_ctx, *C.arrays()), apoe.Queries(gpu_ctx, *Q.arrays()), apoe.Graph(gpu_ctx, rows, entry)
+    ids, dist, _ = apoe.search(gpu_ctx, gc, gq, gg, (1, 1, 1), 64, keyword_filter=True)
+    oid, odist, _ = O.search(C, Q, rows, entry, (1, 1, 1), 64, keyword_filter=True)
+    assert np.array_equal(ids, oid)
+    assert_dist_close(dist, odist, "hits and the empty rest")
+    assert set(ids[0][ids[0] != EMPTY_ID].tolist()) == {v for v in range(n) if flags[v % nt]}
