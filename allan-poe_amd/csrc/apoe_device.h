@@ -39,6 +39,12 @@ __host__ __device__ inline uint32_t desc_nnz_b(uint64_t d) { return (uint32_t)(d
 // Records start on a 128-byte boundary, and so does the term array of a narrow record: a read of
 // a row, of its values or of its terms then starts at a memory line and only its last line is partial.
 constexpr uint32_t REC_ALIGN = 128;
+// Of the 8-bit sketch of a document's dense row (below): dense row ~ scale * codes, Euclidean norm of the difference at
+// most err (infinite: no sketch).
+struct SketchMeta {
+    float scale, err;
+};
+constexpr int SKETCH_BYTES = DIM; // one signed byte a dimension
 struct CorpusView {
     const uint64_t* desc;
     const char* recs;
@@ -612,6 +618,35 @@ __device__ __forceinline__ float dense_finish_lds_half(const DenseRowHalf& d, co
     }
     return dense_mul * wave_sum_dpp(acc);
 }
+// ---- 8-bit sketch of the dense rows: a tighter bound, never a result ----
+// A document's dense row d is kept a second time as signed bytes c with one scale s, and e >= |d - s c|. The query's row p
+// gets codes u, scale t and f >= |p - t u| when the query starts. The inner product of the codes is exact in integers, and
+//   |<p, d> - s t <u, c>| <= |p| |d - s c| + |p - t u| |s c| <= |p| e + f (|d| + e),
+// so 1 KB tells for most candidates that their exact distance lies beyond the pool, and the 4 KB row is read for the others
+// only. On rows of Gaussian entries e is about 0.008 |d|.
+// Lane l holds dimensions 16 l .. 16 l + 15 of either side: one 16-byte load a row and lane, four dot products of four bytes.
+__device__ __forceinline__ float sketch_dot(const uint4 c, const uint4 u) { // wave sum of the code products
+    int a = __builtin_amdgcn_sdot4((int)c.x, (int)u.x, 0, false);
+    a = __builtin_amdgcn_sdot4((int)c.y, (int)u.y, a, false);
+    a = __builtin_amdgcn_sdot4((int)c.z, (int)u.z, a, false);
+    a = __builtin_amdgcn_sdot4((int)c.w, (int)u.w, a, false);
+    return wave_sum_dpp((float)a); // at most 1024 * 127^2 < 2^24 in all: every partial sum is exact
+}
+__device__ __forceinline__ int sketch_code(float x, float per) { return (int)fminf(fmaxf(rintf(x * per), -127.f), 127.f); }
+// Codes of a row whose largest magnitude is `top`: the multiplier (0: the row has no usable scale, all codes are zero).
+__device__ __forceinline__ float sketch_per(float top) { return top > 1e-30f && top < 65504.f ? 127.f / top : 0.f; }
+__device__ __forceinline__ uint32_t sketch_pack(const float4 x, float per) {
+    return (uint32_t)(sketch_code(x.x, per) & 255) | (uint32_t)(sketch_code(x.y, per) & 255) << 8 | (uint32_t)(sketch_code(x.z, per) & 255) << 16 |
+           (uint32_t)(sketch_code(x.w, per) & 255) << 24;
+}
+// Squared difference between four entries and their codes.
+__device__ __forceinline__ float sketch_residual(const float4 x, float per, float scale) {
+    const float a = fmaf(-scale, (float)sketch_code(x.x, per), x.x), b = fmaf(-scale, (float)sketch_code(x.y, per), x.y);
+    const float c = fmaf(-scale, (float)sketch_code(x.z, per), x.z), d = fmaf(-scale, (float)sketch_code(x.w, per), x.w);
+    return a * a + b * b + c * c + d * d;
+}
+__device__ __forceinline__ float max_abs4(const float4 x) { return fmaxf(fmaxf(fabsf(x.x), fabsf(x.y)), fmaxf(fabsf(x.z), fabsf(x.w))); }
+
 __device__ __forceinline__ float pivot_dense_norm_lds(const float4* pivot) {
     const int lane = lane_id();
     float a = 0.f;

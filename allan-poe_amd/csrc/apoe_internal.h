@@ -109,6 +109,8 @@ struct apoe_corpus {
     apoe::DevBuf<uint64_t> desc;
     apoe::DevBuf<char> recs;
     apoe::DevBuf<float> dnorm;
+    apoe::DevBuf<apoe::SketchMeta> sketch_meta; // of the sketch, [n]
+    apoe::DevBuf<uint32_t> sketch; // 8-bit sketch of the dense rows, [n][dim / 4]; absent (null) when device memory is short
     apoe::DevBuf<uint16_t> half; // optional half-precision copy of the dense rows, [n][dim] (apoe_corpus_make_half_rows)
     apoe::CorpusView view() const { return apoe::CorpusView{desc.p, recs.p, dnorm.p, n, narrow ? 1u : 0u}; }
 };
@@ -170,7 +172,7 @@ int copy_out(apoe_ctx* ctx, void* dst_any, const void* src_dev, size_t bytes);
 // Kernel launchers (one per .hip file).
 int launch_pack(apoe_ctx* ctx, uint32_t n, const float* dense, const uint32_t* s_off, const uint32_t* s_idx, const float* s_val,
                 const uint32_t* b_off, const uint32_t* b_idx, const float* b_val, const uint64_t* desc, char* recs, float* dnorm,
-                bool narrow);
+                SketchMeta* sketch_meta, uint32_t* sketch, bool narrow);
 int launch_max_u32(apoe_ctx* ctx, const uint32_t* a_dev, size_t n, uint32_t* out_dev);
 int launch_half_rows(apoe_ctx* ctx, const apoe_corpus* c, uint16_t* out_dev);
 int launch_distance_batch(apoe_ctx* ctx, const apoe_corpus* c, const apoe_queries* q, const float* w3, const uint32_t* ids_dev,

@@ -267,6 +267,13 @@ int apoe_corpus_create(apoe_ctx* ctx, uint32_t n, uint32_t dim, const float* den
         APOE_TRY(c->desc.alloc(n));
         APOE_TRY(c->recs.alloc(c->rec_bytes + ROW_LOAD_SLACK)); // unclamped row loads may read past the last record
         APOE_TRY(c->dnorm.alloc(n));
+        // the sketch saves the search reads but nothing depends on it: a corpus that leaves little of the device does without
+        size_t free_bytes = 0, total_bytes = 0;
+        APOE_HIP(hipMemGetInfo(&free_bytes, &total_bytes));
+        if ((size_t)n * SKETCH_BYTES <= free_bytes / 8) {
+            APOE_TRY(c->sketch.alloc((size_t)n * (SKETCH_BYTES / 4)));
+            APOE_TRY(c->sketch_meta.alloc(n));
+        }
         APOE_TRY(copy_in(ctx, c->desc.p, desc.data(), n * sizeof(uint64_t)));
         APOE_TRY(d_dense.init(ctx, dense, (size_t)n * dim));
         APOE_TRY(d_soff.init(ctx, s_off, n + 1));
@@ -274,7 +281,7 @@ int apoe_corpus_create(apoe_ctx* ctx, uint32_t n, uint32_t dim, const float* den
         APOE_TRY(d_boff.init(ctx, b_off, n + 1));
         APOE_TRY(d_bval.init(ctx, b_val, hb[n]));
         APOE_TRY(launch_pack(ctx, n, d_dense.p, d_soff.p, d_sidx.p, d_sval.p, d_boff.p, d_bidx.p, d_bval.p, c->desc.p, c->recs.p, c->dnorm.p,
-                             c->narrow));
+                             c->sketch_meta.p, c->sketch.p, c->narrow));
         APOE_HIP(hipStreamSynchronize(ctx->stream));
     }
     *out = c.release();
@@ -304,7 +311,7 @@ int apoe_corpus_info(const apoe_corpus* c, uint32_t* info4) {
 
 uint32_t apoe_corpus_pair_bytes(const apoe_corpus* c) { return c ? (c->narrow ? 6u : 8u) : 0u; }
 
-uint64_t apoe_corpus_bytes(const apoe_corpus* c) { return c ? c->rec_bytes + (uint64_t)c->n * 12 + c->half.bytes() : 0; }
+uint64_t apoe_corpus_bytes(const apoe_corpus* c) { return c ? c->rec_bytes + (uint64_t)c->n * 12 + c->sketch.bytes() + c->sketch_meta.bytes() + c->half.bytes() : 0; }
 
 int apoe_queries_create(apoe_ctx* ctx, uint32_t n, uint32_t dim, const float* dense, const uint32_t* s_off, const uint32_t* s_idx,
                         const float* s_val, const uint32_t* b_off, const uint32_t* b_idx, const float* b_val, apoe_queries** out) {

@@ -26,24 +26,37 @@ __global__ __launch_bounds__(256) void pack_kernel(uint32_t n, const float* __re
                                                    const uint32_t* __restrict__ s_idx, const float* __restrict__ s_val,
                                                    const uint32_t* __restrict__ b_off, const uint32_t* __restrict__ b_idx,
                                                    const float* __restrict__ b_val, const uint64_t* __restrict__ desc, char* recs, float* dnorm,
-                                                   uint32_t narrow) {
-    __shared__ float part[4];
+                                                   SketchMeta* sketch_meta, uint32_t* sketch, uint32_t narrow) {
+    __shared__ float part[4], top[4], rest[4];
     for (uint32_t doc = blockIdx.x; doc < n; doc += gridDim.x) {
         const uint64_t d = desc[doc];
         char* rec = recs + desc_off(d) * 16;
         const float4* src = reinterpret_cast<const float4*>(dense + (size_t)doc * DIM);
         float4* dst = reinterpret_cast<float4*>(rec);
-        float sq = 0.f;
-        for (int i = threadIdx.x; i < DIM / 4; i += blockDim.x) {
-            const float4 x = src[i];
-            dst[i] = x;
-            sq += x.x * x.x + x.y * x.y + x.z * x.z + x.w * x.w;
+        static_assert(DIM / 4 == 256, "a thread per float4 of the dense row");
+        const float4 x = src[threadIdx.x];
+        dst[threadIdx.x] = x;
+        const float sq = wave_sum_dpp(x.x * x.x + x.y * x.y + x.z * x.z + x.w * x.w);
+        const float high = -wave_min_dpp(-max_abs4(x));
+        __syncthreads();
+        if (lane_id() == 0) {
+            part[threadIdx.x / WAVE] = sq;
+            top[threadIdx.x / WAVE] = high;
         }
-        sq = wave_sum_dpp(sq);
         __syncthreads();
-        if (lane_id() == 0) part[threadIdx.x / WAVE] = sq;
+        const float norm = sqrtf(part[0] + part[1] + part[2] + part[3]);
+        const float peak = fmaxf(fmaxf(top[0], top[1]), fmaxf(top[2], top[3]));
+        const float per = sketch_per(peak), scale = per > 0.f ? peak / 127.f : 0.f;
+        if (sketch) sketch[(size_t)doc * (SKETCH_BYTES / 4) + threadIdx.x] = sketch_pack(x, per);
+        const float left = wave_sum_dpp(sketch_residual(x, per, scale));
+        if (lane_id() == 0) rest[threadIdx.x / WAVE] = left;
         __syncthreads();
-        if (threadIdx.x == 0) dnorm[doc] = sqrtf(part[0] + part[1] + part[2] + part[3]);
+        if (threadIdx.x == 0) {
+            dnorm[doc] = norm;
+            // rounded up; a row with an entry that is no number or overflows half precision has no sketch (the same bound serves the half-precision rows)
+            const float err = norm < __builtin_inff() && peak < 65504.f ? 1.0001f * sqrtf(rest[0] + rest[1] + rest[2] + rest[3]) : __builtin_inff();
+            if (sketch) sketch_meta[doc] = SketchMeta{scale, err};
+        }
         const uint32_t s0 = s_off[doc], ns = desc_nnz_s(d), b0 = b_off[doc], nb = desc_nnz_b(d), nnz = ns + nb;
         if (narrow) {
             float* vals = reinterpret_cast<float*>(rec + DENSE_BYTES);
@@ -73,10 +86,10 @@ __global__ __launch_bounds__(256) void pack_kernel(uint32_t n, const float* __re
 
 int launch_pack(apoe_ctx* ctx, uint32_t n, const float* dense, const uint32_t* s_off, const uint32_t* s_idx, const float* s_val,
                 const uint32_t* b_off, const uint32_t* b_idx, const float* b_val, const uint64_t* desc, char* recs, float* dnorm,
-                bool narrow) {
+                SketchMeta* sketch_meta, uint32_t* sketch, bool narrow) {
     uint32_t grid = n < 65536u * 16u ? n : 65536u * 16u;
     if (grid == 0) return APOE_OK;
-    pack_kernel<<<grid, 256, 0, ctx->stream>>>(n, dense, s_off, s_idx, s_val, b_off, b_idx, b_val, desc, recs, dnorm, narrow ? 1u : 0u);
+    pack_kernel<<<grid, 256, 0, ctx->stream>>>(n, dense, s_off, s_idx, s_val, b_off, b_idx, b_val, desc, recs, dnorm, sketch_meta, sketch, narrow ? 1u : 0u);
     APOE_HIP(hipGetLastError());
     return APOE_OK;
 }

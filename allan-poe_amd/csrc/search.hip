@@ -14,6 +14,8 @@ constexpr int MAX_NEW = 64;   // fresh candidates per step: one lane each in wav
 constexpr int EVAL_BATCH = 3;  // candidates whose sparse parts a wave keeps in flight together
 constexpr int DENSE_BATCH = 1; // dense rows a wave keeps in flight together
 constexpr int MERGE_ROUNDS = 4; // 64-element rounds of the pool that the merge moves per LDS round trip
+constexpr int STATS = 10;     // counters of a launch; the workspace keeps 16 words for them
+constexpr int SKETCH_BATCH = 4; // sketches a wave keeps in flight together
 constexpr int RING = 32;      // keyword-filter search: evicted keyword hits kept beside the pool (query.cu:18)
 
 // What the kernel does on top of the plain beam search.
@@ -42,8 +44,12 @@ struct SearchArgs {
     uint32_t cands, max_iter, q_count;
     uint32_t* bitmaps;     // one visited bitmap per workgroup
     uint32_t bitmap_words; // multiple of 4
-    unsigned long long* work; // [0] next query, [1] expansions, [2] evaluations, [3] nnz splade, [4] nnz bm25, [5] dense rows read,
-                              // [6] pool entries evaluated again in fp32, [7] their pairs
+    const SketchMeta* sketch_meta;
+    const uint4* sketch;   // null: the corpus has none
+    uint32_t* codes;       // of the query's dense row, 1 KB per workgroup: in device memory (it is read beside sketches, which take longer), since a
+                           // kilobyte of LDS more costs long batches a resident query per CU (12 -> 11: 3 %)
+    unsigned long long* work; // [0] next query, [1] expansions, [2] evaluations, [3] nnz splade, [4] nnz bm25, [5] evaluations that pairs and norms did not settle,
+                              // [6] pool entries evaluated again in fp32, [7] their pairs, [8] sketches read, [9] dense rows (fp32 or half) read in the walk
     uint32_t full_eval;       // 1: read the dense row of every candidate (no bound test)
     const uint16_t* half;     // not null: the walk takes dense parts from the half-precision rows, the final pool is evaluated again in fp32
     uint32_t slots_s, slots_b, ovf_cap; // buckets of the query's SPLADE / BM25 term table, entries of the overflow list
@@ -55,7 +61,7 @@ struct SearchArgs {
 
 // LDS carve-up shared by host (size) and device (pointers).
 struct SearchLds {
-    uint32_t qd, stat, part, tab, ovf, pool_id, pool_dist, pool_ent, pool_hop, new_desc, new_dn, new_id, new_dist, new_ent, new_hop, seed_id, seed_ent, seed_dist, link, ring_id,
+    uint32_t qd, qs, stat, part, tab, ovf, pool_id, pool_dist, pool_ent, pool_hop, new_desc, new_dn, new_id, new_dist, new_ent, new_hop, seed_id, seed_ent, seed_dist, link, ring_id,
         ring_dist, ctl, total;
     __host__ __device__ SearchLds(uint32_t slots_s, uint32_t slots_b, uint32_t ovf_cap, uint32_t cands, int mode) {
         const bool kg = mode == MODE_KG, kwd = mode == MODE_KEYWORD;
@@ -63,7 +69,8 @@ struct SearchLds {
         uint32_t o = 0;
         qd = o; o += DENSE_BYTES;       // the query's dense row, weight applied
         ctl = o; o += 16 * 4;
-        stat = o; o += 8 * 8;           // the workgroup's counters (work[1..7]), sent once when it leaves
+        qs = o; o += 4 * 4;             // scale and error of the codes of the query's dense row
+        stat = o; o += STATS * 8;       // the workgroup's counters (work[1..]), sent once when it leaves
         part = o; o += MAX_NEW * 16;    // sparse sum of a fresh candidate as four partial sums (one per 16 lanes)
         new_desc = o; o += MAX_NEW * 8; // descriptors and dense norms of the fresh candidates
         new_dn = o; o += MAX_NEW * 4;
@@ -297,6 +304,16 @@ __device__ __forceinline__ uint32_t sort_merge(const Pool& P, const Fresh& F, Ri
     return (uint32_t)__builtin_amdgcn_readlane((int)lb, __builtin_ctzll(__ballot(keep && F.rank == 0)));
 }
 
+// A node's row (id wave-uniform) as a scalar global pointer: left alone, the compiler keeps graph + lane in a vector register
+// pair for the whole launch, spills it, and wave 0 of long batches waits for the spill before it sends its loads (3 % of a
+// 10 000-query batch).
+typedef __attribute__((address_space(1))) const uint32_t GlobalWord;
+__device__ __forceinline__ GlobalWord* graph_row(const SearchArgs& a, uint32_t id) {
+    GlobalWord* row = (GlobalWord*)(a.graph + (uint64_t)uniform(id) * a.W);
+    asm volatile("" : "+s"(row));
+    return row;
+}
+
 template <int NW, int MODE, bool NARROW, bool HALF>
 __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE == MODE_PLAIN && !HALF ? APOE_SEARCH_WAVES_PER_EU : 5, 8))) void search_kernel(SearchArgs a) {
     constexpr bool KG = MODE == MODE_KG, KWD = MODE == MODE_KEYWORD;
@@ -321,6 +338,8 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
     P.cands = a.cands;
     uint64_t* new_desc = reinterpret_cast<uint64_t*>(smem + L.new_desc);
     float* new_dn = reinterpret_cast<float*>(smem + L.new_dn);
+    uint32_t* codes = a.codes + (size_t)blockIdx.x * (SKETCH_BYTES / 4);
+    volatile float* qs = reinterpret_cast<volatile float*>(smem + L.qs);
     uint32_t* new_id = reinterpret_cast<uint32_t*>(smem + L.new_id);
     float* new_dist = reinterpret_cast<float*>(smem + L.new_dist);
     uint32_t* new_ent = reinterpret_cast<uint32_t*>(smem + L.new_ent);
@@ -340,7 +359,7 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
     const uint64_t lane_lt = (1ull << lane) - 1;
 
     unsigned long long* stat = reinterpret_cast<unsigned long long*>(smem + L.stat);
-    if (tid < 8) stat[tid] = 0;
+    if (tid < STATS) stat[tid] = 0;
     while (true) {
         __syncthreads();
         if (tid == 0) ctl[CTL_QUERY] = (uint32_t)atomicAdd(a.work, 1ull);
@@ -372,8 +391,28 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
         __syncthreads();
         query_tabs_fill<NARROW, KWD>(T, a.cold->Q, q, a.cold->w_s, a.cold->w_b, a.paths & PATH_SPARSE, a.paths & PATH_BM25, tid, NW * WAVE);
         __syncthreads();
+        float q_scale = 0.f, q_err = 0.f; // of the query's sketch; scale 0: not used
         const float pv_norm = pivot_dense_norm_lds(qd);
-        uint64_t st_exp = 0, st_eval = 0, st_dense = 0, st_again = 0, st_again_pairs = 0; // wave-uniform counters
+        if (a.sketch && (a.paths & PATH_DENSE)) { // every wave works out the scale and the error, all share the codes
+            float4 x[NV];
+            float top = 0.f, left = 0.f;
+#pragma unroll
+            for (int i = 0; i < NV; i++) { x[i] = qd[lane + WAVE * i]; top = fmaxf(top, max_abs4(x[i])); }
+            top = -wave_min_dpp(-top);
+            const float per = sketch_per(top);
+            if (per > 0.f) {
+                q_scale = top / 127.f;
+#pragma unroll
+                for (int i = 0; i < NV; i++) {
+                    left += sketch_residual(x[i], per, q_scale);
+                    if (wave == i % NW) codes[lane + WAVE * i] = sketch_pack(x[i], per);
+                }
+                q_err = 1.0001f * sqrtf(wave_sum_dpp(left));
+            }
+        }
+        if (tid == 0) { qs[0] = q_scale; qs[1] = q_err; }
+        const bool sketched = __builtin_amdgcn_readfirstlane((int)(q_scale > 0.f)) != 0;
+        uint32_t st_exp = 0, st_eval = 0, st_dense = 0, st_again = 0, st_again_pairs = 0, st_sketch = 0, st_rows = 0; // wave-uniform counters of one query
         uint32_t ln_s = 0, ln_b = 0;                    // pairs read for the candidates this lane decided
         Front front; // wave 0: the first unexplored pool entry
         front.id = EMPTY;
@@ -456,6 +495,7 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
                     dense_issue(row, ri.rec);
                     dist = 1.0f - (dense_finish_lds(row, qd, 1.0f) + ssum) - bonus;
                     st_dense++;
+                    st_rows++;
                 }
                 st_eval++;
                 if (lane == 0) {
@@ -502,16 +542,12 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
             // it is reported as INF_DIS and falls off the end of the merge like any other loser
             const float thr = a.full_eval ? __builtin_inff() : P.dist[cands - 1];
             const float thr_eff = thr < INF_DIS ? thr : __builtin_inff();
+            const float span = sketched ? thr_eff - P.dist[0] : __builtin_inff(); // of the pool
             const uint32_t n_ovf = uniform(ctl[CTL_NOVF]);
-            // descriptors and dense norms of all fresh candidates: lane l holds candidate l's
-            uint64_t my_desc = 0;
-            float my_dn = 0.f;
-            if ((uint32_t)lane < n_new) {
-                my_desc = new_desc[lane];
-                my_dn = new_dn[lane];
-            }
+            // descriptors of all fresh candidates: lane l holds candidate l's
+            const uint64_t my_desc = (uint32_t)lane < n_new ? new_desc[lane] : 0;
             if (wave == 0 && front.id != EMPTY) {
-                const uint32_t* row = a.graph + (size_t)(KWD ? front.id & ID_MASK : front.id) * a.W;
+                GlobalWord* row = graph_row(a, KWD ? front.id & ID_MASK : front.id);
                 g_c = lane < (int)a.degree ? row[lane] : EMPTY;
                 if (KWD) g_kw = lane < APOE_KW_SLOTS ? row[a.degree + lane] : 0u;
             }
@@ -559,17 +595,19 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
             wave_fence();
             // the decision for all of the wave's candidates at once, lane l for candidate l: a candidate whose
             // sparse part plus the bound of its dense part cannot reach the pool is reported as INF_DIS
-            uint64_t need; // bit l: candidate l still needs its dense row
+            uint64_t need, asked; // bit l: candidate l still needs its dense row; its sketch comes first
             {
                 const bool mine = (uint32_t)lane < n_new && (uint32_t)(lane & (NW - 1)) == (uint32_t)wave;
-                bool undecided = false;
+                bool undecided = false, wide = false;
                 if (mine) {
                     float bonus = 0.f;
                     if (KG) {
                         if (new_ent[lane] != EMPTY) bonus = a.kg_weight / (float)new_hop[lane]; // query.cu:1759-1760
                     }
                     float ssum = 0.f, v = 0.f;
+                    const float dub = pv_norm * new_dn[lane]; // |<query_d, doc_d>| <= |query_d| * |doc_d|
                     undecided = true;
+                    wide = dub > span;
                     if (a.paths & (PATH_SPARSE | PATH_BM25)) {
                         const float4 p4 = reinterpret_cast<const float4*>(part)[lane];
                         ssum = p4.x + p4.y + p4.z + p4.w; // the order wave_sum_dpp adds its four rows in
@@ -578,7 +616,6 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
                             v = 1.0f - ssum - bonus;
                             undecided = false;
                         } else {
-                            const float dub = pv_norm * my_dn; // |<query_d, doc_d>| <= |query_d| * |doc_d|
                             const float lb = 1.0f - (ssum + dub) - bonus;
                             if (lb > thr_eff + 1e-5f * (fabsf(ssum) + dub + fabsf(bonus) + 1.0f)) {
                                 v = INF_DIS;
@@ -592,9 +629,61 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
                 }
                 st_eval += __popcll(__ballot(mine));
                 need = __ballot(undecided);
+                asked = __ballot(undecided && wide);
+                st_dense += __popcll(need);
             }
             wave_fence();
-            // stage 2: the dense rows of the survivors, DENSE_BATCH rows in flight (two of the half-precision rows)
+            // stage 2: the sketches of the survivors, SKETCH_BATCH in flight, then the same decision with the tighter bound
+            // Asked are candidates whose dense part can move the distance by more than the pool spans: of those few enter the pool
+            // (about span / bound of them), and a sketch that rejects saves three quarters of a row. Where the pairs decide, most
+            // undecided candidates do enter, and the sketch would be a second wait for a row that is read anyway. Both sides, 10 000
+            // queries on 1 M docs: dense rows with neighbours under (49, 1, 1), cands 80 (11 % of the evaluations enter): 4.1 KB of
+            // dense part per evaluation -> 1.7 KB, 35.7 -> 21.6 ms; i.i.d. corpus under (1, 1, 1), cands 256 (13 % are undecided, 11 %
+            // enter): asking always took 42.3 ms, this rule, which asks almost none, 39.0, no sketches 39.3.
+            if (asked) {
+                SketchMeta sm = {0.f, 0.f}; // of candidate l
+                if ((asked >> lane) & 1) sm = a.sketch_meta[new_id[lane]];
+                const uint4 u = reinterpret_cast<const uint4*>(codes)[lane];
+                for (uint64_t left = asked; left;) {
+                    uint4 c[SKETCH_BATCH] = {}; // set on every path: values left open would live, and spill, across the whole walk
+                    uint32_t jj[SKETCH_BATCH];
+#pragma unroll
+                    for (int b = 0; b < SKETCH_BATCH; b++) {
+                        jj[b] = EMPTY;
+                        if (left) {
+                            jj[b] = __builtin_ctzll(left);
+                            left &= left - 1;
+                            c[b] = a.sketch[(size_t)uniform(new_id[jj[b]]) * (SKETCH_BYTES / 16) + lane];
+                        }
+                    }
+#pragma unroll
+                    for (int b = 0; b < SKETCH_BATCH; b++) {
+                        if (jj[b] != EMPTY) {
+                            const float dot = sketch_dot(c[b], u);
+                            if (lane == 0) part[jj[b] * 4] = dot;
+                        }
+                    }
+                }
+                st_sketch += __popcll(asked);
+                wave_fence();
+                bool far = false;
+                if ((asked >> lane) & 1) {
+                    float bonus = 0.f;
+                    if (KG) {
+                        if (new_ent[lane] != EMPTY) bonus = a.kg_weight / (float)new_hop[lane];
+                    }
+                    const float dn = new_dn[lane], ssum = new_dist[lane], dub = pv_norm * dn;
+                    float most = part[lane * 4] * (qs[0] * sm.scale) + pv_norm * sm.err + qs[1] * (dn + sm.err);
+                    if (HALF) most += pv_norm * (4.9e-4f * dn + 1.1e-6f); // the walk's rows are rounded to half precision
+                    const float lb = 1.0f - (ssum + most) - bonus;
+                    far = lb > thr_eff + 1e-5f * (fabsf(ssum) + dub + fabsf(bonus) + 1.0f);
+                    if (far) new_dist[lane] = INF_DIS;
+                }
+                need &= ~__ballot(far);
+                wave_fence();
+            }
+            st_rows += __popcll(need);
+            // stage 3: the dense rows of the survivors, DENSE_BATCH rows in flight (two of the half-precision rows)
             while (HALF && need) {
                 DenseRowHalf row[2];
                 uint32_t jj[2];
@@ -611,7 +700,6 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
                 for (int b = 0; b < 2; b++) {
                     if (jj[b] != EMPTY) {
                         const float dsum = dense_finish_lds_half(row[b], qd, 1.0f);
-                        st_dense++;
                         if (lane == 0) new_dist[jj[b]] = 1.0f - (dsum + new_dist[jj[b]]) - 0.f;
                     }
                 }
@@ -636,7 +724,6 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
                             if (new_ent[jj[b]] != EMPTY) bonus = a.kg_weight / (float)new_hop[jj[b]];
                         }
                         const float dsum = dense_finish_lds(row[b], qd, 1.0f);
-                        st_dense++;
                         if (lane == 0) new_dist[jj[b]] = 1.0f - (dsum + new_dist[jj[b]]) - bonus;
                     }
                 }
@@ -660,7 +747,7 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
                     if (KWD && parent != EMPTY) parent &= ID_MASK;
                 }
                 if (parent != EMPTY && overtaken) {
-                    const uint32_t* row = a.graph + (size_t)parent * a.W;
+                    GlobalWord* row = graph_row(a, parent);
                     g_c = lane < (int)a.degree ? row[lane] : EMPTY;
                     if (KWD) g_kw = lane < APOE_KW_SLOTS ? row[a.degree + lane] : 0u;
                 }
@@ -893,20 +980,22 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
             if (st_dense) atomicAdd(stat + 5, (unsigned long long)st_dense);
             if (st_again) atomicAdd(stat + 6, (unsigned long long)st_again);
             if (st_again_pairs) atomicAdd(stat + 7, (unsigned long long)st_again_pairs);
+            if (st_sketch) atomicAdd(stat + 8, (unsigned long long)st_sketch);
+            if (st_rows) atomicAdd(stat + 9, (unsigned long long)st_rows);
         }
     }
     __syncthreads();
-    if (tid >= 1 && tid < 8 && stat[tid]) atomicAdd(a.work + tid, stat[tid]);
+    if (tid >= 1 && tid < STATS && stat[tid]) atomicAdd(a.work + tid, stat[tid]);
 }
 
 // Counters and once-per-query arguments of a launch, written on the stream (no host copy from a stack frame,
 // no memset node for a caller that records the stream).
 __global__ void search_setup_kernel(unsigned long long* work, SearchCold* dst, SearchCold cold) {
-    if (threadIdx.x < 8) work[threadIdx.x] = 0ull;
+    if (threadIdx.x < STATS) work[threadIdx.x] = 0ull;
     if (threadIdx.x == 0) *dst = cold;
 }
 
-// Workspace of apoe_search_noalloc: counters, once-per-query arguments and the visited bitmaps of as many
+// Workspace of apoe_search_noalloc: counters, once-per-query arguments, the visited bitmaps and query codes of as many
 // workgroups as fit. One copy per GPU, held until the process ends; every call on a GPU uses it, so calls
 // that overlap on one GPU race. Host code never uses the array's name as an address: the device address is
 // asked for once per device (search_static_workspace) and kept.
@@ -1008,6 +1097,8 @@ int launch_search(apoe_ctx* ctx, const apoe_corpus* c, const apoe_queries* q, co
     a.kg_weight = p->kg_weight;
     a.full_eval = (p->variant & 0x100u) ? 1u : 0u;
     a.half = nullptr;
+    a.sketch_meta = c->sketch_meta.p;
+    a.sketch = reinterpret_cast<const uint4*>(c->sketch.p);
     if (p->variant & 0x200u) {
         APOE_REQUIRE(c->half.p != nullptr, "variant 0x200 needs the half-precision rows: call apoe_corpus_make_half_rows first");
         APOE_REQUIRE(kg == nullptr && !p->keyword_filter, "variant 0x200 (half-precision rows) is for the plain search only");
@@ -1036,12 +1127,12 @@ int launch_search(apoe_ctx* ctx, const apoe_corpus* c, const apoe_queries* q, co
     APOE_REQUIRE(L.total <= 64 * 1024, "search needs %u bytes of LDS (query rows with up to %u sparse terms)", L.total, q->max_nnz);
 
     a.bitmap_words = ((c->n + 31) / 32 + 3) & ~3u;
-    // workspace: [counters: 8 x u64][once-per-query arguments][visited bitmaps]
-    const size_t cold_at = 8 * sizeof(unsigned long long), bitmaps_at = (cold_at + sizeof(SearchCold) + 255) & ~(size_t)255;
+    // workspace: [counters: 16 x u64][once-per-query arguments][visited bitmaps][codes of the queries' dense rows]
+    const size_t cold_at = 16 * sizeof(unsigned long long), bitmaps_at = (cold_at + sizeof(SearchCold) + 255) & ~(size_t)255;
     const size_t bitmap_bytes = (size_t)a.bitmap_words * sizeof(uint32_t);
     size_t fit = SIZE_MAX; // workgroups whose visited bitmaps fit the workspace
     if (static_ws) {
-        fit = (APOE_NOALLOC_WS_BYTES - bitmaps_at) / bitmap_bytes;
+        fit = (APOE_NOALLOC_WS_BYTES - bitmaps_at) / (bitmap_bytes + SKETCH_BYTES);
         APOE_REQUIRE(fit >= 1, "the static workspace of %u bytes holds no visited bitmap of %zu bytes", (unsigned)APOE_NOALLOC_WS_BYTES, bitmap_bytes);
     }
 
@@ -1087,12 +1178,13 @@ int launch_search(apoe_ctx* ctx, const apoe_corpus* c, const apoe_queries* q, co
     // persistent grid: as many workgroups as can be resident, never more than queries or bitmaps
     const uint32_t grid = (uint32_t)std::min<size_t>(std::min<size_t>(q_count, fit), (size_t)per_cu * (size_t)ctx->num_cus);
     char* ws = static_ws;
-    if (!static_ws) APOE_TRY(ctx->search_workspace(bitmaps_at + (size_t)grid * bitmap_bytes, &ws));
+    if (!static_ws) APOE_TRY(ctx->search_workspace(bitmaps_at + (size_t)grid * (bitmap_bytes + SKETCH_BYTES), &ws));
     unsigned long long* work = reinterpret_cast<unsigned long long*>(ws);
     search_setup_kernel<<<1, WAVE, 0, ctx->stream>>>(work, reinterpret_cast<SearchCold*>(ws + cold_at), cold);
     APOE_HIP(hipGetLastError());
     a.cold = reinterpret_cast<const SearchCold*>(ws + cold_at);
     a.bitmaps = reinterpret_cast<uint32_t*>(ws + bitmaps_at);
+    a.codes = reinterpret_cast<uint32_t*>(ws + bitmaps_at + (size_t)grid * bitmap_bytes);
     a.work = work;
 
     if (static_ws && !stats) return launch_mode(ctx, mode, nw, a, grid, L.total, nullptr);
@@ -1100,7 +1192,7 @@ int launch_search(apoe_ctx* ctx, const apoe_corpus* c, const apoe_queries* q, co
     APOE_TRY(timed(ctx, &ms, [&]() { return launch_mode(ctx, mode, nw, a, grid, L.total, nullptr); }));
     APOE_HIP(hipStreamSynchronize(ctx->stream));
     if (stats) {
-        unsigned long long h[8];
+        unsigned long long h[STATS];
         APOE_HIP(hipMemcpy(h, work, sizeof(h), hipMemcpyDeviceToHost));
         stats->kernel_ms = ms;
         stats->expansions = h[1];
@@ -1108,8 +1200,8 @@ int launch_search(apoe_ctx* ctx, const apoe_corpus* c, const apoe_queries* q, co
         stats->nnz_sparse = h[3];
         stats->nnz_bm25 = h[4];
         stats->dense_rows = h[5];
-        // dense rows actually needed + pairs + descriptor and dense norm (12 B per evaluation)
-        uint64_t bytes = h[5] * (uint64_t)(a.half ? DENSE_BYTES / 2 : DENSE_BYTES);
+        // dense rows and sketches actually needed (a sketch with its scale and error) + pairs + descriptor and dense norm (12 B per evaluation)
+        uint64_t bytes = h[9] * (uint64_t)(a.half ? DENSE_BYTES / 2 : DENSE_BYTES) + h[8] * (uint64_t)(SKETCH_BYTES + sizeof(SketchMeta));
         bytes += (c->narrow ? 6 : 8) * (h[3] + h[4]) + 12 * h[2];
         bytes += h[6] * (uint64_t)(DENSE_BYTES + 8) + (c->narrow ? 6 : 8) * h[7]; // the pool evaluated again in fp32
         bytes += h[1] * 4ull * a.W;

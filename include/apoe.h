@@ -232,9 +232,10 @@ typedef struct {
     uint64_t evaluations; /* hybrid distance evaluations */
     uint64_t nnz_sparse;  /* SPLADE pairs read by those evaluations (0 if path off) */
     uint64_t nnz_bm25;    /* BM25 pairs read by those evaluations (0 if path off) */
-    uint64_t dense_rows;  /* evaluations that had to read the 4 KB dense row (see variant) */
-    uint64_t algo_bytes;  /* algorithmic HBM bytes: dense rows read + pairs + descriptors + graph
-                             rows + queries + results */
+    uint64_t dense_rows;  /* evaluations that pairs and norms did not settle (see variant): they read the dense
+                             row, or its 1 KB sketch first and the row if that does not settle them either */
+    uint64_t algo_bytes;  /* algorithmic HBM bytes: dense rows and sketches read + pairs + descriptors +
+                             graph rows + queries + results */
 } apoe_search_stats;
 
 /* out_ids/out_dist are [q_count][cands], ascending distance; top_k is the row

@@ -1,0 +1,64 @@
+"""The 8-bit sketch of the dense rows only ever rejects what its 4 KB row would reject: whole rows of results are bit for bit
+those of a walk that reads every row (variant 0x100), on rows where a wrong bound would show: magnitudes from denormal to
+beyond half precision, one-hot rows, zero rows, entries that are no numbers, and weights that make the dense part decide."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+N, D, NQ = 3000, 32, 40
+
+
+def world(kind, seed, wide):
+    rng = np.random.default_rng(seed)
+    centre = rng.standard_normal((8, 1024))
+    dense = (centre[rng.integers(0, 8, N)] + rng.standard_normal((N, 1024))).astype(np.float32)
+    q = (centre[rng.integers(0, 8, NQ)] + rng.standard_normal((NQ, 1024))).astype(np.float32)
+    if kind == "magnitudes":
+        dense *= (10.0 ** rng.choice([-40, -33, -20, -3, 0, 0, 0, 1, 3, 4], N)).astype(np.float32)[:, None]
+        dense[::97] = 0
+        q[::7] *= np.float32(1e-36)
+        q[1] = 0
+    elif kind == "spikes":  # one entry far above the rest: a coarse scale, a large error
+        dense[np.arange(N), rng.integers(0, 1024, N)] *= rng.choice([1, 10, 1000], N).astype(np.float32)
+        dense[::50] = np.eye(1024, dtype=np.float32)[rng.integers(0, 1024, len(dense[::50]))]
+        q[np.arange(NQ), rng.integers(0, 1024, NQ)] *= 100
+    elif kind == "not numbers":
+        dense[5::200, 3] = np.inf
+        dense[7::200, 900] = np.nan
+        dense[9::200, 12] = 7e4
+    idx = (rng.integers(0, 300, (N, 12)).cumsum(1) % 60000).astype(np.uint32) + np.uint32(70000 if wide else 0)
+    off = np.arange(0, 12 * N + 1, 12, dtype=np.uint32)
+    q_off = np.arange(0, 12 * NQ + 1, 12, dtype=np.uint32)
+    corpus = (dense, off, idx.reshape(-1), rng.random(12 * N).astype(np.float32), off, idx[::-1].reshape(-1).copy(), rng.random(12 * N).astype(np.float32))
+    queries = (q, q_off, idx[:NQ].reshape(-1).copy(), rng.random(12 * NQ).astype(np.float32), q_off, idx[-NQ:].reshape(-1).copy(), rng.random(12 * NQ).astype(np.float32))
+    rows = np.zeros((N, D + 8), np.uint32)
+    rows[:, :D] = rng.integers(0, N, (N, D))
+    return corpus, queries, rows, rng.choice(N, D, replace=False).astype(np.uint32)
+
+
+@pytest.mark.parametrize("wide", [False, True])
+@pytest.mark.parametrize("kind", ["plain", "magnitudes", "spikes", "not numbers"])
+def test_rows_are_those_of_reading_every_dense_row(gpu_ctx, kind, wide):
+    import apoe
+    corpus, queries, rows, entry = world(kind, 6, wide)
+    gc, gq, gg = apoe.Corpus(gpu_ctx, *corpus), apoe.Queries(gpu_ctx, *queries), apoe.Graph(gpu_ctx, rows, entry)
+    for w3, cands, shape in (((1, 0, 0), 24, 0), ((49, 1, 1), 64, 4), ((0.01, 1, 1), 33, 3), ((1, 1, 0), 200, 2)):
+        a, ad, sa = apoe.search(gpu_ctx, gc, gq, gg, w3, cands, variant=shape)
+        b, bd, sb = apoe.search(gpu_ctx, gc, gq, gg, w3, cands, variant=shape | 0x100)
+        assert np.array_equal(a, b) and np.array_equal(ad, bd, equal_nan=True), (w3, cands)
+        assert sa.evaluations == sb.evaluations and sa.dense_rows <= sb.dense_rows
+        if kind == "plain" and w3 == (1, 0, 0):
+            assert sa.algo_bytes < 0.8 * sb.algo_bytes  # the sketch is in use
+
+
+@pytest.mark.parametrize("kind", ["plain", "magnitudes", "spikes"])
+def test_half_precision_walk(gpu_ctx, kind):
+    """The walk on half-precision rows under the sketch against the same walk without any bound."""
+    import apoe
+    corpus, queries, rows, entry = world(kind, 8, False)
+    gc, gq, gg = apoe.Corpus(gpu_ctx, *corpus), apoe.Queries(gpu_ctx, *queries), apoe.Graph(gpu_ctx, rows, entry)
+    gc.make_half_rows()
+    for w3 in ((1, 0, 0), (49, 1, 1)):
+        a, ad, _ = apoe.search(gpu_ctx, gc, gq, gg, w3, 48, variant=0x200)
+        b, bd, _ = apoe.search(gpu_ctx, gc, gq, gg, w3, 48, variant=0x300)
+        assert np.array_equal(a, b) and np.array_equal(ad, bd)
