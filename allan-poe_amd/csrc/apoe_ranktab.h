@@ -84,28 +84,6 @@ __device__ __forceinline__ uint32_t ranktab_index(const RankTab& T, uint32_t key
     return ((k * 0x9E3779B1u) >> 12) & (T.index_bits - 1);
 }
 
-// The pairs of the pivots of one group, spread over the threads of the block: thread i holds pair i of every
-// pivot (rows with more pairs than the block has threads read the rest when the table is built). Loaded ahead of
-// time, while the previous group is still being probed, so that a build does not wait for memory.
-constexpr int RT_PV = 1;
-struct PivotRegs {
-    uint2 kv[RT_T][RT_PV]; // raw pairs
-};
-template <typename PivotFn>
-__device__ __forceinline__ void ranktab_pivots_load(PivotRegs& r, PivotFn pivot, uint32_t nt, int tid, int nthreads) {
-#pragma unroll
-    for (int t = 0; t < RT_T; t++) {
-        if ((uint32_t)t < nt) {
-            const Pairs sp = pivot(t);
-#pragma unroll
-            for (int k = 0; k < RT_PV; k++) {
-                const uint32_t j = tid + k * nthreads;
-                r.kv[t][k] = j < sp.nnz ? sp.raw(j) : make_uint2(0u, 0u);
-            }
-        }
-    }
-}
-
 // Bitmap and running counts of the terms that `each` hands out: each(f) calls f(raw pair, is BM25, pivot index) for
 // every pair that this thread is responsible for. All threads of the block call this (the block size is a multiple of
 // 64, at most 1024); `scan` is LDS scratch of 20 words. Returns the number of distinct terms. Does NOT end with a
@@ -216,27 +194,6 @@ __device__ __forceinline__ uint32_t ranktab_build_each(const RankTab& T, EachFn 
         if (ov > RT_OVF) return EMPTY;
     }
     return total;
-}
-
-// The table of pivots [0, nt) (nt <= RT_T) whose pairs are spread over the threads of the block: pivot(t) gives the
-// Pairs of pivot t, `regs` its first pairs (ranktab_pivots_load).
-template <bool NARROW, typename PivotFn>
-__device__ __forceinline__ uint32_t ranktab_build(const RankTab& T, PivotFn pivot, const PivotRegs& regs, uint32_t nt, uint32_t* scan, int tid,
-                                                  int nthreads) {
-    return ranktab_build_each<NARROW>(T, [&](auto f) {
-#pragma unroll
-        for (int t = 0; t < RT_T; t++) {
-            if ((uint32_t)t < nt) {
-                const Pairs sp = pivot(t);
-#pragma unroll
-                for (int k = 0; k < RT_PV; k++) {
-                    const uint32_t j = tid + k * nthreads;
-                    if (j < sp.nnz) f(regs.kv[t][k], j >= sp.ns, t);
-                }
-                for (uint32_t j = tid + RT_PV * nthreads; j < sp.nnz; j += nthreads) f(sp.raw(j), j >= sp.ns, t);
-            }
-        }
-    }, scan, tid, nthreads);
 }
 
 // One pair against the table: acc[t] += value * (pivot t's value of the term). `in` = the lane holds a pair.

@@ -1,13 +1,13 @@
-// NN-Descent step as a local join around the picked neighbour (K = 64).
+// NN-Descent step as a local join around the picked neighbour.
 //
 // The reference's step (index.cu:156-376) lets node u meet the forward list N(v) and the reverse list R(v) of
 // each neighbour v it picks: one pivot against many rows, every row gathered for one evaluation. Here the same
 // pairs are formed the other way round: all pickers of one v are the ROWS of a tile (32 at a time), N(v) and R(v)
 // are its COLUMNS (up to 128), every row of the tile is gathered once and meets every column:
-//   dense part   32 x 128 x 1024 contraction on the matrix cores (fp32 MFMA 32x32x2; eight waves: the 32-column
-//                blocks that exist x equal parts of the dimensions)
+//   dense part   32 x 128 x 1024 contraction on the matrix cores (fp32 MFMA 16x16x4; the waves take the
+//                16-column blocks that exist x equal parts of the dimensions)
 //   sparse part  eight picker rows at a time in an LDS rank table that the column rows probe (apoe_ranktab.h); a
-//                wave keeps the pairs of its sixteen columns in registers, so a row is read from memory once per tile
+//                wave keeps the pairs of its columns (eight or sixteen) in registers, so a row is read from memory once per tile
 //   insertion    a pair closer than the row's last list entry (and not in that list) is offered to the row node
 //                with a 64-bit atomicMin on slot hash(id) of its proposal row: (distance, id), the smallest wins;
 //                in symmetric mode the pair is offered to the column node as well (both endpoints, as the classic
@@ -32,7 +32,12 @@ namespace apoe {
 
 constexpr int JT_ROWS = 32;
 constexpr int JT_COLS = 128;
-constexpr int JT_THREADS = 512;
+// Threads of a tile's workgroup (one per CU: LDS allows no second one). Sixteen waves for narrow corpora: a tile is a chain of
+// short phases with barriers between them (queue, id set, staging, table builds, probes), and four waves per SIMD cover each
+// other's waits where two do not; a wave then owns eight columns, whose pairs fit beside everything else in 128 registers.
+// 100 000 docs K = 64: 117 -> 112 ms over ten steps; 30 011 docs K = 128: step 72 -> 59, prune tiles 30 -> 26 ms. The wide
+// format's row registers (keys of 32 bits, key compares) do not fit 128: it spilled 100 of them and stays at eight waves.
+constexpr int jt_threads(bool narrow) { return narrow ? 1024 : 512; }
 constexpr int JT_STRIDE = JT_COLS + 1;
 constexpr int JT_SEEN = 512; // slots of the id set that removes repeated columns
 // The kernels below are built for lists of KK = 64 and KK = 128 entries (index.cu:6 has K 64; a degree above 32 needs
@@ -41,8 +46,6 @@ constexpr int JT_SEEN = 512; // slots of the id set that removes repeated column
 // 256) are two tiles: the list, then what the reverse list adds to it.
 constexpr int JOIN_PICKS = 4; // index.cu:157,171-181
 constexpr int JOIN_COUNT_PARTS = 256, JOIN_COUNT_AT = 8; // partial insertion counters in the step's work array, one per 64-byte line, from word 8
-constexpr int JT_BATCH = 2;   // column rows a wave probes together
-constexpr int JT_OWN = JT_COLS / (JT_THREADS / WAVE); // columns of a tile that one wave owns: their pairs stay in its registers
 
 __device__ __forceinline__ uint32_t prop_slot(uint32_t id, uint32_t P) { return (uint32_t)(mix64(id) >> 40) & (P - 1); }
 
@@ -222,35 +225,38 @@ __device__ __forceinline__ uint32_t wave_sort_u32(uint32_t v, int lane) {
 
 // The hybrid inner products of a tile, G[r * JT_STRIDE + c] = dense_mul * <row r, column c>_dense + <row r, column c>_sparse for
 // the R rows and M columns whose record addresses and shapes `rowptr` / `rownnz` hold (rows at [0, JT_ROWS), columns at
-// [JT_ROWS, JT_ROWS + JT_COLS): gram_rows_gather). All JT_THREADS threads call it after a barrier behind those arrays; it
+// [JT_ROWS, JT_ROWS + JT_COLS): gram_rows_gather). All threads of the workgroup call it after a barrier behind those arrays; it
 // ends with a barrier. `tabreg` = the table region of JoinLds, `unfit` = counter of rows whose terms did not fit the table.
 template <bool NARROW>
 __device__ __forceinline__ void tile_hybrid_ips(const CorpusView& C, float dense_mul, char* tabreg, const RankTab& T, uint32_t index_bits, uint32_t slot_cap,
                                                 float* G, const unsigned long long* rowptr, const uint32_t* rownnz, uint32_t* scan, uint32_t R,
                                                 uint32_t M, unsigned long long* unfit, int tid, int wave, int lane) {
-    constexpr int NW = JT_THREADS / WAVE;
-    // dense part: the eight waves share the 16-column blocks that exist (8, 4, 2 or 1 by the number of columns) and, for
-    // each block, equal parts of the dimensions (1, 2, 4 or 8): no wave idles when a tile has few columns. The picker
+    constexpr int NT = jt_threads(NARROW), NW = NT / WAVE;
+    constexpr int JT_OWN = JT_COLS / NW;    // columns of a tile that one wave owns: their pairs stay in its registers
+    constexpr int JT_BATCH = NW == 8 ? 2 : 1; // column rows a wave probes together: with four waves per SIMD one at a time covers the waits
+    constexpr int RING = NW == 8 ? 16 : 8;  // column blocks a wave has in flight: 128 per CU either way
+    // dense part: the waves share the 16-column blocks that exist (8, 4, 2 or 1 by the number of columns) and, for
+    // each block, equal parts of the dimensions (1, 2, 4, 8 or 16): no wave idles when a tile has few columns. The picker
     // rows are staged in the table region, which is free until the sparse part. Partial tiles are added into G in a
     // fixed order, a barrier between them.
     {
         const uint32_t nblk = M <= 16 ? 1u : M <= 32 ? 2u : M <= 64 ? 4u : 8u, parts = (uint32_t)NW / nblk;
         const uint32_t blk = (uint32_t)wave % nblk, part = (uint32_t)wave / nblk;
         const bool active = blk * 16 < M;
-        const uint32_t per = (DIM / 16) / parts; // 16-float blocks of the dimensions per part: 64, 32, 16 or 8
+        const uint32_t per = (DIM / 16) / parts; // 16-float blocks of the dimensions per part: 64, 32, 16, 8 or 4
         float4* A = reinterpret_cast<float4*>(tabreg);
         const uint32_t jcol = min(blk * 16 + (uint32_t)(lane & 15), M - 1);
         const float4* pb = reinterpret_cast<const float4*>(rowptr[JT_ROWS + jcol] - DENSE_BYTES) + (lane >> 4);
 #pragma unroll 4
-        for (uint32_t i = tid; i < R * (DIM / 4); i += JT_THREADS) {
+        for (uint32_t i = tid; i < R * (DIM / 4); i += NT) {
             const uint32_t r = i / (DIM / 4), c = i % (DIM / 4);
             A[r * (DIM / 4) + (c ^ (r & 7))] = reinterpret_cast<const float4*>(rowptr[r] - DENSE_BYTES)[c];
         }
         __syncthreads();
         floatx4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
         if (active) {
-            if (per >= 16) join_dense16<16>(A, R, pb, lane, (int)(part * per), (int)((part + 1) * per), acc0, acc1);
-            else join_dense16<8>(A, R, pb, lane, (int)(part * per), (int)((part + 1) * per), acc0, acc1);
+            if (per >= (uint32_t)RING) join_dense16<RING>(A, R, pb, lane, (int)(part * per), (int)((part + 1) * per), acc0, acc1);
+            else join_dense16<RING / 2>(A, R, pb, lane, (int)(part * per), (int)((part + 1) * per), acc0, acc1);
         }
         auto store = [&](bool add) {
 #pragma unroll
@@ -275,8 +281,17 @@ __device__ __forceinline__ void tile_hybrid_ips(const CorpusView& C, float dense
     auto row_pairs = [&](uint32_t i) { Pairs p = gram_row(C, rowptr, rownnz, i); p.narrow = NARROW ? 1u : 0u; return p; };
     auto col_pairs = [&](uint32_t b) { Pairs p = gram_row(C, rowptr + JT_ROWS, rownnz + JT_ROWS, b); p.narrow = NARROW ? 1u : 0u; return p; };
     uint32_t a0 = 0;
-    PivotRegs pv;
-    ranktab_pivots_load(pv, [&](uint32_t t) { return row_pairs(a0 + t); }, min((uint32_t)RT_T, R - a0), tid, JT_THREADS);
+    // a group's pivots, one per wave (as the prune holds its rows): a build hands every wave its own row's pairs, four to a lane
+    RtRow<NARROW> pv;
+    uint32_t pv_shape = 0;
+    auto pivots_load = [&](uint32_t first) {
+        pv_shape = 0;
+        if (wave < RT_T && first + wave < R) {
+            pv_shape = uniform(rownnz[first + wave]);
+            rt_row_load(pv, row_pairs(first + wave), lane);
+        }
+    };
+    pivots_load(0);
     // the wave's columns wave, wave + NW, ...: read once per tile, probed once per group; their shapes
     // (nnz | ns << 16) are wave-uniform and stay in scalar registers
     RtRow<NARROW> own[JT_OWN];
@@ -294,12 +309,12 @@ __device__ __forceinline__ void tile_hybrid_ips(const CorpusView& C, float dense
         uint32_t nt = min((uint32_t)RT_T, R - a0);
         uint32_t built;
         while (true) {
-            built = ranktab_build<NARROW>(T, [&](uint32_t t) { return row_pairs(a0 + t); }, pv, nt, scan, tid, JT_THREADS);
+            built = ranktab_build_rows<NARROW>(T, pv, pv_shape, (uint32_t)wave < nt, wave, row_pairs(min(a0 + wave, R - 1)), scan, tid, NT);
             if (built != EMPTY || nt == 1) break;
             nt = (nt + 1) / 2; // the registers hold the first pivots of the group whatever nt is
         }
         const uint32_t a1 = a0 + nt;
-        if (a1 < R) ranktab_pivots_load(pv, [&](uint32_t t) { return row_pairs(a1 + t); }, min((uint32_t)RT_T, R - a1), tid, JT_THREADS);
+        if (a1 < R) pivots_load(a1);
         if (built == EMPTY) { // one row alone does not fit: its sparse part is missing, the host is told
             if (tid == 0) atomicAdd(unfit, 1ull);
             a0 = a1;
@@ -323,10 +338,12 @@ __device__ __forceinline__ void tile_hybrid_ips(const CorpusView& C, float dense
                     for (int t = 0; t < RT_T; t++) acc[k][t] = 0.f;
                 }
                 ranktab_probe_rows<NARROW, JT_BATCH>(T, rows, shape, [&](int k) { return col_pairs(b0 + k * NW); }, n_ovf, acc, lane);
-                uint32_t t, r;
-                const float z = wave_sum_2x8(acc, lane, &t, &r);
+                uint32_t t, r = 0;
+                float z;
+                if constexpr (JT_BATCH == 2) z = wave_sum_2x8(acc, lane, &t, &r);
+                else z = wave_sum_1x8(acc[0], lane, &t);
                 const uint32_t b = b0 + r * NW;
-                if ((lane & 15) < 4 && t < nt && b < M) G[(a0 + t) * JT_STRIDE + b] += z;
+                if ((lane & 15) < 4 && (JT_BATCH == 2 || lane < 32) && t < nt && b < M) G[(a0 + t) * JT_STRIDE + b] += z;
             }
             __builtin_amdgcn_sched_barrier(0); // one batch at a time: the scheduler must not pile up the reads of all of them
         }
@@ -358,8 +375,9 @@ __device__ __forceinline__ void wave_sort_u32x2(uint32_t& a, uint32_t& b, int la
 }
 
 template <bool NARROW, uint32_t KK>
-__global__ __launch_bounds__(JT_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void join_tile_kernel(JoinArgs a) {
+__global__ __launch_bounds__(jt_threads(NARROW)) __attribute__((amdgpu_waves_per_eu(jt_threads(NARROW) / 256, jt_threads(NARROW) / 256))) void join_tile_kernel(JoinArgs a) {
     constexpr uint32_t HALVES = KK / 64; // tiles per block of picker rows
+    constexpr int NT = jt_threads(NARROW), NW = NT / WAVE;
     a.C.narrow = NARROW ? 1u : 0u;
     extern __shared__ __align__(16) char smem[];
     const JoinLds L(a.index_bits, a.slot_cap, NARROW, KK);
@@ -377,14 +395,13 @@ __global__ __launch_bounds__(JT_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
     volatile uint32_t* ctl = reinterpret_cast<volatile uint32_t*>(smem + L.ctl); // [0] tile, [1] columns
 
     const int tid = threadIdx.x, wave = (int)uniform(tid / WAVE), lane = lane_id();
-    constexpr int NW = JT_THREADS / WAVE;
     const uint32_t n_tiles = a.tile_off[a.n];
 
     if (tid == 0) { ctl[2] = 0; ctl[3] = 0; } // pairs and rows of this workgroup's tiles
     while (true) {
         __syncthreads();
         if (tid == 0) { ctl[0] = (uint32_t)atomicAdd(a.work, 1ull); ctl[1] = 0; }
-        for (uint32_t i = tid; i < JT_SEEN; i += JT_THREADS) seen[i] = EMPTY;
+        for (uint32_t i = tid; i < JT_SEEN; i += NT) seen[i] = EMPTY;
         __syncthreads();
         const uint32_t tile = uniform(ctl[0]);
         if (tile >= n_tiles) break;
@@ -440,8 +457,8 @@ __global__ __launch_bounds__(JT_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
             }
         }
         if ((uint32_t)tid < M) col_worst[tid] = a.symmetric ? a.dist[(size_t)col_id[tid] * KK + KK - 1] : -INF_DIS;
-        gram_rows_gather(a.C, row_id, R, rowptr, rownnz, tid, JT_THREADS);
-        gram_rows_gather(a.C, col_id, M, rowptr + JT_ROWS, rownnz + JT_ROWS, tid, JT_THREADS);
+        gram_rows_gather(a.C, row_id, R, rowptr, rownnz, tid, NT);
+        gram_rows_gather(a.C, col_id, M, rowptr + JT_ROWS, rownnz + JT_ROWS, tid, NT);
         __syncthreads();
         tile_hybrid_ips<NARROW>(a.C, a.dense_mul, smem + L.tab, T, a.index_bits, a.slot_cap, G, rowptr, rownnz, scan, R, M, a.work + 3, tid, wave, lane);
         if (KK == 128) { // the rows' own lists, behind the table (the bytes staged dense rows until now: all waves are past that)
@@ -464,7 +481,7 @@ __global__ __launch_bounds__(JT_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
             __syncthreads();
         }
         // proposals
-        for (uint32_t p = tid; p < R * M; p += JT_THREADS) {
+        for (uint32_t p = tid; p < R * M; p += NT) {
             const uint32_t r = p / M, c = p % M;
             const uint32_t uid = row_id[r], cid = col_id[c];
             if (uid == cid) continue;
@@ -637,7 +654,8 @@ struct GramTileArgs {
 };
 
 template <bool NARROW>
-__global__ __launch_bounds__(JT_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void gram_tile_kernel(GramTileArgs a) {
+__global__ __launch_bounds__(jt_threads(NARROW)) __attribute__((amdgpu_waves_per_eu(jt_threads(NARROW) / 256, jt_threads(NARROW) / 256))) void gram_tile_kernel(GramTileArgs a) {
+    constexpr int NT = jt_threads(NARROW);
     a.C.narrow = NARROW ? 1u : 0u;
     extern __shared__ __align__(16) char smem[];
     const JoinLds L(a.index_bits, a.slot_cap, NARROW);
@@ -681,11 +699,11 @@ __global__ __launch_bounds__(JT_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2
             if ((uint32_t)tid < R) row_id[tid] = valid[r0 + tid];
             if ((uint32_t)tid < M) col_id[tid] = valid[r0 + tid];
             __syncthreads();
-            gram_rows_gather(a.C, row_id, R, rowptr, rownnz, tid, JT_THREADS);
-            gram_rows_gather(a.C, col_id, M, rowptr + JT_ROWS, rownnz + JT_ROWS, tid, JT_THREADS);
+            gram_rows_gather(a.C, row_id, R, rowptr, rownnz, tid, NT);
+            gram_rows_gather(a.C, col_id, M, rowptr + JT_ROWS, rownnz + JT_ROWS, tid, NT);
             __syncthreads();
             tile_hybrid_ips<NARROW>(a.C, a.dense_mul, smem + L.tab, T, a.index_bits, a.slot_cap, G, rowptr, rownnz, scan, R, M, a.work + 3, tid, wave, lane);
-            for (uint32_t p = tid; p < R * M; p += JT_THREADS) {
+            for (uint32_t p = tid; p < R * M; p += NT) {
                 const uint32_t r = p / M, c = p % M;
                 out[(size_t)(r0 + r) * GT_MAX + r0 + c] = G[r * JT_STRIDE + c];
             }
@@ -774,9 +792,9 @@ int launch_nnd_join_iterate(apoe_knn* g) {
                        : (g->corpus->narrow ? &join_tile_kernel<true, 64> : &join_tile_kernel<false, 64>);
     APOE_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)L.total));
     int per_cu = 1;
-    APOE_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(kernel), JT_THREADS, L.total));
+    APOE_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(kernel), jt_threads(g->corpus->narrow), L.total));
     if (per_cu < 1) per_cu = 1;
-    kernel<<<(uint32_t)per_cu * (uint32_t)ctx->num_cus, JT_THREADS, L.total, st>>>(a);
+    kernel<<<(uint32_t)per_cu * (uint32_t)ctx->num_cus, jt_threads(g->corpus->narrow), L.total, st>>>(a);
     APOE_HIP(hipGetLastError());
     if (k128) join_apply_kernel<128><<<(n + 3) / 4, 256, 0, st>>>(n, g->ids.p, g->dist.p, g->prop.p, g->rev.p, g->rev_cnt.p, g->join_work.p + JOIN_COUNT_AT);
     else join_apply_kernel<64><<<(n + 3) / 4, 256, 0, st>>>(n, g->ids.p, g->dist.p, g->prop.p, g->rev.p, g->rev_cnt.p, g->join_work.p + JOIN_COUNT_AT);
@@ -815,9 +833,9 @@ int launch_gram_tiles(apoe_knn* g, uint32_t node0, uint32_t n_nodes, float* gram
     auto kernel = g->corpus->narrow ? &gram_tile_kernel<true> : &gram_tile_kernel<false>;
     APOE_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)L.total));
     int per_cu = 1;
-    APOE_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(kernel), JT_THREADS, L.total));
+    APOE_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(kernel), jt_threads(g->corpus->narrow), L.total));
     if (per_cu < 1) per_cu = 1;
-    kernel<<<(uint32_t)per_cu * (uint32_t)ctx->num_cus, JT_THREADS, L.total, st>>>(a);
+    kernel<<<(uint32_t)per_cu * (uint32_t)ctx->num_cus, jt_threads(g->corpus->narrow), L.total, st>>>(a);
     APOE_HIP(hipGetLastError());
     if (unfit) {
         unsigned long long h[4] = {0, 0, 0, 0};

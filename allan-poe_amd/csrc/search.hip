@@ -583,7 +583,7 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
                     }
                 }
             };
-            if (NW >= 8) { // one or two rows a wave at most expansions: a row that is not there would cost issue slots of a SIMD that four to six waves share
+            if (NW >= 4) { // a few rows a wave at most expansions: a row that is not there would cost issue slots of a SIMD that several waves share
                 for (uint32_t j = wave; j < n_new; j += NW * EVAL_BATCH) {
                     if (j + 2 * NW < n_new) eval_rows(std::integral_constant<int, 3>{}, j);
                     else if (j + NW < n_new) eval_rows(std::integral_constant<int, 2>{}, j);
