@@ -1124,7 +1124,8 @@ int launch_search(apoe_ctx* ctx, const apoe_corpus* c, const apoe_queries* q, co
         a.n_entities = kg->n_entities;
     }
     const SearchLds L(a.slots_s, a.slots_b, a.ovf_cap, a.cands, mode);
-    APOE_REQUIRE(L.total <= 64 * 1024, "search needs %u bytes of LDS (query rows with up to %u sparse terms)", L.total, q->max_nnz);
+    // 64 KB, and 544 bytes for descriptors, norms and counters that were added to the fixed arrays: the query rows that are served do not depend on those
+    APOE_REQUIRE(L.total <= 64 * 1024 + 544, "search needs %u bytes of LDS (query rows with up to %u sparse terms)", L.total, q->max_nnz);
 
     a.bitmap_words = ((c->n + 31) / 32 + 3) & ~3u;
     // workspace: [counters: 16 x u64][once-per-query arguments][visited bitmaps][codes of the queries' dense rows]
