@@ -14,7 +14,7 @@ constexpr int MAX_NEW = 64;   // fresh candidates per step: one lane each in wav
 constexpr int EVAL_BATCH = 3;  // candidates whose sparse parts a wave keeps in flight together
 constexpr int DENSE_BATCH = 1; // dense rows a wave keeps in flight together
 constexpr int MERGE_ROUNDS = 4; // 64-element rounds of the pool that the merge moves per LDS round trip
-constexpr int STATS = 10;     // counters of a launch; the workspace keeps 16 words for them
+constexpr int STATS = 9;      // counters of a launch; the workspace keeps 16 words for them
 constexpr int SKETCH_BATCH = 4; // sketches a wave keeps in flight together
 constexpr int RING = 32;      // keyword-filter search: evicted keyword hits kept beside the pool (query.cu:18)
 
@@ -48,8 +48,8 @@ struct SearchArgs {
     const uint4* sketch;   // null: the corpus has none
     uint32_t* codes;       // of the query's dense row, 1 KB per workgroup: in device memory (it is read beside sketches, which take longer), since a
                            // kilobyte of LDS more costs long batches a resident query per CU (12 -> 11: 3 %)
-    unsigned long long* work; // [0] next query, [1] expansions, [2] evaluations, [3] nnz splade, [4] nnz bm25, [5] evaluations that pairs and norms did not settle,
-                              // [6] pool entries evaluated again in fp32, [7] their pairs, [8] sketches read, [9] dense rows (fp32 or half) read in the walk
+    unsigned long long* work; // [0] next query, [1] expansions, [2] evaluations, [3] nnz splade, [4] nnz bm25, [5] dense rows (fp32 or half) read in the walk,
+                              // [6] pool entries evaluated again in fp32, [7] their pairs, [8] sketches read
     uint32_t full_eval;       // 1: read the dense row of every candidate (no bound test)
     const uint16_t* half;     // not null: the walk takes dense parts from the half-precision rows, the final pool is evaluated again in fp32
     uint32_t slots_s, slots_b, ovf_cap; // buckets of the query's SPLADE / BM25 term table, entries of the overflow list
@@ -70,7 +70,7 @@ struct SearchLds {
         qd = o; o += DENSE_BYTES;       // the query's dense row, weight applied
         ctl = o; o += 16 * 4;
         qs = o; o += 4 * 4;             // scale and error of the codes of the query's dense row
-        stat = o; o += STATS * 8;       // the workgroup's counters (work[1..]), sent once when it leaves
+        stat = o; o += (STATS + 1) / 2 * 16; // the workgroup's counters (work[1..]), sent once when it leaves; `part` is read 16 bytes at a time
         part = o; o += MAX_NEW * 16;    // sparse sum of a fresh candidate as four partial sums (one per 16 lanes)
         new_desc = o; o += MAX_NEW * 8; // descriptors and dense norms of the fresh candidates
         new_dn = o; o += MAX_NEW * 4;
@@ -412,7 +412,7 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
         }
         if (tid == 0) { qs[0] = q_scale; qs[1] = q_err; }
         const bool sketched = __builtin_amdgcn_readfirstlane((int)(q_scale > 0.f)) != 0;
-        uint32_t st_exp = 0, st_eval = 0, st_dense = 0, st_again = 0, st_again_pairs = 0, st_sketch = 0, st_rows = 0; // wave-uniform counters of one query
+        uint32_t st_exp = 0, st_eval = 0, st_dense = 0, st_again = 0, st_again_pairs = 0, st_sketch = 0; // wave-uniform counters of one query
         uint32_t ln_s = 0, ln_b = 0;                    // pairs read for the candidates this lane decided
         Front front; // wave 0: the first unexplored pool entry
         front.id = EMPTY;
@@ -495,7 +495,6 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
                     dense_issue(row, ri.rec);
                     dist = 1.0f - (dense_finish_lds(row, qd, 1.0f) + ssum) - bonus;
                     st_dense++;
-                    st_rows++;
                 }
                 st_eval++;
                 if (lane == 0) {
@@ -630,7 +629,6 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
                 st_eval += __popcll(__ballot(mine));
                 need = __ballot(undecided);
                 asked = __ballot(undecided && wide);
-                st_dense += __popcll(need);
             }
             wave_fence();
             // stage 2: the sketches of the survivors, SKETCH_BATCH in flight, then the same decision with the tighter bound
@@ -682,7 +680,7 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
                 need &= ~__ballot(far);
                 wave_fence();
             }
-            st_rows += __popcll(need);
+            st_dense += __popcll(need);
             // stage 3: the dense rows of the survivors, DENSE_BATCH rows in flight (two of the half-precision rows)
             while (HALF && need) {
                 DenseRowHalf row[2];
@@ -981,7 +979,6 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
             if (st_again) atomicAdd(stat + 6, (unsigned long long)st_again);
             if (st_again_pairs) atomicAdd(stat + 7, (unsigned long long)st_again_pairs);
             if (st_sketch) atomicAdd(stat + 8, (unsigned long long)st_sketch);
-            if (st_rows) atomicAdd(stat + 9, (unsigned long long)st_rows);
         }
     }
     __syncthreads();
@@ -1202,7 +1199,7 @@ int launch_search(apoe_ctx* ctx, const apoe_corpus* c, const apoe_queries* q, co
         stats->nnz_bm25 = h[4];
         stats->dense_rows = h[5];
         // dense rows and sketches actually needed (a sketch with its scale and error) + pairs + descriptor and dense norm (12 B per evaluation)
-        uint64_t bytes = h[9] * (uint64_t)(a.half ? DENSE_BYTES / 2 : DENSE_BYTES) + h[8] * (uint64_t)(SKETCH_BYTES + sizeof(SketchMeta));
+        uint64_t bytes = h[5] * (uint64_t)(a.half ? DENSE_BYTES / 2 : DENSE_BYTES) + h[8] * (uint64_t)(SKETCH_BYTES + sizeof(SketchMeta));
         bytes += (c->narrow ? 6 : 8) * (h[3] + h[4]) + 12 * h[2];
         bytes += h[6] * (uint64_t)(DENSE_BYTES + 8) + (c->narrow ? 6 : 8) * h[7]; // the pool evaluated again in fp32
         bytes += h[1] * 4ull * a.W;

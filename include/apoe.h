@@ -213,7 +213,9 @@ typedef struct {
                                         0x100: read the dense row of every candidate; by
                                         default a candidate whose sparse part plus the Cauchy-Schwarz
                                         bound of its dense part cannot beat the worst entry of the full
-                                        pool is dropped without reading its dense row (same results).
+                                        pool is dropped without reading its dense row, and so is one whose
+                                        dense part is bounded tightly enough by the 8-bit sketch of its row
+                                        (same results).
                                         0x200: while the graph is walked, the dense part of a candidate is
                                         taken from the half-precision copy of the rows (needs
                                         apoe_corpus_make_half_rows; plain search only); when the walk has
@@ -232,8 +234,8 @@ typedef struct {
     uint64_t evaluations; /* hybrid distance evaluations */
     uint64_t nnz_sparse;  /* SPLADE pairs read by those evaluations (0 if path off) */
     uint64_t nnz_bm25;    /* BM25 pairs read by those evaluations (0 if path off) */
-    uint64_t dense_rows;  /* evaluations that pairs and norms did not settle (see variant): they read the dense
-                             row, or its 1 KB sketch first and the row if that does not settle them either */
+    uint64_t dense_rows;  /* evaluations that read the dense row (4 KB, or 2 KB with variant 0x200): neither pairs
+                             and norms nor the 1 KB sketch settled them (see variant) */
     uint64_t algo_bytes;  /* algorithmic HBM bytes: dense rows and sketches read + pairs + descriptors +
                              graph rows + queries + results */
 } apoe_search_stats;
