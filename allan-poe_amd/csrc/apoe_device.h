@@ -399,6 +399,8 @@ __device__ __forceinline__ void query_tabs_clear(const QueryTabs& T, int tid, in
 template <bool NARROW, bool KWD>
 __device__ __forceinline__ void query_tabs_insert(const QueryTabs& T, uint32_t key, float val, bool required) {
     const uint32_t term = key & ~BM25_BIT;
+    // no document holds the id of all 31 bits (the corpus refuses it), and with bit 31 it would read as an empty slot: two terms would share one
+    if (term == ~BM25_BIT) return;
     const uint32_t raw = KWD ? term | (required ? BM25_BIT : 0u) : NARROW ? term : key;
     const uint32_t h = query_hash<NARROW>(term);
     uint4* e = T.b + ((key & BM25_BIT) ? T.mask_s + 1 + (h & T.mask_b) : (h & T.mask_s));

@@ -62,3 +62,36 @@ def test_flags_of_overflow_entries(gpu_ctx, wide, n_flagged):
     assert np.array_equal(ids, oid)
     assert_dist_close(dist, odist, "hits and the empty rest")
     assert set(ids[0][ids[0] != EMPTY_ID].tolist()) == {v for v in range(n) if flags[v % nt]}
+
+
+@pytest.mark.parametrize("wide", [False, True])
+@pytest.mark.parametrize("keyword_filter", [False, True])
+def test_query_terms_that_no_document_can_hold(gpu_ctx, wide, keyword_filter):
+    """The BM25 id 0xFFFFFFFF (0x7FFFFFFF flagged as required) is no document's and reads as an empty table slot. Queries of 192 terms,
+    64 of them that id, the terms that share its bucket handled by other waves: the rows are those of the queries without it."""
+    import apoe
+    n, d, nq, nt = 64, 16, 2000, 192
+    rng = np.random.default_rng(11)
+    k = np.uint64(0x7FFFFFFF)
+    t = np.arange(70000, 200000, dtype=np.uint64) if wide else np.arange(1, 65536, dtype=np.uint64)
+    low = (lambda x: (x ^ (x >> np.uint64(16))) & np.uint64(0xFFFFFF)) if wide else (lambda x: x & np.uint64(0xFFFFFF))
+    bucket = lambda x: (((low(x) * np.uint64(0x9E3779)) & np.uint64(0xFFFFFFFF)) >> np.uint64(10)) % np.uint64(512) # next power of two above 2 * 192 terms
+    same, other = t[bucket(t) == bucket(k)].astype(np.uint32), t[bucket(t) != bucket(k)].astype(np.uint32)
+    terms = np.concatenate([np.full(64, 0xFFFFFFFF, np.uint32), same[:1], other[:63], same[1:2], other[63:126]])
+    dense = rng.standard_normal((n, 1024)).astype(np.float32)
+    none = lambda m: (np.zeros(m + 1, np.uint32), np.zeros(0, np.uint32), np.zeros(0, np.float32))
+    corpus = (dense, *none(n), np.arange(0, 2 * n + 1, 2, dtype=np.uint32), np.tile(same[:2], n), rng.random(2 * n).astype(np.float32) + 1)
+    rows = np.zeros((n, d + 8), np.uint32)
+    rows[:, :d] = (np.arange(n)[:, None] + np.arange(1, d + 1)) % n
+    gc, gg = apoe.Corpus(gpu_ctx, *corpus), apoe.Graph(gpu_ctx, rows, np.arange(d, dtype=np.uint32))
+    assert gc.pair_bytes() == (8 if wide else 6)
+    q = rng.standard_normal((nq, 1024)).astype(np.float32)
+    val = rng.random((nq, nt)).astype(np.float32) + 1
+    flag = np.uint32(KW if keyword_filter else 0)
+    off = lambda m: np.arange(0, m * nq + 1, m, dtype=np.uint32)
+    with_it = apoe.Queries(gpu_ctx, q, *none(nq), off(nt), np.tile(terms | flag, nq), val.reshape(-1))
+    without = apoe.Queries(gpu_ctx, q, *none(nq), off(nt - 64), np.tile(terms[64:] | flag, nq), np.ascontiguousarray(val[:, 64:]).reshape(-1))
+    for variant in (1, 4, 2, 5):
+        a, ad, _ = apoe.search(gpu_ctx, gc, with_it, gg, (0, 0, 1), 40, keyword_filter=keyword_filter, variant=variant)
+        b, bd, _ = apoe.search(gpu_ctx, gc, without, gg, (0, 0, 1), 40, keyword_filter=keyword_filter, variant=variant)
+        assert np.array_equal(a, b) and np.array_equal(ad, bd), (variant, int((a != b).any(axis=1).sum()))
