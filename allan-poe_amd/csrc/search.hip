@@ -61,7 +61,7 @@ struct SearchArgs {
 
 // LDS carve-up shared by host (size) and device (pointers).
 struct SearchLds {
-    uint32_t qd, qs, stat, part, tab, ovf, pool_id, pool_dist, pool_ent, pool_hop, new_desc, new_dn, new_id, new_dist, new_ent, new_hop, seed_id, seed_ent, seed_dist, link, ring_id,
+    uint32_t qd, qs, stat, part, tab, ovf, pool_id, pool_dist, pool_ent, pool_hop, new_id, new_dist, new_ent, new_hop, seed_id, seed_ent, seed_dist, link, ring_id,
         ring_dist, ctl, total;
     __host__ __device__ SearchLds(uint32_t slots_s, uint32_t slots_b, uint32_t ovf_cap, uint32_t cands, int mode) {
         const bool kg = mode == MODE_KG, kwd = mode == MODE_KEYWORD;
@@ -71,9 +71,8 @@ struct SearchLds {
         ctl = o; o += 16 * 4;
         qs = o; o += 4 * 4;             // scale and error of the codes of the query's dense row
         stat = o; o += (STATS + 1) / 2 * 16; // the workgroup's counters (work[1..]), sent once when it leaves; `part` is read 16 bytes at a time
-        part = o; o += MAX_NEW * 16;    // sparse sum of a fresh candidate as four partial sums (one per 16 lanes)
-        new_desc = o; o += MAX_NEW * 8; // descriptors and dense norms of the fresh candidates
-        new_dn = o; o += MAX_NEW * 4;
+        part = o; o += MAX_NEW * 16;    // of a fresh candidate: descriptor and dense norm until its wave takes them up, then its sparse sum as four
+                                        // partial sums (one per 16 lanes)
         new_id = o; o += MAX_NEW * 4;
         new_dist = o; o += MAX_NEW * 4;
         new_ent = o; o += kg || kwd ? MAX_NEW * 4 : 0; // KG: linking entity; keyword search: the hit flag of a fresh candidate
@@ -336,8 +335,9 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
     P.ent = reinterpret_cast<uint32_t*>(smem + L.pool_ent);
     P.hop = reinterpret_cast<uint32_t*>(smem + L.pool_hop);
     P.cands = a.cands;
-    uint64_t* new_desc = reinterpret_cast<uint64_t*>(smem + L.new_desc);
-    float* new_dn = reinterpret_cast<float*>(smem + L.new_dn);
+    auto put_desc = [&](uint32_t pos, uint64_t desc, float dn) { // before the barrier in front of the evaluations
+        reinterpret_cast<float4*>(part)[pos] = make_float4(__uint_as_float((uint32_t)desc), __uint_as_float((uint32_t)(desc >> 32)), dn, 0.f);
+    };
     uint32_t* codes = a.codes + (size_t)blockIdx.x * (SKETCH_BYTES / 4);
     volatile float* qs = reinterpret_cast<volatile float*>(smem + L.qs);
     uint32_t* new_id = reinterpret_cast<uint32_t*>(smem + L.new_id);
@@ -433,8 +433,7 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
                 if (fresh) {
                     const uint32_t pos = __popcll(b & lane_lt);
                     new_id[pos] = c;
-                    new_desc[pos] = a.C.desc[c];
-                    new_dn[pos] = a.C.dnorm[c];
+                    put_desc(pos, a.C.desc[c], a.C.dnorm[c]);
                 }
                 if (lane == 0) { ctl[CTL_NNEW] = __popcll(b); ctl[CTL_PARENT] = 0; }
             }
@@ -543,8 +542,15 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
             const float thr_eff = thr < INF_DIS ? thr : __builtin_inff();
             const float span = sketched ? thr_eff - P.dist[0] : __builtin_inff(); // of the pool
             const uint32_t n_ovf = uniform(ctl[CTL_NOVF]);
-            // descriptors of all fresh candidates: lane l holds candidate l's
-            const uint64_t my_desc = (uint32_t)lane < n_new ? new_desc[lane] : 0;
+            // descriptors and dense norms of this wave's candidates: lane l holds candidate l's
+            const bool mine = (uint32_t)lane < n_new && (uint32_t)(lane & (NW - 1)) == (uint32_t)wave;
+            uint64_t my_desc = 0;
+            float my_dn = 0.f;
+            if (mine) { // no other wave touches the slot from here to the barrier behind the evaluations
+                const float4 s4 = reinterpret_cast<const float4*>(part)[lane];
+                my_desc = (uint64_t)__float_as_uint(s4.y) << 32 | __float_as_uint(s4.x);
+                my_dn = s4.z;
+            }
             if (wave == 0 && front.id != EMPTY) {
                 GlobalWord* row = graph_row(a, KWD ? front.id & ID_MASK : front.id);
                 g_c = lane < (int)a.degree ? row[lane] : EMPTY;
@@ -596,7 +602,6 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
             // sparse part plus the bound of its dense part cannot reach the pool is reported as INF_DIS
             uint64_t need, asked; // bit l: candidate l still needs its dense row; its sketch comes first
             {
-                const bool mine = (uint32_t)lane < n_new && (uint32_t)(lane & (NW - 1)) == (uint32_t)wave;
                 bool undecided = false, wide = false;
                 if (mine) {
                     float bonus = 0.f;
@@ -604,7 +609,7 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
                         if (new_ent[lane] != EMPTY) bonus = a.kg_weight / (float)new_hop[lane]; // query.cu:1759-1760
                     }
                     float ssum = 0.f, v = 0.f;
-                    const float dub = pv_norm * new_dn[lane]; // |<query_d, doc_d>| <= |query_d| * |doc_d|
+                    const float dub = pv_norm * my_dn; // |<query_d, doc_d>| <= |query_d| * |doc_d|
                     undecided = true;
                     wide = dub > span;
                     if (a.paths & (PATH_SPARSE | PATH_BM25)) {
@@ -670,9 +675,9 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
                     if (KG) {
                         if (new_ent[lane] != EMPTY) bonus = a.kg_weight / (float)new_hop[lane];
                     }
-                    const float dn = new_dn[lane], ssum = new_dist[lane], dub = pv_norm * dn;
-                    float most = part[lane * 4] * (qs[0] * sm.scale) + pv_norm * sm.err + qs[1] * (dn + sm.err);
-                    if (HALF) most += pv_norm * (4.9e-4f * dn + 1.1e-6f); // the walk's rows are rounded to half precision
+                    const float ssum = new_dist[lane], dub = pv_norm * my_dn;
+                    float most = part[lane * 4] * (qs[0] * sm.scale) + pv_norm * sm.err + qs[1] * (my_dn + sm.err);
+                    if (HALF) most += pv_norm * (4.9e-4f * my_dn + 1.1e-6f); // the walk's rows are rounded to half precision
                     const float lb = 1.0f - (ssum + most) - bonus;
                     far = lb > thr_eff + 1e-5f * (fabsf(ssum) + dub + fabsf(bonus) + 1.0f);
                     if (far) new_dist[lane] = INF_DIS;
@@ -867,8 +872,7 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
                             g_desc = a.C.desc[c];
                             g_dn = a.C.dnorm[c];
                         }
-                        new_desc[pos] = g_desc;
-                        new_dn[pos] = g_dn;
+                        put_desc(pos, g_desc, g_dn);
                         if (KG) { new_ent[pos] = ent; new_hop[pos] = p_hop + 1; }
                     }
                     n_next = __popcll(b);
@@ -1121,8 +1125,8 @@ int launch_search(apoe_ctx* ctx, const apoe_corpus* c, const apoe_queries* q, co
         a.n_entities = kg->n_entities;
     }
     const SearchLds L(a.slots_s, a.slots_b, a.ovf_cap, a.cands, mode);
-    // 64 KB, and 544 bytes for descriptors, norms and counters that were added to the fixed arrays: the query rows that are served do not depend on those
-    APOE_REQUIRE(L.total <= 64 * 1024 + 544, "search needs %u bytes of LDS (query rows with up to %u sparse terms)", L.total, q->max_nnz);
+    // 64 KB; the fixed arrays were 224 bytes longer when that line was drawn, and the query rows that are served do not depend on their length
+    APOE_REQUIRE(L.total <= 64 * 1024 - 224, "search needs %u bytes of LDS (query rows with up to %u sparse terms)", L.total, q->max_nnz);
 
     a.bitmap_words = ((c->n + 31) / 32 + 3) & ~3u;
     // workspace: [counters: 16 x u64][once-per-query arguments][visited bitmaps][codes of the queries' dense rows]
@@ -1141,10 +1145,12 @@ int launch_search(apoe_ctx* ctx, const apoe_corpus* c, const apoe_queries* q, co
     //    they fit (1 536), e.g. 100 queries at cands 256 in 2.4 instead of 7.9 ms, 1 024 in 5.6 instead of 8.8 ms; four also for batches of up to two rounds of the two-wave
     //    grid (6 144 queries), whose second round ends sooner that way (4-9 % at 4 096 to 6 144 queries, cands 64-512);
     //  * a longer batch is bound by the memory system and runs best with two waves per query and as many queries as fit
-    //    (12 per CU) - unless the pool is so large that LDS leaves room for at most 8 queries on a CU: then four waves
-    //    per query keep twice the loads in flight (1 M docs: 167 against 191 ms at cands 1500, 234 against 290 ms at
-    //    2048, the same at 1024, where 9 queries fit; knowledge-graph search: 66 against 77 ms at cands 512, 150
-    //    against 195 ms at 1024; the keyword search measures the same or worse with four and stays at two).
+    //    (12 per CU) - unless the pool is so large that LDS leaves room for at most 9 queries on a CU: then four waves
+    //    per query keep twice the loads in flight (10 000 queries, 1 M docs, four against two waves: 98.0 against 105.6 ms
+    //    at cands 1024, where 9 queries fit, 185.6 against 248.7 at 2048; knowledge-graph search: 32.8 against 34.6 ms at
+    //    cands 256, where 9 fit, 25.9 against 25.5 at 192, where 10 fit, 129.7 against 184.5 at 1024; the keyword search
+    //    measures the same or worse with four up to cands 768 and stays at two). Plain searches where 10 to 12 queries fit
+    //    measure 1 to 7 % less with four waves as well; the line is one for both modes.
     int nw = 2;
     const uint32_t shape = p->variant & 0xFFu;
     if (shape == 1) nw = 1;
@@ -1169,7 +1175,7 @@ int launch_search(apoe_ctx* ctx, const apoe_corpus* c, const apoe_queries* q, co
         if (at_once <= (size_t)pc16 * ctx->num_cus) { nw = 16; per_cu = pc16; }
         else if (at_once <= (size_t)pc8 * ctx->num_cus) { nw = 8; per_cu = pc8; }
         else if (at_once <= (size_t)pc4 * ctx->num_cus || at_once <= 2 * (size_t)per_cu * ctx->num_cus) { nw = 4; per_cu = pc4; }
-        else if (per_cu <= 8 && mode != MODE_KEYWORD && pc4 * 4 > per_cu * 2) { nw = 4; per_cu = pc4; }
+        else if (per_cu <= 9 && mode != MODE_KEYWORD && pc4 * 4 > per_cu * 2) { nw = 4; per_cu = pc4; }
     } else {
         APOE_TRY(resident_per_cu(nw, &per_cu));
     }

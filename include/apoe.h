@@ -207,7 +207,7 @@ typedef struct {
     uint32_t variant;                /* low byte: launch shape = waves per query. 0 = default: 16 while every query
                                         has a CU of its own, 8 while the whole batch is resident at once that way,
                                         else 4 up to two rounds of the 2-wave grid (about 6 000 queries), else 2 -
-                                        or 4 when the pool is so large that fewer than 9 queries fit a CU (plain
+                                        or 4 when the pool is so large that fewer than 10 queries fit a CU (plain
                                         and KG search). 1/2/3/4/5 = 1/4/8/2/16 waves whatever the batch; other
                                         values are refused. Rows do not depend on it.
                                         0x100: read the dense row of every candidate; by

@@ -120,3 +120,29 @@ def test_large_pool_picks_its_shape_and_unknown_shapes_are_refused(gpu_world):
     assert a[2].evaluations == b[2].evaluations
     with pytest.raises(RuntimeError, match="launch shape"):
         apoe.search(w["ctx"], w["gc"], w["gq"], w["gg"], (1.0, 1.0, 1.0), 32, variant=9)
+
+
+def test_lds_of_a_query_and_the_longest_rows_that_are_served(gpu_ctx):
+    """Query rows of 64 SPLADE and 1 024 BM25 terms (term tables of 128 and 2 048 buckets, 1 088 overflow entries) are served up to
+    cands 2 000. What a query needs there decides how many are resident on a CU: 49 536 bytes and eight a pool entry is the
+    carve-up that the launch shapes were measured with."""
+    import re
+    import apoe
+    import oracle as O
+    n, d, nq = 80, 16, 3
+    rng = np.random.default_rng(5)
+    dense = rng.standard_normal((n, 1024)).astype(np.float32)
+    off = lambda m, k: np.arange(0, m * k + 1, k, dtype=np.uint32)
+    pairs = lambda m, k: (off(m, k), np.tile(np.arange(k, dtype=np.uint32) * 3 + 1, m), rng.random(m * k).astype(np.float32))
+    corpus = (dense, *pairs(n, 5), *pairs(n, 9))
+    queries = (dense[:nq] + 1, *pairs(nq, 64), *pairs(nq, 1024))
+    rows = np.zeros((n, d + 8), np.uint32)
+    rows[:, :d] = (np.arange(n)[:, None] + np.arange(1, d + 1)) % n
+    entry = np.arange(d, dtype=np.uint32)
+    gc, gq, gg = apoe.Corpus(gpu_ctx, *corpus), apoe.Queries(gpu_ctx, *queries), apoe.Graph(gpu_ctx, rows, entry)
+    ids, dist, _ = apoe.search(gpu_ctx, gc, gq, gg, (1, 1, 1), 2000)
+    oid, odist, _ = O.search(O.HybridSet(*corpus), O.HybridSet(*queries), rows, entry, (1, 1, 1), 2000)
+    assert_topk_match(ids, dist, oid, odist, 10, "long query rows, cands 2000")
+    with pytest.raises(apoe.ApoeError, match="bytes of LDS") as e:
+        apoe.search(gpu_ctx, gc, gq, gg, (1, 1, 1), 2001)
+    assert int(re.search(r"needs (\d+) bytes", str(e.value)).group(1)) <= 49536 + 8 * 2001
