@@ -316,6 +316,9 @@ __device__ __forceinline__ GlobalWord* graph_row(const SearchArgs& a, uint32_t i
 template <int NW, int MODE, bool NARROW, bool HALF>
 __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE == MODE_PLAIN && !HALF ? APOE_SEARCH_WAVES_PER_EU : 5, 8))) void search_kernel(SearchArgs a) {
     constexpr bool KG = MODE == MODE_KG, KWD = MODE == MODE_KEYWORD;
+    // Whether wave 0 asks for more than the walk may need (graph row of the first unexplored entry, descriptors of visited neighbours) to
+    // have it early: one query's chain gains, a long batch, whose other queries cover the wait, pays in traffic (figures where the walk starts).
+    constexpr bool AHEAD = NW >= 4;
     a.C.narrow = NARROW ? 1u : 0u; // the pair format as a compile-time constant: no branch at the loads
     extern __shared__ __align__(16) char smem[];
     const SearchLds L(a.slots_s, a.slots_b, a.ovf_cap, a.cands, MODE);
@@ -433,7 +436,7 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
                 if (fresh) {
                     const uint32_t pos = __popcll(b & lane_lt);
                     new_id[pos] = c;
-                    put_desc(pos, a.C.desc[c], a.C.dnorm[c]);
+                    if (AHEAD) put_desc(pos, a.C.desc[c], a.C.dnorm[c]);
                 }
                 if (lane == 0) { ctl[CTL_NNEW] = __popcll(b); ctl[CTL_PARENT] = 0; }
             }
@@ -525,12 +528,15 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
         }
 
         // The next parent is the first unexplored pool entry or a new candidate that goes before it, so it is known BEFORE
-        // the merge: wave 0 starts the parent's three dependent reads (graph row, visited words, descriptors) first and
-        // merges while they are under way; the row of the first unexplored entry is requested while the candidates are
+        // the merge: wave 0 starts the parent's dependent reads (graph row, visited words and, AHEAD, the descriptors) first and
+        // merges while they are under way; AHEAD, the row of the first unexplored entry is requested while the candidates are
         // evaluated. At one query per compute unit the three reads were
         // 2 000 cycles of an iteration after the merge; of them 150 to 280 are left behind it. (Looking one whole expansion ahead,
         // with the visited marks taken back when a candidate overtakes: it is right for 0.55 to 0.64 of the expansions only, and
         // the marks and rows of the others cost long batches 5 %.)
+        // One and two waves per query are for long batches: a row that is overtaken and the descriptors of visited neighbours are
+        // traffic there, and nothing waits for them (10 000 queries, 1 M docs, cands 256 / 512: 1.921e11 -> 1.877e11 bytes and
+        // 30.4 -> 30.1 ms / 55.1 -> 54.3 ms without them).
         uint32_t g_c = EMPTY, g_kw = 0; // lane l: neighbour of `front`, later of the parent; (keyword search) word l of the row's tail
         for (uint32_t it = 0; it <= a.max_iter; it++) {
             // ---- evaluate the fresh candidates: one wave per candidate ----
@@ -546,12 +552,18 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
             const bool mine = (uint32_t)lane < n_new && (uint32_t)(lane & (NW - 1)) == (uint32_t)wave;
             uint64_t my_desc = 0;
             float my_dn = 0.f;
-            if (mine) { // no other wave touches the slot from here to the barrier behind the evaluations
-                const float4 s4 = reinterpret_cast<const float4*>(part)[lane];
-                my_desc = (uint64_t)__float_as_uint(s4.y) << 32 | __float_as_uint(s4.x);
-                my_dn = s4.z;
+            if (mine) {
+                if (AHEAD) { // no other wave touches the slot from here to the barrier behind the evaluations
+                    const float4 s4 = reinterpret_cast<const float4*>(part)[lane];
+                    my_desc = (uint64_t)__float_as_uint(s4.y) << 32 | __float_as_uint(s4.x);
+                    my_dn = s4.z;
+                } else {
+                    const uint32_t cid = new_id[lane];
+                    my_desc = a.C.desc[cid];
+                    my_dn = a.C.dnorm[cid];
+                }
             }
-            if (wave == 0 && front.id != EMPTY) {
+            if (AHEAD && wave == 0 && front.id != EMPTY) {
                 GlobalWord* row = graph_row(a, KWD ? front.id & ID_MASK : front.id);
                 g_c = lane < (int)a.degree ? row[lane] : EMPTY;
                 if (KWD) g_kw = lane < APOE_KW_SLOTS ? row[a.degree + lane] : 0u;
@@ -749,7 +761,7 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
                     }
                     if (KWD && parent != EMPTY) parent &= ID_MASK;
                 }
-                if (parent != EMPTY && overtaken) {
+                if (parent != EMPTY && (overtaken || !AHEAD)) {
                     GlobalWord* row = graph_row(a, parent);
                     g_c = lane < (int)a.degree ? row[lane] : EMPTY;
                     if (KWD) g_kw = lane < APOE_KW_SLOTS ? row[a.degree + lane] : 0u;
@@ -761,8 +773,10 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
                 if (parent != EMPTY && g_c < a.C.n) {
                     const uint32_t bit = 1u << (g_c & 31);
                     fresh = !(atomicOr(&bitmap[g_c >> 5], bit) & bit);
-                    g_desc = a.C.desc[g_c];
-                    g_dn = a.C.dnorm[g_c];
+                    if (AHEAD) {
+                        g_desc = a.C.desc[g_c];
+                        g_dn = a.C.dnorm[g_c];
+                    }
                 }
                 const uint32_t lowest = sort_merge<MODE>(P, F, R);
                 if (parent != EMPTY) {
@@ -868,11 +882,11 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
                     if (alive) {
                         const uint32_t pos = __popcll(b & lane_lt);
                         new_id[pos] = c;
-                        if ((KG || KWD) && !fresh) { // not a graph neighbour: recycled through a keyword or logical edge
+                        if (AHEAD && (KG || KWD) && !fresh) { // not a graph neighbour: recycled through a keyword or logical edge
                             g_desc = a.C.desc[c];
                             g_dn = a.C.dnorm[c];
                         }
-                        put_desc(pos, g_desc, g_dn);
+                        if (AHEAD) put_desc(pos, g_desc, g_dn);
                         if (KG) { new_ent[pos] = ent; new_hop[pos] = p_hop + 1; }
                     }
                     n_next = __popcll(b);
