@@ -1010,11 +1010,13 @@ __global__ void search_setup_kernel(unsigned long long* work, SearchCold* dst, S
     if (threadIdx.x == 0) *dst = cold;
 }
 
-// Workspace of apoe_search_noalloc: counters, once-per-query arguments, the visited bitmaps and query codes of as many
-// workgroups as fit. One copy per GPU, held until the process ends; every call on a GPU uses it, so calls
+// Workspace of apoe_search_noalloc: counters, once-per-query arguments and the visited bitmaps of as many workgroups as fit
+// APOE_NOALLOC_WS_BYTES; behind them the query codes of as many workgroups as a GPU of 256 CUs holds (32 waves a CU), so that
+// the codes take no bitmap's place. One copy per GPU, held until the process ends; every call on a GPU uses it, so calls
 // that overlap on one GPU race. Host code never uses the array's name as an address: the device address is
 // asked for once per device (search_static_workspace) and kept.
-static __device__ __align__(256) unsigned char search_scratch[APOE_NOALLOC_WS_BYTES];
+constexpr uint32_t NOALLOC_CODES = 256 * 32;
+static __device__ __align__(256) unsigned char search_scratch[APOE_NOALLOC_WS_BYTES + NOALLOC_CODES * SKETCH_BYTES];
 
 constexpr int MAX_DEVICES = 64;
 static std::mutex scratch_mutex;
@@ -1148,7 +1150,7 @@ int launch_search(apoe_ctx* ctx, const apoe_corpus* c, const apoe_queries* q, co
     const size_t bitmap_bytes = (size_t)a.bitmap_words * sizeof(uint32_t);
     size_t fit = SIZE_MAX; // workgroups whose visited bitmaps fit the workspace
     if (static_ws) {
-        fit = (APOE_NOALLOC_WS_BYTES - bitmaps_at) / (bitmap_bytes + SKETCH_BYTES);
+        fit = std::min<size_t>((APOE_NOALLOC_WS_BYTES - bitmaps_at) / bitmap_bytes, NOALLOC_CODES);
         APOE_REQUIRE(fit >= 1, "the static workspace of %u bytes holds no visited bitmap of %zu bytes", (unsigned)APOE_NOALLOC_WS_BYTES, bitmap_bytes);
     }
 
@@ -1202,7 +1204,7 @@ int launch_search(apoe_ctx* ctx, const apoe_corpus* c, const apoe_queries* q, co
     APOE_HIP(hipGetLastError());
     a.cold = reinterpret_cast<const SearchCold*>(ws + cold_at);
     a.bitmaps = reinterpret_cast<uint32_t*>(ws + bitmaps_at);
-    a.codes = reinterpret_cast<uint32_t*>(ws + bitmaps_at + (size_t)grid * bitmap_bytes);
+    a.codes = reinterpret_cast<uint32_t*>(static_ws ? static_ws + APOE_NOALLOC_WS_BYTES : ws + bitmaps_at + (size_t)grid * bitmap_bytes);
     a.work = work;
 
     if (static_ws && !stats) return launch_mode(ctx, mode, nw, a, grid, L.total, nullptr);

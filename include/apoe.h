@@ -262,8 +262,8 @@ int apoe_search(apoe_ctx* ctx, const apoe_corpus* c, const apoe_queries* q, cons
  * Same kernels, arguments and results as apoe_search, except that
  *  - out_ids / out_dist must be device memory of the context's GPU (results are written in place);
  *  - the counters, the once-per-query arguments and the visited bitmaps live in one static device array of
- *    APOE_NOALLOC_WS_BYTES that each GPU holds from the first apoe_ctx_create on it until the process
- *    ends; the launch uses as many workgroups as bitmaps of n bits fit there (255 at 1 M documents), so a
+ *    APOE_NOALLOC_WS_BYTES (and 8 MiB more for the 8-bit codes of the running queries) that each GPU holds from
+ *    the first apoe_ctx_create on it until the process ends; the launch uses as many workgroups as bitmaps of n bits fit there (255 at 1 M documents), so a
  *    large batch runs slower than through apoe_search; corpora above APOE_NOALLOC_MAX_DOCS are refused;
  *  - with stats == NULL the call returns with the search still running on the context's stream
  *    (apoe_ctx_synchronize waits for it); with stats it blocks like apoe_search;

@@ -83,3 +83,24 @@ def test_noalloc_refuses_a_query_range_that_wraps(world):
     st = apoe.lib().apoe_search_noalloc(w["ctx"].h, w["gc"].h, w["gq"].h, w["gg"].h, C.c_void_p(0), C.byref(p), C.c_void_p(out_ids.data_ptr()),
                                         C.c_void_p(out_dist.data_ptr()), C.c_void_p(0))
     assert st == -1 and b"beyond" in apoe.lib().apoe_last_error_string()
+
+
+@pytest.mark.parametrize("variant", [1, 4, 5])
+def test_noalloc_with_every_workgroup_the_gpu_holds(world, variant):
+    """5 000 queries (up to 4 096 of them resident) under weights that ask the sketch: every workgroup's codes have a place of their
+    own behind the visited bitmaps, and none takes another's."""
+    import torch
+    import apoe
+    w = world
+    dense, s_off, s_idx, s_val, b_off, b_idx, b_val = w["queries"]
+    m = 25
+    tile_off = lambda o: np.concatenate([[0], np.tile(np.diff(o), m).cumsum()]).astype(np.uint32)
+    gq = apoe.Queries(w["ctx"], np.tile(dense, (m, 1)), tile_off(s_off), np.tile(s_idx, m), np.tile(s_val, m), tile_off(b_off), np.tile(b_idx, m), np.tile(b_val, m))
+    ids, dist, st = apoe.search(w["ctx"], w["gc"], gq, w["gg"], (49.0, 1.0, 1.0), 24, variant=variant)
+    out_ids = torch.full((gq.n, 24), -1, dtype=torch.int32, device="cuda:0")
+    out_dist = torch.full((gq.n, 24), -1.0, dtype=torch.float32, device="cuda:0")
+    st2 = apoe.search_noalloc(w["ctx"], w["gc"], gq, w["gg"], (49.0, 1.0, 1.0), 24, out_ids, out_dist, variant=variant)
+    assert st.dense_rows < st.evaluations  # sketches were asked
+    assert np.array_equal(ids, out_ids.cpu().numpy().view(np.uint32)) and np.array_equal(dist, out_dist.cpu().numpy())
+    assert (st.evaluations, st.dense_rows, st.algo_bytes) == (st2.evaluations, st2.dense_rows, st2.algo_bytes)
+    gq.close()
