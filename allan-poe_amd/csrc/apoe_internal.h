@@ -67,6 +67,16 @@ struct DevBuf {
         n = count;
         return APOE_OK;
     }
+    bool try_alloc(size_t count) { // for what the caller can do without: no error is left behind
+        release();
+        if (hipMalloc((void**)&p, count * sizeof(T)) != hipSuccess) {
+            (void)hipGetLastError();
+            p = nullptr;
+            return false;
+        }
+        n = count;
+        return true;
+    }
     size_t bytes() const { return n * sizeof(T); }
 };
 

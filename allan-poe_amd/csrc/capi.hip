@@ -267,19 +267,19 @@ int apoe_corpus_create(apoe_ctx* ctx, uint32_t n, uint32_t dim, const float* den
         APOE_TRY(c->desc.alloc(n));
         APOE_TRY(c->recs.alloc(c->rec_bytes + ROW_LOAD_SLACK)); // unclamped row loads may read past the last record
         APOE_TRY(c->dnorm.alloc(n));
-        // the sketch saves the search reads but nothing depends on it: a corpus that leaves little of the device does without
         size_t free_bytes = 0, total_bytes = 0;
         APOE_HIP(hipMemGetInfo(&free_bytes, &total_bytes));
-        if ((size_t)n * SKETCH_BYTES <= free_bytes / 8) {
-            APOE_TRY(c->sketch.alloc((size_t)n * (SKETCH_BYTES / 4)));
-            APOE_TRY(c->sketch_meta.alloc(n));
-        }
         APOE_TRY(copy_in(ctx, c->desc.p, desc.data(), n * sizeof(uint64_t)));
         APOE_TRY(d_dense.init(ctx, dense, (size_t)n * dim));
         APOE_TRY(d_soff.init(ctx, s_off, n + 1));
         APOE_TRY(d_sval.init(ctx, s_val, hs[n]));
         APOE_TRY(d_boff.init(ctx, b_off, n + 1));
         APOE_TRY(d_bval.init(ctx, b_val, hb[n]));
+        // The sketch saves the search reads but nothing depends on it: it comes last, after the staged arrays, and a corpus does without
+        // when it cannot be had or when less than ten times its size is free. What is left then holds a K = 128 / degree 64 build (about
+        // 6.3 KB a document) and the half-precision rows (2 KB).
+        if ((size_t)n * SKETCH_BYTES <= free_bytes / 10 && !(c->sketch.try_alloc((size_t)n * (SKETCH_BYTES / 4)) && c->sketch_meta.try_alloc(n)))
+            c->sketch.release();
         APOE_TRY(launch_pack(ctx, n, d_dense.p, d_soff.p, d_sidx.p, d_sval.p, d_boff.p, d_bidx.p, d_bval.p, c->desc.p, c->recs.p, c->dnorm.p,
                              c->sketch_meta.p, c->sketch.p, c->narrow));
         APOE_HIP(hipStreamSynchronize(ctx->stream));
