@@ -73,7 +73,8 @@ int apoe_corpus_make_half_rows(apoe_ctx* ctx, apoe_corpus* c);
 void apoe_corpus_destroy(apoe_corpus* c);
 /* info4 = {n, dim, max splade nnz per row, max bm25 nnz per row} (index.cu:829-835). */
 int apoe_corpus_info(const apoe_corpus* c, uint32_t* info4);
-/* Bytes of the device records: the HBM footprint one full scan reads. */
+/* Bytes of the device records with their descriptors and norms, and of the half-precision rows if they were made: the HBM
+ * footprint one full scan reads. The 8-bit sketch beside them (1 032 bytes a document, when there is room) is not among them. */
 uint64_t apoe_corpus_bytes(const apoe_corpus* c);
 /* Bytes one (term, value) pair takes in the device records: 6 when every term id of the corpus
  * (both paths) is below 65536 (values as f32, ids as u16, the path known from the position),

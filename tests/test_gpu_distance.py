@@ -169,3 +169,23 @@ def test_query_sparse_term_with_bit_31_is_rejected(gpu_ctx):
     q.close()
     with pytest.raises(apoe.ApoeError, match="31 bits"):
         apoe.Queries(gpu_ctx, dense, off, np.array([0x80000007], np.uint32), val, off, np.array([7], np.uint32), val)
+
+
+@pytest.mark.parametrize("wide", [False, True])
+def test_corpus_bytes_are_those_of_a_full_scan(gpu_ctx, wide):
+    """Records (dense row, values, term ids, padded to 128 bytes), descriptor and norm of every document, and the half-precision rows
+    once they are made; the sketch beside them is not part of a scan."""
+    import apoe
+    n, k = 50, 20
+    rng = np.random.default_rng(2)
+    dense = rng.standard_normal((n, 1024)).astype(np.float32)
+    off = np.arange(0, n * k + 1, k, dtype=np.uint32)
+    idx = np.tile(np.arange(k, dtype=np.uint32) + (70000 if wide else 1), n)
+    val = rng.random(n * k).astype(np.float32)
+    gc = apoe.Corpus(gpu_ctx, dense, off, idx, val, off, idx, val)
+    up = lambda b: (b + 127) // 128 * 128
+    record = up(4096 + 8 * 2 * k) if wide else up(up(4096 + 4 * 2 * k) + 2 * 2 * k)
+    assert gc.bytes() == n * (record + 8 + 4)
+    gc.make_half_rows()
+    assert gc.bytes() == n * (record + 8 + 4 + 2048)
+    gc.close()
