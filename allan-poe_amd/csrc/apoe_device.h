@@ -230,7 +230,8 @@ __device__ __forceinline__ void pivot_terms_from_query(uint2* tab, uint32_t mask
         for (uint32_t j = Q.s_off[q] + tid; j < Q.s_off[q + 1]; j += nthreads) term_table_insert(tab, mask, Q.s_idx[j], Q.s_val[j] * w_s);
     if (use_b)
         for (uint32_t j = Q.b_off[q] + tid; j < Q.b_off[q + 1]; j += nthreads)
-            term_table_insert(tab, mask, Q.b_idx[j] | BM25_BIT, Q.b_val[j] * w_b);
+            if ((Q.b_idx[j] | BM25_BIT) != EMPTY) // no document holds that id, and it would read as an empty slot: two terms would share one
+                term_table_insert(tab, mask, Q.b_idx[j] | BM25_BIT, Q.b_val[j] * w_b);
 }
 
 struct EvalOut {

@@ -189,3 +189,29 @@ def test_corpus_bytes_are_those_of_a_full_scan(gpu_ctx, wide):
     gc.make_half_rows()
     assert gc.bytes() == n * (record + 8 + 4 + 2048)
     gc.close()
+
+
+@pytest.mark.parametrize("wide", [False, True])
+def test_query_terms_that_no_document_can_hold(gpu_ctx, wide):
+    """The BM25 id 0xFFFFFFFF is no document's and reads as an empty slot of the query's term table. Queries of 192 terms, 64 of them
+    that id, the terms of its slot handled by other waves: the distances are those of the queries without it, bit for bit."""
+    import apoe
+    n, nq, nt = 16, 2000, 192
+    rng = np.random.default_rng(12)
+    slot = lambda key: ((key.astype(np.uint64) * np.uint64(2654435761)) & np.uint64(0xFFFFFFFF)) >> np.uint64(12) & np.uint64(1023)
+    t = np.arange(70000, 200000, dtype=np.uint32) if wide else np.arange(1, 65536, dtype=np.uint32)
+    here = slot(t | np.uint32(0x80000000)) == slot(np.array([0xFFFFFFFF], np.uint32))
+    same, other = t[here], t[~here]
+    terms = np.concatenate([np.full(64, 0xFFFFFFFF, np.uint32), same[:1], other[:63], same[1:2], other[63:126]])
+    none = lambda m: (np.zeros(m + 1, np.uint32), np.zeros(0, np.uint32), np.zeros(0, np.float32))
+    off = lambda m, k: np.arange(0, m * k + 1, k, dtype=np.uint32)
+    corpus = (rng.standard_normal((n, 1024)).astype(np.float32), *none(n), off(n, 2), np.tile(same[:2], n), rng.random(2 * n).astype(np.float32) + 1)
+    gc = apoe.Corpus(gpu_ctx, *corpus)
+    assert gc.pair_bytes() == (8 if wide else 6)
+    q = rng.standard_normal((nq, 1024)).astype(np.float32)
+    val = rng.random((nq, nt)).astype(np.float32) + 1
+    with_it = apoe.Queries(gpu_ctx, q, *none(nq), off(nq, nt), np.tile(terms, nq), val.reshape(-1))
+    without = apoe.Queries(gpu_ctx, q, *none(nq), off(nq, nt - 64), np.tile(terms[64:], nq), np.ascontiguousarray(val[:, 64:]).reshape(-1))
+    ids = np.tile(np.arange(n, dtype=np.uint32), (nq, 1))
+    a, b = (apoe.distance_batch(gpu_ctx, gc, x, (0, 0, 1), ids) for x in (with_it, without))
+    assert np.array_equal(a, b), int((a != b).any(axis=1).sum())
