@@ -26,6 +26,52 @@ def test_pool_sizes_around_the_merge_groups(gpu_world, cands, variant):
         assert len(set(real.tolist())) == len(real)
 
 
+@pytest.mark.parametrize("variant", [1, 4, 5])
+@pytest.mark.parametrize("cands", [65, 255, 256, 257, 320, 513])
+def test_knowledge_graph_pools_around_the_merge_groups(gpu_world, cands, variant):
+    """Linking entity and hop travel with an entry through the groups: one that goes astray sends the walk to other documents."""
+    import apoe
+    import apoe_synth as S
+    import oracle as O
+    w = gpu_world
+    nq = 24
+    kg = S.to_numpy(S.knowledge_graph(1500, w["C"].n, nq, seed=31, device="cpu", mean_out=6.0))
+    gkg = apoe.KnowledgeGraph(w["ctx"], *kg)
+    ids, dist, st = apoe.search(w["ctx"], w["gc"], w["gq"], w["gg"], (1, 1, 1), cands, kg=gkg, kg_weight=20.0, q_count=nq, variant=variant)
+    oid, odist, cnt = O.search(w["C"], w["Q"].head(nq), w["rows"], w["entry"], (1, 1, 1), cands, kg=O.Kg(*kg), kg_weight=20.0)
+    assert_topk_match(ids, dist, oid, odist, cands, f"kg, cands {cands}")
+    assert_dist_close(dist, odist, f"kg, cands {cands}: pool distances")
+    assert abs(int(st.evaluations) - int(cnt[:, 1].sum())) <= 0.01 * cnt[:, 1].sum()
+    gkg.close()
+
+
+@pytest.mark.parametrize("variant", [1, 4, 5])
+@pytest.mark.parametrize("cands", [65, 66, 80, 129, 130, 257, 321])
+def test_hits_pushed_out_around_the_last_round(gpu_world, cands, variant):
+    """Pools whose last 64-entry round holds one, two or sixteen entries: a merge of up to 32 new candidates pushes out entries of that
+    round and of the one before. Of each query the term that about three tenths of the documents hold is required, and BM25 has no
+    weight: hits enter and leave the pool like any other document, and a row ends with those that were pushed out last."""
+    import apoe
+    import oracle as O
+    w = gpu_world
+    nq = 24
+    qa = list(O.HybridSet(*w["queries"]).head(nq).arrays())
+    off, idx = qa[4], qa[5].copy()
+    df = np.bincount(w["corpus"][5], minlength=int(max(w["corpus"][5].max(), idx.max())) + 1)
+    for q in range(nq):
+        if off[q] < off[q + 1]:
+            idx[off[q] + np.argmin(np.abs(df[idx[off[q]:off[q + 1]]] - 0.3 * w["C"].n))] |= np.uint32(KW)
+    qa[5] = idx
+    gq = apoe.Queries(w["ctx"], *qa)
+    ids, dist, _ = apoe.search(w["ctx"], w["gc"], gq, w["gg"], (1, 1, 0), cands, keyword_filter=True, variant=variant)
+    oid, odist, _ = O.search(w["C"], O.HybridSet(*qa), w["rows"], w["entry"], (1, 1, 0), cands, keyword_filter=True)
+    assert_topk_match(ids, dist, oid, odist, cands, f"keyword, cands {cands}")
+    assert_dist_close(dist, odist, f"keyword, cands {cands}: row distances")
+    worst = O.search(w["C"], w["Q"].head(nq), w["rows"], w["entry"], (1, 1, 0), cands)[1][:, -1]
+    behind = ((oid != EMPTY_ID) & (odist > worst[:, None])).sum(axis=1) # hits beyond the last entry of the pool
+    assert np.median(behind) >= 20
+
+
 def colliding_terms(count, buckets):
     """Term ids below 65 536 whose table bucket is the same: ((term * 0x9E3779) mod 2^32 >> 10) mod buckets."""
     t = np.arange(1, 65536, dtype=np.uint64)

@@ -54,6 +54,32 @@ def test_rows_are_those_of_reading_every_dense_row(gpu_ctx, kind, wide):
             assert read <= 0 and read % (1024 + 8) == 0  # what it costs: a sketch with its scale and error each
 
 
+@pytest.mark.parametrize("wide", [False, True])
+@pytest.mark.parametrize("kind", ["plain", "magnitudes", "spikes", "not numbers"])
+def test_knowledge_graph_and_keyword_search(gpu_ctx, kind, wide):
+    """The bound with the bonus of a linking entity in it, and the walk that keeps hits pushed out of the pool: whole rows bit for bit
+    those of reading every dense row, under weights where the sketch settles evaluations."""
+    import apoe
+    import apoe_synth as S
+    corpus, queries, rows, entry = world(kind, 7, wide)
+    b_idx = queries[5].copy()
+    b_idx[::12] |= np.uint32(0x80000000)  # the first BM25 term of every query is required
+    gc, gq, gg = apoe.Corpus(gpu_ctx, *corpus), apoe.Queries(gpu_ctx, *queries), apoe.Graph(gpu_ctx, rows, entry)
+    gk = apoe.Queries(gpu_ctx, *queries[:5], b_idx, queries[6])
+    kg = apoe.KnowledgeGraph(gpu_ctx, *S.to_numpy(S.knowledge_graph(800, N, NQ, seed=23, device="cpu", mean_out=6.0)))
+    for w3, cands, shape in (((1, 0, 0), 24, 0), ((49, 1, 1), 64, 4), ((49, 1, 1), 300, 2), ((0.01, 1, 1), 33, 3), ((1, 1, 0), 200, 1)):
+        calls = [dict(queries=gq, kg=kg, kg_weight=weight) for weight in (0.5, 40.0, 400.0)] + [dict(queries=gk, keyword_filter=True)]
+        for c in calls:
+            q = c.pop("queries")
+            a, ad, sa = apoe.search(gpu_ctx, gc, q, gg, w3, cands, variant=shape, **c)
+            b, bd, sb = apoe.search(gpu_ctx, gc, q, gg, w3, cands, variant=shape | 0x100, **c)
+            assert np.array_equal(a, b) and np.array_equal(ad, bd, equal_nan=True), (w3, cands, c)
+            assert sa.evaluations == sb.evaluations and sa.dense_rows <= sb.dense_rows == sb.evaluations
+            if kind == "plain" and w3 == (49, 1, 1) and cands == 64:
+                assert sa.dense_rows < 0.6 * sb.dense_rows
+                assert sa.algo_bytes + 4096 * (sb.dense_rows - sa.dense_rows) > sb.algo_bytes + 1032 * 0.3 * sb.evaluations # by sketches, not by the norm bound
+
+
 @pytest.mark.parametrize("kind", ["plain", "magnitudes", "spikes"])
 def test_half_precision_walk(gpu_ctx, kind):
     """The walk on half-precision rows under the sketch against the same walk without any bound."""
