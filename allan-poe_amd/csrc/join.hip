@@ -442,7 +442,7 @@ __global__ __launch_bounds__(jt_threads(NARROW)) __attribute__((amdgpu_waves_per
         const uint32_t M = uniform(ctl[1]);
         if (M == 0) continue;
         // the rows' own lists (who is already a neighbour), the columns' thresholds, where every row's pairs are
-        // each row's list in ascending id order (the proposals look an id up by binary search): wave w reads and sorts rows w, w + 8, ...
+        // each row's list in ascending id order (the proposals look an id up by binary search): wave w reads and sorts rows w, w + NW, ...
         if (KK == 64) {
             uint32_t mine[JT_ROWS / NW];
 #pragma unroll

@@ -1156,10 +1156,11 @@ int launch_search(apoe_ctx* ctx, const apoe_corpus* c, const apoe_queries* q, co
 
     // Launch shape (waves per query). 1, 2, 3, 4, 5: one, four, eight, two, sixteen waves, as the caller says. 0, the default:
     //  * a batch that is resident all at once is bound by the time of ONE query, and that falls with the waves it has
-    //    (alone, cands 256: 4.2 / 2.9 / 2.0 / 1.7 ms with 2 / 4 / 8 / 16 waves): sixteen waves while every query has a
-    //    CU of its own (256), eight while all queries still fit the machine that way (768 at 3 per CU), else four while
-    //    they fit (1 536), e.g. 100 queries at cands 256 in 2.4 instead of 7.9 ms, 1 024 in 5.6 instead of 8.8 ms; four also for batches of up to two rounds of the two-wave
-    //    grid (6 144 queries), whose second round ends sooner that way (4-9 % at 4 096 to 6 144 queries, cands 64-512);
+    //    (128 queries, 1 M docs, cands 256: 4.5 / 3.0 / 2.2 ms with 4 / 8 / 16 waves): sixteen waves while every query has a
+    //    CU of its own (256 queries: 2.30 ms against 3.10 with eight; 300: 3.38 against 3.10), eight while all queries still fit
+    //    the machine that way (768 at 3 per CU: 3.74 against 5.09 with four; 1 024: 5.28 against 5.18), else four while they fit
+    //    (1 536: 6.0 against 8.9 with two); four also for batches of up to two rounds of the two-wave grid (6 144 queries),
+    //    whose second round ends sooner that way (4 096: 13.6 against 15.4 ms, 6 144: 21.1 against 22.6, at cands 64 7.0 against 7.6);
     //  * a longer batch is bound by the memory system and runs best with two waves per query and as many queries as fit
     //    (12 per CU) - unless the pool is so large that LDS leaves room for at most 9 queries on a CU: then four waves
     //    per query keep twice the loads in flight (10 000 queries, 1 M docs, four against two waves: 98.0 against 105.6 ms

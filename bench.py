@@ -30,9 +30,9 @@ HBM_PEAK_GBS = 8000.0
 # (corpus, docs, degree, queries, cands, variant, NN-Descent step) with the profiles/ file that holds the run. Any other
 # workload reports null.
 RECORDED_TRAFFIC = {
-    ("iid", 1_000_000, 48, 10_000, 256, 0, 1): {"default": 1.922e11, "every_dense_row_read": 5.375e11,
+    ("iid", 1_000_000, 48, 10_000, 256, 0, 1): {"default": 1.878e11, "every_dense_row_read": 5.315e11,
                                                  "source": "profiles/bench_1Mdocs_degree48_cands256.md (FETCH_SIZE x 2.000 + WRITE_SIZE x 1.000, factors from a 1 GiB copy)"},
-    ("latent", 1_000_000, 48, 10_000, 80, 0, 1): {"default": 1.123e11, "every_dense_row_read": 1.890e11,
+    ("latent", 1_000_000, 48, 10_000, 80, 0, 1): {"default": 1.105e11, "every_dense_row_read": 1.872e11,
                                                   "source": "profiles/bench_1Mdocs_latent_degree48_cands80.md (FETCH_SIZE x 2.000 + WRITE_SIZE x 1.000, factors from a 1 GiB copy)"},
 }
 
@@ -370,7 +370,7 @@ def main():
                 structured["cands_at_recall_target"], structured["qps_at_recall_target"] = ec, args.queries / (sl.kernel_ms / 1e3)
         if structured["cands_at_recall_target"]:
             # the same walk on half-precision copies of the dense rows, the final pool evaluated again in fp32 (variant | 0x200):
-            # here every evaluation reads its dense row, so the narrower row shows
+            # here pairs and norms settle nothing: what their sketch does not settle reads the narrower row
             gc_l.make_half_rows()
             hc = structured["cands_at_recall_target"]
             apoe.search(ctx, gc_l, gq_l, g_l, w_l, hc, max_iter=iter_cap(hc), variant=0x200)
@@ -561,7 +561,7 @@ def main():
                      "traffic_source": rec_traffic["source"] if rec_traffic else None,
                      "kernel": "search_kernel", "algo_bytes_per_launch": algo_bytes,
                      "at_recall_target": bool(ok),
-                     "mode": "dense row read only when the sparse part plus the bound of the dense part can enter the pool",
+                     "mode": "dense row read only when neither the sparse part plus the norm bound of the dense part nor the 8-bit sketch keeps the candidate out of the pool",
                      # the same evaluations priced as the reference prices them (every evaluation reads its dense row), over the
                      # default mode's time: what a kernel without the bound would have to sustain to be as fast
                      "equivalent_if_every_evaluation_read_its_dense_row": {"bytes_per_launch": full_bytes,

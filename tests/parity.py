@@ -1,7 +1,7 @@
 """Shared parity checks between the HIP path and the CPU oracle."""
 import numpy as np
 
-DIST_RTOL = 1e-4  # hybrid distances within 1e-4 relative
+DIST_RTOL = 1e-4  # the bound on hybrid distances, relative
 
 
 def assert_dist_close(got, want, what=""):
