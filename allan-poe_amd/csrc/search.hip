@@ -318,7 +318,9 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
     constexpr bool KG = MODE == MODE_KG, KWD = MODE == MODE_KEYWORD;
     // Whether wave 0 asks for more than the walk may need (graph row of the first unexplored entry, descriptors of visited neighbours) to
     // have it early: one query's chain gains, a long batch, whose other queries cover the wait, pays in traffic (figures where the walk starts).
-    constexpr bool AHEAD = NW >= 4;
+    // Knowledge-graph search gains in long batches too (ten queries a CU, a longer chain between two walks: 10 000 queries, 1 M docs,
+    // cands 64 / 128 / 160: 10.55 / 18.0 / 22.4 ms ahead, 10.66 / 18.2 / 22.7 when needed).
+    constexpr bool AHEAD = NW >= 4 || KG;
     a.C.narrow = NARROW ? 1u : 0u; // the pair format as a compile-time constant: no branch at the loads
     extern __shared__ __align__(16) char smem[];
     const SearchLds L(a.slots_s, a.slots_b, a.ovf_cap, a.cands, MODE);
@@ -534,7 +536,7 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
         // 2 000 cycles of an iteration after the merge; of them 150 to 280 are left behind it. (Looking one whole expansion ahead,
         // with the visited marks taken back when a candidate overtakes: it is right for 0.55 to 0.64 of the expansions only, and
         // the marks and rows of the others cost long batches 5 %.)
-        // One and two waves per query are for long batches: a row that is overtaken and the descriptors of visited neighbours are
+        // One and two waves per query are for long batches: in plain and keyword search a row that is overtaken and the descriptors of visited neighbours are
         // traffic there, and nothing waits for them (10 000 queries, 1 M docs, cands 256 / 512: 1.921e11 -> 1.877e11 bytes and
         // 30.4 -> 30.1 ms / 55.1 -> 54.3 ms without them).
         uint32_t g_c = EMPTY, g_kw = 0; // lane l: neighbour of `front`, later of the parent; (keyword search) word l of the row's tail
