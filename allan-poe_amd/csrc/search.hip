@@ -521,6 +521,7 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
                     Fresh F;
                     fresh_load<MODE>(F, P, new_id, new_dist, new_ent, new_hop, nb);
                     fresh_rank(F);
+                    F.kept &= __ballot(F.rank < cands); // of more seeds than the pool holds most cannot enter, and the merge's time goes with the kept ones
                     sort_merge<MODE>(P, F, R);
                 }
                 front = pool_front(P, 0);

@@ -27,9 +27,10 @@ def test_pool_sizes_around_the_merge_groups(gpu_world, cands, variant):
 
 
 @pytest.mark.parametrize("variant", [1, 4, 5])
-@pytest.mark.parametrize("cands", [65, 255, 256, 257, 320, 513])
+@pytest.mark.parametrize("cands", [1, 7, 16, 65, 255, 256, 257, 320, 513])
 def test_knowledge_graph_pools_around_the_merge_groups(gpu_world, cands, variant):
-    """Linking entity and hop travel with an entry through the groups: one that goes astray sends the walk to other documents."""
+    """Linking entity and hop travel with an entry through the groups: one that goes astray sends the walk to other documents. The
+    smallest pools hold fewer entries than the walk has seeds."""
     import apoe
     import apoe_synth as S
     import oracle as O
