@@ -6,8 +6,7 @@
 // are its COLUMNS (up to 128), every row of the tile is gathered once and meets every column:
 //   dense part   32 x 128 x 1024 contraction on the matrix cores (fp32 MFMA 16x16x4; the waves take the
 //                16-column blocks that exist x equal parts of the dimensions)
-//   sparse part  eight picker rows at a time in an LDS rank table that the column rows probe (apoe_ranktab.h); a
-//                wave keeps the pairs of its columns (eight or sixteen) in registers, so a row is read from memory once per tile
+//   sparse part  eight picker rows at a time in an LDS rank table that the column rows probe (apoe_ranktab.h)
 //   insertion    a pair closer than the row's last list entry (and not in that list) is offered to the row node
 //                with a 64-bit atomicMin on slot hash(id) of its proposal row: (distance, id), the smallest wins;
 //                in symmetric mode the pair is offered to the column node as well (both endpoints, as the classic
@@ -23,6 +22,7 @@
 #include <hipcub/hipcub.hpp>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "apoe_gram.h"
 #include "apoe_internal.h"
@@ -32,13 +32,16 @@ namespace apoe {
 
 constexpr int JT_ROWS = 32;
 constexpr int JT_COLS = 128;
-// Threads of a tile's workgroup (one per CU: LDS allows no second one). Sixteen waves for narrow corpora: a tile is a chain of
-// short phases with barriers between them (queue, id set, staging, table builds, probes), and four waves per SIMD cover each
-// other's waits where two do not; a wave then owns eight columns, whose pairs fit beside everything else in 128 registers.
-// 100 000 docs K = 64: 117 -> 112 ms over ten steps; 30 011 docs K = 128: step 72 -> 59, prune tiles 30 -> 26 ms. The wide
-// format's row registers (keys of 32 bits, key compares) do not fit 128: it spilled 100 of them and stays at eight waves.
-constexpr int jt_threads(bool narrow) { return narrow ? 1024 : 512; }
+// A tile is a chain of short phases (queue, ids, pairs and table builds, probes, dense rows, proposals) with barriers between
+// them: one phase waits for memory, the next for LDS or the vector units. Two workgroups of eight waves per CU, each with half
+// of the CU's LDS and registers, cover each other's waits; at most a hundred columns meet four to eight pickers in an average
+// tile, so neither workgroup lacks work. Builds of ten steps against one workgroup of sixteen waves (wide pairs: of eight) with the
+// columns' pairs in registers: 100 000 docs K = 64 145.2 -> 113.3 ms, 30 011 docs K = 128 97.3 -> 76.7 ms, 20 000 docs wide 54.5 ->
+// 37.4 ms, 300 000 docs of the i.i.d. corpus 299 -> 254 ms. A corpus whose longest row does not fit the table of the smaller LDS takes one
+// workgroup of sixteen waves per CU (tile_shape).
+constexpr int JT_PAIR_THREADS = 512, JT_SOLO_THREADS = 1024;
 constexpr int JT_STRIDE = JT_COLS + 1;
+constexpr int JT_STAGE_DIMS = 256; // the picker rows are staged at least this many dimensions at a time
 constexpr int JT_SEEN = 512; // slots of the id set that removes repeated columns
 // The kernels below are built for lists of KK = 64 and KK = 128 entries (index.cu:6 has K 64; a degree above 32 needs
 // 2 * degree <= K there, index.cu:702). A node has 2 * KK proposal slots: two proposals of one step whose ids hash to one
@@ -135,51 +138,52 @@ struct JoinArgs {
     uint32_t index_bits, slot_cap, span;
 };
 
+// The table region holds the rank table of the sparse part; behind it in time, the picker rows' own lists (local join only: list
+// entries KK > 0) and, behind those in place, the staged dense rows.
 struct JoinLds {
-    uint32_t G, tab, row_list, rowptr, rownnz, row_id, col_id, row_worst, col_worst, seen, scan, ctl, total;
-    // KK = 64: the picker rows' own lists have an array of their own; KK = 128: they are loaded when the products are done and
-    // sit behind the rank table, inside the region that staged the dense rows before
-    __host__ __device__ JoinLds(uint32_t index_bits, uint32_t slot_cap, bool narrow, uint32_t KK = 64) {
+    uint32_t G, rowptr, rownnz, row_id, row_worst, col_id, col_worst, seen, scan, ctl, tab, stage, stage_bytes, total;
+    __host__ __device__ JoinLds(uint32_t index_bits, uint32_t slot_cap, bool narrow, uint32_t KK) {
         uint32_t o = 0;
         G = o; o += JT_ROWS * JT_STRIDE * 4;
-        row_list = o; o += KK == 64 ? JT_ROWS * 64 * 4 : 0;
         o = (o + 7) & ~7u;
         rowptr = o; o += (JT_ROWS + JT_COLS) * 8;
         rownnz = o; o += (JT_ROWS + JT_COLS) * 4;
         row_id = o; o += JT_ROWS * 4;
-        col_id = o; o += JT_COLS * 4;
         row_worst = o; o += JT_ROWS * 4;
+        col_id = o; o += JT_COLS * 4;
         col_worst = o; o += JT_COLS * 4;
         seen = o; o += JT_SEEN * 4;
         scan = o; o += 20 * 4;
         ctl = o; o += 8 * 4;
         o = (o + 15) & ~15u;
-        // the rank table of the sparse part; before it is built, the same bytes hold the dense parts of the picker rows
-        uint32_t table = (RankTabLds(index_bits, slot_cap, narrow).total + 15) & ~15u;
-        const uint32_t rows = (uint32_t)(JT_ROWS * DENSE_BYTES);
-        if (KK != 64) { row_list = o + table; table += JT_ROWS * KK * 4; }
-        tab = o; o += table > rows ? table : rows;
+        tab = o;
+        const uint32_t lists = JT_ROWS * KK * 4;
+        const uint32_t table = (RankTabLds(index_bits, slot_cap, narrow).total + 15) & ~15u;
+        const uint32_t least = lists + JT_ROWS * JT_STAGE_DIMS * 4;
+        stage = o + lists;
+        o += table > least ? table : least;
+        stage_bytes = o - stage;
         total = o;
     }
 };
 
 // Dense part of a tile on v_mfma_f32_16x16x4_f32. A wave owns 16 columns and a range of 16-float blocks of the
-// dimensions; the picker rows come from LDS (`A`: row r, float4 c at A[r * 256 + (c ^ (r & 7))] -- the swizzle spreads
-// the sixteen rows of a read over the banks without padding), the column rows straight from memory. Lane (j, g), j =
-// lane % 16, g = lane / 16, supplies float4 number 4 b + g of block b for row j (A operand) and for column j (B
-// operand): the four multiplies of a block take one component each, so k-slot g of multiply c stands for dimension
-// 16 b + 4 g + c on both sides. RING column blocks are in flight ahead of the one being multiplied (a ring of
-// registers, refilled as it is consumed). Rows 16..31 of the tile take a second accumulator fed from the same column
-// registers, and only when the tile has them: a tile of at most 16 rows costs half the matrix time.
+// dimensions; the picker rows come from LDS (`A`: row r, float4 c of the staged dimensions at A[r * row4 + (c ^ (r & 7))] -- the
+// swizzle spreads the sixteen rows of a read over the banks without padding), the column rows straight from memory (`pb`: the
+// lane's column at the first staged dimension). Lane (j, g), j = lane % 16, g = lane / 16, supplies float4 number 4 b + g of block
+// b for row j (A operand) and for column j (B operand): the four multiplies of a block take one component each, so k-slot g of
+// multiply c stands for dimension 16 b + 4 g + c on both sides. RING column blocks are in flight ahead of the one being
+// multiplied (a ring of registers, refilled as it is consumed). Rows 16..31 of the tile take a second accumulator fed from the
+// same column registers, and only when the tile has them: a tile of at most 16 rows costs half the matrix time.
 // Result: lane (j, g) holds row 4 g + e (+ 16), column j in acc0[e] (acc1[e]).
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 template <int RING>
-__device__ __forceinline__ void join_dense16(const float4* A, uint32_t nr, const float4* pb, int lane, int b_begin, int b_end, floatx4& acc0,
-                                             floatx4& acc1) {
+__device__ __forceinline__ void join_dense16(const float4* A, uint32_t row4, uint32_t nr, const float4* pb, int lane, int b_begin, int b_end,
+                                             floatx4& acc0, floatx4& acc1) {
     const int j = lane & 15, g = lane >> 4;
     const uint32_t i0 = min((uint32_t)j, nr - 1), i1 = min(16u + (uint32_t)j, nr - 1);
-    const float4* a0 = A + i0 * (DIM / 4);
-    const float4* a1 = A + i1 * (DIM / 4);
+    const float4* a0 = A + i0 * row4;
+    const float4* a1 = A + i1 * row4;
     const uint32_t s0 = i0 & 7, s1 = i1 & 7;
     const bool two = nr > 16; // wave-uniform
     float4 ring[RING];
@@ -223,64 +227,33 @@ __device__ __forceinline__ uint32_t wave_sort_u32(uint32_t v, int lane) {
     return v;
 }
 
-// The hybrid inner products of a tile, G[r * JT_STRIDE + c] = dense_mul * <row r, column c>_dense + <row r, column c>_sparse for
-// the R rows and M columns whose record addresses and shapes `rowptr` / `rownnz` hold (rows at [0, JT_ROWS), columns at
-// [JT_ROWS, JT_ROWS + JT_COLS): gram_rows_gather). All threads of the workgroup call it after a barrier behind those arrays; it
-// ends with a barrier. `tabreg` = the table region of JoinLds, `unfit` = counter of rows whose terms did not fit the table.
+// The pairs of row or column i (wave-uniform) of a tile.
 template <bool NARROW>
-__device__ __forceinline__ void tile_hybrid_ips(const CorpusView& C, float dense_mul, char* tabreg, const RankTab& T, uint32_t index_bits, uint32_t slot_cap,
-                                                float* G, const unsigned long long* rowptr, const uint32_t* rownnz, uint32_t* scan, uint32_t R,
-                                                uint32_t M, unsigned long long* unfit, int tid, int wave, int lane) {
-    constexpr int NT = jt_threads(NARROW), NW = NT / WAVE;
-    constexpr int JT_OWN = JT_COLS / NW;    // columns of a tile that one wave owns: their pairs stay in its registers
-    constexpr int JT_BATCH = NW == 8 ? 2 : 1; // column rows a wave probes together: with four waves per SIMD one at a time covers the waits
-    constexpr int RING = NW == 8 ? 16 : 8;  // column blocks a wave has in flight: 128 per CU either way
-    // dense part: the waves share the 16-column blocks that exist (8, 4, 2 or 1 by the number of columns) and, for
-    // each block, equal parts of the dimensions (1, 2, 4, 8 or 16): no wave idles when a tile has few columns. The picker
-    // rows are staged in the table region, which is free until the sparse part. Partial tiles are added into G in a
-    // fixed order, a barrier between them.
-    {
-        const uint32_t nblk = M <= 16 ? 1u : M <= 32 ? 2u : M <= 64 ? 4u : 8u, parts = (uint32_t)NW / nblk;
-        const uint32_t blk = (uint32_t)wave % nblk, part = (uint32_t)wave / nblk;
-        const bool active = blk * 16 < M;
-        const uint32_t per = (DIM / 16) / parts; // 16-float blocks of the dimensions per part: 64, 32, 16, 8 or 4
-        float4* A = reinterpret_cast<float4*>(tabreg);
-        const uint32_t jcol = min(blk * 16 + (uint32_t)(lane & 15), M - 1);
-        const float4* pb = reinterpret_cast<const float4*>(rowptr[JT_ROWS + jcol] - DENSE_BYTES) + (lane >> 4);
-#pragma unroll 4
-        for (uint32_t i = tid; i < R * (DIM / 4); i += NT) {
-            const uint32_t r = i / (DIM / 4), c = i % (DIM / 4);
-            A[r * (DIM / 4) + (c ^ (r & 7))] = reinterpret_cast<const float4*>(rowptr[r] - DENSE_BYTES)[c];
-        }
-        __syncthreads();
-        floatx4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
-        if (active) {
-            if (per >= (uint32_t)RING) join_dense16<RING>(A, R, pb, lane, (int)(part * per), (int)((part + 1) * per), acc0, acc1);
-            else join_dense16<RING / 2>(A, R, pb, lane, (int)(part * per), (int)((part + 1) * per), acc0, acc1);
-        }
-        auto store = [&](bool add) {
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                float* at = &G[(4 * (lane >> 4) + e) * JT_STRIDE + blk * 16 + (lane & 15)];
-                *at = add ? *at + dense_mul * acc0[e] : dense_mul * acc0[e];
-                if (R > 16) {
-                    float* at1 = at + 16 * JT_STRIDE;
-                    *at1 = add ? *at1 + dense_mul * acc1[e] : dense_mul * acc1[e];
-                }
-            }
-        };
-        for (uint32_t ph = 0; ph < parts; ph++) {
-            if (active && part == ph) store(ph != 0);
-            if (ph + 1 < parts) __syncthreads();
-        }
-    }
-    __syncthreads();
-    // sparse part: groups of eight rows in the rank table, every column probes it once per group. The pairs of a
-    // group's rows are requested while the group before it is probed; the pairs of a wave's columns stay in its
-    // registers for the whole tile: a build and the probes find their operands there.
-    auto row_pairs = [&](uint32_t i) { Pairs p = gram_row(C, rowptr, rownnz, i); p.narrow = NARROW ? 1u : 0u; return p; };
-    auto col_pairs = [&](uint32_t b) { Pairs p = gram_row(C, rowptr + JT_ROWS, rownnz + JT_ROWS, b); p.narrow = NARROW ? 1u : 0u; return p; };
-    uint32_t a0 = 0;
+__device__ __forceinline__ Pairs tile_pairs(const unsigned long long* rowptr, const uint32_t* rownnz, uint32_t i) {
+    const unsigned long long at = rowptr[i];
+    Pairs p;
+    p.base = reinterpret_cast<const char*>((unsigned long long)uniform((uint32_t)(at >> 32)) << 32 | uniform((uint32_t)at));
+    const uint32_t w = uniform(rownnz[i]);
+    p.nnz = w & 0xFFFFu;
+    p.ns = w >> 16;
+    p.narrow = NARROW ? 1u : 0u;
+    return p;
+}
+
+// Sparse part of a tile: G[r * JT_STRIDE + c] = <row r, column c>_sparse for the R rows and M columns whose record addresses and
+// shapes `rowptr` / `rownnz` hold (rows at [0, JT_ROWS), columns at [JT_ROWS, JT_ROWS + JT_COLS): gram_rows_gather). Groups of
+// eight rows in the rank table, every column probes it once per group. All threads of the workgroup call it after a barrier behind
+// those arrays; it ends with a barrier. `unfit` = counter of rows whose terms did not fit the table.
+// The pairs of a group's rows are requested while the group before it is probed, those of a wave's columns TILE_AHEAD columns ahead
+// (a tile has one group in most cases: with the columns held in registers for all groups a wave needs 96 of them and a CU holds
+// one workgroup only).
+template <bool NARROW, int NT>
+__device__ __forceinline__ void tile_sparse(const RankTab& T, float* G, const unsigned long long* rowptr, const uint32_t* rownnz, uint32_t* scan, uint32_t R,
+                                            uint32_t M, unsigned long long* unfit, int tid, int wave, int lane) {
+    constexpr int NW = NT / WAVE, TILE_AHEAD = NARROW ? 3 : 2;
+    static_assert(NW >= RT_T, "a wave per pivot of a group");
+    auto row_pairs = [&](uint32_t i) { return tile_pairs<NARROW>(rowptr, rownnz, i); };
+    auto col_pairs = [&](uint32_t b) { return tile_pairs<NARROW>(rowptr, rownnz, JT_ROWS + b); };
     // a group's pivots, one per wave (as the prune holds its rows): a build hands every wave its own row's pairs, four to a lane
     RtRow<NARROW> pv;
     uint32_t pv_shape = 0;
@@ -291,20 +264,20 @@ __device__ __forceinline__ void tile_hybrid_ips(const CorpusView& C, float dense
             rt_row_load(pv, row_pairs(first + wave), lane);
         }
     };
+    // the wave's columns wave, wave + NW, ...; shapes (nnz | ns << 16) are wave-uniform. Slot s holds columns wave + (s + k * TILE_AHEAD) * NW
+    RtRow<NARROW> col[TILE_AHEAD];
+    uint32_t col_shape[TILE_AHEAD];
+    auto col_load = [&](int s, uint32_t b) {
+        col_shape[s] = uniform(rownnz[JT_ROWS + b]);
+        rt_row_load(col[s], col_pairs(b), lane);
+    };
     pivots_load(0);
-    // the wave's columns wave, wave + NW, ...: read once per tile, probed once per group; their shapes
-    // (nnz | ns << 16) are wave-uniform and stay in scalar registers
-    RtRow<NARROW> own[JT_OWN];
-    uint32_t own_shape[JT_OWN];
 #pragma unroll
-    for (int k = 0; k < JT_OWN; k++) {
-        const uint32_t b = wave + k * NW;
-        own_shape[k] = 0;
-        if (b < M) {
-            own_shape[k] = uniform(rownnz[JT_ROWS + b]);
-            rt_row_load(own[k], col_pairs(b), lane);
-        }
+    for (int s = 0; s < TILE_AHEAD; s++) {
+        col_shape[s] = 0;
+        if (wave + s * NW < (int)M) col_load(s, wave + s * NW);
     }
+    uint32_t a0 = 0;
     while (a0 < R) {
         uint32_t nt = min((uint32_t)RT_T, R - a0);
         uint32_t built;
@@ -317,37 +290,83 @@ __device__ __forceinline__ void tile_hybrid_ips(const CorpusView& C, float dense
         if (a1 < R) pivots_load(a1);
         if (built == EMPTY) { // one row alone does not fit: its sparse part is missing, the host is told
             if (tid == 0) atomicAdd(unfit, 1ull);
+            for (uint32_t c = tid; c < M; c += NT) G[a0 * JT_STRIDE + c] = 0.f;
             a0 = a1;
             continue;
         }
         const uint32_t n_ovf = NARROW ? 0u : uniform(min(scan[16], (uint32_t)RT_OVF));
+        for (uint32_t b0 = wave; b0 < M; b0 += TILE_AHEAD * NW) {
 #pragma unroll
-        for (int q = 0; q < JT_OWN / JT_BATCH; q++) {
-            const uint32_t b0 = wave + q * JT_BATCH * NW;
-            if (b0 < M) { // wave-uniform
-                float acc[JT_BATCH][RT_T];
-                RtRow<NARROW> rows[JT_BATCH];
-                uint32_t shape[JT_BATCH];
+            for (int s = 0; s < TILE_AHEAD; s++) {
+                const uint32_t b = b0 + s * NW;
+                if (b < M) { // wave-uniform
+                    float acc[1][RT_T];
+                    RtRow<NARROW> rows[1] = {col[s]};
+                    const uint32_t shape[1] = {col_shape[s]};
+                    const uint32_t next = b + TILE_AHEAD * NW;
+                    if (next < M) col_load(s, next);
+                    else if (a1 < R) col_load(s, wave + s * NW); // the first of the slot again, for the next group
 #pragma unroll
-                for (int k = 0; k < JT_BATCH; k++) {
-                    rows[k] = own[q * JT_BATCH + k];
-                    rows[k].touch();
-                    shape[k] = own_shape[q * JT_BATCH + k];
-                    asm volatile("" : "+s"(shape[k])); // as touch(): the lane masks of a row are made where they are used
-#pragma unroll
-                    for (int t = 0; t < RT_T; t++) acc[k][t] = 0.f;
+                    for (int t = 0; t < RT_T; t++) acc[0][t] = 0.f;
+                    ranktab_probe_rows<NARROW, 1>(T, rows, shape, [&](int) { return col_pairs(b); }, n_ovf, acc, lane);
+                    uint32_t t;
+                    const float z = wave_sum_1x8(acc[0], lane, &t);
+                    if ((lane & 15) < 4 && lane < 32 && t < nt) G[(a0 + t) * JT_STRIDE + b] = z;
                 }
-                ranktab_probe_rows<NARROW, JT_BATCH>(T, rows, shape, [&](int k) { return col_pairs(b0 + k * NW); }, n_ovf, acc, lane);
-                uint32_t t, r = 0;
-                float z;
-                if constexpr (JT_BATCH == 2) z = wave_sum_2x8(acc, lane, &t, &r);
-                else z = wave_sum_1x8(acc[0], lane, &t);
-                const uint32_t b = b0 + r * NW;
-                if ((lane & 15) < 4 && (JT_BATCH == 2 || lane < 32) && t < nt && b < M) G[(a0 + t) * JT_STRIDE + b] += z;
+                __builtin_amdgcn_sched_barrier(0); // one column at a time: the scheduler must not pile up the reads of all of them
             }
-            __builtin_amdgcn_sched_barrier(0); // one batch at a time: the scheduler must not pile up the reads of all of them
         }
         a0 = a1;
+        __syncthreads();
+    }
+}
+
+// Dense part of a tile: adds dense_mul * <row r, column c>_dense to G for the R rows and the M columns. The waves share the 16-column
+// blocks that exist (8, 4, 2 or 1 by the number of columns) and, for each block, equal parts of the dimensions: no wave idles
+// when a tile has few columns. The picker rows are staged in `stage`, all dimensions at once if they fit, else a half or a quarter
+// at a time. Partial tiles are added into G in a fixed order, a barrier between them. All threads of the workgroup call it after a barrier; it ends with a
+// barrier.
+template <int NT>
+__device__ __forceinline__ void tile_dense(float dense_mul, char* stage, uint32_t stage_bytes, float* G, const unsigned long long* rowptr, uint32_t R,
+                                           uint32_t M, int tid, int wave, int lane) {
+    constexpr int NW = NT / WAVE;
+    constexpr int RING = 8; // column blocks a wave has in flight: 128 KB per CU
+    static_assert(DIM == 4 * JT_STAGE_DIMS, "a row is staged whole, in halves or in quarters");
+    const uint32_t nblk = M <= 16 ? 1u : M <= 32 ? 2u : M <= 64 ? 4u : 8u, parts = (uint32_t)NW / nblk;
+    const uint32_t blk = (uint32_t)wave % nblk, part = (uint32_t)wave / nblk;
+    const bool active = blk * 16 < M;
+    const uint32_t fit = stage_bytes / (4 * R);
+    const uint32_t dims = fit >= DIM ? (uint32_t)DIM : fit >= DIM / 2 ? (uint32_t)DIM / 2 : (uint32_t)DIM / 4;
+    const uint32_t per = dims / 16 / parts; // 16-float blocks of the staged dimensions per part: 64 ... 1
+    float4* A = reinterpret_cast<float4*>(stage);
+    const uint32_t row4 = dims / 4;
+    const uint32_t jcol = min(blk * 16 + (uint32_t)(lane & 15), M - 1);
+    const float4* pb = reinterpret_cast<const float4*>(rowptr[JT_ROWS + jcol] - DENSE_BYTES) + (lane >> 4);
+    floatx4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
+    for (uint32_t d4 = 0; d4 < DIM / 4; d4 += row4) {
+        if (d4) __syncthreads();
+#pragma unroll 4
+        for (uint32_t i = tid; i < R * row4; i += NT) {
+            const uint32_t r = i / row4, c = i % row4;
+            A[r * row4 + (c ^ (r & 7))] = reinterpret_cast<const float4*>(rowptr[r] - DENSE_BYTES)[d4 + c];
+        }
+        __syncthreads();
+        if (active) {
+            const int b0 = (int)(part * per), b1 = b0 + (int)per;
+            if (per >= (uint32_t)RING) join_dense16<RING>(A, row4, R, pb + d4, lane, b0, b1, acc0, acc1);
+            else if (per >= 4) join_dense16<4>(A, row4, R, pb + d4, lane, b0, b1, acc0, acc1);
+            else join_dense16<1>(A, row4, R, pb + d4, lane, b0, b1, acc0, acc1);
+        }
+    }
+    for (uint32_t ph = 0; ph < parts; ph++) {
+        if (active && part == ph && blk * 16 + (uint32_t)(lane & 15) < M) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                float* at = &G[(4 * (lane >> 4) + e) * JT_STRIDE + blk * 16 + (lane & 15)];
+                *at += dense_mul * acc0[e];
+                if (R > 16) at[16 * JT_STRIDE] += dense_mul * acc1[e];
+            }
+        }
         __syncthreads();
     }
 }
@@ -374,16 +393,16 @@ __device__ __forceinline__ void wave_sort_u32x2(uint32_t& a, uint32_t& b, int la
     }
 }
 
-template <bool NARROW, uint32_t KK>
-__global__ __launch_bounds__(jt_threads(NARROW)) __attribute__((amdgpu_waves_per_eu(jt_threads(NARROW) / 256, jt_threads(NARROW) / 256))) void join_tile_kernel(JoinArgs a) {
+template <bool NARROW, uint32_t KK, int NT>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void join_tile_kernel(JoinArgs a) {
     constexpr uint32_t HALVES = KK / 64; // tiles per block of picker rows
-    constexpr int NT = jt_threads(NARROW), NW = NT / WAVE;
+    constexpr int NW = NT / WAVE;
     a.C.narrow = NARROW ? 1u : 0u;
     extern __shared__ __align__(16) char smem[];
     const JoinLds L(a.index_bits, a.slot_cap, NARROW, KK);
     const RankTab T = ranktab_at(smem + L.tab, a.index_bits, a.slot_cap, a.span, NARROW);
     float* G = reinterpret_cast<float*>(smem + L.G);
-    uint32_t* row_list = reinterpret_cast<uint32_t*>(smem + L.row_list);
+    uint32_t* row_list = reinterpret_cast<uint32_t*>(smem + L.tab); // behind the sparse part
     unsigned long long* rowptr = reinterpret_cast<unsigned long long*>(smem + L.rowptr);
     uint32_t* rownnz = reinterpret_cast<uint32_t*>(smem + L.rownnz);
     uint32_t* row_id = reinterpret_cast<uint32_t*>(smem + L.row_id);
@@ -441,45 +460,34 @@ __global__ __launch_bounds__(jt_threads(NARROW)) __attribute__((amdgpu_waves_per
         __syncthreads();
         const uint32_t M = uniform(ctl[1]);
         if (M == 0) continue;
-        // the rows' own lists (who is already a neighbour), the columns' thresholds, where every row's pairs are
-        // each row's list in ascending id order (the proposals look an id up by binary search): wave w reads and sorts rows w, w + NW, ...
-        if (KK == 64) {
-            uint32_t mine[JT_ROWS / NW];
-#pragma unroll
-            for (int k = 0; k < JT_ROWS / NW; k++) {
-                const uint32_t r = wave + k * NW;
-                mine[k] = r < R ? a.ids[(size_t)row_id[r] * KK + lane] & ~FLAG : 0u;
-            }
-#pragma unroll
-            for (int k = 0; k < JT_ROWS / NW; k++) {
-                const uint32_t r = wave + k * NW;
-                if (r < R) row_list[r * KK + lane] = wave_sort_u32(mine[k], lane);
-            }
-        }
         if ((uint32_t)tid < M) col_worst[tid] = a.symmetric ? a.dist[(size_t)col_id[tid] * KK + KK - 1] : -INF_DIS;
         gram_rows_gather(a.C, row_id, R, rowptr, rownnz, tid, NT);
         gram_rows_gather(a.C, col_id, M, rowptr + JT_ROWS, rownnz + JT_ROWS, tid, NT);
         __syncthreads();
-        tile_hybrid_ips<NARROW>(a.C, a.dense_mul, smem + L.tab, T, a.index_bits, a.slot_cap, G, rowptr, rownnz, scan, R, M, a.work + 3, tid, wave, lane);
-        if (KK == 128) { // the rows' own lists, behind the table (the bytes staged dense rows until now: all waves are past that)
-            uint32_t lo[JT_ROWS / NW], hi[JT_ROWS / NW];
+        tile_sparse<NARROW, NT>(T, G, rowptr, rownnz, scan, R, M, a.work + 3, tid, wave, lane);
+        // the rows' own lists (who is already a neighbour), each in ascending id order (the proposals look an id up by binary search):
+        // wave w reads and sorts rows w, w + NW, ... into the table's bytes
+        {
+            constexpr int KL = KK / WAVE;
+            uint32_t own[JT_ROWS / NW][KL];
 #pragma unroll
             for (int k = 0; k < JT_ROWS / NW; k++) {
                 const uint32_t r = wave + k * NW;
-                lo[k] = r < R ? a.ids[(size_t)row_id[r] * KK + lane] & ~FLAG : 0u;
-                hi[k] = r < R ? a.ids[(size_t)row_id[r] * KK + WAVE + lane] & ~FLAG : 0u;
+#pragma unroll
+                for (int l = 0; l < KL; l++) own[k][l] = r < R ? a.ids[(size_t)row_id[r] * KK + l * WAVE + lane] & ~FLAG : 0u;
             }
 #pragma unroll
             for (int k = 0; k < JT_ROWS / NW; k++) {
                 const uint32_t r = wave + k * NW;
-                if (r < R) {
-                    wave_sort_u32x2(lo[k], hi[k], lane);
-                    row_list[r * KK + lane] = lo[k];
-                    row_list[r * KK + WAVE + lane] = hi[k];
+                if (r < R) { // wave-uniform
+                    if constexpr (KL == 1) own[k][0] = wave_sort_u32(own[k][0], lane);
+                    else wave_sort_u32x2(own[k][0], own[k][KL - 1], lane);
+#pragma unroll
+                    for (int l = 0; l < KL; l++) row_list[r * KK + l * WAVE + lane] = own[k][l];
                 }
             }
-            __syncthreads();
         }
+        tile_dense<NT>(a.dense_mul, smem + L.stage, L.stage_bytes, G, rowptr, R, M, tid, wave, lane);
         // proposals
         for (uint32_t p = tid; p < R * M; p += NT) {
             const uint32_t r = p / M, c = p % M;
@@ -653,12 +661,11 @@ struct GramTileArgs {
     uint32_t index_bits, slot_cap, span;
 };
 
-template <bool NARROW>
-__global__ __launch_bounds__(jt_threads(NARROW)) __attribute__((amdgpu_waves_per_eu(jt_threads(NARROW) / 256, jt_threads(NARROW) / 256))) void gram_tile_kernel(GramTileArgs a) {
-    constexpr int NT = jt_threads(NARROW);
+template <bool NARROW, int NT>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void gram_tile_kernel(GramTileArgs a) {
     a.C.narrow = NARROW ? 1u : 0u;
     extern __shared__ __align__(16) char smem[];
-    const JoinLds L(a.index_bits, a.slot_cap, NARROW);
+    const JoinLds L(a.index_bits, a.slot_cap, NARROW, 0);
     const RankTab T = ranktab_at(smem + L.tab, a.index_bits, a.slot_cap, a.span, NARROW);
     float* G = reinterpret_cast<float*>(smem + L.G);
     unsigned long long* rowptr = reinterpret_cast<unsigned long long*>(smem + L.rowptr);
@@ -702,7 +709,8 @@ __global__ __launch_bounds__(jt_threads(NARROW)) __attribute__((amdgpu_waves_per
             gram_rows_gather(a.C, row_id, R, rowptr, rownnz, tid, NT);
             gram_rows_gather(a.C, col_id, M, rowptr + JT_ROWS, rownnz + JT_ROWS, tid, NT);
             __syncthreads();
-            tile_hybrid_ips<NARROW>(a.C, a.dense_mul, smem + L.tab, T, a.index_bits, a.slot_cap, G, rowptr, rownnz, scan, R, M, a.work + 3, tid, wave, lane);
+            tile_sparse<NARROW, NT>(T, G, rowptr, rownnz, scan, R, M, a.work + 3, tid, wave, lane);
+            tile_dense<NT>(a.dense_mul, smem + L.stage, L.stage_bytes, G, rowptr, R, M, tid, wave, lane);
             for (uint32_t p = tid; p < R * M; p += NT) {
                 const uint32_t r = p / M, c = p % M;
                 out[(size_t)(r0 + r) * GT_MAX + r0 + c] = G[r * JT_STRIDE + c];
@@ -712,11 +720,38 @@ __global__ __launch_bounds__(jt_threads(NARROW)) __attribute__((amdgpu_waves_per
     }
 }
 
-static void join_table_shape(const apoe_corpus* c, uint32_t* index_bits, uint32_t* slot_cap, uint32_t* span) {
-    *span = next_pow2(std::max(c->max_term + 1, 1024u));
-    *index_bits = c->narrow ? 2 * *span : 65536u;
-    const uint32_t want = RT_T * (c->max_nnz_s + c->max_nnz_b);
-    *slot_cap = std::min<uint32_t>(std::max<uint32_t>((want + 63) & ~63u, 256u), (uint32_t)APOE_JOIN_MAX_ROW_TERMS);
+// Table of a tile, and whether two workgroups share a CU (half of its LDS each). The table then takes as many slots as fit, up to
+// eight rows of the longest kind: an average group of eight rows of 180 terms has 1 000 distinct ones, 1 344 slots fit beside a
+// bitmap for a vocabulary of 32 768. A group that exceeds them is done in halves; a corpus with a single row that does
+// would lose that row, so it takes the whole LDS.
+struct TileShape {
+    uint32_t index_bits, slot_cap, span, lds;
+    bool pair;
+};
+static TileShape tile_shape(const apoe_ctx* ctx, const apoe_corpus* c, uint32_t KK) {
+    TileShape s;
+    s.span = next_pow2(std::max(c->max_term + 1, 1024u));
+    s.index_bits = c->narrow ? 2 * s.span : 65536u;
+    const uint32_t longest = c->max_nnz_s + c->max_nnz_b, want = std::max<uint32_t>((RT_T * longest + 63) & ~63u, 256u);
+    const uint32_t half = (uint32_t)(ctx->lds_per_block / 2), floor_slots = std::max(longest, 256u);
+    s.slot_cap = want;
+    while (s.slot_cap > floor_slots && JoinLds(s.index_bits, s.slot_cap, c->narrow, KK).total > half) s.slot_cap -= 64;
+    s.pair = s.slot_cap >= floor_slots && JoinLds(s.index_bits, s.slot_cap, c->narrow, KK).total <= half;
+    if (!s.pair) s.slot_cap = std::min<uint32_t>(want, (uint32_t)APOE_JOIN_MAX_ROW_TERMS);
+    s.lds = JoinLds(s.index_bits, s.slot_cap, c->narrow, KK).total;
+    return s;
+}
+
+// A persistent grid of tile workgroups.
+template <typename Args>
+static int launch_tiles(apoe_ctx* ctx, void (*kernel)(Args), const TileShape& shape, const Args& a) {
+    const int threads = shape.pair ? JT_PAIR_THREADS : JT_SOLO_THREADS;
+    APOE_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)shape.lds));
+    int per_cu = 1;
+    APOE_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(kernel), threads, shape.lds));
+    kernel<<<(uint32_t)std::max(per_cu, 1) * (uint32_t)ctx->num_cus, threads, shape.lds, ctx->stream>>>(a);
+    APOE_HIP(hipGetLastError());
+    return APOE_OK;
 }
 
 int join_alloc(apoe_knn* g) {
@@ -748,10 +783,8 @@ int launch_nnd_join_iterate(apoe_knn* g) {
     const bool k128 = g->K == 128;
     const uint32_t halves = g->K / 64;
     if (!g->prop.p) APOE_TRY(join_alloc(g));
-    uint32_t index_bits, slot_cap, span;
-    join_table_shape(g->corpus, &index_bits, &slot_cap, &span);
-    const JoinLds L(index_bits, slot_cap, g->corpus->narrow, g->K);
-    APOE_REQUIRE(L.total <= ctx->lds_per_block, "the local-join tile needs %u bytes of LDS, a workgroup may have %zu", L.total, ctx->lds_per_block);
+    const TileShape shape = tile_shape(ctx, g->corpus, g->K);
+    APOE_REQUIRE(shape.lds <= ctx->lds_per_block, "the local-join tile needs %u bytes of LDS, a workgroup may have %zu", shape.lds, ctx->lds_per_block);
 
     APOE_HIP(hipMemsetAsync(g->counter.p, 0, sizeof(unsigned long long), st)); // [0] inserted; [2], [3] accumulate over the build
     fill_u32_kernel2<<<1024, 256, 0, st>>>(g->pick_cnt.p, (uint64_t)n + 1, 0u);
@@ -785,17 +818,17 @@ int launch_nnd_join_iterate(apoe_knn* g) {
     a.tile_v = g->tile_v.p;
     a.prop = g->prop.p;
     a.work = g->join_work.p;
-    a.index_bits = index_bits;
-    a.slot_cap = slot_cap;
-    a.span = span;
-    auto kernel = k128 ? (g->corpus->narrow ? &join_tile_kernel<true, 128> : &join_tile_kernel<false, 128>)
-                       : (g->corpus->narrow ? &join_tile_kernel<true, 64> : &join_tile_kernel<false, 64>);
-    APOE_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)L.total));
-    int per_cu = 1;
-    APOE_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(kernel), jt_threads(g->corpus->narrow), L.total));
-    if (per_cu < 1) per_cu = 1;
-    kernel<<<(uint32_t)per_cu * (uint32_t)ctx->num_cus, jt_threads(g->corpus->narrow), L.total, st>>>(a);
-    APOE_HIP(hipGetLastError());
+    a.index_bits = shape.index_bits;
+    a.slot_cap = shape.slot_cap;
+    a.span = shape.span;
+    const bool narrow = g->corpus->narrow;
+    auto kernel_of = [&](auto threads) {
+        constexpr int NT = decltype(threads)::value;
+        return k128 ? (narrow ? &join_tile_kernel<true, 128, NT> : &join_tile_kernel<false, 128, NT>)
+                    : (narrow ? &join_tile_kernel<true, 64, NT> : &join_tile_kernel<false, 64, NT>);
+    };
+    APOE_TRY(launch_tiles(ctx, shape.pair ? kernel_of(std::integral_constant<int, JT_PAIR_THREADS>{}) : kernel_of(std::integral_constant<int, JT_SOLO_THREADS>{}),
+                          shape, a));
     if (k128) join_apply_kernel<128><<<(n + 3) / 4, 256, 0, st>>>(n, g->ids.p, g->dist.p, g->prop.p, g->rev.p, g->rev_cnt.p, g->join_work.p + JOIN_COUNT_AT);
     else join_apply_kernel<64><<<(n + 3) / 4, 256, 0, st>>>(n, g->ids.p, g->dist.p, g->prop.p, g->rev.p, g->rev_cnt.p, g->join_work.p + JOIN_COUNT_AT);
     APOE_HIP(hipGetLastError());
@@ -811,10 +844,8 @@ int launch_gram_tiles(apoe_knn* g, uint32_t node0, uint32_t n_nodes, float* gram
     hipStream_t st = ctx->stream;
     APOE_REQUIRE(g->K <= GT_MAX, "Gram tiles are built for lists of at most %u entries", GT_MAX);
     if (!g->join_work.p) APOE_TRY(g->join_work.alloc(JOIN_COUNT_AT + JOIN_COUNT_PARTS * 8));
-    uint32_t index_bits, slot_cap, span;
-    join_table_shape(g->corpus, &index_bits, &slot_cap, &span);
-    const JoinLds L(index_bits, slot_cap, g->corpus->narrow);
-    APOE_REQUIRE(L.total <= ctx->lds_per_block, "a Gram tile needs %u bytes of LDS, a workgroup may have %zu", L.total, ctx->lds_per_block);
+    const TileShape shape = tile_shape(ctx, g->corpus, 0);
+    APOE_REQUIRE(shape.lds <= ctx->lds_per_block, "a Gram tile needs %u bytes of LDS, a workgroup may have %zu", shape.lds, ctx->lds_per_block);
     fill_u64_kernel<<<1, 64, 0, st>>>(g->join_work.p, 8, 0ull);
     APOE_HIP(hipGetLastError());
     GramTileArgs a{};
@@ -827,16 +858,15 @@ int launch_gram_tiles(apoe_knn* g, uint32_t node0, uint32_t n_nodes, float* gram
     a.dist = g->dist.p;
     a.gram = gram;
     a.work = g->join_work.p;
-    a.index_bits = index_bits;
-    a.slot_cap = slot_cap;
-    a.span = span;
-    auto kernel = g->corpus->narrow ? &gram_tile_kernel<true> : &gram_tile_kernel<false>;
-    APOE_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)L.total));
-    int per_cu = 1;
-    APOE_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(kernel), jt_threads(g->corpus->narrow), L.total));
-    if (per_cu < 1) per_cu = 1;
-    kernel<<<(uint32_t)per_cu * (uint32_t)ctx->num_cus, jt_threads(g->corpus->narrow), L.total, st>>>(a);
-    APOE_HIP(hipGetLastError());
+    a.index_bits = shape.index_bits;
+    a.slot_cap = shape.slot_cap;
+    a.span = shape.span;
+    auto kernel_of = [&](auto threads) {
+        constexpr int NT = decltype(threads)::value;
+        return g->corpus->narrow ? &gram_tile_kernel<true, NT> : &gram_tile_kernel<false, NT>;
+    };
+    APOE_TRY(launch_tiles(ctx, shape.pair ? kernel_of(std::integral_constant<int, JT_PAIR_THREADS>{}) : kernel_of(std::integral_constant<int, JT_SOLO_THREADS>{}),
+                          shape, a));
     if (unfit) {
         unsigned long long h[4] = {0, 0, 0, 0};
         APOE_HIP(hipMemcpyAsync(h, g->join_work.p, sizeof(h), hipMemcpyDeviceToHost, st));
@@ -849,9 +879,7 @@ int launch_gram_tiles(apoe_knn* g, uint32_t node0, uint32_t n_nodes, float* gram
 // Whether launch_gram_tiles can serve this handle: lists of at most 128 entries, rows that fit a tile's table, LDS for a tile.
 bool gram_tiles_fit(const apoe_knn* g) {
     if (g->K > GT_MAX || g->corpus->max_nnz_s + g->corpus->max_nnz_b > (uint32_t)APOE_JOIN_MAX_ROW_TERMS) return false;
-    uint32_t index_bits, slot_cap, span;
-    join_table_shape(g->corpus, &index_bits, &slot_cap, &span);
-    return JoinLds(index_bits, slot_cap, g->corpus->narrow).total <= g->ctx->lds_per_block;
+    return tile_shape(g->ctx, g->corpus, 0).lds <= g->ctx->lds_per_block;
 }
 
 // Pairs evaluated and rows gathered by the tiles of the last step, and whether a row did not fit the table.

@@ -35,3 +35,63 @@ def test_first_step_on_lists_of_few_documents(gpu_world, columns):
     assert same.mean() >= 0.99
     assert_dist_close(gd[same], st.dist[same], "stored distances")
     knn.close()
+
+
+def step_equals_oracle(ctx, corpus, oracle_corpus, ids, K):
+    """One join step from the lists `ids` (reverse lists empty), row for row the oracle's."""
+    import apoe
+    import oracle as O
+    n = len(ids)
+    dist = np.sort(np.random.default_rng(1).random((n, K)).astype(np.float32) + 900, axis=1)
+    st = O.nnd_init(n, K, 1)
+    st.ids[:] = ids
+    st.dist[:] = dist
+    knn = apoe.Knn(ctx, corpus, K, 7.0)
+    knn.upload(ids, dist)
+    knn.set_join(1)
+    ins = knn.iterate(last=True)
+    oins, _ = O.join_iterate(oracle_corpus, 7.0, st, slots=2 * K)
+    got, gd = knn.download()
+    assert abs(ins - oins) <= 0.001 * oins + 1
+    same = np.all(got == (st.ids & 0x7FFFFFFF), axis=1)
+    assert same.mean() >= 0.99
+    assert_dist_close(gd[same], st.dist[same], "stored distances")
+    knn.close()
+
+
+@pytest.mark.parametrize("K", [64, 128])
+@pytest.mark.parametrize("pickers", [1, 8, 9, 11, 12, 13, 16, 17, 22, 25, 26, 31, 32, 33])
+def test_tiles_of_a_given_number_of_pickers(gpu_world, pickers, K):
+    """Blocks of `pickers` documents pick the same four nodes: tiles of that many rows (staged whole, in halves or in quarters;
+    one or two accumulators; groups of eight pivots whole and partial) with the 64 or 128 columns of a full list."""
+    w = gpu_world
+    n = w["C"].n
+    rng = np.random.default_rng(pickers)
+    ids = np.stack([rng.choice(n, K, replace=False) for _ in range(n)]).astype(np.uint32)
+    ids[:, :4] = 4 * (np.arange(n) // pickers)[:, None] % (n - 4) + np.arange(4)
+    step_equals_oracle(w["ctx"], w["gc"], w["C"], ids, K)
+
+
+@pytest.mark.parametrize("shift,terms", [(0, 1200), (0, 1345), (0, 1700), (70000, 900), (70000, 1100)])
+def test_a_row_that_takes_the_whole_table(gpu_ctx, shift, terms):
+    """One document's row fills the table that two workgroups per CU leave room for, or exceeds it: then one workgroup per CU runs
+    the tiles (`shift`: term ids past 65535 take the wide pair format, whose table hashes)."""
+    import apoe
+    import apoe_synth as S
+    import oracle as O
+    n, K, row = 600, 64, 17
+    dense, s_off, s_idx, s_val, b_off, b_idx, b_val = S.to_numpy(S.corpus(n, seed=5, device="cpu"))
+    rng = np.random.default_rng(terms)
+    cnt = np.diff(s_off.astype(np.int64))
+    cnt[row] = terms
+    off = np.concatenate([[0], np.cumsum(cnt)]).astype(np.uint32)
+    keep = lambda a, new: np.concatenate([a[:s_off[row]], new, a[s_off[row + 1]:]]).astype(a.dtype)
+    idx = keep(s_idx, np.sort(rng.choice(30000, terms, replace=False)))
+    val = keep(s_val, rng.uniform(0.5, 2.0, terms))
+    arrays = (dense, off, idx, val, b_off, (b_idx + np.uint32(shift)).astype(np.uint32), b_val)
+    gc = apoe.Corpus(gpu_ctx, *arrays)
+    assert gc.pair_bytes() == (8 if shift else 6)
+    ids = np.stack([rng.choice(n, K, replace=False) for _ in range(n)]).astype(np.uint32)
+    ids[:, 0] = row  # every document picks the long row, and it is a column wherever it is not
+    step_equals_oracle(gpu_ctx, gc, O.HybridSet(*arrays), ids, K)
+    gc.close()
