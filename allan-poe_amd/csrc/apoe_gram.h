@@ -117,19 +117,21 @@ __device__ __forceinline__ uint2 row_pairs_get(const RowPairs& r, int c, uint32_
     return kv;
 }
 
-// The 64 gathered rows are kept in LDS as the address of the pair array and one word with
-// nnz (low half) and nnz_s (high half); nnz <= 2 * DESC_NNZ_MAX fits 16 bits.
+// The gathered rows are kept in LDS as the byte offset of their pair array in the record buffer and one word with
+// nnz (low half) and nnz_s (high half); nnz <= 2 * DESC_NNZ_MAX fits 16 bits. Offsets and not addresses: the compiler knows
+// C.recs + offset for device memory, while an address read from LDS may point anywhere and its loads are flat ones, which count
+// as LDS accesses too: every wait for a table read behind them waits for the rows that were requested ahead.
 __device__ __forceinline__ void gram_rows_gather(const CorpusView& C, const uint32_t* ids, uint32_t m, unsigned long long* rowptr, uint32_t* rownnz,
                                                  int tid, int nthreads) {
     for (uint32_t i = tid; i < m; i += nthreads) {
         const uint64_t d = C.desc[ids[i]];
-        rowptr[i] = (unsigned long long)(C.recs + desc_off(d) * 16 + DENSE_BYTES);
+        rowptr[i] = desc_off(d) * 16 + DENSE_BYTES;
         rownnz[i] = (desc_nnz_s(d) + desc_nnz_b(d)) | (desc_nnz_s(d) << 16);
     }
 }
 __device__ __forceinline__ Pairs gram_row(const CorpusView& C, const unsigned long long* rowptr, const uint32_t* rownnz, uint32_t i) {
     Pairs p;
-    p.base = reinterpret_cast<const char*>(rowptr[i]);
+    p.base = C.recs + rowptr[i];
     const uint32_t w = rownnz[i];
     p.nnz = w & 0xFFFFu;
     p.ns = w >> 16;

@@ -165,6 +165,7 @@ struct apoe_knn {
     // local-join step (apoe_knn_set_join): the picks of a step grouped by the picked node, the tiles, the proposal rows
     int join = 0; // 0: expansion step, 1: local join, 2: local join that offers a pair to both endpoints
     bool join_symmetric = false;
+    bool settled = false; // few pairs of a join step still enter a list: the next one asks the sketches before it reads dense rows
     apoe::DevBuf<uint32_t> picks, pick_cnt, pick_off, pick_fill, pick_src, tile_cnt, tile_off, tile_v;
     apoe::DevBuf<unsigned long long> prop, join_work;
     apoe::DevBuf<char> scan_tmp;
@@ -195,7 +196,7 @@ int search_static_workspace(int device, char** out); // device address of the st
 int launch_nnd_init(apoe_knn* g, uint64_t seed);
 int launch_nnd_iterate(apoe_knn* g, uint64_t* inserted);
 int launch_nnd_join_iterate(apoe_knn* g);
-int join_step_counters(apoe_knn* g, unsigned long long* out3);
+int join_step_finish(apoe_knn* g, unsigned long long* unfit);
 int launch_gram_tiles(apoe_knn* g, uint32_t node0, uint32_t n_nodes, float* gram, unsigned long long* unfit);
 bool gram_tiles_fit(const apoe_knn* g);
 int launch_nnd_merge_reverse(apoe_knn* g);

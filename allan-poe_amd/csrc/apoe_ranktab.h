@@ -147,8 +147,9 @@ __device__ __forceinline__ uint32_t ranktab_slot(uint2 w, uint32_t idx) {
 // must hand out the same pairs both times). Returns the number of distinct terms, or EMPTY if they
 // exceed the slot capacity or the overflow list (the table is then unusable: the caller retries with fewer pivots).
 // Ends with a barrier: the table is ready on return.
+// A group of at most four pivots needs the first plane of the values only (`planes` = 1, wave-uniform).
 template <bool NARROW, typename EachFn>
-__device__ __forceinline__ uint32_t ranktab_build_each(const RankTab& T, EachFn each, uint32_t* scan, int tid, int nthreads) {
+__device__ __forceinline__ uint32_t ranktab_build_each(const RankTab& T, EachFn each, uint32_t* scan, int tid, int nthreads, int planes = RT_T / 4) {
     const uint32_t total = ranktab_build_bits<NARROW>(T, each, T.slot_cap, scan, tid, nthreads);
     if (total > T.slot_cap) {
         __syncthreads();
@@ -156,7 +157,7 @@ __device__ __forceinline__ uint32_t ranktab_build_each(const RankTab& T, EachFn 
     }
     for (uint32_t s = tid; s < total; s += nthreads) {
         T.vals[s] = make_float4(0.f, 0.f, 0.f, 0.f);
-        T.vals[T.slot_cap + s] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (planes > 1) T.vals[T.slot_cap + s] = make_float4(0.f, 0.f, 0.f, 0.f);
     }
     if (!NARROW) {
         for (uint32_t s = tid; s < total; s += nthreads) T.keys[s] = EMPTY;
@@ -297,7 +298,7 @@ __device__ __forceinline__ void rt_row_load(RtRow<false>& r, const Pairs& sp, in
 // register window only. Everything else as ranktab_build_each.
 template <bool NARROW>
 __device__ __forceinline__ uint32_t ranktab_build_rows(const RankTab& T, const RtRow<NARROW>& pr, uint32_t shape, bool mine, int t, const Pairs& tail,
-                                                       uint32_t* scan, int tid, int nthreads) {
+                                                       uint32_t* scan, int tid, int nthreads, int planes = RT_T / 4) {
     const int lane = tid & (WAVE - 1);
     const uint32_t nnz = mine ? shape & 0xFFFFu : 0u, ns = shape >> 16;
     return ranktab_build_each<NARROW>(T, [&](auto f) {
@@ -307,27 +308,31 @@ __device__ __forceinline__ uint32_t ranktab_build_rows(const RankTab& T, const R
             if (j < nnz) f(make_uint2(pr.key(c), pr.v[c]), NARROW ? j >= ns : false, t);
         }
         for (uint32_t j = RT_CHUNKS * WAVE + lane; j < nnz; j += WAVE) f(tail.raw(j), j >= ns, t);
-    }, scan, tid, nthreads);
+    }, scan, tid, nthreads, planes);
 }
 
 // NB streamed rows against the table at once: acc[r][0..7] += per-pivot sums of this lane's pairs of row r.
 // All bitmap reads of the batch are issued before the first value read; the value reads follow in two halves (chunks
 // 0-1, then 2-3 of every row), each issued whole before its multiplies: three LDS round trips per batch whatever NB
 // is, and at most NB x 2 x 8 value registers in flight. shape[r] = nnz | ns << 16 of row r (wave-uniform;
-// 0: the row is not there); tail(r) gives the Pairs of row r for the pairs beyond the register window.
-template <bool NARROW, int NB, typename TailFn>
+// 0: the row is not there); tail(r) gives the Pairs of row r for the pairs beyond the register window. NP = 4: the group has
+// at most four pivots, the second plane is not read.
+template <bool NARROW, int NB, int NP = RT_T, typename TailFn>
 __device__ __forceinline__ void ranktab_probe_rows(const RankTab& T, const RtRow<NARROW> (&rows)[NB], const uint32_t (&shape)[NB], TailFn tail,
-                                                   uint32_t n_ovf, float (&acc)[NB][RT_T], int lane) {
+                                                   uint32_t n_ovf, float (&acc)[NB][NP], int lane) {
+    static_assert(NP == 4 || NP == RT_T, "one or both planes");
     static_assert(RT_CHUNKS % 2 == 0, "the value reads go out in two halves");
     auto add8 = [&](int r, float m, const float4& lo, const float4& hi) {
         acc[r][0] = fmaf(m, lo.x, acc[r][0]);
         acc[r][1] = fmaf(m, lo.y, acc[r][1]);
         acc[r][2] = fmaf(m, lo.z, acc[r][2]);
         acc[r][3] = fmaf(m, lo.w, acc[r][3]);
-        acc[r][4] = fmaf(m, hi.x, acc[r][4]);
-        acc[r][5] = fmaf(m, hi.y, acc[r][5]);
-        acc[r][6] = fmaf(m, hi.z, acc[r][6]);
-        acc[r][7] = fmaf(m, hi.w, acc[r][7]);
+        if constexpr (NP > 4) {
+            acc[r][4] = fmaf(m, hi.x, acc[r][4]);
+            acc[r][5] = fmaf(m, hi.y, acc[r][5]);
+            acc[r][6] = fmaf(m, hi.z, acc[r][6]);
+            acc[r][7] = fmaf(m, hi.w, acc[r][7]);
+        }
     };
     auto overflow = [&](int r, uint32_t key, uint32_t val_bits, bool in) {
         for (uint32_t o = 0; o < n_ovf; o++) { // wave-uniform count, zero for narrow corpora
@@ -360,13 +365,17 @@ __device__ __forceinline__ void ranktab_probe_rows(const RankTab& T, const RtRow
                 const bool in = rt_pair(h + c, lane) < nnz;
                 p[r][c] = ranktab_locate<NARROW>(T, w[r][h + c], index_of(r, h + c), rows[r].v[h + c], in);
                 lo[r][c] = T.vals[p[r][c].slot];
-                hi[r][c] = T.vals[T.slot_cap + p[r][c].slot];
+                if constexpr (NP > 4) hi[r][c] = T.vals[T.slot_cap + p[r][c].slot];
+                else hi[r][c] = make_float4(0.f, 0.f, 0.f, 0.f);
                 ok[r][c] = true;
                 if (!NARROW) ok[r][c] = p[r][c].mul == 0.f || T.keys[p[r][c].slot] == rows[r].key(h + c);
             }
         }
 #pragma unroll
-        for (int r = 0; r < NB; r++) asm volatile("" : "+v"(lo[r][0].x), "+v"(lo[r][1].x), "+v"(hi[r][0].x), "+v"(hi[r][1].x));
+        for (int r = 0; r < NB; r++) {
+            if constexpr (NP > 4) asm volatile("" : "+v"(lo[r][0].x), "+v"(lo[r][1].x), "+v"(hi[r][0].x), "+v"(hi[r][1].x));
+            else asm volatile("" : "+v"(lo[r][0].x), "+v"(lo[r][1].x));
+        }
 #pragma unroll
         for (int r = 0; r < NB; r++) {
             const uint32_t nnz = shape[r] & 0xFFFFu;
@@ -391,7 +400,7 @@ __device__ __forceinline__ void ranktab_probe_rows(const RankTab& T, const RtRow
                 const uint32_t ix = ranktab_index<NARROW>(T, kv.x, NARROW ? j >= ns : (int)kv.x < 0);
                 const uint2 ww = T.word[in ? ix >> 5 : 0u];
                 const RankProbe q = ranktab_locate<NARROW>(T, ww, ix, kv.y, in);
-                const float4 vl = T.vals[q.slot], vh = T.vals[T.slot_cap + q.slot];
+                const float4 vl = T.vals[q.slot], vh = NP > 4 ? T.vals[T.slot_cap + q.slot] : make_float4(0.f, 0.f, 0.f, 0.f);
                 bool good = true;
                 if (!NARROW) good = q.mul == 0.f || T.keys[q.slot] == kv.x;
                 add8(r, good ? q.mul : 0.f, vl, vh);

@@ -528,6 +528,7 @@ int apoe_nnd_init(apoe_knn* g, uint64_t seed) {
     APOE_TRY(timed(g->ctx, &ms, [&]() { return launch_nnd_init(g, seed); }));
     g->elapsed_ms = ms;
     g->ready = true;
+    g->settled = false; // random lists
     g->pruned = false;
     return APOE_OK;
 }
@@ -552,11 +553,11 @@ int apoe_nnd_iterate(apoe_knn* g, int last, uint64_t* inserted) {
         *inserted = h;
     }
     if (g->join) { // a picker row whose terms did not fit the tile's table was evaluated without its sparse part
-        unsigned long long c3[3] = {0, 0, 0};
-        APOE_TRY(join_step_counters(g, c3));
-        if (c3[2]) g->ready = false;
-        APOE_REQUIRE_STATE(c3[2] == 0, "the local-join step could not hold the sparse terms of %llu rows in its table (too many terms share table "
-                           "slots): the lists of this handle are not valid, build again with the expansion step (apoe_knn_set_join(..., 0))", c3[2]);
+        unsigned long long unfit = 0;
+        APOE_TRY(join_step_finish(g, &unfit));
+        if (unfit) g->ready = false;
+        APOE_REQUIRE_STATE(unfit == 0, "the local-join step could not hold the sparse terms of %llu rows in its table (too many terms share table "
+                           "slots): the lists of this handle are not valid, build again with the expansion step (apoe_knn_set_join(..., 0))", unfit);
     }
     return APOE_OK;
 }
@@ -637,6 +638,7 @@ int apoe_knn_upload(apoe_knn* g, const uint32_t* ids, const float* dist) {
     APOE_TRY(launch_norms(g->ctx, g->corpus, g->dense_scale, g->norms.p));
     APOE_HIP(hipStreamSynchronize(st));
     g->ready = true;
+    g->settled = true; // lists worth saving
     g->pruned = false;
     return APOE_OK;
 }

@@ -293,7 +293,7 @@ __global__ __launch_bounds__(PS_THREADS) void prune_select_kernel(CorpusView C, 
     uint32_t* o_fwd = reinterpret_cast<uint32_t*>(smem + L.o_fwd);
     uint32_t* o_det = reinterpret_cast<uint32_t*>(smem + L.o_det);
     uint32_t* o_kw = reinterpret_cast<uint32_t*>(smem + L.o_kw);
-    volatile uint32_t* ctl = reinterpret_cast<volatile uint32_t*>(smem + L.ctl);
+    uint32_t* ctl = reinterpret_cast<uint32_t*>(smem + L.ctl);
 
     const int tid = threadIdx.x, wave = tid / WAVE, lane = lane_id();
     constexpr uint32_t NWV = PS_THREADS / WAVE;
@@ -699,7 +699,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
     uint32_t* o_fwd = reinterpret_cast<uint32_t*>(smem + L.o_fwd);
     uint32_t* o_det = reinterpret_cast<uint32_t*>(smem + L.o_det);
     uint32_t* o_kw = reinterpret_cast<uint32_t*>(smem + L.o_kw);
-    volatile uint32_t* ctl = reinterpret_cast<volatile uint32_t*>(smem + L.ctl);
+    uint32_t* ctl = reinterpret_cast<uint32_t*>(smem + L.ctl);
 
     const int tid = threadIdx.x, wave = (int)uniform(tid / WAVE), lane = lane_id();
     const uint32_t u = blockIdx.x, umask = umap_slots - 1, mmask = map_slots - 1;
@@ -933,10 +933,10 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
     __syncthreads();
     if (rank) {
         const RankTab T = ranktab_at(reinterpret_cast<char*>(tabs), rank_bits, rank_slots, rank_span, NARROW);
-        gram_sparse_rank<NARROW>(C, m, G, T, ovf_cnt, rowptr, rownnz, own, own_shape, (uint32_t*)&ctl[PC_FAIL], tid, NT);
-    } else if (union_slots) gram_sparse_union(C, nb_id, m, G, reinterpret_cast<char*>(tabs), union_slots, ovf_cnt, rowptr, rownnz, (uint32_t*)&ctl[PC_FAIL], tid, NT);
-    else if (tgroup == 8) gram_sparse_64<8>(C, nb_id, m, G, tabs, term_slots, ovf_cnt, rowptr, rownnz, (uint32_t*)&ctl[PC_FAIL], tid, NT);
-    else gram_sparse_64<4>(C, nb_id, m, G, tabs, term_slots, ovf_cnt, rowptr, rownnz, (uint32_t*)&ctl[PC_FAIL], tid, NT);
+        gram_sparse_rank<NARROW>(C, m, G, T, ovf_cnt, rowptr, rownnz, own, own_shape, &ctl[PC_FAIL], tid, NT);
+    } else if (union_slots) gram_sparse_union(C, nb_id, m, G, reinterpret_cast<char*>(tabs), union_slots, ovf_cnt, rowptr, rownnz, &ctl[PC_FAIL], tid, NT);
+    else if (tgroup == 8) gram_sparse_64<8>(C, nb_id, m, G, tabs, term_slots, ovf_cnt, rowptr, rownnz, &ctl[PC_FAIL], tid, NT);
+    else gram_sparse_64<4>(C, nb_id, m, G, tabs, term_slots, ovf_cnt, rowptr, rownnz, &ctl[PC_FAIL], tid, NT);
     // keyword flags of all pairs at once (index.cu:637,651-654): flag(c, s) = (R[s] & ~R[c]) != 0. A thread takes one row c and
     // one of its two flag words: its own mask stays in registers (the first four words), the lanes of a wave read the same R[s]
     if (tid < 2 * (int)K) {

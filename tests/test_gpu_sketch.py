@@ -91,3 +91,44 @@ def test_half_precision_walk(gpu_ctx, kind):
         a, ad, _ = apoe.search(gpu_ctx, gc, gq, gg, w3, 48, variant=0x200)
         b, bd, _ = apoe.search(gpu_ctx, gc, gq, gg, w3, 48, variant=0x300)
         assert np.array_equal(a, b) and np.array_equal(ad, bd)
+
+
+@pytest.mark.parametrize("K,mode", [(64, 1), (64, 2), (128, 1)])
+@pytest.mark.parametrize("wide", [False, True])
+@pytest.mark.parametrize("kind", ["plain", "spikes"])
+def test_join_step_from_settled_lists(gpu_ctx, kind, wide, K, mode):
+    """Uploaded lists count as settled: a join step asks the sketches which columns of a tile it can leave out. From the exact lists with
+    three entries in ten replaced by random documents, a step's lists hold the oracle's distances, row for row."""
+    import apoe
+    import oracle as O
+    corpus, _, _, _ = world(kind, 6, wide)
+    dense = corpus[0] / np.linalg.norm(corpus[0], axis=1, keepdims=True) * np.random.default_rng(8).uniform(0.5, 2.0, (N, 1)).astype(np.float32)
+    dense[::97] = 0
+    idx = np.random.default_rng(9).integers(1, 300, (N, 12)).cumsum(1).astype(np.uint32) + np.uint32(70000 if wide else 0)  # no term twice in a row
+    corpus = (dense.astype(np.float32), corpus[1], idx.reshape(-1), corpus[3], corpus[4], idx[::-1].reshape(-1).copy(), corpus[6])
+    C = O.HybridSet(*corpus)
+    rng = np.random.default_rng(K)
+    ids, _ = O.bruteforce_knn_self(C, 7.0, K)
+    some = rng.random(ids.shape) < 0.3
+    ids[some] = rng.integers(0, N, int(some.sum()))
+    dist = O.distance_pairs(C, 7.0, np.repeat(np.arange(N, dtype=np.uint32), K), ids.reshape(-1)).reshape(N, K)
+    order = np.argsort(dist, 1, kind="stable")
+    ids, dist = np.take_along_axis(ids, order, 1), np.take_along_axis(dist, order, 1)
+    st = O.nnd_init(N, K, 1)  # its reverse lists are empty
+    st.ids[:], st.dist[:] = ids, dist
+    gc = apoe.Corpus(gpu_ctx, *corpus)
+    knn = apoe.Knn(gpu_ctx, gc, K, 7.0)
+    knn.upload(ids, dist)
+    knn.set_join(mode)
+    ins = knn.iterate(last=True)
+    oins, _ = O.join_iterate(C, 7.0, st, slots=2 * K, symmetric=mode == 2)
+    got, gd = knn.download()
+    assert 0 < ins and abs(ins - oins) <= 0.002 * oins + 2
+    # a list that lost an entry differs from there on by the gap between two entries, about a hundredth of its range of 50; a different
+    # order of the float sums moves a distance by at most 1024 x 2^-24 = 6e-5 of it, and may swap neighbours
+    scale = np.maximum(1.0, np.abs(st.dist))
+    same = np.all(np.abs(gd - st.dist) <= 6e-5 * scale, axis=1)
+    assert same.mean() >= 0.999, np.flatnonzero(~same)[:10]
+    assert np.mean(got == (st.ids & 0x7FFFFFFF)) >= 0.99
+    knn.close()
+    gc.close()
