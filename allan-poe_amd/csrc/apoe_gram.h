@@ -75,13 +75,16 @@ __device__ __forceinline__ void gram_dense_upper(const CorpusView& C, const uint
     }
 }
 
+// The product of rows i < j goes to G[j][i], below the diagonal (the sparse part stands at G[i][j]).
 __device__ __forceinline__ void gram_dense_store(float* G, int tile, int lane, const floatx16& acc, float dense_mul, bool add) {
     const int ti = tile >> 1, tj = tile & 1;
 #pragma unroll
     for (int v = 0; v < 16; v++) {
-        const int i = 8 * (v / 4) + 4 * (lane >> 5) + (v % 4), j = lane & 31;
-        float* at = &G[(ti * 32 + i) * GRAM_STRIDE + tj * 32 + j];
-        *at = add ? *at + dense_mul * acc[v] : dense_mul * acc[v];
+        const int i = ti * 32 + 8 * (v / 4) + 4 * (lane >> 5) + (v % 4), j = tj * 32 + (lane & 31);
+        if (i < j) {
+            float* at = &G[j * GRAM_STRIDE + i];
+            *at = add ? *at + dense_mul * acc[v] : dense_mul * acc[v];
+        }
     }
 }
 
@@ -92,8 +95,7 @@ __device__ __forceinline__ void gram_dense_store(float* G, int tile, int lane, c
 // probe loop: a lane issues the reads for all its terms and all T pivots back to back.
 // Every later row is read once per group (pairs in registers, the next row's loads already
 // in flight), per-lane partial sums are reduced once per (row, pivot) with DPP adds, and
-// lane 0 adds the result to G. Two barriers per group of T pivots; the lower triangle is
-// mirrored at the end.
+// lane 0 adds the result to G (above the diagonal). Two barriers per group of T pivots.
 constexpr int GRAM_CHUNKS = 5;  // 64-pair chunks of a row kept in registers (320 pairs)
 constexpr int GRAM_OVF = 32;    // overflow entries per pivot table
 
@@ -154,7 +156,7 @@ __device__ __forceinline__ Slots3 gram_slots3(uint32_t key, uint32_t mask) {
 // tabs: T tables of `slots` entries, then T overflow lists of GRAM_OVF entries; ovf_cnt[T];
 // rowptr/rownnz: LDS scratch for 64 rows; *fail is set when an overflow list is too short
 // (the caller must then discard G). All threads of the block call it; G must already hold
-// the dense part. slots >= 2 x the longest row.
+// zeros above the diagonal. slots >= 2 x the longest row.
 template <int T>
 __device__ __forceinline__ void gram_sparse_64(const CorpusView& C, const uint32_t* ids, uint32_t m, float* G, uint2* tabs, uint32_t slots,
                                                uint32_t* ovf_cnt, unsigned long long* rowptr, uint32_t* rownnz, uint32_t* fail, int tid,
@@ -260,11 +262,6 @@ __device__ __forceinline__ void gram_sparse_64(const CorpusView& C, const uint32
         }
         __syncthreads();
     }
-    for (uint32_t t = tid; t < m * m; t += nthreads) {
-        const uint32_t i = t / m, j = t % m;
-        if (i > j) G[i * GRAM_STRIDE + j] = G[j * GRAM_STRIDE + i];
-    }
-    __syncthreads();
 }
 
 // ---- sparse part, union-table form ----
@@ -471,11 +468,6 @@ __device__ __forceinline__ void gram_sparse_union(const CorpusView& C, const uin
         __syncthreads();
         a0 += nt;
     }
-    for (uint32_t t = tid; t < m * m; t += nthreads) {
-        const uint32_t i = t / m, j = t % m;
-        if (i > j) G[i * GRAM_STRIDE + j] = G[j * GRAM_STRIDE + i];
-    }
-    __syncthreads();
 }
 
 #endif // __HIPCC__

@@ -171,6 +171,7 @@ struct apoe_knn {
     apoe::DevBuf<char> scan_tmp;
     // prune outputs
     apoe::DevBuf<uint32_t> fwd, det, cnt, kw;
+    apoe::DevBuf<uint32_t> open; // prune: which nodes the bounds left open [n], how many, and which
 };
 
 namespace apoe {
@@ -197,7 +198,7 @@ int launch_nnd_init(apoe_knn* g, uint64_t seed);
 int launch_nnd_iterate(apoe_knn* g, uint64_t* inserted);
 int launch_nnd_join_iterate(apoe_knn* g);
 int join_step_finish(apoe_knn* g, unsigned long long* unfit);
-int launch_gram_tiles(apoe_knn* g, uint32_t node0, uint32_t n_nodes, float* gram, unsigned long long* unfit);
+int launch_gram_tiles(apoe_knn* g, const uint32_t* nodes, uint32_t node0, uint32_t n_nodes, float* gram, unsigned long long* unfit);
 bool gram_tiles_fit(const apoe_knn* g);
 int launch_nnd_merge_reverse(apoe_knn* g);
 int launch_prune(apoe_knn* g, uint32_t degree);

@@ -46,7 +46,7 @@ struct PruneLds {
     }
 };
 
-enum { PC_M = 0, PC_NSEL = 1, PC_REJECT = 2, PC_ALLFLAG = 3, PC_CNT = 4, PC_FAIL = 5 };
+enum { PC_M = 0, PC_NSEL = 1, PC_REJECT = 2, PC_ALLFLAG = 3, PC_CNT = 4, PC_FAIL = 5, PC_OPEN = 6, PC_STILL_OPEN = 7 };
 
 // allan_poe (index.cu:539-714) for node u = blockIdx.x:
 //  (a) detour counts over u's sorted list; (b) order by (detour, rank);
@@ -239,6 +239,471 @@ __global__ __launch_bounds__(PR_THREADS) void prune_kernel(CorpusView C, float d
     if (tid == 0) cnt_out[u] = ctl[PC_CNT];
 }
 
+// ---- keys in an LDS map of (key, value) words, open addressing ----
+
+__device__ __forceinline__ void lds_map_insert(uint2* map, uint32_t mask, uint32_t key, uint32_t val) { // a key that is there keeps its value
+    uint32_t h = term_hash(key, mask);
+    while (true) {
+        const uint32_t old = atomicCAS(&map[h].x, EMPTY, key);
+        if (old == EMPTY) { map[h].y = val; return; }
+        if (old == key) return;
+        h = (h + 1) & mask;
+    }
+}
+// The entries of N keys (EMPTY: none): e[k].x == key[k] where it is found. The first slots of all keys are read before any is
+// compared, then the second ones of those that met another key, and so on: as many LDS round trips as the longest chain, not N times that.
+template <int N>
+__device__ __forceinline__ void lds_map_find(const uint2* map, uint32_t mask, const uint32_t (&key)[N], uint2 (&e)[N]) {
+    uint32_t h[N];
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+        h[k] = term_hash(key[k], mask);
+        e[k] = map[h[k]];
+    }
+    while (true) {
+        bool more = false;
+#pragma unroll
+        for (int k = 0; k < N; k++) {
+            const bool go = e[k].x != key[k] && e[k].x != EMPTY && key[k] != EMPTY;
+            h[k] = (h[k] + 1) & mask;
+            if (go) e[k] = map[h[k]];
+            more |= go;
+        }
+        if (__ballot(more) == 0) break;
+    }
+}
+
+// ---- the prune where bounds settle it ----
+//
+// The selection (below) asks of two neighbours c and s of a node only whether <c, s> exceeds either one's norm. |<c, s>_dense - the
+// product of the sketches| has a bound (apoe_device.h), |<c, s>_sparse| is at most the product of the two sparse norms; on a corpus
+// whose dense rows have neighbours that answers all pairs of most nodes (100 000 docs, dense_mul 49: 86 of 100), and neither a dense row nor a
+// pair of terms but the keys of the BM25 terms is read. A node with an open pair sets open[u] and leaves nothing else.
+// Small in LDS and registers, so that many nodes share a CU: it is a chain of short phases (five nodes of 64 rows a CU;
+// 100 000 docs 3.8 ms, with the 14 000 open nodes behind it 6.0 ms, where Gram matrices and selection took 25.4; 30 011 docs K = 128 28.9 -> 10.4 ms).
+template <uint32_t K>
+struct BoundLds {
+    uint32_t stage, row, F, above, below, rowptr, rownnz, idmap, umap, R, nb_id, nb_dist, nrm, det, order, o_fwd, o_det, o_kw, ctl, total;
+    __host__ __device__ BoundLds(uint32_t umap_slots, uint32_t map_slots, uint32_t words) {
+        uint32_t o = 0;
+        // the sketches, a quarter of the dimensions at a time; then what the later phases need
+        stage = o;
+        idmap = o; o += map_slots * 8;
+        umap = o; o += umap_slots * 8;
+        R = o; o += K * words * 4;
+        o = (o + 7) & ~7u;
+        F = o; o += K * (K / 8);
+        if (o < K * (SKETCH_BYTES / 4)) o = K * (SKETCH_BYTES / 4);
+        row = o; o += K * 16;
+        above = o; o += K * (K / 8);
+        below = o; o += K * (K / 8);
+        rowptr = o; o += K * 8;
+        rownnz = o; o += K * 4;
+        nb_id = o; o += K * 4;
+        nb_dist = o; o += K * 4;
+        nrm = o; o += K * 4;
+        det = o; o += K * 4;
+        order = o; o += K * 4;
+        o_fwd = o; o += WAVE * 4;
+        o_det = o; o += WAVE * 4;
+        o_kw = o; o += (1 + APOE_KW_CAND) * 4;
+        ctl = o; o += 16 * 4;
+        total = o;
+    }
+};
+typedef int intx4 __attribute__((ext_vector_type(4)));
+template <uint32_t K, bool NARROW>
+__global__ __launch_bounds__(K * 4) __attribute__((amdgpu_waves_per_eu(4, 8))) void prune_bound_kernel(CorpusView C, float dense_mul, const float* __restrict__ norms,
+                                                               const uint32_t* __restrict__ ids, const float* __restrict__ dist, uint32_t d, uint32_t* fwd,
+                                                               uint32_t* det_out, uint32_t* cnt_out, uint32_t* kw_out, uint32_t umap_slots, uint32_t map_slots,
+                                                               uint32_t words, const SketchMeta* __restrict__ sketch_meta, const uint4* __restrict__ sketch,
+                                                               uint32_t* open) {
+    constexpr int NT = K * 4, NWAVES = NT / WAVE, KL = K / WAVE;
+    constexpr int OWN = K / NWAVES; // rows a wave looks after: wave, wave + NWAVES, ...
+    static_assert(OWN == 16, "two batches of eight rows");
+    C.narrow = NARROW ? 1u : 0u;
+    extern __shared__ __align__(16) char smem[];
+    const BoundLds<K> L(umap_slots, map_slots, words);
+    intx4* stage = reinterpret_cast<intx4*>(smem + L.stage);
+    uint2* idmap = reinterpret_cast<uint2*>(smem + L.idmap);
+    uint2* umap = reinterpret_cast<uint2*>(smem + L.umap);
+    uint32_t* R = reinterpret_cast<uint32_t*>(smem + L.R);
+    uint64_t* F = reinterpret_cast<uint64_t*>(smem + L.F); // [K][KL], as above and below
+    uint64_t* above = reinterpret_cast<uint64_t*>(smem + L.above);
+    uint64_t* below = reinterpret_cast<uint64_t*>(smem + L.below);
+    float4* row = reinterpret_cast<float4*>(smem + L.row); // dense norm, scale and error of the sketch, bound of the norm of the sparse part
+    unsigned long long* rowptr = reinterpret_cast<unsigned long long*>(smem + L.rowptr);
+    uint32_t* rownnz = reinterpret_cast<uint32_t*>(smem + L.rownnz);
+    uint32_t* nb_id = reinterpret_cast<uint32_t*>(smem + L.nb_id);
+    float* nb_dist = reinterpret_cast<float*>(smem + L.nb_dist);
+    float* nrm = reinterpret_cast<float*>(smem + L.nrm);
+    uint32_t* det = reinterpret_cast<uint32_t*>(smem + L.det);
+    uint32_t* order = reinterpret_cast<uint32_t*>(smem + L.order);
+    uint32_t* o_fwd = reinterpret_cast<uint32_t*>(smem + L.o_fwd);
+    uint32_t* o_det = reinterpret_cast<uint32_t*>(smem + L.o_det);
+    uint32_t* o_kw = reinterpret_cast<uint32_t*>(smem + L.o_kw);
+    uint32_t* ctl = reinterpret_cast<uint32_t*>(smem + L.ctl);
+
+    const int tid = threadIdx.x, wave = (int)uniform(tid / WAVE), lane = lane_id();
+    const uint32_t u = blockIdx.x, umask = umap_slots - 1, mmask = map_slots - 1;
+    const size_t base = (size_t)u * K;
+    const uint64_t lane_lt = (1ull << lane) - 1;
+
+    for (uint32_t i = tid; i < K * KL; i += NT) above[i] = below[i] = 0;
+    for (uint32_t i = tid; i < K; i += NT) det[i] = 0;
+    if (tid < 16) ctl[tid] = 0;
+    // valid list entries, in list order
+    if (wave == 0) {
+        uint32_t m = 0;
+#pragma unroll
+        for (int q = 0; q < KL; q++) {
+            const uint32_t v = ids[base + q * WAVE + lane] & ~FLAG;
+            const float dv = dist[base + q * WAVE + lane];
+            const bool ok = dv < INF_DIS && v < C.n && v != u;
+            const uint64_t b = __ballot(ok);
+            if (ok) {
+                const uint32_t pos = m + __popcll(b & lane_lt);
+                nb_id[pos] = v;
+                nb_dist[pos] = dv;
+            }
+            m += __popcll(b);
+        }
+        if (lane == 0) ctl[PC_M] = m;
+    }
+    __syncthreads();
+    const uint32_t m = uniform(ctl[PC_M]);
+    // the code products of all pairs: 16 x 16 blocks (bi <= bj), dealt out to the waves; a quarter of the dimensions is staged while the
+    // next one is on its way. Lane (j, g), j = lane % 16, g = lane / 16, supplies codes 64 b + 16 g .. of row j of a block and holds row 4 g + e, column j
+    constexpr int NB = K / 16, BLOCKS = NB * (NB + 1) / 2, PER = (BLOCKS + NWAVES - 1) / NWAVES;
+    constexpr uint32_t UNITS = SKETCH_BYTES / 4 / 16; // 16-byte units of a row in a quarter
+    const int j = lane & 15, g = lane >> 4;
+    uint32_t bi[PER], bj[PER]; // wave-uniform; bj = NB: none
+    intx4 acc[PER];
+#pragma unroll
+    for (int q = 0; q < PER; q++) {
+        uint32_t t = wave + q * NWAVES, i = 0;
+        while (i < NB && t >= NB - i) { t -= NB - i; i++; }
+        bi[q] = uniform(i);
+        bj[q] = uniform(i < NB ? i + t : (uint32_t)NB);
+        acc[q] = intx4{0, 0, 0, 0};
+    }
+    if (m > 0) {
+        constexpr int LOADS = K * UNITS / NT;
+        const intx4* from[LOADS]; // rows that are not there: the last one again
+        intx4 ahead[LOADS];
+#pragma unroll
+        for (int k = 0; k < LOADS; k++) {
+            const uint32_t i = tid + k * NT;
+            from[k] = reinterpret_cast<const intx4*>(sketch) + (size_t)nb_id[min(i / UNITS, m - 1)] * (SKETCH_BYTES / 16) + i % UNITS;
+            ahead[k] = from[k][0];
+        }
+        if (tid < (int)m) { // meanwhile: what the tests and the later phases need of a row
+            const uint32_t v = nb_id[tid];
+            const uint64_t desc = C.desc[v];
+            const float nv = norms[v], dn = C.dnorm[v];
+            const SketchMeta sm = sketch_meta[v];
+            nrm[tid] = nv;
+            // what the hybrid norm leaves to the sparse part, with room for the rounding of both norms
+            row[tid] = make_float4(dn, sm.scale, sm.err, sqrtf(fmaxf(nv - dense_mul * dn * dn, 0.f) + 1e-5f * (nv + dense_mul * dn * dn)));
+            rowptr[tid] = desc_off(desc) * 16 + DENSE_BYTES;
+            rownnz[tid] = (desc_nnz_s(desc) + desc_nnz_b(desc)) | (desc_nnz_s(desc) << 16);
+        }
+        // On a corpus whose pairs decide, the longest rows sit in every list, and next to a shorter one the product of the sparse norms tells
+        // nothing: if even the largest dense part cannot take a pair out of reach of the smaller norm, the node is open without a look at
+        // the sketches (100 000 i.i.d. docs, where all are: 0.2 ms instead of 3.5).
+        __syncthreads();
+        if (wave == 0) {
+            float longest = 0.f, top_dense = 0.f;
+#pragma unroll
+            for (int q = 0; q < KL; q++) {
+                const float4 x = q * WAVE + (uint32_t)lane < m ? row[q * WAVE + lane] : make_float4(0.f, 0.f, 0.f, 0.f);
+                longest = fmaxf(longest, x.w);
+                top_dense = fmaxf(top_dense, x.x);
+            }
+            longest = -wave_min_dpp(-longest);
+            top_dense = -wave_min_dpp(-top_dense);
+#pragma unroll
+            for (int q = 0; q < KL; q++) {
+                const uint32_t i = q * WAVE + lane;
+                // the row of the longest sparse part is not compared with itself
+                const float dense = i < m ? row[i].x : 0.f;
+                if (i < m && row[i].w < longest && longest * row[i].w - dense_mul * dense * top_dense > nrm[i]) ctl[PC_OPEN] = 1;
+            }
+        }
+        __syncthreads();
+        if (uniform(ctl[PC_OPEN])) {
+            if (tid == 0) open[u] = 1;
+            return;
+        }
+#pragma unroll 1
+        for (uint32_t quarter = 0; quarter < 4; quarter++) {
+            if (quarter) __syncthreads();
+#pragma unroll
+            for (int k = 0; k < LOADS; k++) {
+                const uint32_t i = tid + k * NT, r = i / UNITS, c = i % UNITS;
+                stage[r * UNITS + (c ^ (r & (UNITS - 1)))] = ahead[k];
+            }
+            __syncthreads();
+            if (quarter < 3) {
+#pragma unroll
+                for (int k = 0; k < LOADS; k++) ahead[k] = from[k][(quarter + 1) * UNITS];
+            }
+#pragma unroll
+            for (int q = 0; q < PER; q++) {
+                if (16 * bj[q] < m) { // wave-uniform; a block that is not there starts at K >= m
+                    const uint32_t ra = min(16 * bi[q] + (uint32_t)j, m - 1), rb = min(16 * bj[q] + (uint32_t)j, m - 1);
+#pragma unroll
+                    for (int k = 0; k < (int)UNITS / 4; k++) {
+                        const uint32_t c = 4 * k + g;
+                        const intx4 a = stage[ra * UNITS + (c ^ (ra & (UNITS - 1)))], b = stage[rb * UNITS + (c ^ (rb & (UNITS - 1)))];
+                        acc[q] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, acc[q], 0, 0, 0);
+                    }
+                }
+            }
+        }
+    }
+    bool undecided = false;
+#pragma unroll
+    for (int q = 0; q < PER; q++) {
+        if (16 * bj[q] < m) {
+            const uint32_t c = 16 * bj[q] + j;
+            const float4 rc = c < m ? row[c] : make_float4(0.f, 0.f, 0.f, 0.f);
+            const float nc = c < m ? nrm[c] : 0.f;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const uint32_t r = 16 * bi[q] + 4 * g + e;
+                if (r < c && c < m) {
+                    const float4 rr = row[r];
+                    const float nr = nrm[r];
+                    const float p = dense_mul * ((float)acc[q][e] * (rr.y * rc.y));
+                    const float off = dense_mul * (rr.x * rc.z + rr.z * (rc.x + rc.z)) + rr.w * rc.w + 1e-5f * (dense_mul * rr.x * rc.x + rr.w * rc.w + 1.0f);
+                    undecided |= !(fabsf(p - nr) > off && fabsf(p - nc) > off); // not a number: open
+                    auto set = [&](uint64_t* masks, uint32_t of, uint32_t bit) { atomicOr(reinterpret_cast<uint32_t*>(masks) + of * (2 * KL) + (bit >> 5), 1u << (bit & 31)); };
+                    if (nr < p) { set(above, r, c); set(below, c, r); }
+                    if (nc < p) { set(above, c, r); set(below, r, c); }
+                }
+            }
+        }
+    }
+    if (undecided) ctl[PC_OPEN] = 1;
+    __syncthreads();
+    if (uniform(ctl[PC_OPEN])) {
+        if (tid == 0) open[u] = 1;
+        return;
+    }
+    // the staged sketches make room
+    for (uint32_t i = tid; i < map_slots; i += NT) idmap[i] = make_uint2(EMPTY, 0u);
+    for (uint32_t i = tid; i < umap_slots; i += NT) umap[i] = make_uint2(EMPTY, 0u);
+    for (uint32_t i = tid; i < K * words; i += NT) R[i] = 0;
+    __syncthreads();
+    if (tid < (int)m) lds_map_insert(idmap, mmask, nb_id[tid], tid);
+    {   // u's BM25 terms -> index
+        const uint64_t du = C.desc[u];
+        const Pairs sp = record_pairs(C, du);
+        const uint32_t ns = desc_nnz_s(du), nb = desc_nnz_b(du);
+        for (uint32_t i = tid; i < nb; i += NT) lds_map_insert(umap, umask, sp.key(ns + i), i);
+    }
+    __syncthreads();
+    // (a) detour counts, eight list entries of a thread at a time
+#pragma unroll 1
+    for (uint32_t t0 = 0; t0 < m * K; t0 += 8 * NT) {
+        uint32_t xs[8];
+        float dxs[8];
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            const uint32_t t = t0 + tid + k * NT;
+            xs[k] = EMPTY;
+            dxs[k] = 0.f;
+            if (t < m * K) {
+                const size_t at = (size_t)nb_id[t / K] * K + t % K;
+                xs[k] = ids[at] & ~FLAG;
+                dxs[k] = dist[at];
+            }
+        }
+        uint2 e[8];
+        lds_map_find(idmap, mmask, xs, e);
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            const uint32_t r = (t0 + tid + k * NT) / K;
+            if (xs[k] != EMPTY && e[k].x == xs[k] && e[k].y > r && dxs[k] < nb_dist[e[k].y]) atomicAdd(&det[e[k].y], 1u);
+        }
+    }
+    // R[r] = bits of u's BM25 terms that row r holds too: one wave per row, the first 64 BM25 terms of eight rows at a time
+#pragma unroll 1
+    for (int half = 0; half < 2; half++) {
+        uint32_t key[8], nbs[8];
+        auto row_pairs = [&](uint32_t r) {
+            Pairs sp = gram_row(C, rowptr, rownnz, r);
+            sp.narrow = NARROW ? 1u : 0u;
+            return sp;
+        };
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            const uint32_t r = wave + NWAVES * (8 * half + k);
+            nbs[k] = 0;
+            key[k] = EMPTY;
+            if (r < m) { // wave-uniform
+                const Pairs sp = row_pairs(r);
+                nbs[k] = uniform(sp.nnz - sp.ns);
+                if ((uint32_t)lane < nbs[k]) key[k] = sp.raw(sp.ns + lane).x; // the path bit follows where the key is used
+            }
+        }
+        uint2 e[8];
+#pragma unroll
+        for (int k = 0; k < 8; k++) key[k] |= BM25_BIT;
+        lds_map_find(umap, umask, key, e);
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            const uint32_t r = wave + NWAVES * (8 * half + k);
+            if (key[k] != EMPTY && e[k].x == key[k]) atomicOr(&R[r * words + (e[k].y >> 5)], 1u << (e[k].y & 31));
+            if (nbs[k] > WAVE) {
+                const Pairs sp = row_pairs(r);
+                for (uint32_t i = WAVE + lane; i < nbs[k]; i += WAVE) {
+                    const uint32_t x[1] = {sp.key(sp.ns + i)};
+                    uint2 f[1];
+                    lds_map_find(umap, umask, x, f);
+                    if (f[0].x == x[0]) atomicOr(&R[r * words + (f[0].y >> 5)], 1u << (f[0].y & 31));
+                }
+            }
+        }
+    }
+    __syncthreads();
+    // (b) stable order by detour count: the last wave; keyword flags of all pairs: flag(c, s) = (R[s] & ~R[c]) != 0, lane s for one c at a time
+    if (wave == NWAVES - 1) {
+        uint32_t key[KL], rank[KL];
+#pragma unroll
+        for (int q = 0; q < KL; q++) {
+            const uint32_t i = q * WAVE + lane;
+            key[q] = i < m ? (det[i] << 16) | i : ~0u;
+            rank[q] = 0;
+        }
+#pragma unroll
+        for (int q = 0; q < KL; q++) {
+            for (uint32_t i = 0; i < WAVE && q * WAVE + i < m; i++) {
+                const uint32_t x = (uint32_t)__builtin_amdgcn_readlane((int)key[q], (int)i);
+#pragma unroll
+                for (int p = 0; p < KL; p++) rank[p] += x < key[p];
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < KL; q++)
+            if (q * WAVE + (uint32_t)lane < m) order[rank[q]] = q * WAVE + lane;
+    }
+    for (uint32_t c = wave; c < m; c += NWAVES) {
+#pragma unroll
+        for (int q = 0; q < KL; q++) {
+            const uint32_t s = q * WAVE + lane;
+            uint32_t any = 0;
+            for (uint32_t w = 0; w < words; w++) any |= (s < m ? R[s * words + w] : 0u) & ~R[c * words + w];
+            const uint64_t f = __ballot(any != 0);
+            if (lane == 0) F[c * KL + q] = f;
+        }
+    }
+    __syncthreads();
+    // (c)+(d) sequential selection as in prune_gram_kernel: position 64 q + lane of the order in register q
+    if (wave == 0) {
+        uint32_t ord[KL], id_o[KL], det_o[KL];
+        uint64_t up[KL][KL], dn[KL][KL], fl[KL][KL], live[KL] = {}, taken[KL] = {}, flagged[KL] = {};
+        bool plain = true;
+#pragma unroll
+        for (int q = 0; q < KL; q++) {
+            const uint32_t t = q * WAVE + lane;
+            ord[q] = t < m ? order[t] : 0u;
+            id_o[q] = t < m ? nb_id[ord[q]] : EMPTY;
+            det_o[q] = t < m ? det[ord[q]] : 0u;
+#pragma unroll
+            for (int w = 0; w < KL; w++) {
+                up[q][w] = t < m ? above[ord[q] * KL + w] : 0ull;
+                dn[q][w] = t < m ? below[ord[q] * KL + w] : 0ull;
+                fl[q][w] = t < m ? F[ord[q] * KL + w] : 0ull;
+                plain = plain && (up[q][w] | dn[q][w]) == 0;
+            }
+        }
+        plain = __ballot(!plain) == 0; // no product exceeds a norm: all are taken and stay
+#pragma unroll
+        for (int q = 0; q < KL; q++) {
+            for (uint32_t i = 0; i < WAVE && q * WAVE + i < m; i++) {
+                const uint32_t c = (uint32_t)__builtin_amdgcn_readlane((int)ord[q], (int)i);
+                bool reject = false, allflag = q * WAVE + i > 0;
+#pragma unroll
+                for (int w = 0; w < KL; w++) {
+                    allflag = allflag && (live[w] & ~readlane64(fl[q][w], i)) == 0;
+                    if (!plain) {
+                        reject = reject || (readlane64(up[q][w], i) & live[w]) != 0;
+                    }
+                }
+                if (!plain) {
+#pragma unroll
+                    for (int w = 0; w < KL; w++) live[w] &= ~readlane64(dn[q][w], i);
+                }
+                if (!reject) {
+#pragma unroll
+                    for (int w = 0; w < KL; w++) live[w] |= (c >> 6) == (uint32_t)w ? 1ull << (c & 63) : 0ull;
+                    taken[q] |= 1ull << i;
+                    if (allflag) flagged[q] |= 1ull << i;
+                }
+            }
+        }
+        // (e) emit: live members in selection order fill the row, flagged ones beyond d become keyword candidates
+        bool alive[KL];
+        uint64_t lb[KL];
+        uint32_t n_live = 0, n_kw = 0;
+#pragma unroll
+        for (int q = 0; q < KL; q++) {
+            uint64_t lw = live[0];
+#pragma unroll
+            for (int w = 1; w < KL; w++) lw = (ord[q] >> 6) == (uint32_t)w ? live[w] : lw;
+            alive[q] = ((taken[q] >> lane) & 1) && ((lw >> (ord[q] & 63)) & 1);
+            lb[q] = __ballot(alive[q]);
+            const uint32_t pos = n_live + __popcll(lb[q] & lane_lt);
+            if (alive[q] && pos < d) { o_fwd[pos] = id_o[q]; o_det[pos] = det_o[q]; }
+            const bool kwc = alive[q] && pos >= d && ((flagged[q] >> lane) & 1);
+            const uint64_t kb = __ballot(kwc);
+            const uint32_t kpos = n_kw + __popcll(kb & lane_lt);
+            if (kwc && kpos < APOE_KW_CAND) o_kw[1 + kpos] = id_o[q];
+            n_live += __popcll(lb[q]);
+            n_kw += __popcll(kb);
+        }
+        uint32_t cnt = min(n_live, d);
+        const uint32_t nkw = min(n_kw, (uint32_t)APOE_KW_CAND);
+        if (cnt < d) { // fewer survivors than the row has slots: the remaining neighbours in order, each id once
+            bool add[KL];
+#pragma unroll
+            for (int q = 0; q < KL; q++) add[q] = q * WAVE + (uint32_t)lane < m;
+#pragma unroll
+            for (int p = 0; p < KL; p++) {
+                for (uint64_t rest = lb[p]; rest; rest &= rest - 1) {
+                    const uint32_t x = (uint32_t)__builtin_amdgcn_readlane((int)id_o[p], __builtin_ctzll(rest));
+#pragma unroll
+                    for (int q = 0; q < KL; q++) add[q] = add[q] && x != id_o[q];
+                }
+                for (uint32_t i = 0; i < WAVE && p * WAVE + i < m; i++) {
+                    const uint32_t x = (uint32_t)__builtin_amdgcn_readlane((int)id_o[p], (int)i);
+#pragma unroll
+                    for (int q = 0; q < KL; q++) add[q] = add[q] && !(q * WAVE + (uint32_t)lane > p * WAVE + i && x == id_o[q]);
+                }
+            }
+#pragma unroll
+            for (int q = 0; q < KL; q++) {
+                const uint64_t ab = __ballot(add[q]);
+                const uint32_t at = cnt + __popcll(ab & lane_lt);
+                if (add[q] && at < d) { o_fwd[at] = id_o[q]; o_det[at] = det_o[q]; }
+                cnt = min(d, cnt + (uint32_t)__popcll(ab));
+            }
+        }
+        if (lane == 0) { ctl[PC_CNT] = cnt; o_kw[0] = nkw; }
+        for (uint32_t i = cnt + lane; i < d; i += WAVE) { o_fwd[i] = u; o_det[i] = EMPTY; }
+        for (uint32_t i = nkw + lane; i < APOE_KW_CAND; i += WAVE) o_kw[1 + i] = 0;
+    }
+    __syncthreads();
+    for (uint32_t i = tid; i < d; i += NT) {
+        fwd[(size_t)u * d + i] = o_fwd[i];
+        det_out[(size_t)u * d + i] = o_det[i];
+    }
+    for (uint32_t i = tid; i < 1 + APOE_KW_CAND; i += NT) kw_out[(size_t)u * (1 + APOE_KW_CAND) + i] = o_kw[i];
+    if (tid == 0) cnt_out[u] = ctl[PC_CNT];
+}
+
 // ---- the prune on a Gram matrix that the tile kernel of join.hip has left in memory (lists of up to 128 entries) ----
 
 constexpr uint32_t PS_MAX = 128;            // longest list
@@ -267,7 +732,7 @@ struct SelectLds {
     }
 };
 
-// allan_poe (index.cu:539-714) for node u = node0 + blockIdx.x, as prune_kernel, with every inner product <c, s> read from the
+// allan_poe (index.cu:539-714) for node u = node0 + blockIdx.x (nodes: the list's entry there), as prune_kernel, with every inner product <c, s> read from the
 // node's Gram matrix gram[blockIdx.x][i][j] (i <= j: positions in the list of valid entries) instead of being evaluated:
 // detour counts and the (detour, rank) order as there; the keyword flag of a pair from bit masks R[i] = the BM25 terms of u
 // that row i holds (flag(c, s) = R[s] has a bit that R[c] lacks); the sequential selection by wave 0 alone, two selected
@@ -275,7 +740,7 @@ struct SelectLds {
 // requested from the matrix in memory while the current candidate is decided. The workgroup keeps no copy of the matrix:
 // several nodes share a CU, and the others cover the selection's waits.
 __global__ __launch_bounds__(PS_THREADS) void prune_select_kernel(CorpusView C, const float* __restrict__ norms, uint32_t K, const uint32_t* __restrict__ ids,
-                                                                  const float* __restrict__ dist, uint32_t d, uint32_t node0, const float* __restrict__ gram,
+                                                                  const float* __restrict__ dist, uint32_t d, const uint32_t* __restrict__ nodes, uint32_t node0, const float* __restrict__ gram,
                                                                   uint32_t* fwd, uint32_t* det_out, uint32_t* cnt_out, uint32_t* kw_out, uint32_t umap_slots,
                                                                   uint32_t map_slots, uint32_t words) {
     extern __shared__ __align__(16) char smem[];
@@ -297,7 +762,7 @@ __global__ __launch_bounds__(PS_THREADS) void prune_select_kernel(CorpusView C, 
 
     const int tid = threadIdx.x, wave = tid / WAVE, lane = lane_id();
     constexpr uint32_t NWV = PS_THREADS / WAVE;
-    const uint32_t u = node0 + blockIdx.x, umask = umap_slots - 1, mmask = map_slots - 1;
+    const uint32_t u = nodes ? nodes[node0 + blockIdx.x] : node0 + blockIdx.x, umask = umap_slots - 1, mmask = map_slots - 1;
     const size_t base = (size_t)u * K;
     const uint64_t lane_lt = (1ull << lane) - 1;
     const float* gu = gram + (size_t)blockIdx.x * PS_MAX * PS_MAX;
@@ -564,7 +1029,7 @@ constexpr int PRUNE_DENSE_NB = 2; // 8-float blocks of the rows a wave requests 
 constexpr int GRAM_THREADS = 512; // 8 waves share one node's tables: more lookups in flight per byte of LDS
 
 struct GramPruneLds {
-    uint32_t G, tabs, ovf_cnt, rowptr, rownnz, umap, R, F, idmap, nb_id, nb_dist, nrm, det, order, o_fwd, o_det, o_kw, ctl, total;
+    uint32_t G, tabs, ovf_cnt, rowptr, rownnz, umap, R, F, above, below, row, idmap, nb_id, nb_dist, nrm, det, order, o_fwd, o_det, o_kw, ctl, total;
     // union_slots != 0: the table region holds one union table (apoe_gram.h) instead of tgroup pivot tables;
     // rank_slots != 0: it holds a rank table (apoe_ranktab.h) of rank_bits index bits instead
     __host__ __device__ __forceinline__ GramPruneLds(uint32_t term_slots, uint32_t tgroup, uint32_t umap_slots, uint32_t map_slots, uint32_t words,
@@ -581,7 +1046,10 @@ struct GramPruneLds {
         umap = o; o += umap_slots * 8;
         idmap = o; o += map_slots * 8;
         R = o; o += GRAM_ROWS * words * 4;
-        F = o; o += GRAM_ROWS * 2 * 4; // keyword-flag matrix: bit s of row c = "s holds a term of u that c lacks"
+        F = o; o += GRAM_ROWS * 8; // keyword-flag matrix: bit s of row c = "s holds a term of u that c lacks"
+        above = o; o += GRAM_ROWS * 8; // bit s of row c: <c, s> exceeds c's norm ...
+        below = o; o += GRAM_ROWS * 8; // ... and s's norm
+        row = o; o += GRAM_ROWS * 16;  // dense norm, scale and error of the sketch, norm of the sparse part
         nb_id = o; o += GRAM_ROWS * 4;
         nb_dist = o; o += GRAM_ROWS * 4;
         nrm = o; o += GRAM_ROWS * 4;
@@ -658,18 +1126,270 @@ __device__ __forceinline__ void gram_sparse_rank(const CorpusView& C, uint32_t m
             __syncthreads(); // the table is rebuilt next
         }
     }
-    for (uint32_t t = tid; t < m * m; t += nthreads) {
-        const uint32_t i = t / m, j = t % m;
-        if (i > j) G[i * GRAM_STRIDE + j] = G[j * GRAM_STRIDE + i];
+}
+
+// Sparse part of the Gram matrix from one numbering of the terms that at least two of the rows hold (narrow corpora; a term of one row
+// only multiplies nothing). A bitmap over the term space counts a term's first and second appearance,
+// the rank of its second-appearance bit is its slot; every wave writes the slots of its rows' pairs in place of their terms, drops the
+// pairs without one (a third of them, for 64 rows of 180 Zipf terms) and deals the rest out to the lanes, 64 to a chunk. A group of
+// eight pivots is then written straight into a table of eight values a slot (one word per pair, no clearing: a wave takes its pivot's words
+// out again and puts the next in) and a row reads eight values per pair: no bitmap, no key, no hit test, empty lanes read a slot of zeros.
+// Per node of 64 rows of 180 terms (1 290 shared ones) against the group-by-group rank table: 106 000 cycles
+// instead of 151 000 (two nodes a CU), of them 31 000 for the numbering; what is left is bound by the 16-byte table reads (100 000 i.i.d.
+// docs: prune 22.1 -> 16.4 ms).
+// `region` / `bytes`: LDS for bitmap and table, one after the other. Returns false (for all threads alike, nothing written to G) when
+// the slots do not fit the table or a row keeps more than 256 pairs. All threads call it; it ends with a barrier.
+constexpr int GS_CHUNKS = 4;
+struct SharedRow {
+    float v[GS_CHUNKS];
+    uint32_t s2[GS_CHUNKS / 2]; // slots of two pairs a word
+    __device__ __forceinline__ uint32_t slot(int c) const { return (c & 1) ? s2[c >> 1] >> 16 : s2[c >> 1] & 0xFFFFu; }
+};
+__device__ __forceinline__ void gram_shared_groups(uint32_t m, float* G, float4* table, uint32_t plane, const SharedRow (&own)[GR_OWN], uint32_t chunks, int wave,
+                                                   int lane) {
+    // group g = rows 8 g .. 8 g + 7, row r in own[r / 8] of wave r % 8: wave w's pivot of group g is its own[g]; `chunks`: lane k holds the
+    // chunks of own[k]
+    float* words = reinterpret_cast<float*>(table) + ((wave >> 2) * plane * 4 + (wave & 3)); // this wave's word of slot 0
+    const uint32_t ng = m >= 2 ? (m - 2) / 8 + 1 : 0; // the last row is never a pivot
+    SharedRow pr = own[0];
+    for (uint32_t g = 0; g < ng; g++) {
+#pragma unroll
+        for (int k = 1; k < GR_OWN; k++) { // wave-uniform selects, so that own[] stays in registers
+            const bool take = g == (uint32_t)k;
+#pragma unroll
+            for (int c = 0; c < GS_CHUNKS; c++) pr.v[c] = take ? own[k].v[c] : pr.v[c];
+#pragma unroll
+            for (int c = 0; c < GS_CHUNKS / 2; c++) pr.s2[c] = take ? own[k].s2[c] : pr.s2[c];
+        }
+#pragma unroll
+        for (int c = 0; c < GS_CHUNKS; c++) words[pr.slot(c) * 4] = pr.v[c]; // an empty lane's value is zero: the slot of zeros stays one
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < GR_OWN; k++) {
+            const uint32_t nc = (uint32_t)__builtin_amdgcn_readlane((int)chunks, k), b = wave + 8 * k;
+            if (b > 8 * g && nc != 0) { // wave-uniform
+                float acc[8];
+#pragma unroll
+                for (int t = 0; t < 8; t++) acc[t] = 0.f;
+                auto add = [&](float v, const float4& lo, const float4& hi) {
+                    acc[0] = fmaf(v, lo.x, acc[0]);
+                    acc[1] = fmaf(v, lo.y, acc[1]);
+                    acc[2] = fmaf(v, lo.z, acc[2]);
+                    acc[3] = fmaf(v, lo.w, acc[3]);
+                    acc[4] = fmaf(v, hi.x, acc[4]);
+                    acc[5] = fmaf(v, hi.y, acc[5]);
+                    acc[6] = fmaf(v, hi.z, acc[6]);
+                    acc[7] = fmaf(v, hi.w, acc[7]);
+                };
+                SharedRow r = own[k];
+                asm volatile("" : "+v"(r.s2[0]), "+v"(r.s2[1])); // addresses are worked out here, not kept for all rows and groups
+                // the reads of three chunks together, whether the row has them or not (an average row keeps 122 to 135 pairs), a fourth where it has
+                float4 lo[GS_CHUNKS - 1], hi[GS_CHUNKS - 1];
+#pragma unroll
+                for (int c = 0; c < GS_CHUNKS - 1; c++) {
+                    lo[c] = table[r.slot(c)];
+                    hi[c] = table[plane + r.slot(c)];
+                }
+                asm volatile("" : "+v"(lo[0].x), "+v"(lo[1].x), "+v"(lo[2].x), "+v"(hi[0].x), "+v"(hi[1].x), "+v"(hi[2].x));
+#pragma unroll
+                for (int c = 0; c < GS_CHUNKS - 1; c++) add(r.v[c], lo[c], hi[c]);
+                if (nc == GS_CHUNKS) add(r.v[GS_CHUNKS - 1], table[r.slot(GS_CHUNKS - 1)], table[plane + r.slot(GS_CHUNKS - 1)]);
+                uint32_t t;
+                const float z = wave_sum_1x8(acc, lane, &t);
+                const uint32_t p = 8 * g + t;
+                if ((lane & 15) < 4 && (lane & 32) == 0 && p < b) G[p * GRAM_STRIDE + b] = z;
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int c = 0; c < GS_CHUNKS; c++) words[pr.slot(c) * 4] = 0.f;
     }
     __syncthreads();
 }
+template <typename TailFn> // tail(k): the Pairs of own row k, for those beyond the register window
+__device__ __forceinline__ bool gram_sparse_shared(uint32_t m, float* G, char* region, uint32_t bytes, uint32_t index_bits, uint32_t span, uint32_t* scan,
+                                                   const RtRow<true> (&rows)[GR_OWN], const uint32_t (&shapes)[GR_OWN], TailFn tail, int tid, int wave, int lane) {
+    constexpr int NT = 8 * WAVE;
+    constexpr uint32_t WINDOW = RT_CHUNKS * WAVE, KEPT = GS_CHUNKS * WAVE;
+    RankTab T; // the bitmap: x = terms seen at least twice, y = terms seen, then the count of the x bits before
+    T.word = reinterpret_cast<uint2*>(region);
+    T.index_bits = index_bits;
+    T.span = span;
+    const uint32_t W = index_bits / 32, counts = W * 8;
+    uint2* out = reinterpret_cast<uint2*>(region + counts) + wave * GS_CHUNKS * WAVE; // a row's pairs on their way to other lanes
+    if (counts + 8 * GS_CHUNKS * WAVE * 8 > bytes) return false;
+    for (uint32_t w = tid; w < W; w += NT) T.word[w] = make_uint2(0u, 0u);
+    uint32_t* overfull = scan + 17;
+    if (tid == 0) *overfull = 0;
+    __syncthreads();
+    auto seen = [&](uint32_t idx) {
+        const uint32_t bit = 1u << (idx & 31);
+        if (atomicOr(&T.word[idx >> 5].y, bit) & bit) atomicOr(&T.word[idx >> 5].x, bit);
+    };
+    auto index_of = [&](int k, int c) { return ranktab_index<true>(T, rows[k].key(c), rt_pair(c, lane) >= (shapes[k] >> 16)); };
+#pragma unroll
+    for (int k = 0; k < GR_OWN; k++) {
+        const uint32_t nnz = shapes[k] & 0xFFFFu;
+        uint32_t idx[GS_CHUNKS], old[GS_CHUNKS];
+#pragma unroll
+        for (int c = 0; c < GS_CHUNKS; c++) {
+            idx[c] = index_of(k, c);
+            old[c] = 0;
+            if (rt_pair(c, lane) < nnz) old[c] = atomicOr(&T.word[idx[c] >> 5].y, 1u << (idx[c] & 31));
+        }
+#pragma unroll
+        for (int c = 0; c < GS_CHUNKS; c++) {
+            const uint32_t bit = 1u << (idx[c] & 31);
+            if (old[c] & bit) atomicOr(&T.word[idx[c] >> 5].x, bit);
+        }
+        if (nnz > WINDOW) {
+            const Pairs sp = tail(k);
+            for (uint32_t j = WINDOW + lane; j < nnz; j += WAVE) seen(ranktab_index<true>(T, sp.raw(j).x, j >= sp.ns));
+        }
+    }
+    __syncthreads();
+    // counts: thread i owns the words [i * per, (i + 1) * per), two words (16 bytes) at a time
+    const uint32_t per = ((W + NT - 1) / NT + 1) & ~1u;
+    uint4* word2 = reinterpret_cast<uint4*>(T.word);
+    uint32_t some = 0;
+    for (uint32_t k = 0; k < per; k += 2) {
+        const uint32_t w = tid * per + k;
+        if (w < W) {
+            const uint4 two = word2[w >> 1];
+            some += __popc(two.x) + __popc(two.z);
+        }
+    }
+    const uint32_t incl = wave_scan_add_dpp(some);
+    if (lane == WAVE - 1) scan[wave] = incl;
+    __syncthreads();
+    uint32_t before = incl - some, total = 0;
+    for (int w = 0; w < 8; w++) {
+        const uint32_t x = scan[w];
+        if (w < wave) before += x;
+        total += x;
+    }
+    const uint32_t plane = total + 1; // the last slot stays zero
+    if (plane * 32 > bytes || plane > 0xFFFFu) {
+        __syncthreads();
+        return false;
+    }
+    for (uint32_t k = 0; k < per; k += 2) {
+        const uint32_t w = tid * per + k;
+        if (w < W) {
+            uint4 two = word2[w >> 1];
+            two.y = before;
+            before += __popc(two.x);
+            two.w = before;
+            before += __popc(two.z);
+            word2[w >> 1] = two;
+        }
+    }
+    __syncthreads();
+    SharedRow own[GR_OWN];
+    uint32_t chunks = 0;
+#pragma unroll
+    for (int k = 0; k < GR_OWN; k++) {
+        const uint32_t nnz = shapes[k] & 0xFFFFu;
+        uint32_t slot[GS_CHUNKS], mine = 0;
+#pragma unroll
+        for (int c = 0; c < GS_CHUNKS; c++) {
+            slot[c] = EMPTY;
+            if (rt_pair(c, lane) < nnz) {
+                const uint32_t idx = index_of(k, c);
+                slot[c] = ranktab_slot(T.word[idx >> 5], idx);
+            }
+            mine += slot[c] != EMPTY;
+        }
+        const uint32_t upto = wave_scan_add_dpp(mine);
+        uint32_t all = (uint32_t)__builtin_amdgcn_readlane((int)upto, WAVE - 1);
+        uint32_t at = upto - mine;
+#pragma unroll
+        for (int c = 0; c < GS_CHUNKS; c++)
+            if (slot[c] != EMPTY) out[at++] = make_uint2(slot[c], rows[k].v[c]);
+        if (nnz > WINDOW) {
+            const Pairs sp = tail(k);
+            for (uint32_t j0 = WINDOW; j0 < nnz; j0 += WAVE) {
+                const uint32_t j = j0 + lane;
+                uint32_t sl = EMPTY;
+                uint2 kv = make_uint2(0u, 0u);
+                if (j < nnz) {
+                    kv = sp.raw(j);
+                    const uint32_t idx = ranktab_index<true>(T, kv.x, j >= sp.ns);
+                    sl = ranktab_slot(T.word[idx >> 5], idx);
+                }
+                const uint64_t keep = __ballot(sl != EMPTY);
+                const uint32_t to = all + __popcll(keep & ((1ull << lane) - 1));
+                if (sl != EMPTY && to < KEPT) out[to] = make_uint2(sl, kv.y);
+                all += __popcll(keep);
+            }
+            if (all > KEPT) *overfull = 1;
+        }
+        wave_fence_lds();
+#pragma unroll
+        for (int c = 0; c < GS_CHUNKS; c++) {
+            uint2 x = make_uint2(total, 0u);
+            if ((uint32_t)(c * WAVE + lane) < all) x = out[c * WAVE + lane];
+            own[k].v[c] = __uint_as_float(x.y);
+            if (c & 1) own[k].s2[c >> 1] |= x.x << 16;
+            else own[k].s2[c >> 1] = x.x;
+        }
+        wave_fence_lds();
+        const uint32_t nc = (all + WAVE - 1) / WAVE;
+        chunks = lane == k ? nc : chunks;
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    __syncthreads(); // the bitmap is done with
+    if (uniform(*overfull)) {
+        __syncthreads();
+        return false;
+    }
+    float4* table = reinterpret_cast<float4*>(region);
+    for (uint32_t i = tid; i < 2 * plane; i += NT) table[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+    __syncthreads();
+    gram_shared_groups(m, G, table, plane, own, chunks, wave, lane);
+    return true;
+}
 
-// Same result as prune_kernel, different traffic: the node's <= 64 neighbour rows are read
-// once, their hybrid Gram matrix is built in LDS (dense part on the matrix cores), every
-// row's overlap with the centre node's BM25 terms becomes a bit mask, and the sequential
-// RNG-IP selection with its keyword flags then runs on LDS only:
-//   <c,s> = G[c][s];   flag(c,s) = (R[s] & ~R[c]) != 0   with R[x] = bm25(x) ∩ bm25(u).
+// Code products of up to 64 sketches (apoe_device.h), added as integers to the words above the diagonal of G, which hold zeros: wave w takes
+// the codes 128 w .. 128 w + 127 of every row, so every sketch is read once; two v_mfma_i32_16x16x64_i8 per 16 x 16 block. Integer sums are
+// exact: they do not depend on the order of the atomics. Lane (j, g), j = lane % 16, g = lane / 16, supplies codes 64 b + 16 g .. of
+// block b for row j of a block and holds row 4 g + e, column j of a product.
+__device__ __forceinline__ void gram_sketch_upper(const uint4* sketch, const uint32_t* ids, uint32_t m, int* Gi, int wave, int lane) {
+    constexpr int NB = GRAM_ROWS / 16, KB = SKETCH_BYTES / 8 / 64;
+    const int j = lane & 15, g = lane >> 4;
+    intx4 x[NB][KB];
+#pragma unroll
+    for (int b = 0; b < NB; b++) {
+        const uint4* p = sketch + (size_t)ids[min((uint32_t)(16 * b + j), m - 1)] * (SKETCH_BYTES / 16) + wave * (SKETCH_BYTES / 8 / 16) + g;
+#pragma unroll
+        for (int k = 0; k < KB; k++) x[b][k] = __builtin_bit_cast(intx4, p[4 * k]);
+    }
+#pragma unroll
+    for (int bi = 0; bi < NB; bi++) {
+#pragma unroll
+        for (int bj = bi; bj < NB; bj++) {
+            if (16 * bj >= (int)m) continue; // wave-uniform
+            intx4 acc = {0, 0, 0, 0};
+#pragma unroll
+            for (int k = 0; k < KB; k++) acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(x[bi][k], x[bj][k], acc, 0, 0, 0);
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int r = 16 * bi + 4 * g + e, c = 16 * bj + j;
+                if (r < c && c < (int)m) atomicAdd(&Gi[r * GRAM_STRIDE + c], acc[e]);
+            }
+        }
+    }
+}
+
+// Same result as prune_kernel, different traffic. The selection asks of two neighbours c and s of the node only whether <c, s> exceeds
+// either one's norm, and mostly bounds tell: the dense part from the 8-bit sketches (64 KB a node instead of 256), the sparse part
+// first as the product of the two sparse norms and, where that leaves a pair open, as the exact sparse Gram matrix of the node's rows (rank
+// table, apoe_ranktab.h). A node with a pair that is open even then, and a corpus without sketches, takes the dense Gram matrix on the fp32
+// matrix cores. The answers are two 64-bit masks per row, every row's overlap with the centre node's BM25 terms is a bit
+// mask too, and the sequential RNG-IP selection with its keyword flags is a few scalar instructions per neighbour:
+//   rejected(c) = above[c] & live;   live &= ~below[c];   flag(c, s) = (R[s] & ~R[c]) != 0   with R[x] = bm25(x) ∩ bm25(u).
+// (100 000 docs, every node: cycles of wave 0 on one CU's two nodes, with the Gram matrix / as it is: dense part and its sums 68 000 / 6 000,
+// keyword masks and flags 35 000 / 25 000, selection 28 000 / 2 500.)
 template <int NT, bool NARROW>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void prune_gram_kernel(CorpusView C, float dense_mul, const float* __restrict__ norms,
                                                                 const uint32_t* __restrict__ ids, const float* __restrict__ dist,
@@ -677,12 +1397,15 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
                                                                 uint32_t* kw_out, uint32_t term_slots, uint32_t tgroup,
                                                                 uint32_t umap_slots, uint32_t map_slots, uint32_t words,
                                                                 uint32_t union_slots, uint32_t rank_bits, uint32_t rank_slots,
-                                                                uint32_t rank_span, unsigned long long* gfail) {
+                                                                uint32_t rank_span, const SketchMeta* __restrict__ sketch_meta,
+                                                                const uint4* __restrict__ sketch, const uint32_t* __restrict__ nodes, unsigned long long* gfail) {
     constexpr uint32_t K = GRAM_ROWS;
+    constexpr int NWAVES = NT / WAVE;
+    static_assert(NWAVES == 8, "dimensions and rows are dealt out to eight waves");
     C.narrow = NARROW ? 1u : 0u; // the pair format as a compile-time constant: no branch at the loads
     extern __shared__ __align__(16) char smem[];
     const GramPruneLds L(term_slots, tgroup, umap_slots, map_slots, words, union_slots, rank_bits, rank_slots, NARROW);
-    float* G = reinterpret_cast<float*>(smem + L.G);
+    float* G = reinterpret_cast<float*>(smem + L.G); // [i][j], i < j: sparse part of <i, j>; [j][i]: its dense part
     uint2* tabs = reinterpret_cast<uint2*>(smem + L.tabs);
     uint32_t* ovf_cnt = reinterpret_cast<uint32_t*>(smem + L.ovf_cnt);
     unsigned long long* rowptr = reinterpret_cast<unsigned long long*>(smem + L.rowptr);
@@ -690,7 +1413,10 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
     uint2* umap = reinterpret_cast<uint2*>(smem + L.umap);
     uint2* idmap = reinterpret_cast<uint2*>(smem + L.idmap);
     uint32_t* R = reinterpret_cast<uint32_t*>(smem + L.R);
-    uint32_t* F = reinterpret_cast<uint32_t*>(smem + L.F);
+    uint64_t* F = reinterpret_cast<uint64_t*>(smem + L.F);
+    uint64_t* above = reinterpret_cast<uint64_t*>(smem + L.above);
+    uint64_t* below = reinterpret_cast<uint64_t*>(smem + L.below);
+    float4* row = reinterpret_cast<float4*>(smem + L.row); // dense norm, scale and error of the sketch, bound of the norm of the sparse part
     uint32_t* nb_id = reinterpret_cast<uint32_t*>(smem + L.nb_id);
     float* nb_dist = reinterpret_cast<float*>(smem + L.nb_dist);
     float* nrm = reinterpret_cast<float*>(smem + L.nrm);
@@ -702,7 +1428,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
     uint32_t* ctl = reinterpret_cast<uint32_t*>(smem + L.ctl);
 
     const int tid = threadIdx.x, wave = (int)uniform(tid / WAVE), lane = lane_id();
-    const uint32_t u = blockIdx.x, umask = umap_slots - 1, mmask = map_slots - 1;
+    const uint32_t u = nodes ? nodes[blockIdx.x] : blockIdx.x, umask = umap_slots - 1, mmask = map_slots - 1;
     const size_t base = (size_t)u * K;
     const uint64_t lane_lt = (1ull << lane) - 1;
 
@@ -710,7 +1436,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
     for (uint32_t i = tid; i < umap_slots; i += NT) umap[i] = make_uint2(EMPTY, 0u);
     for (uint32_t i = tid; i < K * words; i += NT) R[i] = 0;
     for (uint32_t i = tid; i < K; i += NT) det[i] = 0;
-    for (uint32_t i = tid; i < K * 2; i += NT) F[i] = 0;
+    for (uint32_t i = tid; i < K * GRAM_STRIDE; i += NT) G[i] = 0.f;
     if (tid < 16) ctl[tid] = 0;
     __syncthreads();
 
@@ -721,70 +1447,31 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
         const uint64_t b = __ballot(ok);
         if (ok) {
             const uint32_t pos = __popcll(b & lane_lt);
+            const uint64_t desc = C.desc[v];
+            const float nv = norms[v], dn = C.dnorm[v];
+            SketchMeta sm = {0.f, 0.f};
+            if (sketch) sm = sketch_meta[v];
             nb_id[pos] = v;
             nb_dist[pos] = dv;
-            nrm[pos] = norms[v];
+            nrm[pos] = nv;
+            // what the hybrid norm leaves to the sparse part, with room for the rounding of both norms
+            row[pos] = make_float4(dn, sm.scale, sm.err, sqrtf(fmaxf(nv - dense_mul * dn * dn, 0.f) + 1e-5f * (nv + dense_mul * dn * dn)));
+            rowptr[pos] = desc_off(desc) * 16 + DENSE_BYTES;
+            rownnz[pos] = (desc_nnz_s(desc) + desc_nnz_b(desc)) | (desc_nnz_s(desc) << 16);
+            lds_map_insert(idmap, mmask, v, pos);
         }
         if (lane == 0) ctl[PC_M] = __popcll(b);
-    }
-    if (!(NARROW && rank_slots != 0)) {   // u's BM25 terms -> index (the rank path of narrow corpora numbers them through the rank table)
+    } else { // u's BM25 terms -> index
         const uint64_t du = C.desc[u];
         const Pairs sp = record_pairs(C, du);
         const uint32_t ns = desc_nnz_s(du), nb = desc_nnz_b(du);
-        for (uint32_t j = tid; j < nb; j += NT) {
-            const uint32_t key = sp.key(ns + j);
-            uint32_t h = term_hash(key, umask);
-            while (true) {
-                const uint32_t old = atomicCAS(&umap[h].x, EMPTY, key);
-                if (old == EMPTY) { umap[h].y = j; break; }
-                if (old == key) break;
-                h = (h + 1) & umask;
-            }
-        }
+        for (uint32_t j = tid - WAVE; j < nb; j += NT - WAVE) lds_map_insert(umap, umask, sp.key(ns + j), j);
     }
     __syncthreads();
     const uint32_t m = uniform(ctl[PC_M]);
+    if (sketch && m) gram_sketch_upper(sketch, nb_id, m, reinterpret_cast<int*>(G), wave, lane);
 
-    const bool rank = rank_slots != 0; // the sparse part runs on the rank table with the rows held in registers
-    if (rank) gram_rows_gather(C, nb_id, m, rowptr, rownnz, tid, NT);
-    // (a) detour counts (as prune_kernel)
-    for (uint32_t i = tid; i < m; i += NT) {
-        const uint32_t key = nb_id[i];
-        uint32_t h = term_hash(key, mmask);
-        while (true) {
-            const uint32_t old = atomicCAS(&idmap[h].x, EMPTY, key);
-            if (old == EMPTY) { idmap[h].y = i; break; }
-            if (old == key) break;
-            h = (h + 1) & mmask;
-        }
-    }
-    // R[r] = bits of u's BM25 terms that row r holds too: one wave per row, lanes over its BM25 pairs
-    auto mark = [&](uint32_t r, uint32_t key) {
-        uint32_t h = term_hash(key, umask);
-        while (true) {
-            const uint2 e = umap[h];
-            if (e.x == key) { atomicOr(&R[r * words + (e.y >> 5)], 1u << (e.y & 31)); break; }
-            if (e.x == EMPTY) break;
-            h = (h + 1) & umask;
-        }
-    };
-    for (uint32_t r = wave; r < (rank ? 0u : m); r += NT / WAVE) {
-        const uint64_t dr = C.desc[nb_id[r]];
-        const Pairs sp = record_pairs(C, dr);
-        const uint32_t ns = desc_nnz_s(dr), nb = desc_nnz_b(dr);
-        for (uint32_t j = lane; j < nb; j += WAVE) {
-            const uint32_t key = sp.key(ns + j);
-            uint32_t h = term_hash(key, umask);
-            while (true) {
-                const uint2 e = umap[h];
-                if (e.x == key) { atomicOr(&R[r * words + (e.y >> 5)], 1u << (e.y & 31)); break; }
-                if (e.x == EMPTY) break;
-                h = (h + 1) & umask;
-            }
-        }
-    }
-    __syncthreads();
-    {   // all list entries of this thread are requested before the first one is looked up
+    {   // (a) detour counts: all list entries of this thread are requested before the first one is looked up
         constexpr uint32_t PER = K * K / NT;
         uint32_t xs[PER];
         float dxs[PER];
@@ -799,212 +1486,219 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
                 dxs[k] = dist[at];
             }
         }
+        uint2 e[PER];
+        lds_map_find(idmap, mmask, xs, e);
 #pragma unroll
         for (uint32_t k = 0; k < PER; k++) {
-            const uint32_t r = (tid + k * NT) / K, x = xs[k];
-            if (x == EMPTY) continue;
-            uint32_t h = term_hash(x, mmask);
-            while (true) {
-                const uint2 e = idmap[h];
-                if (e.x == x) {
-                    if (e.y > r && dxs[k] < nb_dist[e.y]) atomicAdd(&det[e.y], 1u);
-                    break;
-                }
-                if (e.x == EMPTY) break;
-                h = (h + 1) & mmask;
-            }
+            const uint32_t r = (tid + k * NT) / K;
+            if (xs[k] != EMPTY && e[k].x == xs[k] && e[k].y > r && dxs[k] < nb_dist[e[k].y]) atomicAdd(&det[e[k].y], 1u);
         }
     }
-    __syncthreads();
-    // hybrid Gram matrix of the m rows. Only the upper triangle of G is used (the sparse part is added there and the
-    // lower triangle is mirrored from it at the end). Every wave takes an eighth of the dimensions and computes the
-    // three upper tiles for it from one read of the rows; the partial tiles are added into G in a fixed order
-    // (barriers between them): the result does not depend on timing.
-    constexpr int NWAVES = NT / WAVE, BLOCKS = DIM / 8;
-    static_assert(NWAVES == 8, "dimensions and rows are dealt out to eight waves");
-    floatx16 dacc00, dacc01, dacc11;
-    gram_dense_upper<PRUNE_DENSE_NB>(C, nb_id, m, lane, wave * (BLOCKS / NWAVES), (wave + 1) * (BLOCKS / NWAVES), dacc00, dacc01, dacc11);
-    // this wave's rows w, w + 8, ...: requested as soon as the wave's dense tile is done (its operands need the registers), used from the keyword masks on
-    static_assert(NT / WAVE == 8 || NT / WAVE == 4, "rows are dealt out to eight waves");
-    RtRow<NARROW> own[GR_OWN];
-    uint32_t own_shape[GR_OWN];
-#pragma unroll
-    for (int k = 0; k < GR_OWN; k++) {
-        const uint32_t b = wave + 8 * k;
-        own_shape[k] = 0;
-        if (rank && b < m) {
-            own_shape[k] = uniform(rownnz[b]);
-            Pairs sp = gram_row(C, rowptr, rownnz, b);
+    {   // R[r] = bits of u's BM25 terms that row r holds too: one wave per row, the first 64 BM25 terms of all its rows requested at once
+        uint32_t key[GR_OWN], nbs[GR_OWN];
+        auto row_pairs = [&](uint32_t r) {
+            Pairs sp = gram_row(C, rowptr, rownnz, r);
             sp.narrow = NARROW ? 1u : 0u;
-            rt_row_load(own[k], sp, lane);
-        }
-    }
-    // (b) stable order by detour count (LDS only: runs while the rows arrive)
-    for (uint32_t i = tid; i < m; i += NT) {
-        const uint32_t key = (det[i] << 16) | i;
-        uint32_t r = 0;
-        for (uint32_t j = 0; j < m; j++) r += ((det[j] << 16) | j) < key;
-        order[r] = i;
-    }
-    for (int ph = 0; ph < NWAVES; ph++) {
-        if (wave == ph && m > 0) {
-            gram_dense_store(G, 0, lane, dacc00, dense_mul, ph != 0);
-            if (m > 32) {
-                gram_dense_store(G, 1, lane, dacc01, dense_mul, ph != 0);
-                gram_dense_store(G, 3, lane, dacc11, dense_mul, ph != 0);
-            }
-        }
-        if (ph + 1 < NWAVES) __syncthreads();
-    }
-    if (rank && NARROW) {
-        // keyword masks through the rank table: u's BM25 terms alone go into the bitmap (no values), a term's slot -- its
-        // rank among them -- is its bit in the masks, and every wave looks the BM25 pairs of its rows up with one 8-byte
-        // read each: no hash collisions, no probe loop
-        const RankTab T = ranktab_at(reinterpret_cast<char*>(tabs), rank_bits, rank_slots, rank_span, NARROW);
-        const uint64_t du = C.desc[u];
-        const Pairs up = record_pairs(C, du);
-        const uint32_t ns_u = desc_nnz_s(du), nb_u = desc_nnz_b(du);
-        ranktab_build_bits<NARROW>(T, [&](auto f) {
-            for (uint32_t j = tid; j < nb_u; j += NT) f(up.raw(ns_u + j), true, 0);
-        }, ~0u, ovf_cnt, tid, NT);
-        __syncthreads();
-        auto mark_bit = [&](uint32_t r, uint2 w, uint32_t idx) {
-            const uint32_t e = ranktab_slot(w, idx);
-            if (e != EMPTY) atomicOr(&R[r * words + (e >> 5)], 1u << (e & 31));
+            return sp;
         };
 #pragma unroll
         for (int k = 0; k < GR_OWN; k++) {
-            const uint32_t nnz = own_shape[k] & 0xFFFFu, ns = own_shape[k] >> 16, r = wave + 8 * k;
-            if (nnz > ns) { // wave-uniform: the row has BM25 pairs
-                uint32_t idx[RT_CHUNKS];
-                uint2 w[RT_CHUNKS];
-#pragma unroll
-                for (int c = 0; c < RT_CHUNKS; c++) {
-                    const uint32_t j = rt_pair(c, lane);
-                    idx[c] = ranktab_index<NARROW>(T, own[k].key(c), true);
-                    w[c] = T.word[j >= ns && j < nnz ? idx[c] >> 5 : 0u];
-                }
-#pragma unroll
-                for (int c = 0; c < RT_CHUNKS; c++) {
-                    const uint32_t j = rt_pair(c, lane);
-                    if (j >= ns && j < nnz) mark_bit(r, w[c], idx[c]);
-                }
-                if (nnz > RT_CHUNKS * WAVE) {
-                    Pairs sp = gram_row(C, rowptr, rownnz, r);
-                    sp.narrow = NARROW ? 1u : 0u;
-                    for (uint32_t j = max(ns, (uint32_t)(RT_CHUNKS * WAVE)) + lane; j < nnz; j += WAVE) {
-                        const uint32_t ix = ranktab_index<NARROW>(T, sp.raw(j).x, true);
-                        mark_bit(r, T.word[ix >> 5], ix);
-                    }
-                }
+            const uint32_t r = wave + NWAVES * k;
+            nbs[k] = 0;
+            key[k] = EMPTY;
+            if (r < m) { // wave-uniform
+                const Pairs sp = row_pairs(r);
+                nbs[k] = uniform(sp.nnz - sp.ns);
+                if ((uint32_t)lane < nbs[k]) key[k] = sp.raw(sp.ns + lane).x; // the path bit follows where the key is used
             }
         }
-    } else if (rank) {
+        uint2 e[GR_OWN];
+#pragma unroll
+        for (int k = 0; k < GR_OWN; k++) key[k] |= BM25_BIT;
+        lds_map_find(umap, umask, key, e);
 #pragma unroll
         for (int k = 0; k < GR_OWN; k++) {
-            const uint32_t nnz = own_shape[k] & 0xFFFFu, ns = own_shape[k] >> 16, r = wave + 8 * k;
-            if (nnz > ns) { // wave-uniform: the row has BM25 pairs
-                // the first table slot of all four pairs is read before any is compared; the probe loop is for the
-                // pairs whose slot holds another term
-                uint32_t key[RT_CHUNKS], h[RT_CHUNKS];
-                uint2 e[RT_CHUNKS];
-#pragma unroll
-                for (int c = 0; c < RT_CHUNKS; c++) {
-                    key[c] = own[k].key(c) | (NARROW ? 0x80000000u : 0u);
-                    h[c] = term_hash(key[c], umask);
-                    e[c] = umap[h[c]];
-                }
-#pragma unroll
-                for (int c = 0; c < RT_CHUNKS; c++) {
-                    const uint32_t j = rt_pair(c, lane);
-                    if (j >= ns && j < nnz) {
-                        if (e[c].x == key[c]) atomicOr(&R[r * words + (e[c].y >> 5)], 1u << (e[c].y & 31));
-                        else if (e[c].x != EMPTY) mark(r, key[c]);
-                    }
-                }
-                if (nnz > RT_CHUNKS * WAVE) {
-                    Pairs sp = gram_row(C, rowptr, rownnz, r);
-                    sp.narrow = NARROW ? 1u : 0u;
-                    for (uint32_t j = max(ns, (uint32_t)(RT_CHUNKS * WAVE)) + lane; j < nnz; j += WAVE) mark(r, sp.key(j));
+            const uint32_t r = wave + NWAVES * k;
+            if (key[k] != EMPTY && e[k].x == key[k]) atomicOr(&R[r * words + (e[k].y >> 5)], 1u << (e[k].y & 31));
+            if (nbs[k] > WAVE) {
+                const Pairs sp = row_pairs(r);
+                for (uint32_t j = WAVE + lane; j < nbs[k]; j += WAVE) {
+                    const uint32_t x[1] = {sp.key(sp.ns + j)};
+                    uint2 f[1];
+                    lds_map_find(umap, umask, x, f);
+                    if (f[0].x == x[0]) atomicOr(&R[r * words + (f[0].y >> 5)], 1u << (f[0].y & 31));
                 }
             }
         }
     }
     __syncthreads();
-    if (rank) {
-        const RankTab T = ranktab_at(reinterpret_cast<char*>(tabs), rank_bits, rank_slots, rank_span, NARROW);
-        gram_sparse_rank<NARROW>(C, m, G, T, ovf_cnt, rowptr, rownnz, own, own_shape, &ctl[PC_FAIL], tid, NT);
-    } else if (union_slots) gram_sparse_union(C, nb_id, m, G, reinterpret_cast<char*>(tabs), union_slots, ovf_cnt, rowptr, rownnz, &ctl[PC_FAIL], tid, NT);
-    else if (tgroup == 8) gram_sparse_64<8>(C, nb_id, m, G, tabs, term_slots, ovf_cnt, rowptr, rownnz, &ctl[PC_FAIL], tid, NT);
-    else gram_sparse_64<4>(C, nb_id, m, G, tabs, term_slots, ovf_cnt, rowptr, rownnz, &ctl[PC_FAIL], tid, NT);
-    // keyword flags of all pairs at once (index.cu:637,651-654): flag(c, s) = (R[s] & ~R[c]) != 0. A thread takes one row c and
-    // one of its two flag words: its own mask stays in registers (the first four words), the lanes of a wave read the same R[s]
-    if (tid < 2 * (int)K) {
-        const uint32_t c = (uint32_t)tid % K, q = (uint32_t)tid / K;
-        uint32_t rc[4], word = 0;
+    // (b) stable order by detour count
+    if (wave == 0) {
+        const uint32_t key = (uint32_t)lane < m ? (det[lane] << 16) | (uint32_t)lane : ~0u;
+        uint32_t r = 0;
+        for (uint32_t j = 0; j < m; j++) r += (uint32_t)__builtin_amdgcn_readlane((int)key, (int)j) < key;
+        if ((uint32_t)lane < m) order[r] = lane;
+    }
+    // keyword flags of all pairs (index.cu:637,651-654): flag(c, s) = (R[s] & ~R[c]) != 0, lane s of a wave for one c at a time
+    {
+        uint32_t rs[4];
 #pragma unroll
-        for (int w = 0; w < 4; w++) rc[w] = (uint32_t)w < words && c < m ? R[c * words + w] : 0u;
-        for (uint32_t b = 0; b < 32 && q * 32 + b < m; b++) {
-            const uint32_t sidx = q * 32 + b;
+        for (int w = 0; w < 4; w++) rs[w] = (uint32_t)w < words && (uint32_t)lane < m ? R[lane * words + w] : 0u;
+        for (uint32_t c = wave; c < m; c += NWAVES) {
             uint32_t any = 0;
 #pragma unroll
             for (int w = 0; w < 4; w++)
-                if ((uint32_t)w < words) any |= R[sidx * words + w] & ~rc[w];
-            for (uint32_t w = 4; w < words; w++) any |= R[sidx * words + w] & ~(c < m ? R[c * words + w] : 0u);
-            word |= (any != 0 ? 1u : 0u) << b;
+                if ((uint32_t)w < words) any |= rs[w] & ~(uint32_t)__builtin_amdgcn_readlane((int)rs[w], (int)c);
+            for (uint32_t w = 4; w < words; w++) any |= ((uint32_t)lane < m ? R[lane * words + w] : 0u) & ~R[c * words + w];
+            const uint64_t f = __ballot(any != 0);
+            if (lane == 0) F[c] = f;
         }
-        F[c * 2 + q] = c < m ? word : 0u;
     }
-    __syncthreads();
-    // (c)+(d) sequential selection on the Gram matrix: wave 0, lane i keeps selected member i in registers and the
-    // candidate at position i of the order (its Gram row, norm and flag word are handed out with readlane); the Gram
-    // entries of step t + 1 are requested before step t is decided (the lane that would hold candidate t as a new
-    // member asks for its entry too), so a step waits for no memory
+    // the dense Gram matrix on the matrix cores, below the diagonal: every wave takes an eighth of the dimensions and computes the
+    // three tiles for it from one read of the rows; the partial tiles are added in a fixed order (barriers between them): the
+    // result does not depend on timing
+    auto dense_all = [&]() {
+        constexpr int BLOCKS = DIM / 8;
+        floatx16 dacc00, dacc01, dacc11;
+        gram_dense_upper<PRUNE_DENSE_NB>(C, nb_id, m, lane, wave * (BLOCKS / NWAVES), (wave + 1) * (BLOCKS / NWAVES), dacc00, dacc01, dacc11);
+        for (int ph = 0; ph < NWAVES; ph++) {
+            if (wave == ph && m > 0) {
+                gram_dense_store(G, 0, lane, dacc00, dense_mul, ph != 0);
+                if (m > 32) {
+                    gram_dense_store(G, 1, lane, dacc01, dense_mul, ph != 0);
+                    gram_dense_store(G, 3, lane, dacc11, dense_mul, ph != 0);
+                }
+            }
+            __syncthreads();
+        }
+    };
+    auto code_product = [&](uint32_t i, uint32_t j) { // i < j
+        return dense_mul * ((float)reinterpret_cast<const int*>(G)[i * GRAM_STRIDE + j] * (row[i].y * row[j].y));
+    };
+    // above[c], below[c] from what is known; returns whether a pair of the node stays open. bounded: the dense parts are within the sketches'
+    // error, and until the sparse parts are `summed` they stand above the diagonal as integers; until then the sparse parts are known to lie
+    // within the product of the sparse norms. any_open: an LDS word of this call, cleared
+    auto decide = [&](bool bounded, bool summed, uint32_t& any_open) -> bool {
+        bool open = false;
+        const float4 rs = (uint32_t)lane < m ? row[lane] : make_float4(0.f, 0.f, 0.f, 0.f);
+        const float ns = (uint32_t)lane < m ? nrm[lane] : 0.f;
+        for (uint32_t c = wave; c < m; c += NWAVES) {
+            const uint32_t lo = min(c, (uint32_t)lane), hi = max(c, (uint32_t)lane);
+            const bool pair = (uint32_t)lane < m && (uint32_t)lane != c;
+            const float4 rc = row[c];
+            const float nc = nrm[c];
+            float p = 0.f;
+            if (pair) {
+                if (bounded && !summed) p = code_product(lo, hi);
+                else p = G[lo * GRAM_STRIDE + hi] + G[hi * GRAM_STRIDE + lo];
+            }
+            float e = 0.f; // p is exact but for e
+            if (bounded) e = dense_mul * (rs.x * rc.z + rs.z * (rc.x + rc.z));
+            if (!summed) e += rs.w * rc.w;
+            if (bounded || !summed) e += 1e-5f * (dense_mul * rs.x * rc.x + rs.w * rc.w + 1.0f);
+            const bool up = pair && nc < p, dn = pair && ns < p;
+            if (bounded || !summed) open |= pair && !(fabsf(p - nc) > e && fabsf(p - ns) > e); // not a number: open
+            const uint64_t a = __ballot(up), b = __ballot(dn);
+            if (lane == 0) { above[c] = a; below[c] = b; }
+        }
+        if (open) any_open = 1;
+        __syncthreads();
+        return uniform(any_open) != 0;
+    };
+    const bool bounded = sketch != nullptr;
+    if (bounded) __syncthreads(); // the order and the flags are behind one barrier with the code products
+    else dense_all();
+    if (decide(bounded, false, ctl[PC_OPEN])) {
+        if (bounded) { // code products above the diagonal -> dense parts below it
+            for (uint32_t t = tid; t < m * K; t += NT) {
+                const uint32_t i = t / K, j = t % K;
+                if (i < j && j < m) {
+                    G[j * GRAM_STRIDE + i] = code_product(i, j);
+                    G[i * GRAM_STRIDE + j] = 0.f;
+                }
+            }
+            __syncthreads();
+        }
+        if (rank_slots != 0) { // the rank table, with this wave's rows w, w + 8, ... in registers
+            auto own_rows = [&](RtRow<NARROW> (&own)[GR_OWN], uint32_t (&own_shape)[GR_OWN]) {
+#pragma unroll
+                for (int k = 0; k < GR_OWN; k++) {
+                    const uint32_t b = wave + 8 * k;
+                    own_shape[k] = 0;
+                    if (b < m) {
+                        own_shape[k] = uniform(rownnz[b]);
+                        Pairs sp = gram_row(C, rowptr, rownnz, b);
+                        sp.narrow = NARROW ? 1u : 0u;
+                        rt_row_load(own[k], sp, lane);
+                    }
+                }
+            };
+            bool summed = false;
+            if constexpr (NARROW) {
+                RtRow<NARROW> own[GR_OWN];
+                uint32_t own_shape[GR_OWN];
+                own_rows(own, own_shape);
+                summed = gram_sparse_shared(m, G, reinterpret_cast<char*>(tabs), RankTabLds(rank_bits, rank_slots, true).total, rank_bits, rank_span, ovf_cnt, own, own_shape,
+                                            [&](int k) {
+                                                Pairs sp = gram_row(C, rowptr, rownnz, wave + 8 * k);
+                                                sp.narrow = 1u;
+                                                return sp;
+                                            }, tid, wave, lane);
+            }
+            if (!summed) {
+                RtRow<NARROW> own[GR_OWN];
+                uint32_t own_shape[GR_OWN];
+                own_rows(own, own_shape);
+                const RankTab T = ranktab_at(reinterpret_cast<char*>(tabs), rank_bits, rank_slots, rank_span, NARROW);
+                gram_sparse_rank<NARROW>(C, m, G, T, ovf_cnt, rowptr, rownnz, own, own_shape, &ctl[PC_FAIL], tid, NT);
+            }
+        } else if (union_slots) gram_sparse_union(C, nb_id, m, G, reinterpret_cast<char*>(tabs), union_slots, ovf_cnt, rowptr, rownnz, &ctl[PC_FAIL], tid, NT);
+        else if (tgroup == 8) gram_sparse_64<8>(C, nb_id, m, G, tabs, term_slots, ovf_cnt, rowptr, rownnz, &ctl[PC_FAIL], tid, NT);
+        else gram_sparse_64<4>(C, nb_id, m, G, tabs, term_slots, ovf_cnt, rowptr, rownnz, &ctl[PC_FAIL], tid, NT);
+        if (decide(bounded, true, ctl[PC_STILL_OPEN])) {
+            dense_all();
+            decide(false, true, ctl[PC_STILL_OPEN]);
+        }
+    }
+    // (c)+(d) sequential selection, wave 0: lane t holds the masks of the candidate at position t of the order; `live` = the selected
+    // members that are not tombstoned, `taken` = the positions that were selected
     if (wave == 0 && m > 0) {
         const uint32_t ord = (uint32_t)lane < m ? order[lane] : order[0];
-        const float nrm_o = nrm[ord];
-        const uint32_t f_lo = F[ord * 2], f_hi = F[ord * 2 + 1];
-        const uint32_t id_o = nb_id[ord], det_o = det[ord];
-        uint32_t n_sel = 1;
-        uint32_t my_gi = (uint32_t)__builtin_amdgcn_readlane((int)ord, 0), my_kw = 0;
-        bool my_live = lane == 0;
-        float my_nrm = readlane_f32(nrm_o, 0);
-        float p_next = 0.f;
-        if (m > 1) p_next = G[(uint32_t)__builtin_amdgcn_readlane((int)ord, 1) * GRAM_STRIDE + my_gi];
-        for (uint32_t t = 1; t < m; t++) {
-            const uint32_t c = (uint32_t)__builtin_amdgcn_readlane((int)ord, (int)t);
-            const float norm_c = readlane_f32(nrm_o, t);
-            const uint64_t fc = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)f_hi, (int)t) << 32) | (uint32_t)__builtin_amdgcn_readlane((int)f_lo, (int)t);
-            const float p = p_next;
-            if (t + 1 < m) {
-                const uint32_t cn = (uint32_t)__builtin_amdgcn_readlane((int)ord, (int)(t + 1));
-                p_next = G[cn * GRAM_STRIDE + ((uint32_t)lane == n_sel ? c : my_gi)];
+        const uint64_t up = above[ord], dn = below[ord], fl = F[ord];
+        uint64_t live = 1ull << (uint32_t)__builtin_amdgcn_readlane((int)ord, 0), taken = 1, flagged = 0;
+        if (__ballot((uint32_t)lane < m && (up | dn) != 0) == 0) { // no product exceeds a norm: all are taken, a flag needs what stands before only
+            uint64_t before = (uint32_t)lane < m ? 1ull << ord : 0ull;
+            for (int o = 1; o < WAVE; o <<= 1) {
+                const uint64_t x = ((uint64_t)(uint32_t)__shfl_up((uint32_t)(before >> 32), o, WAVE) << 32) | (uint32_t)__shfl_up((uint32_t)before, o, WAVE);
+                if (lane >= o) before |= x;
             }
-            const bool act = (uint32_t)lane < n_sel && my_live;
-            const bool rej = act && norm_c < p, tomb = act && my_nrm < p, noflag = act && !((fc >> my_gi) & 1ull);
-            const bool reject = __ballot(rej) != 0;
-            const bool allflag = __ballot(noflag) == 0;
-            if (tomb) my_live = false;
+            live = taken = m == 64 ? ~0ull : (1ull << m) - 1;
+            flagged = __ballot(lane > 0 && (uint32_t)lane < m && (before & ~(1ull << ord) & ~fl) == 0);
+        } else for (uint32_t t = 1; t < m; t++) {
+            const uint32_t c = (uint32_t)__builtin_amdgcn_readlane((int)ord, (int)t);
+            const bool reject = (readlane64(up, t) & live) != 0, allflag = (live & ~readlane64(fl, t)) == 0;
+            live &= ~readlane64(dn, t);
             if (!reject) {
-                if ((uint32_t)lane == n_sel) { my_gi = c; my_live = true; my_nrm = norm_c; my_kw = allflag ? 1u : 0u; }
-                n_sel++;
+                live |= 1ull << c;
+                taken |= 1ull << t;
+                if (allflag) flagged |= 1ull << t;
             }
         }
         // (e) emit: live members in selection order fill the row, flagged ones beyond d become keyword candidates
-        const bool live = (uint32_t)lane < n_sel && my_live;
-        const uint64_t lb = __ballot(live);
+        const uint32_t id_o = nb_id[ord], det_o = det[ord];
+        const bool alive = ((taken >> lane) & 1) && ((live >> ord) & 1);
+        const uint64_t lb = __ballot(alive);
         const uint32_t pos = __popcll(lb & lane_lt);
-        const uint32_t my_id = nb_id[my_gi], my_det = det[my_gi];
-        if (live && pos < d) { o_fwd[pos] = my_id; o_det[pos] = my_det; }
+        if (alive && pos < d) { o_fwd[pos] = id_o; o_det[pos] = det_o; }
         uint32_t cnt = min((uint32_t)__popcll(lb), d);
-        const bool kwc = live && pos >= d && my_kw;
+        const bool kwc = alive && pos >= d && ((flagged >> lane) & 1);
         const uint64_t kb = __ballot(kwc);
         const uint32_t kpos = __popcll(kb & lane_lt);
-        if (kwc && kpos < APOE_KW_CAND) o_kw[1 + kpos] = my_id;
+        if (kwc && kpos < APOE_KW_CAND) o_kw[1 + kpos] = id_o;
         const uint32_t nkw = min((uint32_t)__popcll(kb), (uint32_t)APOE_KW_CAND);
         if (cnt < d) { // fewer survivors than the row has slots: the remaining neighbours in order, each id once
             bool add = (uint32_t)lane < m;
-            for (uint64_t rest = lb; rest; rest &= rest - 1) add = add && (uint32_t)__builtin_amdgcn_readlane((int)my_id, __builtin_ctzll(rest)) != id_o;
+            for (uint64_t rest = lb; rest; rest &= rest - 1) add = add && (uint32_t)__builtin_amdgcn_readlane((int)id_o, __builtin_ctzll(rest)) != id_o;
             for (uint32_t t = 0; t + 1 < m; t++) add = add && !((uint32_t)lane > t && (uint32_t)__builtin_amdgcn_readlane((int)id_o, (int)t) == id_o);
             const uint64_t ab = __ballot(add);
             const uint32_t at = cnt + __popcll(ab & lane_lt);
@@ -1155,6 +1849,43 @@ __global__ __launch_bounds__(256) void final_rows_kernel(uint32_t n, uint32_t d,
 
 static uint32_t doc_term_slots(const apoe_corpus* c) { return next_pow2(std::max(64u, 2 * (c->max_nnz_s + c->max_nnz_b))); }
 
+// The nodes whose flag is set, in no order: one atomic per wave (one per node on a single counter is 19 ns each, one after the other).
+__global__ __launch_bounds__(256) void open_nodes_kernel(uint32_t n, const uint32_t* __restrict__ flag, uint32_t* count, uint32_t* nodes) {
+    const uint32_t u = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint64_t b = __ballot(u < n && flag[u] != 0);
+    if (b == 0) return;
+    uint32_t at = 0;
+    if (lane_id() == 0) at = atomicAdd(count, (uint32_t)__popcll(b));
+    at = uniform(at) + __popcll(b & ((1ull << lane_id()) - 1));
+    if ((b >> lane_id()) & 1) nodes[at] = u;
+}
+
+// Prunes the nodes that bounds settle (prune_bound_kernel). *n_open, *nodes: the others, a device list in no order; without sketches all of
+// them (*nodes null: 0 .. n).
+static int launch_prune_bounds(apoe_knn* g, uint32_t degree, uint32_t umap_slots, uint32_t map_slots, uint32_t words, uint32_t* n_open, const uint32_t** nodes) {
+    apoe_ctx* ctx = g->ctx;
+    *n_open = g->n;
+    *nodes = nullptr;
+    const uint32_t lds = g->K == 64 ? BoundLds<64>(umap_slots, map_slots, words).total : BoundLds<128>(umap_slots, map_slots, words).total;
+    if (!g->corpus->sketch.p || lds > ctx->lds_per_block) return APOE_OK;
+    if (!g->open.p) APOE_TRY(g->open.alloc(2 * (size_t)g->n + 1)); // flags, number, nodes
+    APOE_HIP(hipMemsetAsync(g->open.p, 0, ((size_t)g->n + 1) * sizeof(uint32_t), ctx->stream));
+    auto kernel = g->K == 64 ? (g->corpus->narrow ? &prune_bound_kernel<64, true> : &prune_bound_kernel<64, false>)
+                             : (g->corpus->narrow ? &prune_bound_kernel<128, true> : &prune_bound_kernel<128, false>);
+    APOE_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    kernel<<<g->n, g->K * 4, lds, ctx->stream>>>(g->corpus->view(), g->dense_scale * g->dense_scale, g->norms.p, g->ids.p, g->dist.p, degree, g->fwd.p, g->det.p,
+                                                 g->cnt.p, g->kw.p, umap_slots, map_slots, words, g->corpus->sketch_meta.p,
+                                                 reinterpret_cast<const uint4*>(g->corpus->sketch.p), g->open.p);
+    APOE_HIP(hipGetLastError());
+    uint32_t *count = g->open.p + g->n, *list = count + 1;
+    open_nodes_kernel<<<(g->n + 255) / 256, 256, 0, ctx->stream>>>(g->n, g->open.p, count, list);
+    APOE_HIP(hipGetLastError());
+    APOE_HIP(hipMemcpyAsync(n_open, count, sizeof(uint32_t), hipMemcpyDeviceToHost, ctx->stream));
+    APOE_HIP(hipStreamSynchronize(ctx->stream));
+    *nodes = list;
+    return APOE_OK;
+}
+
 int launch_prune(apoe_knn* g, uint32_t degree) {
     apoe_ctx* ctx = g->ctx;
     const uint32_t term_slots = doc_term_slots(g->corpus);
@@ -1188,13 +1919,20 @@ int launch_prune(apoe_knn* g, uint32_t degree) {
         }
     }
     const GramPruneLds GL(gram_slots, tgroup, uset_slots, map_slots, words, union_slots, rank_bits, rank_slots, narrow);
-    if (g->K == GRAM_ROWS && GL.total <= lds_budget && !g->force_sequential_prune) {
+    const bool gathered = !g->force_sequential_prune && (g->K == GRAM_ROWS ? GL.total <= lds_budget : g->K <= PS_MAX && gram_tiles_fit(g));
+    // nodes that bounds settle are done here; the others are left in a list
+    uint32_t n_open = g->n;
+    const uint32_t* open = nullptr;
+    if (gathered) APOE_TRY(launch_prune_bounds(g, degree, uset_slots, map_slots, words, &n_open, &open));
+    if (gathered && n_open == 0) return APOE_OK;
+    if (g->K == GRAM_ROWS && gathered) {
         APOE_HIP(hipMemsetAsync(g->counter.p + 1, 0, sizeof(unsigned long long), ctx->stream));
         auto kernel = g->corpus->narrow ? &prune_gram_kernel<GRAM_THREADS, true> : &prune_gram_kernel<GRAM_THREADS, false>;
         APOE_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)GL.total));
-        kernel<<<g->n, GRAM_THREADS, GL.total, ctx->stream>>>(g->corpus->view(), g->dense_scale * g->dense_scale, g->norms.p, g->ids.p, g->dist.p, degree,
-                                                              g->fwd.p, g->det.p, g->cnt.p, g->kw.p, gram_slots, tgroup, uset_slots, map_slots, words,
-                                                              union_slots, rank_bits, rank_slots, rank_span, g->counter.p + 1);
+        kernel<<<n_open, GRAM_THREADS, GL.total, ctx->stream>>>(g->corpus->view(), g->dense_scale * g->dense_scale, g->norms.p, g->ids.p, g->dist.p, degree,
+                                                                g->fwd.p, g->det.p, g->cnt.p, g->kw.p, gram_slots, tgroup, uset_slots, map_slots, words,
+                                                                union_slots, rank_bits, rank_slots, rank_span, g->corpus->sketch_meta.p,
+                                                                reinterpret_cast<const uint4*>(g->corpus->sketch.p), open, g->counter.p + 1);
         APOE_HIP(hipGetLastError());
         unsigned long long failed = 0;
         APOE_HIP(hipMemcpyAsync(&failed, g->counter.p + 1, sizeof(failed), hipMemcpyDeviceToHost, ctx->stream));
@@ -1204,19 +1942,19 @@ int launch_prune(apoe_knn* g, uint32_t degree) {
     }
     // lists longer than 64 entries: Gram matrices by the tile kernel of the local join, a batch of nodes at a time, and the
     // selection on them; a row too long for a tile's table sends the whole prune to the table-probing kernel below
-    if (g->K > GRAM_ROWS && g->K <= PS_MAX && !g->force_sequential_prune && gram_tiles_fit(g)) {
+    if (g->K > GRAM_ROWS && gathered) {
         const SelectLds SL(uset_slots, map_slots, words);
         if (SL.total <= ctx->lds_per_block) {
-            const uint32_t batch = std::min<uint32_t>(g->n, 32768u);
+            const uint32_t batch = std::min<uint32_t>(n_open, 32768u);
             DevBuf<float> gram;
             APOE_TRY(gram.alloc((size_t)batch * PS_MAX * PS_MAX));
             APOE_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&prune_select_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)SL.total));
             unsigned long long unfit = 0;
-            for (uint32_t node0 = 0; node0 < g->n && !unfit; node0 += batch) {
-                const uint32_t cnt = std::min(batch, g->n - node0);
-                APOE_TRY(launch_gram_tiles(g, node0, cnt, gram.p, &unfit));
+            for (uint32_t node0 = 0; node0 < n_open && !unfit; node0 += batch) {
+                const uint32_t cnt = std::min(batch, n_open - node0);
+                APOE_TRY(launch_gram_tiles(g, open, node0, cnt, gram.p, &unfit));
                 if (unfit) break;
-                prune_select_kernel<<<cnt, PS_THREADS, SL.total, ctx->stream>>>(g->corpus->view(), g->norms.p, g->K, g->ids.p, g->dist.p, degree, node0, gram.p,
+                prune_select_kernel<<<cnt, PS_THREADS, SL.total, ctx->stream>>>(g->corpus->view(), g->norms.p, g->K, g->ids.p, g->dist.p, degree, open, node0, gram.p,
                                                                               g->fwd.p, g->det.p, g->cnt.p, g->kw.p, uset_slots, map_slots, words);
                 APOE_HIP(hipGetLastError());
             }
