@@ -38,6 +38,8 @@ __host__ __device__ inline uint32_t desc_nnz_b(uint64_t d) { return (uint32_t)(d
 // A corpus is narrow when every term id of both paths is below 65536 (6 instead of 8 bytes a pair).
 // Records start on a 128-byte boundary, and so does the term array of a narrow record: a read of
 // a row, of its values or of its terms then starts at a memory line and only its last line is partial.
+// Coded records (narrow ones, unless memory is short): behind the terms nnz signed bytes and one scale per path, value ~ scale * byte to
+// half a step. Terms, bytes and scales are one read of 3 nnz + 8 bytes, from which a search bounds the sparse part (below).
 constexpr uint32_t REC_ALIGN = 128;
 // Of the 8-bit sketch of a document's dense row (below): dense row ~ scale * codes, Euclidean norm of the difference at
 // most err (infinite: no sketch).
@@ -56,8 +58,10 @@ struct CorpusView {
 __host__ __device__ inline uint32_t narrow_keys_offset(uint32_t nnz) { // of the term array, from the first value
     return (4u * nnz + REC_ALIGN - 1) & ~(REC_ALIGN - 1);
 }
-__host__ __device__ inline uint64_t record_units(uint32_t nnz, bool narrow) { // 16-byte units of one record
-    const uint64_t bytes = (uint64_t)DENSE_BYTES + (narrow ? (uint64_t)narrow_keys_offset(nnz) + 2ull * nnz : 8ull * nnz);
+__host__ __device__ inline uint32_t codes_offset(uint32_t nnz) { return narrow_keys_offset(nnz) + 2u * nnz; }          // from the first value
+__host__ __device__ inline uint32_t code_scales_offset(uint32_t nnz) { return (codes_offset(nnz) + nnz + 3u) & ~3u; } // two floats: SPLADE, BM25
+__host__ __device__ inline uint64_t record_units(uint32_t nnz, bool narrow, bool coded) { // 16-byte units of one record
+    const uint64_t bytes = (uint64_t)DENSE_BYTES + (coded ? (uint64_t)code_scales_offset(nnz) + 8 : narrow ? (uint64_t)narrow_keys_offset(nnz) + 2ull * nnz : 8ull * nnz);
     return (bytes + REC_ALIGN - 1) / REC_ALIGN * (REC_ALIGN / 16);
 }
 
@@ -529,6 +533,99 @@ __device__ __forceinline__ float row_probe(const CorpusView& C, const RowLoad& r
             const bool b = NARROW ? j >= s.ns : (int)kv.x < 0;
             query_match<NARROW, KWD>((b ? tab_b : tab_s)[query_hash<NARROW>(kv.x) & (b ? T.mask_b : T.mask_s)], kv.x, kv.y, true, b, acc, hit);
             query_overflow<NARROW, KWD>(T, n_ovf, kv.x, kv.y, true, b, acc, hit);
+        }
+    }
+    return acc;
+}
+
+// ---- codes of a record's values: a bound of the sparse part, never a result ----
+// value = scale * code + rest, |rest| <= scale / 2, so the sparse sum is at most the sum over the matched terms of q * scale * code +
+// |q| * scale / 2. CODE_STEP has 0.01 of a step of room for what either sum rounds: a lane's chain of c products and the six additions
+// behind it err by at most (c + 6) 2^-24 * 127.5 steps, which reaches 0.005 at c = 650, and LDS holds no query of 64 * 650 terms.
+// A row with a value that is no number or infinite has an infinite scale: its bound is not a number and settles nothing.
+constexpr float CODE_STEP = 0.51f;
+struct CodeLoad {
+    uint32_t k[3];
+    int v[3];
+    float scale_s, scale_b;
+    int n, nsr; // wave-uniform: pairs of the paths in use (0 for a candidate that is not there), SPLADE pairs among them
+};
+__device__ __forceinline__ void code_issue(CodeLoad& r, const CorpusView& C, uint64_t desc, bool live, uint32_t paths) {
+    const int lane = lane_id();
+    const uint32_t ns = desc_nnz_s(desc), nnz = ns + desc_nnz_b(desc), begin = (paths & PATH_SPARSE) ? 0u : ns;
+    r.n = live ? (int)(((paths & PATH_BM25) ? nnz : ns) - begin) : 0;
+    r.nsr = (int)(ns - begin);
+    const char* base = C.recs + desc_off(desc) * 16 + DENSE_BYTES;
+    const uint16_t* keys = reinterpret_cast<const uint16_t*>(base + narrow_keys_offset(nnz)) + begin;
+    const signed char* codes = reinterpret_cast<const signed char*>(base + codes_offset(nnz)) + begin;
+    const float* scales = reinterpret_cast<const float*>(base + code_scales_offset(nnz));
+#pragma unroll
+    for (int c = 0; c < 3; c++) { // not clamped to the row, as row_issue
+        r.k[c] = keys[lane + WAVE * c];
+        r.v[c] = codes[lane + WAVE * c];
+    }
+    r.scale_s = scales[0];
+    r.scale_b = scales[1];
+}
+// This lane's part of the upper bound of the candidate's sparse sum; hit as row_probe. desc(): the candidate's descriptor again, for a row
+// that is longer than the loads (what follows from it is not kept in scalar registers for a whole batch).
+template <bool KWD, typename Desc>
+__device__ __forceinline__ float code_probe(const CorpusView& C, const CodeLoad& r, Desc desc, uint32_t paths, const QueryTabs& T, uint32_t n_ovf, bool& hit) {
+    const int lane = lane_id();
+    float acc = 0.f;
+    bool in[3], bm[3];
+    uint4 e[3];
+    const uint4* tab_s = T.b;
+    const uint4* tab_b = T.b + T.mask_s + 1;
+    auto bucket = [&](uint32_t key, bool b) { return (b ? tab_b : tab_s)[query_hash<true>(key) & (b ? T.mask_b : T.mask_s)]; };
+    auto more = [&](float q, int code, bool b) {
+        const float t = q * (b ? r.scale_b : r.scale_s);
+        return fmaf((float)code, t, fmaf(CODE_STEP, fabsf(t), acc));
+    };
+    auto match = [&](const uint4 x, uint32_t key, int code, bool valid, bool b) {
+        constexpr uint32_t cmp = KWD ? ~BM25_BIT : ~0u;
+        const bool m0 = ((x.x ^ key) & cmp) == 0, m1 = ((x.z ^ key) & cmp) == 0;
+        const float next = more(__uint_as_float(m0 ? x.y : x.w), code, b);
+        acc = valid && (m0 || m1) ? next : acc;
+        if (KWD) hit |= valid && b && ((m0 && (int)x.x < 0) || (m1 && (int)x.z < 0));
+    };
+    auto overflow = [&](uint32_t raw, int code, bool valid, bool b) {
+        const uint32_t key = raw | (b ? BM25_BIT : 0u);
+        const uint32_t front = KWD ? n_ovf & 0xFFFFu : n_ovf, all = KWD ? front + (n_ovf >> 16) : n_ovf;
+        for (uint32_t i = 0; i < all; i++) {
+            const bool required = KWD && i >= front;
+            const uint2 o = T.ovf[required ? T.ovf_cap - 1 - (i - front) : i];
+            if (valid && o.x == key) {
+                acc = more(__uint_as_float(o.y), code, b);
+                if (KWD) hit |= required;
+            }
+        }
+    };
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+        in[c] = lane < r.n - WAVE * c;
+        bm[c] = lane >= r.nsr - WAVE * c;
+        e[c] = bucket(r.k[c], bm[c]);
+    }
+    asm volatile("" : "+v"(e[0].x), "+v"(e[1].x), "+v"(e[2].x)); // the three reads together, as row_probe
+#pragma unroll
+    for (int c = 0; c < 3; c++) match(e[c], r.k[c], r.v[c], in[c], bm[c]);
+    if (n_ovf) {
+#pragma unroll
+        for (int c = 0; c < 3; c++) overflow(r.k[c], r.v[c], in[c], bm[c]);
+    }
+    if (r.n > 3 * WAVE) { // rows with more than 192 pairs
+        const uint64_t d = desc();
+        const uint32_t ns = desc_nnz_s(d), nnz = ns + desc_nnz_b(d), begin = (paths & PATH_SPARSE) ? 0u : ns;
+        const char* base = C.recs + desc_off(d) * 16 + DENSE_BYTES;
+        const uint16_t* keys = reinterpret_cast<const uint16_t*>(base + narrow_keys_offset(nnz));
+        const signed char* codes = reinterpret_cast<const signed char*>(base + codes_offset(nnz));
+        for (uint32_t j = begin + 3 * WAVE + lane; j < begin + (uint32_t)r.n; j += WAVE) {
+            const uint32_t key = keys[j];
+            const int code = codes[j];
+            const bool b = j >= ns;
+            match(bucket(key, b), key, code, true, b);
+            overflow(key, code, true, b);
         }
     }
     return acc;

@@ -114,8 +114,9 @@ struct apoe_corpus {
     apoe_ctx* ctx = nullptr;
     uint32_t n = 0, dim = 0, max_nnz_s = 0, max_nnz_b = 0;
     uint32_t max_term = 0; // largest term id of either path
-    uint64_t rec_bytes = 0, total_pairs = 0;
+    uint64_t rec_bytes = 0, total_pairs = 0; // bytes without the codes: what a scan of all rows reads
     bool narrow = false; // pair format of the records (6 instead of 8 bytes a pair when every term id is below 65536)
+    bool coded = false;  // narrow records carry byte codes of their values (a bound for the search)
     apoe::DevBuf<uint64_t> desc;
     apoe::DevBuf<char> recs;
     apoe::DevBuf<float> dnorm;
@@ -183,7 +184,7 @@ int copy_out(apoe_ctx* ctx, void* dst_any, const void* src_dev, size_t bytes);
 // Kernel launchers (one per .hip file).
 int launch_pack(apoe_ctx* ctx, uint32_t n, const float* dense, const uint32_t* s_off, const uint32_t* s_idx, const float* s_val,
                 const uint32_t* b_off, const uint32_t* b_idx, const float* b_val, const uint64_t* desc, char* recs, float* dnorm,
-                SketchMeta* sketch_meta, uint32_t* sketch, bool narrow);
+                SketchMeta* sketch_meta, uint32_t* sketch, bool narrow, bool coded);
 int launch_max_u32(apoe_ctx* ctx, const uint32_t* a_dev, size_t n, uint32_t* out_dev);
 int launch_half_rows(apoe_ctx* ctx, const apoe_corpus* c, uint16_t* out_dev);
 int launch_distance_batch(apoe_ctx* ctx, const apoe_corpus* c, const apoe_queries* q, const float* w3, const uint32_t* ids_dev,

@@ -255,17 +255,36 @@ int apoe_corpus_create(apoe_ctx* ctx, uint32_t n, uint32_t dim, const float* den
         c->narrow = max_term < 65536u;
         c->max_term = max_term;
         std::vector<uint64_t> desc(n);
-        uint64_t off16 = 0;
+        const bool codes = c->narrow;
+        uint64_t off16 = 0, with_codes = 0;
         for (uint32_t i = 0; i < n; i++) {
             const uint32_t ns = hs[i + 1] - hs[i], nb = hb[i + 1] - hb[i];
-            desc[i] = make_desc(off16, ns, nb);
-            off16 += record_units(ns + nb, c->narrow);
+            desc[i] = make_desc(codes ? with_codes : off16, ns, nb);
+            off16 += record_units(ns + nb, c->narrow, false);
+            with_codes += record_units(ns + nb, c->narrow, codes);
         }
         APOE_REQUIRE(off16 < (1ull << DESC_OFF_BITS), "corpus of %llu bytes exceeds the record address range", (unsigned long long)off16 * 16);
         c->rec_bytes = off16 * 16;
         c->total_pairs = (uint64_t)hs[n] + hb[n];
         APOE_TRY(c->desc.alloc(n));
-        APOE_TRY(c->recs.alloc(c->rec_bytes + ROW_LOAD_SLACK)); // unclamped row loads may read past the last record
+        if (codes) {
+            // Nothing depends on the codes (about 4 % of the records): a corpus that would take more than a quarter of the free device memory with
+            // them does without.
+            size_t free_now = 0, total_now = 0;
+            APOE_HIP(hipMemGetInfo(&free_now, &total_now));
+            c->coded = with_codes < (1ull << DESC_OFF_BITS) && with_codes * 16 <= free_now / 4 && c->recs.try_alloc(with_codes * 16 + ROW_LOAD_SLACK);
+        }
+        if (!c->coded) {
+            if (codes) {
+                off16 = 0;
+                for (uint32_t i = 0; i < n; i++) {
+                    const uint32_t ns = hs[i + 1] - hs[i], nb = hb[i + 1] - hb[i];
+                    desc[i] = make_desc(off16, ns, nb);
+                    off16 += record_units(ns + nb, true, false);
+                }
+            }
+            APOE_TRY(c->recs.alloc(c->rec_bytes + ROW_LOAD_SLACK)); // unclamped row loads may read past the last record
+        }
         APOE_TRY(c->dnorm.alloc(n));
         size_t free_bytes = 0, total_bytes = 0;
         APOE_HIP(hipMemGetInfo(&free_bytes, &total_bytes));
@@ -281,7 +300,7 @@ int apoe_corpus_create(apoe_ctx* ctx, uint32_t n, uint32_t dim, const float* den
         if ((size_t)n * SKETCH_BYTES <= free_bytes / 10 && !(c->sketch.try_alloc((size_t)n * (SKETCH_BYTES / 4)) && c->sketch_meta.try_alloc(n)))
             c->sketch.release();
         APOE_TRY(launch_pack(ctx, n, d_dense.p, d_soff.p, d_sidx.p, d_sval.p, d_boff.p, d_bidx.p, d_bval.p, c->desc.p, c->recs.p, c->dnorm.p,
-                             c->sketch_meta.p, c->sketch.p, c->narrow));
+                             c->sketch_meta.p, c->sketch.p, c->narrow, c->coded));
         APOE_HIP(hipStreamSynchronize(ctx->stream));
     }
     *out = c.release();

@@ -26,8 +26,8 @@ __global__ __launch_bounds__(256) void pack_kernel(uint32_t n, const float* __re
                                                    const uint32_t* __restrict__ s_idx, const float* __restrict__ s_val,
                                                    const uint32_t* __restrict__ b_off, const uint32_t* __restrict__ b_idx,
                                                    const float* __restrict__ b_val, const uint64_t* __restrict__ desc, char* recs, float* dnorm,
-                                                   SketchMeta* sketch_meta, uint32_t* sketch, uint32_t narrow) {
-    __shared__ float part[4], top[4], rest[4];
+                                                   SketchMeta* sketch_meta, uint32_t* sketch, uint32_t narrow, uint32_t coded) {
+    __shared__ float part[4], top[4], rest[4], most[2][4];
     for (uint32_t doc = blockIdx.x; doc < n; doc += gridDim.x) {
         const uint64_t d = desc[doc];
         char* rec = recs + desc_off(d) * 16;
@@ -69,16 +69,42 @@ __global__ __launch_bounds__(256) void pack_kernel(uint32_t n, const float* __re
                 vals[ns + j] = b_val[b0 + j];
                 keys[ns + j] = (uint16_t)b_idx[b0 + j];
             }
-            // fill the two alignment gaps so that a record never holds stale bytes
+            // fill the alignment gaps so that a record never holds stale bytes
             for (uint32_t j = nnz + threadIdx.x; j < narrow_keys_offset(nnz) / 4; j += blockDim.x) vals[j] = 0.f;
-            const uint32_t key_slots = (uint32_t)(record_units(nnz, true) * 16 - DENSE_BYTES - narrow_keys_offset(nnz)) / 2;
-            for (uint32_t j = nnz + threadIdx.x; j < key_slots; j += blockDim.x) keys[j] = 0xFFFFu;
+            const uint32_t end = (uint32_t)(record_units(nnz, true, coded) * 16 - DENSE_BYTES);
+            if (!coded) {
+                for (uint32_t j = nnz + threadIdx.x; j < (end - narrow_keys_offset(nnz)) / 2; j += blockDim.x) keys[j] = 0xFFFFu;
+            } else {
+                float high[2] = {0.f, 0.f}; // largest magnitude per path; a value that is no number counts as infinite
+                auto raise = [](float& to, float v) { to = v == v ? fmaxf(to, fabsf(v)) : __builtin_inff(); };
+                for (uint32_t j = threadIdx.x; j < ns; j += blockDim.x) raise(high[0], s_val[s0 + j]);
+                for (uint32_t j = threadIdx.x; j < nb; j += blockDim.x) raise(high[1], b_val[b0 + j]);
+                for (int p = 0; p < 2; p++) {
+                    const float m = -wave_min_dpp(-high[p]);
+                    if (lane_id() == 0) most[p][threadIdx.x / WAVE] = m; // last read before the barriers at the next document's start
+                }
+                __syncthreads();
+                float per[2], step[2];
+                for (int p = 0; p < 2; p++) {
+                    const float m = fmaxf(fmaxf(most[p][0], most[p][1]), fmaxf(most[p][2], most[p][3]));
+                    const bool usable = m > 1e-30f; // below, half a step of 2e-30 covers the value
+                    per[p] = usable ? 127.f / m : 0.f;
+                    step[p] = usable ? m / 127.f : m > 0.f ? 2e-30f : 0.f;
+                }
+                signed char* codes = reinterpret_cast<signed char*>(rec + DENSE_BYTES + codes_offset(nnz));
+                for (uint32_t j = threadIdx.x; j < ns; j += blockDim.x) codes[j] = (signed char)sketch_code(s_val[s0 + j], per[0]);
+                for (uint32_t j = threadIdx.x; j < nb; j += blockDim.x) codes[ns + j] = (signed char)sketch_code(b_val[b0 + j], per[1]);
+                const uint32_t scales = code_scales_offset(nnz);
+                if (threadIdx.x < 2) reinterpret_cast<float*>(rec + DENSE_BYTES + scales)[threadIdx.x] = step[threadIdx.x];
+                if (threadIdx.x < scales - codes_offset(nnz) - nnz) codes[nnz + threadIdx.x] = 0;
+                for (uint32_t j = scales + 8 + 4 * threadIdx.x; j < end; j += 4 * blockDim.x) *reinterpret_cast<uint32_t*>(rec + DENSE_BYTES + j) = ~0u;
+            }
         } else {
             uint2* sp = reinterpret_cast<uint2*>(rec + DENSE_BYTES);
             for (uint32_t j = threadIdx.x; j < ns; j += blockDim.x) sp[j] = make_uint2(s_idx[s0 + j], __float_as_uint(s_val[s0 + j]));
             for (uint32_t j = threadIdx.x; j < nb; j += blockDim.x)
                 sp[ns + j] = make_uint2(b_idx[b0 + j] | BM25_BIT, __float_as_uint(b_val[b0 + j]));
-            const uint32_t pair_slots = (uint32_t)(record_units(nnz, false) * 16 - DENSE_BYTES) / 8;
+            const uint32_t pair_slots = (uint32_t)(record_units(nnz, false, false) * 16 - DENSE_BYTES) / 8;
             for (uint32_t j = nnz + threadIdx.x; j < pair_slots; j += blockDim.x) sp[j] = make_uint2(EMPTY, 0u);
         }
     }
@@ -86,10 +112,10 @@ __global__ __launch_bounds__(256) void pack_kernel(uint32_t n, const float* __re
 
 int launch_pack(apoe_ctx* ctx, uint32_t n, const float* dense, const uint32_t* s_off, const uint32_t* s_idx, const float* s_val,
                 const uint32_t* b_off, const uint32_t* b_idx, const float* b_val, const uint64_t* desc, char* recs, float* dnorm,
-                SketchMeta* sketch_meta, uint32_t* sketch, bool narrow) {
+                SketchMeta* sketch_meta, uint32_t* sketch, bool narrow, bool coded) {
     uint32_t grid = n < 65536u * 16u ? n : 65536u * 16u;
     if (grid == 0) return APOE_OK;
-    pack_kernel<<<grid, 256, 0, ctx->stream>>>(n, dense, s_off, s_idx, s_val, b_off, b_idx, b_val, desc, recs, dnorm, sketch_meta, sketch, narrow ? 1u : 0u);
+    pack_kernel<<<grid, 256, 0, ctx->stream>>>(n, dense, s_off, s_idx, s_val, b_off, b_idx, b_val, desc, recs, dnorm, sketch_meta, sketch, narrow ? 1u : 0u, coded ? 1u : 0u);
     APOE_HIP(hipGetLastError());
     return APOE_OK;
 }

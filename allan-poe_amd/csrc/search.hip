@@ -12,9 +12,10 @@ constexpr int MAX_NEW = 64;   // fresh candidates per step: one lane each in wav
 // Tuning constants: the measured best on MI355X.
 #define APOE_SEARCH_WAVES_PER_EU 6 // plain search: 12 queries per CU fit its LDS; the other modes need more LDS per query and stay at 5 (a macro: it sits in an attribute)
 constexpr int EVAL_BATCH = 3;  // candidates whose sparse parts a wave keeps in flight together
+constexpr int CODE_BATCH = 3;  // rows whose codes a wave keeps in flight together
 constexpr int DENSE_BATCH = 1; // dense rows a wave keeps in flight together
 constexpr int MERGE_ROUNDS = 4; // 64-element rounds of the pool that the merge moves per LDS round trip
-constexpr int STATS = 9;      // counters of a launch; the workspace keeps 16 words for them
+constexpr int STATS = 10;     // counters of a launch; the workspace keeps 16 words for them
 constexpr int SKETCH_BATCH = 4; // sketches a wave keeps in flight together
 constexpr int RING = 32;      // keyword-filter search: evicted keyword hits kept beside the pool (query.cu:18)
 
@@ -49,7 +50,8 @@ struct SearchArgs {
     uint32_t* codes;       // of the query's dense row, 1 KB per workgroup: in device memory (it is read beside sketches, which take longer), since a
                            // kilobyte of LDS more costs long batches a resident query per CU (12 -> 11: 3 %)
     unsigned long long* work; // [0] next query, [1] expansions, [2] evaluations, [3] nnz splade, [4] nnz bm25, [5] dense rows (fp32 or half) read in the walk,
-                              // [6] pool entries evaluated again in fp32, [7] their pairs, [8] sketches read
+                              // [6] pool entries evaluated again in fp32, [7] their pairs, [8] sketches read, [9] pairs of the evaluations that codes settled
+    uint32_t coded;           // 1: the records carry codes of their values and the search may ask them
     uint32_t full_eval;       // 1: read the dense row of every candidate (no bound test)
     const uint16_t* half;     // not null: the walk takes dense parts from the half-precision rows, the final pool is evaluated again in fp32
     uint32_t slots_s, slots_b, ovf_cap; // buckets of the query's SPLADE / BM25 term table, entries of the overflow list
@@ -313,7 +315,8 @@ __device__ __forceinline__ GlobalWord* graph_row(const SearchArgs& a, uint32_t i
     return row;
 }
 
-template <int NW, int MODE, bool NARROW, bool HALF>
+// CODES: pairs are bounded by the codes of their values before they are read (figures where that is done).
+template <int NW, int MODE, bool NARROW, bool HALF, bool CODES>
 __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE == MODE_PLAIN && !HALF ? APOE_SEARCH_WAVES_PER_EU : 5, 8))) void search_kernel(SearchArgs a) {
     constexpr bool KG = MODE == MODE_KG, KWD = MODE == MODE_KEYWORD;
     // Whether wave 0 asks for more than the walk may need (graph row of the first unexplored entry, descriptors of visited neighbours) to
@@ -420,7 +423,7 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
         if (tid == 0) { qs[0] = q_scale; qs[1] = q_err; }
         const bool sketched = __builtin_amdgcn_readfirstlane((int)(q_scale > 0.f)) != 0;
         uint32_t st_exp = 0, st_eval = 0, st_dense = 0, st_again = 0, st_again_pairs = 0, st_sketch = 0; // wave-uniform counters of one query
-        uint32_t ln_s = 0, ln_b = 0;                    // pairs read for the candidates this lane decided
+        uint32_t ln_s = 0, ln_b = 0, ln_coded = 0;      // pairs read for the candidates this lane decided; of those that codes settled
         Front front; // wave 0: the first unexplored pool entry
         front.id = EMPTY;
         front.slot = 0;
@@ -573,16 +576,21 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
                 g_c = lane < (int)a.degree ? row[lane] : EMPTY;
                 if (KWD) g_kw = lane < APOE_KW_SLOTS ? row[a.degree + lane] : 0u;
             }
-            // stage 1: the sparse parts of this wave's candidates (wave + k * NW), EVAL_BATCH of them in flight.
-            // No branch on whether a candidate of the batch exists: one that does not is a row of no pairs,
-            // so the loads of the whole batch are issued back to back.
-            auto eval_rows = [&](auto nb, uint32_t j) {
+            // Stage 1: the sparse parts of this wave's candidates (wave + k * NW), several rows in flight. No branch on whether a candidate
+            // of the batch exists: one that does not is a row of no pairs, so the loads of the whole batch are issued back to back.
+            // With codes, an upper bound of the sparse part from the terms and a byte a value instead (3 bytes a pair, not 6, CODE_BATCH rows in
+            // flight); decision and sketches go by that bound, and the pairs of the few candidates that stay open come with their dense rows.
+            // 10 000 queries on 1 M docs: i.i.d. at cands 256 38.4 -> 36.0 ms (the vector units are busy for 0.66 of the cycles now, 0.44 before: a coded
+            // row takes more instructions), with dense neighbours at cands 80 21.5 -> 19.5; three or four rows in flight measure the same, and so do
+            // pairs and rows of two open candidates together. Short batches, four and more waves a query, are bound by the chain of one query,
+            // which a second read of the open candidates' pairs would lengthen: they read the pairs at once.
+            auto eval_rows = [&](auto nb, auto at) { // at(b): the b-th candidate, n_new or more: there is none
                 constexpr int NB = decltype(nb)::value;
                 RowLoad rl[NB];
                 RowInfo ri[NB];
 #pragma unroll
                 for (int b = 0; b < NB; b++) {
-                    const uint32_t jj = j + b * NW;
+                    const uint32_t jj = at(b);
                     row_issue<NARROW>(rl[b], ri[b], a.C, readlane64(my_desc, jj & (WAVE - 1)), jj < n_new, a.paths);
                 }
                 float acc[NB];
@@ -594,6 +602,33 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
                 }
 #pragma unroll
                 for (int b = 0; b < NB; b++) {
+                    const uint32_t jj = at(b);
+                    const float rs = row_sum_dpp(acc[b]);
+                    if (jj < n_new) {
+                        if ((lane & 15) == 0) part[jj * 4 + (lane >> 4)] = rs;
+                        if (KWD) {
+                            const bool kw_hit = __ballot(hit[b]) != 0;
+                            if (lane == 0) new_ent[jj] = kw_hit ? 1u : 0u;
+                        }
+                    }
+                }
+            };
+            auto code_rows = [&](uint32_t j) {
+                CodeLoad rl[CODE_BATCH];
+#pragma unroll
+                for (int b = 0; b < CODE_BATCH; b++) {
+                    const uint32_t jj = j + b * NW;
+                    code_issue(rl[b], a.C, readlane64(my_desc, jj & (WAVE - 1)), jj < n_new, a.paths);
+                }
+                float acc[CODE_BATCH];
+                bool hit[CODE_BATCH];
+#pragma unroll
+                for (int b = 0; b < CODE_BATCH; b++) {
+                    hit[b] = false;
+                    acc[b] = code_probe<KWD>(a.C, rl[b], [&]() { return readlane64(my_desc, (j + b * NW) & (WAVE - 1)); }, a.paths, T, n_ovf, hit[b]);
+                }
+#pragma unroll
+                for (int b = 0; b < CODE_BATCH; b++) {
                     const uint32_t jj = j + b * NW;
                     const float rs = row_sum_dpp(acc[b]);
                     if (jj < n_new) {
@@ -605,14 +640,18 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
                     }
                 }
             };
-            if (NW >= 4) { // a few rows a wave at most expansions: a row that is not there would cost issue slots of a SIMD that several waves share
+            const bool by_codes = CODES && thr_eff < __builtin_inff();
+            if (CODES && by_codes) {
+                for (uint32_t j = wave; j < n_new; j += NW * CODE_BATCH) code_rows(j);
+            } else if (NW >= 4) { // a few rows a wave at most expansions: a row that is not there would cost issue slots of a SIMD that several waves share
                 for (uint32_t j = wave; j < n_new; j += NW * EVAL_BATCH) {
-                    if (j + 2 * NW < n_new) eval_rows(std::integral_constant<int, 3>{}, j);
-                    else if (j + NW < n_new) eval_rows(std::integral_constant<int, 2>{}, j);
-                    else eval_rows(std::integral_constant<int, 1>{}, j);
+                    auto at = [&](int b) { return j + b * NW; };
+                    if (j + 2 * NW < n_new) eval_rows(std::integral_constant<int, 3>{}, at);
+                    else if (j + NW < n_new) eval_rows(std::integral_constant<int, 2>{}, at);
+                    else eval_rows(std::integral_constant<int, 1>{}, at);
                 }
             } else {
-                for (uint32_t j = wave; j < n_new; j += NW * EVAL_BATCH) eval_rows(std::integral_constant<int, EVAL_BATCH>{}, j);
+                for (uint32_t j = wave; j < n_new; j += NW * EVAL_BATCH) eval_rows(std::integral_constant<int, EVAL_BATCH>{}, [&](int b) { return j + b * NW; });
             }
             wave_fence();
             // the decision for all of the wave's candidates at once, lane l for candidate l: a candidate whose
@@ -702,9 +741,11 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
                 need &= ~__ballot(far);
                 wave_fence();
             }
+            if (CODES && by_codes && mine && !((need >> lane) & 1))
+                ln_coded += ((a.paths & PATH_SPARSE) ? desc_nnz_s(my_desc) : 0u) + ((a.paths & PATH_BM25) ? desc_nnz_b(my_desc) : 0u);
+            // stage 3: the dense rows of the survivors, DENSE_BATCH rows in flight (two of the half-precision rows); behind codes the pairs with them
             st_dense += __popcll(need);
-            // stage 3: the dense rows of the survivors, DENSE_BATCH rows in flight (two of the half-precision rows)
-            while (HALF && need) {
+            while (HALF && !CODES && need) {
                 DenseRowHalf row[2];
                 uint32_t jj[2];
 #pragma unroll
@@ -724,7 +765,7 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
                     }
                 }
             }
-            while (!HALF && need) {
+            while (!HALF && !CODES && need) {
                 DenseRow row[DENSE_BATCH];
                 uint32_t jj[DENSE_BATCH];
 #pragma unroll
@@ -745,6 +786,42 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
                         }
                         const float dsum = dense_finish_lds(row[b], qd, 1.0f);
                         if (lane == 0) new_dist[jj[b]] = 1.0f - (dsum + new_dist[jj[b]]) - bonus;
+                    }
+                }
+            }
+            constexpr int ROWS = HALF ? 2 : DENSE_BATCH;
+            while (CODES && need) {
+                std::conditional_t<HALF, DenseRowHalf, DenseRow> row[ROWS] = {}; // set on every path, as the sketches
+                RowLoad rl[ROWS] = {};
+                RowInfo ri[ROWS] = {};
+                uint32_t jj[ROWS];
+#pragma unroll
+                for (int b = 0; b < ROWS; b++) {
+                    jj[b] = EMPTY;
+                    if (need) {
+                        jj[b] = __builtin_ctzll(need);
+                        need &= need - 1;
+                        const uint64_t desc = readlane64(my_desc, jj[b]);
+                        if (by_codes) row_issue<NARROW>(rl[b], ri[b], a.C, desc, true, a.paths);
+                        if constexpr (HALF) dense_issue_half(row[b], a.half + (size_t)uniform(new_id[jj[b]]) * DIM);
+                        else dense_issue(row[b], a.C.recs + desc_off(desc) * 16);
+                    }
+                }
+#pragma unroll
+                for (int b = 0; b < ROWS; b++) {
+                    if (jj[b] != EMPTY) {
+                        float bonus = 0.f;
+                        if (KG) {
+                            if (new_ent[jj[b]] != EMPTY) bonus = a.kg_weight / (float)new_hop[jj[b]];
+                        }
+                        float ssum, dsum;
+                        if (by_codes) {
+                            bool hit = false; // known from the codes already
+                            ssum = wave_sum_dpp(row_probe<NARROW, KWD>(a.C, rl[b], ri[b], T, n_ovf, hit));
+                        } else ssum = new_dist[jj[b]];
+                        if constexpr (HALF) dsum = dense_finish_lds_half(row[b], qd, 1.0f);
+                        else dsum = dense_finish_lds(row[b], qd, 1.0f);
+                        if (lane == 0) new_dist[jj[b]] = 1.0f - (dsum + ssum) - bonus;
                     }
                 }
             }
@@ -992,6 +1069,7 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
         for (int o = WAVE / 2; o > 0; o >>= 1) {
             st_ns += __shfl_xor(st_ns, o, WAVE);
             st_nb += __shfl_xor(st_nb, o, WAVE);
+            if (CODES) ln_coded += __shfl_xor(ln_coded, o, WAVE);
         }
         if (lane == 0) { // summed in LDS over the workgroup's queries: seven atomics per query on one memory line would queue up
             if (st_exp) atomicAdd(stat + 1, (unsigned long long)st_exp);
@@ -1002,6 +1080,7 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
             if (st_again) atomicAdd(stat + 6, (unsigned long long)st_again);
             if (st_again_pairs) atomicAdd(stat + 7, (unsigned long long)st_again_pairs);
             if (st_sketch) atomicAdd(stat + 8, (unsigned long long)st_sketch);
+            if (CODES && ln_coded) atomicAdd(stat + 9, (unsigned long long)ln_coded);
         }
     }
     __syncthreads();
@@ -1041,18 +1120,21 @@ int search_static_workspace(int device, char** out) {
     return APOE_OK;
 }
 
-template <int NW, int MODE, bool NARROW, bool HALF = false>
+template <int NW, int MODE, bool NARROW, bool HALF = false, bool CODES = false>
 static int launch_format(apoe_ctx* ctx, const SearchArgs& a, uint32_t grid, size_t lds, int* per_cu) {
-    if constexpr (MODE == MODE_PLAIN && !HALF) {
+    if constexpr (MODE == MODE_PLAIN && !HALF && !CODES) {
         if (a.half) return launch_format<NW, MODE, NARROW, true>(ctx, a, grid, lds, per_cu);
     }
-    const void* fn = reinterpret_cast<const void*>(&search_kernel<NW, MODE, NARROW, HALF>);
+    if constexpr (NARROW && NW <= 2 && !CODES) {
+        if (a.coded) return launch_format<NW, MODE, NARROW, HALF, true>(ctx, a, grid, lds, per_cu);
+    }
+    const void* fn = reinterpret_cast<const void*>(&search_kernel<NW, MODE, NARROW, HALF, CODES>);
     APOE_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     if (per_cu) { // occupancy query only
         APOE_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, fn, NW * WAVE, lds));
         return APOE_OK;
     }
-    search_kernel<NW, MODE, NARROW, HALF><<<grid, NW * WAVE, lds, ctx->stream>>>(a);
+    search_kernel<NW, MODE, NARROW, HALF, CODES><<<grid, NW * WAVE, lds, ctx->stream>>>(a);
     APOE_HIP(hipGetLastError());
     return APOE_OK;
 }
@@ -1135,6 +1217,11 @@ int launch_search(apoe_ctx* ctx, const apoe_corpus* c, const apoe_queries* q, co
         APOE_REQUIRE(c->n < (1u << 30), "keyword-filter search keeps two flag bits on a document id: %u documents are too many", c->n);
         a.paths = PATH_DENSE | PATH_SPARSE | PATH_BM25; // query.cu:2005-2007: always the three-path loop
     }
+    // The codes pay where dense rows or sketches are read as well and memory bounds a long batch: 10 000 queries on 1 M docs with / without them,
+    // i.i.d. at cands 256 36.0 / 38.4 ms, with dense neighbours at cands 80 19.5 / 21.5, knowledge graph at cands 128 21.4 / 22.1. A search of pairs alone is bound by vector instructions,
+    // of which a coded row takes more (SPLADE alone, cands 256: 25.8 against 24.5 ms). The codes are kernels of their own: with both ways in one,
+    // the registers it spills cost the searches without codes 3 %.
+    a.coded = c->coded && !a.full_eval && (a.paths & PATH_DENSE) && (a.paths & (PATH_SPARSE | PATH_BM25)) ? 1u : 0u;
     if (use_kg) {
         APOE_REQUIRE(kg->n_queries >= p->q_begin + q_count, "knowledge graph holds entities for %u queries, %u needed", kg->n_queries, p->q_begin + q_count);
         a.e2e_off = kg->e2e_off.p;
@@ -1229,6 +1316,7 @@ int launch_search(apoe_ctx* ctx, const apoe_corpus* c, const apoe_queries* q, co
         // dense rows and sketches actually needed (a sketch with its scale and error) + pairs + descriptor and dense norm (12 B per evaluation)
         uint64_t bytes = h[5] * (uint64_t)(a.half ? DENSE_BYTES / 2 : DENSE_BYTES) + h[8] * (uint64_t)(SKETCH_BYTES + sizeof(SketchMeta));
         bytes += (c->narrow ? 6 : 8) * (h[3] + h[4]) + 12 * h[2];
+        bytes -= 3 * h[9]; // where codes settle an evaluation: a byte instead of the value
         bytes += h[6] * (uint64_t)(DENSE_BYTES + 8) + (c->narrow ? 6 : 8) * h[7]; // the pool evaluated again in fp32
         bytes += h[1] * 4ull * a.W;
         uint64_t qbytes = (uint64_t)q_count * DENSE_BYTES + 8 * (q->h_s_off[p->q_begin + q_count] - q->h_s_off[p->q_begin]) +

@@ -1,0 +1,58 @@
+"""The byte codes of a record's values only ever reject what the pairs themselves would reject: whole rows of results are bit for bit
+those of a walk without any bound (variant 0x100), on values where a wrong bound would show: magnitudes from denormal to 1e30, negative
+ones, values that are no numbers, rows without pairs, of one path and longer than a wave's loads, in each mode that asks the codes."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+N, D, NQ, VOCAB = 3000, 32, 40, 400
+
+
+def rows_of(rng, n, lengths, kind):
+    off = np.zeros(n + 1, np.uint32)
+    off[1:] = np.cumsum(rng.choice(lengths, n))
+    idx = np.concatenate([rng.choice(VOCAB, off[i + 1] - off[i], replace=False) for i in range(n)]).astype(np.uint32) * 163
+    val = rng.gamma(1.0, 1.0, len(idx)).astype(np.float32)
+    if kind == "magnitudes":
+        val *= (10.0 ** rng.choice([-44, -38, -30, -9, 0, 0, 0, 2, 8], len(val))).astype(np.float32)
+    elif kind == "negative":
+        val *= rng.choice([-1, 1, 1], len(val)).astype(np.float32)
+    elif kind == "not numbers":
+        val[::997] = np.inf
+        val[5::997] = np.nan
+    return off, idx, val
+
+
+def world(kind, seed):
+    rng = np.random.default_rng(seed)
+    dense = rng.standard_normal((N, 1024)).astype(np.float32) * np.float32(0.1)
+    q = rng.standard_normal((NQ, 1024)).astype(np.float32) * np.float32(0.1)
+    corpus = (dense, *rows_of(rng, N, [0, 1, 63, 64, 65, 130, 250], kind), *rows_of(rng, N, [0, 1, 31, 64, 129], kind))
+    queries = (q, *rows_of(rng, NQ, [1, 20, 60], "negative" if kind == "negative" else "plain"), *rows_of(rng, NQ, [1, 20, 60], "plain"))
+    rows = np.zeros((N, D + 8), np.uint32)
+    rows[:, :D] = rng.integers(0, N, (N, D))
+    return corpus, queries, rows, rng.choice(N, D, replace=False).astype(np.uint32)
+
+
+@pytest.mark.parametrize("kind", ["plain", "magnitudes", "negative", "not numbers"])
+def test_rows_are_those_of_a_walk_without_bounds(gpu_ctx, kind):
+    import apoe
+    import apoe_synth as S
+    corpus, queries, rows, entry = world(kind, 3)
+    b_idx = queries[5].copy()
+    b_idx[queries[4][:-1]] |= np.uint32(0x80000000)  # the first BM25 term of every query is required
+    gc, gq, gg = apoe.Corpus(gpu_ctx, *corpus), apoe.Queries(gpu_ctx, *queries), apoe.Graph(gpu_ctx, rows, entry)
+    gk = apoe.Queries(gpu_ctx, *queries[:5], b_idx, queries[6])
+    kg = apoe.KnowledgeGraph(gpu_ctx, *S.to_numpy(S.knowledge_graph(800, N, NQ, seed=23, device="cpu", mean_out=6.0)))
+    gc.make_half_rows()
+    for w3, cands, shape in (((0.01, 1, 1), 24, 4), ((1, 1, 1), 24, 4), ((49, 1, 1), 64, 1), ((1, 3, 0), 33, 1), ((0.5, 0, 2), 100, 4)):
+        for query, more in ((gq, {}), (gk, dict(keyword_filter=True)), (gq, dict(kg=kg, kg_weight=5.0))):
+            a, ad, sa = apoe.search(gpu_ctx, gc, query, gg, w3, cands, variant=shape, **more)
+            b, bd, sb = apoe.search(gpu_ctx, gc, query, gg, w3, cands, variant=shape | 0x100, **more)
+            assert np.array_equal(a, b) and np.array_equal(ad, bd, equal_nan=True), (w3, cands, sorted(more))
+            assert sa.evaluations == sb.evaluations and sa.dense_rows <= sb.dense_rows
+            if kind == "plain" and w3 == (0.01, 1, 1):  # codes are in use (and no sketches, the dense parts are small): values of settled pairs are not read
+                assert sa.algo_bytes + 4096 * (sb.dense_rows - sa.dense_rows) < sb.algo_bytes
+        a, ad, _ = apoe.search(gpu_ctx, gc, gq, gg, w3, cands, variant=shape | 0x200)
+        b, bd, _ = apoe.search(gpu_ctx, gc, gq, gg, w3, cands, variant=shape | 0x300)
+        assert np.array_equal(a, b) and np.array_equal(ad, bd, equal_nan=True), (w3, cands, "half")
