@@ -580,8 +580,8 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
             // of the batch exists: one that does not is a row of no pairs, so the loads of the whole batch are issued back to back.
             // With codes, an upper bound of the sparse part from the terms and a byte a value instead (3 bytes a pair, not 6, CODE_BATCH rows in
             // flight); decision and sketches go by that bound, and the pairs of the few candidates that stay open come with their dense rows.
-            // 10 000 queries on 1 M docs: i.i.d. at cands 256 38.4 -> 36.0 ms (the vector units are busy for 0.66 of the cycles now, 0.44 before: a coded
-            // row takes more instructions), with dense neighbours at cands 80 21.5 -> 19.5; three or four rows in flight measure the same, and so do
+            // 10 000 queries on 1 M docs with dense neighbours at cands 80: 21.5 -> 19.5 ms (a coded row takes more vector instructions, 119 against 84 an
+            // evaluation on i.i.d. rows, which then bound the batch); three or four rows in flight measure the same, and so do
             // pairs and rows of two open candidates together. Short batches, four and more waves a query, are bound by the chain of one query,
             // which a second read of the open candidates' pairs would lengthen: they read the pairs at once.
             auto eval_rows = [&](auto nb, auto at) { // at(b): the b-th candidate, n_new or more: there is none
@@ -1217,11 +1217,12 @@ int launch_search(apoe_ctx* ctx, const apoe_corpus* c, const apoe_queries* q, co
         APOE_REQUIRE(c->n < (1u << 30), "keyword-filter search keeps two flag bits on a document id: %u documents are too many", c->n);
         a.paths = PATH_DENSE | PATH_SPARSE | PATH_BM25; // query.cu:2005-2007: always the three-path loop
     }
-    // The codes pay where dense rows or sketches are read as well and memory bounds a long batch: 10 000 queries on 1 M docs with / without them,
-    // i.i.d. at cands 256 36.0 / 38.4 ms, with dense neighbours at cands 80 19.5 / 21.5, knowledge graph at cands 128 21.4 / 22.1. A search of pairs alone is bound by vector instructions,
-    // of which a coded row takes more (SPLADE alone, cands 256: 25.8 against 24.5 ms). The codes are kernels of their own: with both ways in one,
-    // the registers it spills cost the searches without codes 3 %.
-    a.coded = c->coded && !a.full_eval && (a.paths & PATH_DENSE) && (a.paths & (PATH_SPARSE | PATH_BM25)) ? 1u : 0u;
+    // The codes pay where the dense part decides, so that pairs settle little and memory bounds a long batch: 10 000 queries on 1 M docs with / without them,
+    // dense neighbours under (49, 1, 1) at cands 80 19.5 / 21.5 ms, i.i.d. under (1729, 6.28, 1) at cands 256 45.7 / 49.3. Under (1, 1, 1) it is the graph
+    // that tells (i.i.d. at cands 256: lists of near rows 36.0 / 38.4, a built index, whose hubs stay in the cache, 30.7 / 29.9, at cands 64 10.9 / 10.0),
+    // and pairs alone are bound by vector instructions, of which a coded row takes more (SPLADE, cands 256: 25.8 / 24.5). The line lies between the
+    // measured ratios of 1 and 49. The codes are kernels of their own: with both ways in one, spilled registers cost searches without codes 3 %.
+    a.coded = c->coded && !a.full_eval && p->w_dense >= 8.f * fmaxf(p->w_sparse, p->w_bm25) && (a.paths & PATH_DENSE) && (a.paths & (PATH_SPARSE | PATH_BM25)) ? 1u : 0u;
     if (use_kg) {
         APOE_REQUIRE(kg->n_queries >= p->q_begin + q_count, "knowledge graph holds entities for %u queries, %u needed", kg->n_queries, p->q_begin + q_count);
         a.e2e_off = kg->e2e_off.p;
