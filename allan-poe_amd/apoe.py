@@ -41,7 +41,7 @@ EXPORTS = [
     "apoe_kg_create", "apoe_kg_destroy", "apoe_calibrate_weights", "apoe_hybrid_distance_batch", "apoe_hybrid_distance_pairs", "apoe_norms",
     "apoe_knn_create", "apoe_knn_destroy", "apoe_knn_use_half_rows", "apoe_knn_set_join", "apoe_nnd_init", "apoe_nnd_iterate", "apoe_nnd_merge_reverse",
     "apoe_knn_download", "apoe_knn_upload", "apoe_knn_download_reverse", "apoe_knn_upload_reverse", "apoe_knn_set_prune_form", "apoe_prune", "apoe_prune_download", "apoe_finalize_graph",
-    "apoe_knn_elapsed_ms", "apoe_knn_counters", "apoe_graph_create", "apoe_graph_destroy", "apoe_graph_info", "apoe_graph_download",
+    "apoe_knn_elapsed_ms", "apoe_knn_counters", "apoe_knn_read_counters", "apoe_graph_create", "apoe_graph_destroy", "apoe_graph_info", "apoe_graph_download",
     "apoe_search", "apoe_search_noalloc",
 ]
 
@@ -310,6 +310,12 @@ class Knn:
         out = (C.c_uint64 * 2)()
         _check(lib().apoe_knn_counters(self.h, out))
         return int(out[0]), int(out[1])
+
+    def read_counters(self):
+        """(dense rows, rows of pairs, sketches) that the NN-Descent steps since init read."""
+        out = (C.c_uint64 * 3)()
+        _check(lib().apoe_knn_read_counters(self.h, out))
+        return int(out[0]), int(out[1]), int(out[2])
 
     def close(self):
         if self.h:

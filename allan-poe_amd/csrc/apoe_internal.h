@@ -149,6 +149,9 @@ struct apoe_graph {
     apoe::DevBuf<uint32_t> rows, entry;
 };
 
+// Counts of a K-NN handle: the entries that the last step inserted, a flag of the calls that check something, and sums since apoe_nnd_init.
+enum { KC_INSERTED = 0, KC_FLAG = 1, KC_EVALUATIONS = 2, KC_DENSE_ROWS = 3, KC_JOIN_EVALUATIONS = 4, KC_JOIN_PAIR_ROWS = 5, KC_SKETCHES = 6, KC_WORDS = 8 };
+
 struct apoe_knn {
     apoe_ctx* ctx = nullptr;
     const apoe_corpus* corpus = nullptr;
@@ -162,7 +165,7 @@ struct apoe_knn {
     apoe::DevBuf<uint32_t> ids, rev_cnt;
     apoe::DevBuf<unsigned long long> rev; // [n][K] reverse lists: (distance key << 32 | id) per slot
     apoe::DevBuf<float> dist, norms;
-    apoe::DevBuf<unsigned long long> counter;
+    apoe::DevBuf<unsigned long long> counter; // KC_ words
     // local-join step (apoe_knn_set_join): the picks of a step grouped by the picked node, the tiles, the proposal rows
     int join = 0; // 0: expansion step, 1: local join, 2: local join that offers a pair to both endpoints
     bool join_symmetric = false;

@@ -134,7 +134,7 @@ struct JoinArgs {
     const unsigned long long* rev;
     const uint32_t *pick_off, *pick_src, *tile_off, *tile_v;
     unsigned long long* prop;
-    unsigned long long* work; // [0] next tile, [1] pairs evaluated, [2] rows gathered, [3] a row did not fit the table
+    unsigned long long* work; // [0] next tile, [1] pairs evaluated, [2] dense rows read, [3] a row did not fit the table, [5] rows whose pairs were read
     uint32_t index_bits, slot_cap, span;
     const SketchMeta* sketch_meta;
     const uint4* sketch; // null: every dense row is read
@@ -514,14 +514,14 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
     uint8_t* seen_col = reinterpret_cast<uint8_t*>(smem + L.seen_col); // ... and their numbers; NO_COL: not a column of this tile
     constexpr uint8_t NO_COL = 0xFF;
     uint32_t* scan = reinterpret_cast<uint32_t*>(smem + L.scan);
-    uint32_t* ctl = reinterpret_cast<uint32_t*>(smem + L.ctl); // [0] tile, [1] columns, [4] columns whose dense rows are read
+    uint32_t* ctl = reinterpret_cast<uint32_t*>(smem + L.ctl); // [0] tile, [1] columns, [4] columns whose dense rows are read; [2], [3], [5] counts (below)
     TileSketch* S = reinterpret_cast<TileSketch*>(seen); // once the rows' lists are looked up
     static_assert(sizeof(TileSketch) <= JT_SEEN * 4, "the id set's bytes hold what the sketches tell");
 
     const int wave = (int)uniform(threadIdx.x / WAVE);
     const uint32_t n_tiles = a.tile_off[a.n];
 
-    if (threadIdx.x == 0) { ctl[2] = 0; ctl[3] = 0; } // pairs and rows of this workgroup's tiles
+    if (threadIdx.x == 0) { ctl[2] = 0; ctl[3] = 0; ctl[5] = 0; } // pairs evaluated, dense rows and rows of pairs read by this workgroup's tiles
     while (true) {
         // opaque to the compiler: what follows from a thread's number is worked out where a tile needs it, not once for all tiles and spilled
         int tid = threadIdx.x;
@@ -650,13 +650,15 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
         }
         if (tid == 0) { // summed here, sent once when the workgroup leaves: a million atomics on one address per step would queue up
             ctl[2] += R * M;
-            ctl[3] += R + M;
+            ctl[3] += Mc ? R + Mc : 0;
+            ctl[5] += R + M;
             if (ctl[2] >= 0x40000000u) { atomicAdd(a.work + 1, (unsigned long long)ctl[2]); ctl[2] = 0; }
         }
     }
     if (threadIdx.x == 0) {
         atomicAdd(a.work + 1, (unsigned long long)ctl[2]);
         atomicAdd(a.work + 2, (unsigned long long)ctl[3]);
+        atomicAdd(a.work + 5, (unsigned long long)ctl[5]);
     }
 }
 
@@ -769,13 +771,17 @@ __global__ __launch_bounds__(256) void join_apply_kernel(uint32_t n, uint32_t* i
     }
 }
 
-// work[4] = entries that entered a list in this step, beside the pairs for the host.
-__global__ static void join_account_kernel(unsigned long long* work, unsigned long long* counter) {
-    counter[2] += work[1]; // pairs evaluated
-    counter[3] += work[2]; // rows gathered (each read in full, dense part included)
+// work[4] = entries that entered a list in this step, beside the pairs for the host. settled: the step asked the sketches, one for every
+// row and column of a tile.
+__global__ static void join_account_kernel(unsigned long long* work, unsigned long long* counter, uint32_t settled) {
+    counter[KC_EVALUATIONS] += work[1];
+    counter[KC_DENSE_ROWS] += work[2];
+    counter[KC_JOIN_EVALUATIONS] += work[1];
+    counter[KC_JOIN_PAIR_ROWS] += work[5];
+    if (settled) counter[KC_SKETCHES] += work[5];
     unsigned long long inserted = 0; // the partial counts of join_apply_kernel
     for (int p = 0; p < JOIN_COUNT_PARTS; p++) inserted += work[JOIN_COUNT_AT + p * 8];
-    counter[0] = inserted;
+    counter[KC_INSERTED] = inserted;
     work[4] = inserted;
 }
 
@@ -935,7 +941,7 @@ int launch_nnd_join_iterate(apoe_knn* g) {
     const TileShape shape = tile_shape(ctx, g->corpus);
     APOE_REQUIRE(shape.lds <= ctx->lds_per_block, "the local-join tile needs %u bytes of LDS, a workgroup may have %zu", shape.lds, ctx->lds_per_block);
 
-    APOE_HIP(hipMemsetAsync(g->counter.p, 0, sizeof(unsigned long long), st)); // [0] inserted; [2], [3] accumulate over the build
+    APOE_HIP(hipMemsetAsync(g->counter.p, 0, sizeof(unsigned long long), st)); // the inserted entries; the counts behind them run over the build
     fill_u32_kernel2<<<1024, 256, 0, st>>>(g->pick_cnt.p, (uint64_t)n + 1, 0u);
     fill_u32_kernel2<<<1024, 256, 0, st>>>(g->pick_fill.p, (uint64_t)n + 1, 0u);
     fill_u64_kernel<<<8, 256, 0, st>>>(g->join_work.p, JOIN_COUNT_AT + JOIN_COUNT_PARTS * 8, 0ull);
@@ -983,7 +989,7 @@ int launch_nnd_join_iterate(apoe_knn* g) {
     if (k128) join_apply_kernel<128><<<(n + 3) / 4, 256, 0, st>>>(n, g->ids.p, g->dist.p, g->prop.p, g->rev.p, g->rev_cnt.p, g->join_work.p + JOIN_COUNT_AT);
     else join_apply_kernel<64><<<(n + 3) / 4, 256, 0, st>>>(n, g->ids.p, g->dist.p, g->prop.p, g->rev.p, g->rev_cnt.p, g->join_work.p + JOIN_COUNT_AT);
     APOE_HIP(hipGetLastError());
-    join_account_kernel<<<1, 1, 0, st>>>(g->join_work.p, g->counter.p);
+    join_account_kernel<<<1, 1, 0, st>>>(g->join_work.p, g->counter.p, a.sketch != nullptr);
     APOE_HIP(hipGetLastError());
     return APOE_OK;
 }

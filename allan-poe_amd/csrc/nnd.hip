@@ -367,7 +367,7 @@ static uint32_t doc_term_slots(const apoe_corpus* c) { return next_pow2(std::max
 
 int launch_nnd_init(apoe_knn* g, uint64_t seed) {
     apoe_ctx* ctx = g->ctx;
-    APOE_HIP(hipMemsetAsync(g->counter.p, 0, 4 * sizeof(unsigned long long), ctx->stream));
+    APOE_HIP(hipMemsetAsync(g->counter.p, 0, KC_WORDS * sizeof(unsigned long long), ctx->stream));
     const uint64_t total = (uint64_t)g->n * g->K;
     const uint32_t grid = (uint32_t)std::min<uint64_t>((total + 255) / 256, 1u << 20);
     nnd_init_kernel<<<grid, 256, 0, ctx->stream>>>(g->n, g->K, seed, g->ids.p, g->dist.p, g->rev.p, g->rev_cnt.p);
@@ -393,7 +393,7 @@ int launch_nnd_iterate(apoe_knn* g, uint64_t* inserted) {
     const NndLds L(term_slots, seen_slots, g->K);
     APOE_REQUIRE(L.total <= 64 * 1024, "NN-Descent needs %u bytes of LDS (rows with up to %u sparse terms)", L.total,
                  g->corpus->max_nnz_s + g->corpus->max_nnz_b);
-    APOE_HIP(hipMemsetAsync(g->counter.p, 0, sizeof(unsigned long long), ctx->stream)); // [0] inserted; [2], [3] accumulate over the build
+    APOE_HIP(hipMemsetAsync(g->counter.p, 0, sizeof(unsigned long long), ctx->stream)); // the inserted entries; the counts behind them run over the build
     auto kernel = g->half_rows ? (g->corpus->narrow ? &nnd_iterate_kernel<true, true> : &nnd_iterate_kernel<false, true>)
                                : (g->corpus->narrow ? &nnd_iterate_kernel<true, false> : &nnd_iterate_kernel<false, false>);
     APOE_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)L.total));
@@ -496,7 +496,7 @@ int apoe_knn_create(apoe_ctx* ctx, const apoe_corpus* c, uint32_t K, float dense
     APOE_TRY(g->rev.alloc(total));
     APOE_TRY(g->rev_cnt.alloc(c->n));
     APOE_TRY(g->norms.alloc(c->n));
-    APOE_TRY(g->counter.alloc(4));
+    APOE_TRY(g->counter.alloc(KC_WORDS));
     *out = g.release();
     return APOE_OK;
 }
@@ -713,14 +713,29 @@ int apoe_knn_upload_reverse(apoe_knn* g, const uint32_t* rev_ids, const float* r
 
 float apoe_knn_elapsed_ms(const apoe_knn* g) { return g ? g->elapsed_ms : 0.f; }
 
+static int read_counts(apoe_knn* g, unsigned long long* h) {
+    APOE_HIP(hipSetDevice(g->ctx->device));
+    APOE_HIP(hipStreamSynchronize(g->ctx->stream));
+    APOE_HIP(hipMemcpy(h, g->counter.p, KC_WORDS * sizeof(*h), hipMemcpyDeviceToHost));
+    return APOE_OK;
+}
+
 int apoe_knn_counters(apoe_knn* g, uint64_t* out2) {
     APOE_REQUIRE(g && out2, "null argument");
-    APOE_HIP(hipSetDevice(g->ctx->device));
-    unsigned long long h[4] = {0, 0, 0, 0};
-    APOE_HIP(hipStreamSynchronize(g->ctx->stream));
-    APOE_HIP(hipMemcpy(h, g->counter.p, sizeof(h), hipMemcpyDeviceToHost));
-    out2[0] = h[2];
-    out2[1] = h[3];
+    unsigned long long h[KC_WORDS] = {};
+    APOE_TRY(read_counts(g, h));
+    out2[0] = h[KC_EVALUATIONS];
+    out2[1] = h[KC_DENSE_ROWS];
+    return APOE_OK;
+}
+
+int apoe_knn_read_counters(apoe_knn* g, uint64_t* out3) {
+    APOE_REQUIRE(g && out3, "null argument");
+    unsigned long long h[KC_WORDS] = {};
+    APOE_TRY(read_counts(g, h));
+    out3[0] = h[KC_DENSE_ROWS];
+    out3[1] = h[KC_EVALUATIONS] - h[KC_JOIN_EVALUATIONS] + h[KC_JOIN_PAIR_ROWS]; // an expansion step reads the pairs of every evaluation
+    out3[2] = h[KC_SKETCHES];
     return APOE_OK;
 }
 

@@ -58,13 +58,14 @@ def build_index(apoe, ctx, gc, args, join, keep_lists=False):
         knn.iterate(last=(it == args.nnd_iters - 1))
     nnd_ms = knn.elapsed_ms()
     evals, rows = knn.counters()
+    _, pair_rows, sketches = knn.read_counters()
     knn.merge_reverse()
     lists = knn.download()[0] if keep_lists else None
     knn.prune(args.degree)
     graph = knn.finalize()
     total_ms = knn.elapsed_ms()
     knn.close()
-    return graph, dict(nnd_ms=nnd_ms, total_ms=total_ms, wall_s=time.time() - t0, evaluations=evals, rows_read=rows), lists
+    return graph, dict(nnd_ms=nnd_ms, total_ms=total_ms, wall_s=time.time() - t0, evaluations=evals, rows_read=rows, pair_rows=pair_rows, sketches=sketches), lists
 
 
 def main():
@@ -130,21 +131,17 @@ def main():
 
     # ---- index build (NN-Descent + reverse merge + RNG-IP prune + final rows), with both NN-Descent steps ----
     mean_pairs = (corpus[2].numel() + corpus[5].numel()) / args.docs
-    row_bytes = 4096 + gc.pair_bytes() * mean_pairs + 12
     builds = {}
     graph = None
     lists = None
     for join in sorted({0, args.join}):
         g, tm, ls = build_index(apoe, ctx, gc, args, join, keep_lists=True)
-        if join == 0:
-            # expansion step: an evaluation reads pairs + descriptor, and the dense row when the bound does not settle it
-            tm["algo_bytes"] = tm["rows_read"] * 4096 + tm["evaluations"] * (gc.pair_bytes() * mean_pairs + 12)
-        else:
-            # join: every row of a tile is read once, in full
-            tm["algo_bytes"] = tm["rows_read"] * row_bytes
+        # dense rows + rows of pairs with their descriptors and norms (expansion step: one an evaluation, join: one per row and column of a
+        # tile) + sketches of the join steps that asked them
+        tm["algo_bytes"] = tm["rows_read"] * 4096 + tm["pair_rows"] * (gc.pair_bytes() * mean_pairs + 12) + tm["sketches"] * 1032
         builds[join] = tm
         log(f"[bench] build (NN-Descent step {join}): {tm['total_ms'] / 1e3:.2f}s GPU time ({tm['wall_s']:.2f}s wall); NN-Descent {tm['nnd_ms'] / 1e3:.2f}s, "
-            f"{tm['evaluations'] / 1e9:.2f}G pair evaluations, {tm['rows_read'] / 1e9:.3f}G rows read, {tm['algo_bytes'] / (tm['nnd_ms'] / 1e3) / 1e12:.2f} TB/s algorithmic")
+            f"{tm['evaluations'] / 1e9:.2f}G pair evaluations, {tm['rows_read'] / 1e9:.3f}G dense rows read, {tm['algo_bytes'] / (tm['nnd_ms'] / 1e3) / 1e12:.2f} TB/s algorithmic")
         if join == args.join:
             graph, lists = g, ls
         else:

@@ -186,9 +186,12 @@ int apoe_finalize_graph(apoe_knn* g, apoe_graph** out);
  * calls on this handle so far: the reference's "Indexing time" region (index.cu:889-908). */
 float apoe_knn_elapsed_ms(const apoe_knn* g);
 /* out2 = {hybrid distance evaluations, dense rows read} of the NN-Descent steps since apoe_nnd_init
- * (a candidate whose sparse part plus the bound of its dense part cannot enter the list is not
- * read in full). No counterpart in the reference; used to price the build against the HBM roofline. */
+ * (an expansion step does not read the dense row of a candidate whose sparse part plus the bound of its dense part cannot
+ * enter the list; a join step reads a row once per tile, and once the lists have settled not those of columns that the sketches
+ * rule out). No counterpart in the reference; used to price the build against the HBM roofline. */
 int apoe_knn_counters(apoe_knn* g, uint64_t* out2);
+/* out3 = {dense rows, rows whose (term, value) pairs, 8-bit sketches (1 032 bytes each)} that those steps read. */
+int apoe_knn_read_counters(apoe_knn* g, uint64_t* out3);
 
 /* ---- graph handle: the .poe payload (index.cu:927-939, query.cu:35-62) ---- */
 int apoe_graph_create(apoe_ctx* ctx, uint32_t n, uint32_t width, const uint32_t* rows,
