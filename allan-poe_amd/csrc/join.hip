@@ -794,7 +794,7 @@ __global__ __launch_bounds__(256) static void fill_u32_kernel2(uint32_t* p, uint
 
 // ---- hybrid Gram matrices of whole neighbour lists, tile by tile (the prune of lists longer than 64 entries) ----
 //
-// For node u = node0 + q (or the list's entry there) the valid entries of its list (distance below INF_DIS, a document, not u itself),
+// For node u = nodes[node0 + q] the valid entries of its list (distance below INF_DIS, a document, not u itself),
 // in list order, are the rows and columns of a Gram matrix of at most 128 x 128. Tile t computes rows
 // [32 t, 32 t + 32) against the columns [32 t, m): the upper triangle, diagonal blocks whole. The products go to
 // gram[q * 128 * 128 + i * 128 + j] for i <= j (entries below the diagonal of a diagonal block are
@@ -805,7 +805,7 @@ struct GramTileArgs {
     CorpusView C;
     float dense_mul;
     uint32_t K, node0, n_nodes;
-    const uint32_t* nodes; // not null: node q of the batch is nodes[node0 + q]
+    const uint32_t* nodes; // node q of the batch is nodes[node0 + q]
     const uint32_t* ids;
     const float* dist;
     float* gram;
@@ -839,7 +839,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
         __syncthreads();
         const uint32_t slot = uniform(ctl[0]);
         if (slot >= a.n_nodes) break;
-        const uint32_t u = a.nodes ? uniform(a.nodes[a.node0 + slot]) : a.node0 + slot;
+        const uint32_t u = uniform(a.nodes[a.node0 + slot]);
         if (wave == 0) {
             const size_t base = (size_t)u * a.K;
             uint32_t m = 0;
@@ -994,7 +994,7 @@ int launch_nnd_join_iterate(apoe_knn* g) {
     return APOE_OK;
 }
 
-// Gram matrices (upper triangles) of the lists of nodes [node0, node0 + n_nodes) (or of those entries of the list `nodes`) into gram[n_nodes][128][128]. *unfit = rows
+// Gram matrices (upper triangles) of the lists of nodes[node0 .. node0 + n_nodes) into gram[n_nodes][128][128]. *unfit = rows
 // whose sparse terms did not fit the tile's table (their products lack the sparse part: the caller must not use the result).
 int launch_gram_tiles(apoe_knn* g, const uint32_t* nodes, uint32_t node0, uint32_t n_nodes, float* gram, unsigned long long* unfit) {
     apoe_ctx* ctx = g->ctx;

@@ -46,9 +46,13 @@ struct PruneLds {
     }
 };
 
-enum { PC_M = 0, PC_NSEL = 1, PC_REJECT = 2, PC_ALLFLAG = 3, PC_CNT = 4, PC_FAIL = 5, PC_OPEN = 6, PC_STILL_OPEN = 7 };
+enum { PC_M = 0, PC_NSEL = 1, PC_REJECT = 2, PC_ALLFLAG = 3, PC_CNT = 4, PC_FAIL = 5, PC_OPEN = 6, PC_STILL_OPEN = 7, PC_TABLE = 8 };
 
-// allan_poe (index.cu:539-714) for node u = blockIdx.x:
+// What a node leaves to another form of the prune: a pair that bounds do not settle, or a neighbour whose norm is not finite. The gathered forms
+// multiply a value by zero where a row lacks its term, which an infinite one does not survive; the table-probing kernel multiplies hits only.
+enum { NODE_SETTLED = 0, NODE_OPEN = 1, NODE_TABLE = 2 };
+
+// allan_poe (index.cu:539-714) for node u = blockIdx.x (nodes: the list's entry there):
 //  (a) detour counts over u's sorted list; (b) order by (detour, rank);
 //  (c) sequential RNG-IP selection: candidate c is the pivot, each live selected s is
 //      evaluated against it by one wave; norm[c] < <c,s> rejects c, norm[s] < <c,s>
@@ -57,8 +61,8 @@ enum { PC_M = 0, PC_NSEL = 1, PC_REJECT = 2, PC_ALLFLAG = 3, PC_CNT = 4, PC_FAIL
 //      forward row, flagged live ones beyond become keyword-edge candidates.
 __global__ __launch_bounds__(PR_THREADS) void prune_kernel(CorpusView C, float dense_mul, const float* __restrict__ norms, uint32_t K,
                                                            const uint32_t* __restrict__ ids, const float* __restrict__ dist, uint32_t d,
-                                                           uint32_t* fwd, uint32_t* det_out, uint32_t* cnt_out, uint32_t* kw_out,
-                                                           uint32_t term_slots, uint32_t uset_slots, uint32_t map_slots) {
+                                                           const uint32_t* __restrict__ nodes, uint32_t* fwd, uint32_t* det_out, uint32_t* cnt_out,
+                                                           uint32_t* kw_out, uint32_t term_slots, uint32_t uset_slots, uint32_t map_slots) {
     extern __shared__ __align__(16) char smem[];
     const PruneLds L(term_slots, uset_slots, map_slots, K);
     uint2* tab = reinterpret_cast<uint2*>(smem + L.tab);
@@ -79,7 +83,7 @@ __global__ __launch_bounds__(PR_THREADS) void prune_kernel(CorpusView C, float d
     volatile uint32_t* ctl = reinterpret_cast<volatile uint32_t*>(smem + L.ctl);
 
     const int tid = threadIdx.x, wave = tid / WAVE, lane = lane_id();
-    const uint32_t u = blockIdx.x, tmask = term_slots - 1, umask = uset_slots - 1, mmask = map_slots - 1;
+    const uint32_t u = nodes ? nodes[blockIdx.x] : blockIdx.x, tmask = term_slots - 1, umask = uset_slots - 1, mmask = map_slots - 1;
     const size_t base = (size_t)u * K;
     const uint64_t lane_lt = (1ull << lane) - 1;
 
@@ -278,7 +282,8 @@ __device__ __forceinline__ void lds_map_find(const uint2* map, uint32_t mask, co
 // The selection (below) asks of two neighbours c and s of a node only whether <c, s> exceeds either one's norm. |<c, s>_dense - the
 // product of the sketches| has a bound (apoe_device.h), |<c, s>_sparse| is at most the product of the two sparse norms; on a corpus
 // whose dense rows have neighbours that answers all pairs of most nodes (100 000 docs, dense_mul 49: 86 of 100), and neither a dense row nor a
-// pair of terms but the keys of the BM25 terms is read. A node with an open pair sets open[u] and leaves nothing else.
+// pair of terms but the keys of the BM25 terms is read. A node with an open pair sets open[u] = NODE_OPEN, one with a norm that is not finite NODE_TABLE, and
+// leaves nothing else.
 // Small in LDS and registers, so that many nodes share a CU: it is a chain of short phases (five nodes of 64 rows a CU;
 // 100 000 docs 3.8 ms, with the 14 000 open nodes behind it 6.0 ms, where Gram matrices and selection took 25.4; 30 011 docs K = 128 28.9 -> 10.4 ms).
 template <uint32_t K>
@@ -403,6 +408,7 @@ __global__ __launch_bounds__(K * 4) __attribute__((amdgpu_waves_per_eu(4, 8))) v
             const float nv = norms[v], dn = C.dnorm[v];
             const SketchMeta sm = sketch_meta[v];
             nrm[tid] = nv;
+            if (!(nv < __builtin_inff())) ctl[PC_OPEN] = ctl[PC_TABLE] = 1;
             // what the hybrid norm leaves to the sparse part, with room for the rounding of both norms
             row[tid] = make_float4(dn, sm.scale, sm.err, sqrtf(fmaxf(nv - dense_mul * dn * dn, 0.f) + 1e-5f * (nv + dense_mul * dn * dn)));
             rowptr[tid] = desc_off(desc) * 16 + DENSE_BYTES;
@@ -432,7 +438,7 @@ __global__ __launch_bounds__(K * 4) __attribute__((amdgpu_waves_per_eu(4, 8))) v
         }
         __syncthreads();
         if (uniform(ctl[PC_OPEN])) {
-            if (tid == 0) open[u] = 1;
+            if (tid == 0) open[u] = ctl[PC_TABLE] ? NODE_TABLE : NODE_OPEN;
             return;
         }
 #pragma unroll 1
@@ -488,7 +494,7 @@ __global__ __launch_bounds__(K * 4) __attribute__((amdgpu_waves_per_eu(4, 8))) v
     if (undecided) ctl[PC_OPEN] = 1;
     __syncthreads();
     if (uniform(ctl[PC_OPEN])) {
-        if (tid == 0) open[u] = 1;
+        if (tid == 0) open[u] = NODE_OPEN;
         return;
     }
     // the staged sketches make room
@@ -732,7 +738,7 @@ struct SelectLds {
     }
 };
 
-// allan_poe (index.cu:539-714) for node u = node0 + blockIdx.x (nodes: the list's entry there), as prune_kernel, with every inner product <c, s> read from the
+// allan_poe (index.cu:539-714) for node u = nodes[node0 + blockIdx.x], as prune_kernel, with every inner product <c, s> read from the
 // node's Gram matrix gram[blockIdx.x][i][j] (i <= j: positions in the list of valid entries) instead of being evaluated:
 // detour counts and the (detour, rank) order as there; the keyword flag of a pair from bit masks R[i] = the BM25 terms of u
 // that row i holds (flag(c, s) = R[s] has a bit that R[c] lacks); the sequential selection by wave 0 alone, two selected
@@ -762,7 +768,7 @@ __global__ __launch_bounds__(PS_THREADS) void prune_select_kernel(CorpusView C, 
 
     const int tid = threadIdx.x, wave = tid / WAVE, lane = lane_id();
     constexpr uint32_t NWV = PS_THREADS / WAVE;
-    const uint32_t u = nodes ? nodes[node0 + blockIdx.x] : node0 + blockIdx.x, umask = umap_slots - 1, mmask = map_slots - 1;
+    const uint32_t u = nodes[node0 + blockIdx.x], umask = umap_slots - 1, mmask = map_slots - 1;
     const size_t base = (size_t)u * K;
     const uint64_t lane_lt = (1ull << lane) - 1;
     const float* gu = gram + (size_t)blockIdx.x * PS_MAX * PS_MAX;
@@ -1428,7 +1434,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
     uint32_t* ctl = reinterpret_cast<uint32_t*>(smem + L.ctl);
 
     const int tid = threadIdx.x, wave = (int)uniform(tid / WAVE), lane = lane_id();
-    const uint32_t u = nodes ? nodes[blockIdx.x] : blockIdx.x, umask = umap_slots - 1, mmask = map_slots - 1;
+    const uint32_t u = nodes[blockIdx.x], umask = umap_slots - 1, mmask = map_slots - 1;
     const size_t base = (size_t)u * K;
     const uint64_t lane_lt = (1ull << lane) - 1;
 
@@ -1849,40 +1855,66 @@ __global__ __launch_bounds__(256) void final_rows_kernel(uint32_t n, uint32_t d,
 
 static uint32_t doc_term_slots(const apoe_corpus* c) { return next_pow2(std::max(64u, 2 * (c->max_nnz_s + c->max_nnz_b))); }
 
-// The nodes whose flag is set, in no order: one atomic per wave (one per node on a single counter is 19 ns each, one after the other).
-__global__ __launch_bounds__(256) void open_nodes_kernel(uint32_t n, const uint32_t* __restrict__ flag, uint32_t* count, uint32_t* nodes) {
-    const uint32_t u = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint64_t b = __ballot(u < n && flag[u] != 0);
-    if (b == 0) return;
-    uint32_t at = 0;
-    if (lane_id() == 0) at = atomicAdd(count, (uint32_t)__popcll(b));
-    at = uniform(at) + __popcll(b & ((1ull << lane_id()) - 1));
-    if ((b >> lane_id()) & 1) nodes[at] = u;
+// Where no bounds can be asked (a corpus without sketches): every node is open, but for those that the table-probing kernel takes. One wave per node.
+__global__ __launch_bounds__(256) void prune_triage_kernel(uint32_t n, uint32_t K, const uint32_t* __restrict__ ids, const float* __restrict__ dist,
+                                                           const float* __restrict__ norms, uint32_t* open) {
+    const uint32_t u = blockIdx.x * (256 / WAVE) + threadIdx.x / WAVE, lane = lane_id();
+    if (u >= n) return;
+    bool far = false;
+    for (uint32_t i = lane; i < K; i += WAVE) {
+        const uint32_t v = ids[(size_t)u * K + i] & ~FLAG;
+        if (dist[(size_t)u * K + i] < INF_DIS && v < n && v != u) far |= !(norms[v] < __builtin_inff());
+    }
+    const bool table = __ballot(far) != 0;
+    if (lane == 0) open[u] = table ? NODE_TABLE : NODE_OPEN;
 }
 
-// Prunes the nodes that bounds settle (prune_bound_kernel). *n_open, *nodes: the others, a device list in no order; without sketches all of
-// them (*nodes null: 0 .. n).
-static int launch_prune_bounds(apoe_knn* g, uint32_t degree, uint32_t umap_slots, uint32_t map_slots, uint32_t words, uint32_t* n_open, const uint32_t** nodes) {
+// The nodes of either flag, in no order: those of NODE_OPEN from the front of the list, those of NODE_TABLE from its end (`table` = 0: they
+// count as open). One atomic per wave and flag (one per node on a single counter is 19 ns each, one after the other).
+__global__ __launch_bounds__(256) void open_nodes_kernel(uint32_t n, uint32_t table, const uint32_t* __restrict__ flag, uint32_t* count, uint32_t* nodes) {
+    const uint32_t u = blockIdx.x * blockDim.x + threadIdx.x, f = u < n ? flag[u] : (uint32_t)NODE_SETTLED;
+    const bool to_table = table && f == NODE_TABLE;
+    for (int side = 0; side < 2; side++) {
+        const uint64_t b = __ballot(side ? to_table : f != NODE_SETTLED && !to_table);
+        if (b == 0) continue;
+        uint32_t at = 0;
+        if (lane_id() == 0) at = atomicAdd(count + side, (uint32_t)__popcll(b));
+        at = uniform(at) + __popcll(b & ((1ull << lane_id()) - 1));
+        if ((b >> lane_id()) & 1) nodes[side ? n - 1 - at : at] = u;
+    }
+}
+
+// Prunes the nodes that bounds settle (prune_bound_kernel) and lists the others, in no order.
+struct OpenNodes {
+    uint32_t open = 0, table = 0; // how many are left to the gathered forms and to the table-probing kernel
+    const uint32_t *open_nodes = nullptr, *table_nodes = nullptr;
+};
+static int launch_prune_bounds(apoe_knn* g, uint32_t degree, uint32_t umap_slots, uint32_t map_slots, uint32_t words, bool table_form, OpenNodes* left) {
     apoe_ctx* ctx = g->ctx;
-    *n_open = g->n;
-    *nodes = nullptr;
+    const uint32_t n = g->n;
     const uint32_t lds = g->K == 64 ? BoundLds<64>(umap_slots, map_slots, words).total : BoundLds<128>(umap_slots, map_slots, words).total;
-    if (!g->corpus->sketch.p || lds > ctx->lds_per_block) return APOE_OK;
-    if (!g->open.p) APOE_TRY(g->open.alloc(2 * (size_t)g->n + 1)); // flags, number, nodes
-    APOE_HIP(hipMemsetAsync(g->open.p, 0, ((size_t)g->n + 1) * sizeof(uint32_t), ctx->stream));
-    auto kernel = g->K == 64 ? (g->corpus->narrow ? &prune_bound_kernel<64, true> : &prune_bound_kernel<64, false>)
-                             : (g->corpus->narrow ? &prune_bound_kernel<128, true> : &prune_bound_kernel<128, false>);
-    APOE_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    kernel<<<g->n, g->K * 4, lds, ctx->stream>>>(g->corpus->view(), g->dense_scale * g->dense_scale, g->norms.p, g->ids.p, g->dist.p, degree, g->fwd.p, g->det.p,
-                                                 g->cnt.p, g->kw.p, umap_slots, map_slots, words, g->corpus->sketch_meta.p,
-                                                 reinterpret_cast<const uint4*>(g->corpus->sketch.p), g->open.p);
+    if (!g->open.p) APOE_TRY(g->open.alloc(2 * (size_t)n + 2)); // flags, numbers, nodes
+    APOE_HIP(hipMemsetAsync(g->open.p, 0, ((size_t)n + 2) * sizeof(uint32_t), ctx->stream));
+    if (g->corpus->sketch.p && lds <= ctx->lds_per_block) {
+        auto kernel = g->K == 64 ? (g->corpus->narrow ? &prune_bound_kernel<64, true> : &prune_bound_kernel<64, false>)
+                                 : (g->corpus->narrow ? &prune_bound_kernel<128, true> : &prune_bound_kernel<128, false>);
+        APOE_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        kernel<<<n, g->K * 4, lds, ctx->stream>>>(g->corpus->view(), g->dense_scale * g->dense_scale, g->norms.p, g->ids.p, g->dist.p, degree, g->fwd.p, g->det.p,
+                                                  g->cnt.p, g->kw.p, umap_slots, map_slots, words, g->corpus->sketch_meta.p,
+                                                  reinterpret_cast<const uint4*>(g->corpus->sketch.p), g->open.p);
+    } else {
+        prune_triage_kernel<<<(n + 3) / 4, 256, 0, ctx->stream>>>(n, g->K, g->ids.p, g->dist.p, g->norms.p, g->open.p);
+    }
     APOE_HIP(hipGetLastError());
-    uint32_t *count = g->open.p + g->n, *list = count + 1;
-    open_nodes_kernel<<<(g->n + 255) / 256, 256, 0, ctx->stream>>>(g->n, g->open.p, count, list);
+    uint32_t *count = g->open.p + n, *list = count + 2, h[2] = {0, 0};
+    open_nodes_kernel<<<(n + 255) / 256, 256, 0, ctx->stream>>>(n, table_form, g->open.p, count, list);
     APOE_HIP(hipGetLastError());
-    APOE_HIP(hipMemcpyAsync(n_open, count, sizeof(uint32_t), hipMemcpyDeviceToHost, ctx->stream));
+    APOE_HIP(hipMemcpyAsync(h, count, sizeof(h), hipMemcpyDeviceToHost, ctx->stream));
     APOE_HIP(hipStreamSynchronize(ctx->stream));
-    *nodes = list;
+    left->open = h[0];
+    left->table = h[1];
+    left->open_nodes = list;
+    left->table_nodes = list + (n - h[1]);
     return APOE_OK;
 }
 
@@ -1920,19 +1952,30 @@ int launch_prune(apoe_knn* g, uint32_t degree) {
     }
     const GramPruneLds GL(gram_slots, tgroup, uset_slots, map_slots, words, union_slots, rank_bits, rank_slots, narrow);
     const bool gathered = !g->force_sequential_prune && (g->K == GRAM_ROWS ? GL.total <= lds_budget : g->K <= PS_MAX && gram_tiles_fit(g));
-    // nodes that bounds settle are done here; the others are left in a list
-    uint32_t n_open = g->n;
-    const uint32_t* open = nullptr;
-    if (gathered) APOE_TRY(launch_prune_bounds(g, degree, uset_slots, map_slots, words, &n_open, &open));
-    if (gathered && n_open == 0) return APOE_OK;
+    const PruneLds L(term_slots, uset_slots, map_slots, g->K);
+    const bool table_fits = L.total <= 64 * 1024;
+    auto table_form = [&](uint32_t count, const uint32_t* nodes) -> int { // the table-probing kernel; null: all nodes
+        APOE_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&prune_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)L.total));
+        prune_kernel<<<count, PR_THREADS, L.total, ctx->stream>>>(g->corpus->view(), g->dense_scale * g->dense_scale, g->norms.p, g->K, g->ids.p, g->dist.p, degree,
+                                                                  nodes, g->fwd.p, g->det.p, g->cnt.p, g->kw.p, term_slots, uset_slots, map_slots);
+        APOE_HIP(hipGetLastError());
+        return APOE_OK;
+    };
+    // nodes that bounds settle are done here; the others are left in two lists
+    OpenNodes left;
+    if (gathered) {
+        APOE_TRY(launch_prune_bounds(g, degree, uset_slots, map_slots, words, table_fits, &left));
+        if (left.table) APOE_TRY(table_form(left.table, left.table_nodes));
+        if (left.open == 0) return APOE_OK;
+    }
     if (g->K == GRAM_ROWS && gathered) {
         APOE_HIP(hipMemsetAsync(g->counter.p + 1, 0, sizeof(unsigned long long), ctx->stream));
         auto kernel = g->corpus->narrow ? &prune_gram_kernel<GRAM_THREADS, true> : &prune_gram_kernel<GRAM_THREADS, false>;
         APOE_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)GL.total));
-        kernel<<<n_open, GRAM_THREADS, GL.total, ctx->stream>>>(g->corpus->view(), g->dense_scale * g->dense_scale, g->norms.p, g->ids.p, g->dist.p, degree,
+        kernel<<<left.open, GRAM_THREADS, GL.total, ctx->stream>>>(g->corpus->view(), g->dense_scale * g->dense_scale, g->norms.p, g->ids.p, g->dist.p, degree,
                                                                 g->fwd.p, g->det.p, g->cnt.p, g->kw.p, gram_slots, tgroup, uset_slots, map_slots, words,
                                                                 union_slots, rank_bits, rank_slots, rank_span, g->corpus->sketch_meta.p,
-                                                                reinterpret_cast<const uint4*>(g->corpus->sketch.p), open, g->counter.p + 1);
+                                                                reinterpret_cast<const uint4*>(g->corpus->sketch.p), left.open_nodes, g->counter.p + 1);
         APOE_HIP(hipGetLastError());
         unsigned long long failed = 0;
         APOE_HIP(hipMemcpyAsync(&failed, g->counter.p + 1, sizeof(failed), hipMemcpyDeviceToHost, ctx->stream));
@@ -1945,16 +1988,16 @@ int launch_prune(apoe_knn* g, uint32_t degree) {
     if (g->K > GRAM_ROWS && gathered) {
         const SelectLds SL(uset_slots, map_slots, words);
         if (SL.total <= ctx->lds_per_block) {
-            const uint32_t batch = std::min<uint32_t>(n_open, 32768u);
+            const uint32_t batch = std::min<uint32_t>(left.open, 32768u);
             DevBuf<float> gram;
             APOE_TRY(gram.alloc((size_t)batch * PS_MAX * PS_MAX));
             APOE_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&prune_select_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)SL.total));
             unsigned long long unfit = 0;
-            for (uint32_t node0 = 0; node0 < n_open && !unfit; node0 += batch) {
-                const uint32_t cnt = std::min(batch, n_open - node0);
-                APOE_TRY(launch_gram_tiles(g, open, node0, cnt, gram.p, &unfit));
+            for (uint32_t node0 = 0; node0 < left.open && !unfit; node0 += batch) {
+                const uint32_t cnt = std::min(batch, left.open - node0);
+                APOE_TRY(launch_gram_tiles(g, left.open_nodes, node0, cnt, gram.p, &unfit));
                 if (unfit) break;
-                prune_select_kernel<<<cnt, PS_THREADS, SL.total, ctx->stream>>>(g->corpus->view(), g->norms.p, g->K, g->ids.p, g->dist.p, degree, open, node0, gram.p,
+                prune_select_kernel<<<cnt, PS_THREADS, SL.total, ctx->stream>>>(g->corpus->view(), g->norms.p, g->K, g->ids.p, g->dist.p, degree, left.open_nodes, node0, gram.p,
                                                                               g->fwd.p, g->det.p, g->cnt.p, g->kw.p, uset_slots, map_slots, words);
                 APOE_HIP(hipGetLastError());
             }
@@ -1962,15 +2005,8 @@ int launch_prune(apoe_knn* g, uint32_t degree) {
             if (!unfit) return APOE_OK;
         }
     }
-    const PruneLds L(term_slots, uset_slots, map_slots, g->K);
-    APOE_REQUIRE(L.total <= 64 * 1024, "prune needs %u bytes of LDS (rows with up to %u sparse terms)", L.total,
-                 g->corpus->max_nnz_s + g->corpus->max_nnz_b);
-    APOE_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&prune_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)L.total));
-    prune_kernel<<<g->n, PR_THREADS, L.total, ctx->stream>>>(g->corpus->view(), g->dense_scale * g->dense_scale, g->norms.p, g->K, g->ids.p,
-                                                             g->dist.p, degree, g->fwd.p, g->det.p, g->cnt.p, g->kw.p, term_slots, uset_slots,
-                                                             map_slots);
-    APOE_HIP(hipGetLastError());
-    return APOE_OK;
+    APOE_REQUIRE(table_fits, "prune needs %u bytes of LDS (rows with up to %u sparse terms)", L.total, g->corpus->max_nnz_s + g->corpus->max_nnz_b);
+    return table_form(g->n, nullptr);
 }
 
 int launch_final_graph(apoe_knn* g, uint32_t* rows_dev) {

@@ -172,7 +172,8 @@ int apoe_knn_upload_reverse(apoe_knn* g, const uint32_t* rev_ids, const float* r
  *   0  (default) the forms that gather every neighbour row once: for K = 64 one workgroup builds the node's hybrid Gram
  *      matrix in LDS and selects on it; for K = 128 the Gram matrices of a batch of nodes are computed by the tile kernel
  *      of the local join (32 rows x up to 128 columns of a list at a time) into device memory and a second kernel selects
- *      on them. A corpus whose rows do not fit the tables of these forms falls back to form 1 by itself;
+ *      on them. A corpus whose rows do not fit the tables of these forms falls back to form 1 by itself, and so does a node with
+ *      a neighbour whose norm is not finite;
  *   1  the table-probing kernel: the candidate is the pivot, one wave per live selected member evaluates its product,
  *      rows are read again at every selection step (what the reference does). */
 int apoe_knn_set_prune_form(apoe_knn* g, int form);
