@@ -14,8 +14,10 @@
 // and a second kernel merges every node's proposals into its sorted list (wave-level rank merge, new before old
 // on equal distance, index.cu:333-351) and registers the entries that are new in a list with their nodes' reverse
 // lists (slot = registrations so far, modulo K; every registration a 64-bit atomicMin, so beyond K the closer entry
-// of a slot stays, index.cu:362-372). Lists are read as the step found them and proposals are minima under a total
-// order, so the lists a step leaves do not depend on the order in which tiles run. The reverse lists are append-only
+// of a slot stays, index.cu:362-372). Lists are read as the step found them, proposals are minima under a total
+// order, and the bits of a distance do not depend on which of a node's pickers share a tile (tile_dense; in the wide pair
+// format the last bit may, where two terms of a group sit on one table slot), so the lists a step leaves do not depend on the
+// order in which pickers arrive and tiles run. The reverse lists are append-only
 // over the steps: a node that later drops v stays in R(v) (a stale column costs one evaluation and can never enter a
 // list wrongly: its distance is computed again), and while a list has fewer than K registrations its content does
 // not depend on the order either; beyond K, which entries share a slot follows the arrival order of the counter.
@@ -328,16 +330,20 @@ __device__ __forceinline__ void tile_sparse(const char* recs, const RankTab& T, 
 // when a tile has few columns. The picker rows are staged in `stage`, all dimensions at once if they fit, else a half or a quarter
 // at a time. Partial tiles are added into G in a fixed order, a barrier between them. All threads of the workgroup call it after a barrier; it ends with a
 // barrier.
+// How the dimensions are split into partial sums follows from split_rows (staging) and split_cols (parts) alone. A node whose pickers fill
+// several tiles gives JT_ROWS and all its columns: which pickers are this tile's, and so R and the columns they leave open, is up to the order of
+// their arrival, and the sums must not be. That leaves waves idle where few columns are left (last step, K = 128, 200 000 docs 15.7 -> 16.4 ms;
+// K = 64, 1 M docs 58.3 -> 58.7); a node of one tile has the same R and columns in every run and splits by them.
 template <int NT>
 __device__ __forceinline__ void tile_dense(const char* recs, float dense_mul, char* stage, uint32_t stage_bytes, float* G, const unsigned long long* rowptr, const uint32_t* cols,
-                                           uint32_t R, uint32_t M, int tid, int wave, int lane) {
+                                           uint32_t R, uint32_t M, uint32_t split_rows, uint32_t split_cols, int tid, int wave, int lane) {
     constexpr int NW = NT / WAVE;
     constexpr int RING = 8; // column blocks a wave has in flight: 128 KB per CU
     static_assert(DIM == 4 * JT_STAGE_DIMS, "a row is staged whole, in halves or in quarters");
-    const uint32_t nblk = M <= 16 ? 1u : M <= 32 ? 2u : M <= 64 ? 4u : 8u, parts = (uint32_t)NW / nblk;
+    const uint32_t nblk = split_cols <= 16 ? 1u : split_cols <= 32 ? 2u : split_cols <= 64 ? 4u : 8u, parts = (uint32_t)NW / nblk;
     const uint32_t blk = (uint32_t)wave % nblk, part = (uint32_t)wave / nblk;
     const bool active = blk * 16 < M;
-    const uint32_t fit = stage_bytes / (4 * R);
+    const uint32_t fit = stage_bytes / (4 * split_rows);
     const uint32_t dims = fit >= DIM ? (uint32_t)DIM : fit >= DIM / 2 ? (uint32_t)DIM / 2 : (uint32_t)DIM / 4;
     const uint32_t per = dims / 16 / parts; // 16-float blocks of the staged dimensions per part: 64 ... 1
     float4* A = reinterpret_cast<float4*>(stage);
@@ -638,7 +644,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
             cols = S->cols;
             Mc = uniform(ctl[4]);
         }
-        if (Mc) tile_dense<NT>(a.C.recs, a.dense_mul, smem + L.tab, L.tab_bytes, G, rowptr, cols, R, Mc, tid, wave, lane);
+        if (Mc) tile_dense<NT>(a.C.recs, a.dense_mul, smem + L.tab, L.tab_bytes, G, rowptr, cols, R, Mc, cnt > JT_ROWS ? (uint32_t)JT_ROWS : R, cnt > JT_ROWS ? M : Mc, tid, wave, lane);
         // proposals
         for (uint32_t p = tid; p < R * Mc; p += NT) {
             const uint32_t r = p / Mc, c = cols ? cols[p % Mc] : p % Mc;
@@ -865,7 +871,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
             gram_rows_gather(a.C, col_id, M, rowptr + JT_ROWS, rownnz + JT_ROWS, tid, NT);
             __syncthreads();
             tile_sparse<NARROW, NT>(a.C.recs, T, G, rowptr, rownnz, scan, R, M, a.work + 3, tid, wave, lane, [] {});
-            tile_dense<NT>(a.C.recs, a.dense_mul, smem + L.tab, L.tab_bytes, G, rowptr, nullptr, R, M, tid, wave, lane);
+            tile_dense<NT>(a.C.recs, a.dense_mul, smem + L.tab, L.tab_bytes, G, rowptr, nullptr, R, M, R, M, tid, wave, lane);
             for (uint32_t p = tid; p < R * M; p += NT) {
                 const uint32_t r = p / M, c = p % M;
                 out[(size_t)(r0 + r) * GT_MAX + r0 + c] = G[r * JT_STRIDE + c];
