@@ -1050,12 +1050,13 @@ struct GramPruneLds {
         rowptr = o; o += GRAM_ROWS * 8;
         rownnz = o; o += GRAM_ROWS * 4;
         umap = o; o += umap_slots * 8;
-        idmap = o; o += map_slots * 8;
+        idmap = o; // for the detour counts; then, in the same bytes, what the tests of the pairs need:
+        row = o;                       // dense norm, scale and error of the sketch, norm of the sparse part
+        above = row + GRAM_ROWS * 16;  // bit s of row c: <c, s> exceeds c's norm ...
+        below = above + GRAM_ROWS * 8; // ... and s's norm
+        o += map_slots * 8 > GRAM_ROWS * 32 ? map_slots * 8 : GRAM_ROWS * 32;
         R = o; o += GRAM_ROWS * words * 4;
         F = o; o += GRAM_ROWS * 8; // keyword-flag matrix: bit s of row c = "s holds a term of u that c lacks"
-        above = o; o += GRAM_ROWS * 8; // bit s of row c: <c, s> exceeds c's norm ...
-        below = o; o += GRAM_ROWS * 8; // ... and s's norm
-        row = o; o += GRAM_ROWS * 16;  // dense norm, scale and error of the sketch, norm of the sparse part
         nb_id = o; o += GRAM_ROWS * 4;
         nb_dist = o; o += GRAM_ROWS * 4;
         nrm = o; o += GRAM_ROWS * 4;
@@ -1454,14 +1455,9 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
         if (ok) {
             const uint32_t pos = __popcll(b & lane_lt);
             const uint64_t desc = C.desc[v];
-            const float nv = norms[v], dn = C.dnorm[v];
-            SketchMeta sm = {0.f, 0.f};
-            if (sketch) sm = sketch_meta[v];
             nb_id[pos] = v;
             nb_dist[pos] = dv;
-            nrm[pos] = nv;
-            // what the hybrid norm leaves to the sparse part, with room for the rounding of both norms
-            row[pos] = make_float4(dn, sm.scale, sm.err, sqrtf(fmaxf(nv - dense_mul * dn * dn, 0.f) + 1e-5f * (nv + dense_mul * dn * dn)));
+            nrm[pos] = norms[v];
             rowptr[pos] = desc_off(desc) * 16 + DENSE_BYTES;
             rownnz[pos] = (desc_nnz_s(desc) + desc_nnz_b(desc)) | (desc_nnz_s(desc) << 16);
             lds_map_insert(idmap, mmask, v, pos);
@@ -1538,6 +1534,15 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
         }
     }
     __syncthreads();
+    // the last wave, which has the fewest rows, reads what the tests need of a row: the map's bytes are free now
+    if (wave == NWAVES - 1 && (uint32_t)lane < m) {
+        const uint32_t v = nb_id[lane];
+        const float nv = nrm[lane], dn = C.dnorm[v];
+        SketchMeta sm = {0.f, 0.f};
+        if (sketch) sm = sketch_meta[v];
+        // what the hybrid norm leaves to the sparse part, with room for the rounding of both norms
+        row[lane] = make_float4(dn, sm.scale, sm.err, sqrtf(fmaxf(nv - dense_mul * dn * dn, 0.f) + 1e-5f * (nv + dense_mul * dn * dn)));
+    }
     // (b) stable order by detour count
     if (wave == 0) {
         const uint32_t key = (uint32_t)lane < m ? (det[lane] << 16) | (uint32_t)lane : ~0u;
