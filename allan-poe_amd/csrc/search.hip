@@ -50,7 +50,7 @@ struct SearchArgs {
     uint32_t* codes;       // of the query's dense row, 1 KB per workgroup: in device memory (it is read beside sketches, which take longer), since a
                            // kilobyte of LDS more costs long batches a resident query per CU (12 -> 11: 3 %)
     unsigned long long* work; // [0] next query, [1] expansions, [2] evaluations, [3] nnz splade, [4] nnz bm25, [5] dense rows (fp32 or half) read in the walk,
-                              // [6] pool entries evaluated again in fp32, [7] their pairs, [8] sketches read, [9] pairs of the evaluations that codes settled
+                              // [6] pool entries evaluated again in fp32, [7] their pairs, [8] sketches read, [9] pairs of the evaluations that codes left open less those that they settled
     uint32_t coded;           // 1: the records carry codes of their values and the search may ask them
     uint32_t full_eval;       // 1: read the dense row of every candidate (no bound test)
     const uint16_t* half;     // not null: the walk takes dense parts from the half-precision rows, the final pool is evaluated again in fp32
@@ -424,6 +424,7 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
         const bool sketched = __builtin_amdgcn_readfirstlane((int)(q_scale > 0.f)) != 0;
         uint32_t st_exp = 0, st_eval = 0, st_dense = 0, st_again = 0, st_again_pairs = 0, st_sketch = 0; // wave-uniform counters of one query
         uint32_t ln_s = 0, ln_b = 0, ln_coded = 0;      // pairs read for the candidates this lane decided; of those that codes settled
+        uint32_t st_reread = 0;                         // wave-uniform: pairs of the candidates that codes left open
         Front front; // wave 0: the first unexplored pool entry
         front.id = EMPTY;
         front.slot = 0;
@@ -802,7 +803,10 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
                         jj[b] = __builtin_ctzll(need);
                         need &= need - 1;
                         const uint64_t desc = readlane64(my_desc, jj[b]);
-                        if (by_codes) row_issue<NARROW>(rl[b], ri[b], a.C, desc, true, a.paths);
+                        if (by_codes) {
+                            row_issue<NARROW>(rl[b], ri[b], a.C, desc, true, a.paths);
+                            st_reread += (uint32_t)ri[b].n;
+                        }
                         if constexpr (HALF) dense_issue_half(row[b], a.half + (size_t)uniform(new_id[jj[b]]) * DIM);
                         else dense_issue(row[b], a.C.recs + desc_off(desc) * 16);
                     }
@@ -1080,7 +1084,7 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
             if (st_again) atomicAdd(stat + 6, (unsigned long long)st_again);
             if (st_again_pairs) atomicAdd(stat + 7, (unsigned long long)st_again_pairs);
             if (st_sketch) atomicAdd(stat + 8, (unsigned long long)st_sketch);
-            if (CODES && ln_coded) atomicAdd(stat + 9, (unsigned long long)ln_coded);
+            if (CODES) atomicAdd(stat + 9, (unsigned long long)st_reread - ln_coded);
         }
     }
     __syncthreads();
@@ -1317,7 +1321,7 @@ int launch_search(apoe_ctx* ctx, const apoe_corpus* c, const apoe_queries* q, co
         // dense rows and sketches actually needed (a sketch with its scale and error) + pairs + descriptor and dense norm (12 B per evaluation)
         uint64_t bytes = h[5] * (uint64_t)(a.half ? DENSE_BYTES / 2 : DENSE_BYTES) + h[8] * (uint64_t)(SKETCH_BYTES + sizeof(SketchMeta));
         bytes += (c->narrow ? 6 : 8) * (h[3] + h[4]) + 12 * h[2];
-        bytes -= 3 * h[9]; // where codes settle an evaluation: a byte instead of the value
+        bytes += 3 * h[9]; // codes are three bytes a pair with their terms: instead of the pair, or beside it where it was read after all
         bytes += h[6] * (uint64_t)(DENSE_BYTES + 8) + (c->narrow ? 6 : 8) * h[7]; // the pool evaluated again in fp32
         bytes += h[1] * 4ull * a.W;
         uint64_t qbytes = (uint64_t)q_count * DENSE_BYTES + 8 * (q->h_s_off[p->q_begin + q_count] - q->h_s_off[p->q_begin]) +

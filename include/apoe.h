@@ -241,7 +241,7 @@ typedef struct {
     uint64_t nnz_bm25;    /* BM25 pairs read by those evaluations (0 if path off) */
     uint64_t dense_rows;  /* evaluations that read the dense row (4 KB, or 2 KB with variant 0x200): neither pairs
                              and norms nor the 1 KB sketch settled them (see variant) */
-    uint64_t algo_bytes;  /* algorithmic HBM bytes: dense rows and sketches read + pairs (or their byte codes) + descriptors +
+    uint64_t algo_bytes;  /* algorithmic HBM bytes: dense rows and sketches read + pairs (and byte codes where they are asked) + descriptors +
                              graph rows + queries + results */
 } apoe_search_stats;
 

@@ -56,3 +56,28 @@ def test_rows_are_those_of_a_walk_without_bounds(gpu_ctx, kind):
         a, ad, _ = apoe.search(gpu_ctx, gc, gq, gg, w3, cands, variant=shape | 0x200)
         b, bd, _ = apoe.search(gpu_ctx, gc, gq, gg, w3, cands, variant=shape | 0x300)
         assert np.array_equal(a, b) and np.array_equal(ad, bd, equal_nan=True), (w3, cands, "half")
+
+
+def test_bytes_of_evaluations_that_the_codes_leave_open(gpu_ctx):
+    """Documents that no bound tells apart (all alike): whatever the codes are asked for stays open, and what was read is codes (a byte and a
+    16-bit term a pair) and sketch beside what a walk without bounds reads."""
+    import apoe
+    rng = np.random.default_rng(8)
+    pairs_s, pairs_b = 40, 20
+    off = lambda n, m: np.arange(n + 1, dtype=np.uint32) * np.uint32(m)
+    same = lambda x, n: np.ascontiguousarray(np.broadcast_to(x, (n, len(x)))).astype(x.dtype)
+    dense, terms = rng.standard_normal(1024).astype(np.float32), np.arange(64, dtype=np.uint32)
+    val = rng.gamma(1.0, 1.0, 64).astype(np.float32)
+    corpus = (same(dense, N), off(N, pairs_s), same(terms[:pairs_s], N).ravel(), same(val[:pairs_s], N).ravel(),
+              off(N, pairs_b), same(terms[:pairs_b], N).ravel(), same(val[:pairs_b], N).ravel())
+    queries = (same(dense, NQ), off(NQ, 10), same(terms[:10], NQ).ravel(), same(val[:10], NQ).ravel(),
+               off(NQ, 10), same(terms[:10], NQ).ravel(), same(val[:10], NQ).ravel())
+    rows = np.zeros((N, D + 8), np.uint32)
+    rows[:, :D] = rng.integers(0, N, (N, D))
+    gc, gq, gg = apoe.Corpus(gpu_ctx, *corpus), apoe.Queries(gpu_ctx, *queries), apoe.Graph(gpu_ctx, rows, np.arange(D, dtype=np.uint32))
+    for w3, pairs in (((49, 1, 1), pairs_s + pairs_b), ((49, 1, 0), pairs_s)):
+        _, _, sa = apoe.search(gpu_ctx, gc, gq, gg, w3, 24, variant=4)
+        _, _, sb = apoe.search(gpu_ctx, gc, gq, gg, w3, 24, variant=4 | 0x100)
+        assert sa.evaluations == sa.dense_rows == sb.evaluations == sb.dense_rows
+        coded, rest = divmod(sa.algo_bytes - sb.algo_bytes, 3 * pairs + 1032)
+        assert rest == 0 and 0 < coded < sa.evaluations, (coded, rest)
