@@ -16,6 +16,7 @@ LIB_PATH = os.path.join(_HERE, "libapoe.so")
 INF_DIS = 1000000.0
 KW_SLOTS = 8
 KW_CAND = 32
+WITHOUT_CODES, WITHOUT_SKETCHES = 1, 2
 
 _lib = None
 
@@ -36,7 +37,7 @@ class SearchStats(C.Structure):
 
 
 EXPORTS = [
-    "apoe_last_error_string", "apoe_ctx_create", "apoe_ctx_destroy", "apoe_ctx_synchronize", "apoe_corpus_create",
+    "apoe_last_error_string", "apoe_ctx_create", "apoe_ctx_destroy", "apoe_ctx_synchronize", "apoe_corpus_create", "apoe_corpus_create_without",
     "apoe_corpus_destroy", "apoe_corpus_info", "apoe_corpus_bytes", "apoe_corpus_pair_bytes", "apoe_corpus_make_half_rows", "apoe_queries_create", "apoe_queries_destroy",
     "apoe_kg_create", "apoe_kg_destroy", "apoe_calibrate_weights", "apoe_hybrid_distance_batch", "apoe_hybrid_distance_pairs", "apoe_norms",
     "apoe_knn_create", "apoe_knn_destroy", "apoe_knn_use_half_rows", "apoe_knn_set_join", "apoe_nnd_init", "apoe_nnd_iterate", "apoe_nnd_merge_reverse",
@@ -119,13 +120,13 @@ class Context:
 
 
 class Corpus:
-    def __init__(self, ctx, dense, s_off, s_idx, s_val, b_off, b_idx, b_val):
+    def __init__(self, ctx, dense, s_off, s_idx, s_val, b_off, b_idx, b_val, without=0):
         self.ctx = ctx
         n, dim = dense.shape
         keep = [_ptr(dense, np.float32), _ptr(s_off, np.uint32), _ptr(s_idx, np.uint32), _ptr(s_val, np.float32),
                 _ptr(b_off, np.uint32), _ptr(b_idx, np.uint32), _ptr(b_val, np.float32)]
         self.h = C.c_void_p()
-        _check(lib().apoe_corpus_create(ctx.h, C.c_uint32(n), C.c_uint32(dim), *[k[1] for k in keep], C.byref(self.h)))
+        _check(lib().apoe_corpus_create_without(ctx.h, C.c_uint32(without), C.c_uint32(n), C.c_uint32(dim), *[k[1] for k in keep], C.byref(self.h)))
         self.n, self.dim = n, dim
 
     def info(self):

@@ -213,8 +213,14 @@ int apoe_ctx_synchronize(apoe_ctx* ctx) {
 
 int apoe_corpus_create(apoe_ctx* ctx, uint32_t n, uint32_t dim, const float* dense, const uint32_t* s_off, const uint32_t* s_idx,
                        const float* s_val, const uint32_t* b_off, const uint32_t* b_idx, const float* b_val, apoe_corpus** out) {
+    return apoe_corpus_create_without(ctx, 0, n, dim, dense, s_off, s_idx, s_val, b_off, b_idx, b_val, out);
+}
+
+int apoe_corpus_create_without(apoe_ctx* ctx, uint32_t without, uint32_t n, uint32_t dim, const float* dense, const uint32_t* s_off, const uint32_t* s_idx,
+                               const float* s_val, const uint32_t* b_off, const uint32_t* b_idx, const float* b_val, apoe_corpus** out) {
     APOE_REQUIRE(ctx && out, "ctx/out is null");
     *out = nullptr;
+    APOE_REQUIRE((without & ~(APOE_WITHOUT_CODES | APOE_WITHOUT_SKETCHES)) == 0, "unknown flags 0x%x", without);
     APOE_REQUIRE(dim == DIM, "dim must be %d, got %u", DIM, dim);
     APOE_REQUIRE(n >= 1 && n < (1u << 30), "document count %u outside [1, 2^30)", n);
     APOE_REQUIRE(dense && s_off && b_off, "dense/s_off/b_off is null");
@@ -255,7 +261,7 @@ int apoe_corpus_create(apoe_ctx* ctx, uint32_t n, uint32_t dim, const float* den
         c->narrow = max_term < 65536u;
         c->max_term = max_term;
         std::vector<uint64_t> desc(n);
-        const bool codes = c->narrow;
+        const bool codes = c->narrow && !(without & APOE_WITHOUT_CODES);
         uint64_t off16 = 0, with_codes = 0;
         for (uint32_t i = 0; i < n; i++) {
             const uint32_t ns = hs[i + 1] - hs[i], nb = hb[i + 1] - hb[i];
@@ -297,7 +303,7 @@ int apoe_corpus_create(apoe_ctx* ctx, uint32_t n, uint32_t dim, const float* den
         // The sketch saves the search reads but nothing depends on it: it comes last, after the staged arrays, and a corpus does without
         // when it cannot be had or when less than ten times its size is free. What is left then holds a K = 128 / degree 64 build (about
         // 6.3 KB a document) and the half-precision rows (2 KB).
-        if ((size_t)n * SKETCH_BYTES <= free_bytes / 10 && !(c->sketch.try_alloc((size_t)n * (SKETCH_BYTES / 4)) && c->sketch_meta.try_alloc(n)))
+        if (!(without & APOE_WITHOUT_SKETCHES) && (size_t)n * SKETCH_BYTES <= free_bytes / 10 && !(c->sketch.try_alloc((size_t)n * (SKETCH_BYTES / 4)) && c->sketch_meta.try_alloc(n)))
             c->sketch.release();
         APOE_TRY(launch_pack(ctx, n, d_dense.p, d_soff.p, d_sidx.p, d_sval.p, d_boff.p, d_bidx.p, d_bval.p, c->desc.p, c->recs.p, c->dnorm.p,
                              c->sketch_meta.p, c->sketch.p, c->narrow, c->coded));

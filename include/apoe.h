@@ -63,6 +63,16 @@ int apoe_corpus_create(apoe_ctx* ctx, uint32_t n, uint32_t dim, const float* den
                        const uint32_t* s_off, const uint32_t* s_idx, const float* s_val,
                        const uint32_t* b_off, const uint32_t* b_idx, const float* b_val,
                        apoe_corpus** out);
+/* apoe_corpus_create without some of what a corpus does without when device memory is short; results are the same.
+ * APOE_WITHOUT_CODES: no byte codes of the values in the records (4 % of them; a narrow corpus goes without when it would take
+ * more than a quarter of the free memory), APOE_WITHOUT_SKETCHES: no 8-bit sketches of the dense rows (1 032 bytes a document;
+ * left out when they would take more than a tenth). */
+#define APOE_WITHOUT_CODES 1u
+#define APOE_WITHOUT_SKETCHES 2u
+int apoe_corpus_create_without(apoe_ctx* ctx, uint32_t without, uint32_t n, uint32_t dim, const float* dense,
+                               const uint32_t* s_off, const uint32_t* s_idx, const float* s_val,
+                               const uint32_t* b_off, const uint32_t* b_idx, const float* b_val,
+                               apoe_corpus** out);
 /* Optional second copy of the dense rows in half precision (IEEE binary16, round to nearest even; 2 KB per
  * row beside the 4 KB fp32 row, which stays). The reference keeps ONLY such a copy and multiplies and adds in
  * half precision (f2h, utils.cuh:78-83; query.cu:459-465); here it is an option for callers that trade
@@ -74,7 +84,8 @@ void apoe_corpus_destroy(apoe_corpus* c);
 /* info4 = {n, dim, max splade nnz per row, max bm25 nnz per row} (index.cu:829-835). */
 int apoe_corpus_info(const apoe_corpus* c, uint32_t* info4);
 /* Bytes of the device records with their descriptors and norms, and of the half-precision rows if they were made: the HBM
- * footprint one full scan reads. The 8-bit sketch beside them (1 032 bytes a document, when there is room) is not among them. */
+ * footprint one full scan reads. The byte codes in the records (4 % of them, narrow corpora) and the 8-bit sketches beside them
+ * (1 032 bytes a document), both when there is room, are not among them. */
 uint64_t apoe_corpus_bytes(const apoe_corpus* c);
 /* Bytes one (term, value) pair takes in the device records: 6 when every term id of the corpus
  * (both paths) is below 65536 (values as f32, ids as u16, the path known from the position),

@@ -37,10 +37,7 @@ def make(kind, wide):
     return tuple(a)
 
 
-@pytest.mark.parametrize("wide", [False, True])
-@pytest.mark.parametrize("K,degree", [(64, 32), (64, 64), (128, 48)])
-@pytest.mark.parametrize("kind", ["bounds settle", "pairs decide", "near twins", "rich rows", "odd rows"])
-def test_prune_matches_oracle(gpu_ctx, kind, K, degree, wide):
+def check(gpu_ctx, kind, K, degree, wide, without=0):
     import apoe
     import oracle as O
     arrays = make(kind, wide)
@@ -49,7 +46,7 @@ def test_prune_matches_oracle(gpu_ctx, kind, K, degree, wide):
     counts = [c for c in (0, 1, 2, 15, 16, 17, 31, 32, 33, 48, 49, 63, 64, 65, 96, 113, 127) if c < K]
     for i, u in enumerate(np.random.default_rng(6).choice(N, 6 * len(counts), replace=False)):
         dist[u, counts[i % len(counts)]:] = apoe.INF_DIS
-    gc = apoe.Corpus(gpu_ctx, *arrays)
+    gc = apoe.Corpus(gpu_ctx, *arrays, without=without)
     knn = apoe.Knn(gpu_ctx, gc, K, 7.0)
     knn.upload(ids, dist)
     knn.prune(degree)
@@ -63,3 +60,10 @@ def test_prune_matches_oracle(gpu_ctx, kind, K, degree, wide):
     assert np.all(g_kw == c_kw, axis=1)[same].mean() >= 0.995
     if kind == "near twins":
         assert np.any(c_cnt < min(degree, K - 1))  # the rule does reject here
+
+
+@pytest.mark.parametrize("wide", [False, True])
+@pytest.mark.parametrize("K,degree", [(64, 32), (64, 64), (128, 48)])
+@pytest.mark.parametrize("kind", ["bounds settle", "pairs decide", "near twins", "rich rows", "odd rows"])
+def test_prune_matches_oracle(gpu_ctx, kind, K, degree, wide):
+    check(gpu_ctx, kind, K, degree, wide)
