@@ -117,6 +117,8 @@ struct apoe_corpus {
     uint64_t rec_bytes = 0, total_pairs = 0; // bytes without the codes: what a scan of all rows reads
     bool narrow = false; // pair format of the records (6 instead of 8 bytes a pair when every term id is below 65536)
     bool coded = false;  // narrow records carry byte codes of their values (a bound for the search)
+    uint64_t pairs_s = 0;           // SPLADE pairs of all rows
+    double mean_sq[3] = {0, 0, 0};  // coded: mean squared norm of a row's dense, SPLADE and BM25 part, over a sample
     apoe::DevBuf<uint64_t> desc;
     apoe::DevBuf<char> recs;
     apoe::DevBuf<float> dnorm;
@@ -188,6 +190,9 @@ int copy_out(apoe_ctx* ctx, void* dst_any, const void* src_dev, size_t bytes);
 int launch_pack(apoe_ctx* ctx, uint32_t n, const float* dense, const uint32_t* s_off, const uint32_t* s_idx, const float* s_val,
                 const uint32_t* b_off, const uint32_t* b_idx, const float* b_val, const uint64_t* desc, char* recs, float* dnorm,
                 SketchMeta* sketch_meta, uint32_t* sketch, bool narrow, bool coded);
+constexpr uint32_t ROW_SCALE_PARTS = 256;
+int launch_row_scale(apoe_ctx* ctx, uint32_t n, uint32_t sample, const float* dense, const uint32_t* s_off, const float* s_val, const uint32_t* b_off, const float* b_val,
+                     float* out_dev); // out[ROW_SCALE_PARTS][3]: squares summed over `sample` rows
 int launch_max_u32(apoe_ctx* ctx, const uint32_t* a_dev, size_t n, uint32_t* out_dev);
 int launch_half_rows(apoe_ctx* ctx, const apoe_corpus* c, uint16_t* out_dev);
 int launch_distance_batch(apoe_ctx* ctx, const apoe_corpus* c, const apoe_queries* q, const float* w3, const uint32_t* ids_dev,

@@ -249,9 +249,9 @@ int apoe_corpus_create_without(apoe_ctx* ctx, uint32_t without, uint32_t n, uint
         APOE_TRY(d_sidx.init(ctx, s_idx, hs[n]));
         APOE_TRY(d_bidx.init(ctx, b_idx, hb[n]));
         // the pair format follows from the largest term id of either path
-        DevBuf<uint32_t> d_max;
+        DevBuf<uint32_t> d_max; // behind it: the sums of the sample below
         uint32_t max_term = 0;
-        APOE_TRY(d_max.alloc(1));
+        APOE_TRY(d_max.alloc(1 + 3 * ROW_SCALE_PARTS));
         APOE_TRY(copy_in(ctx, d_max.p, &max_term, sizeof(uint32_t)));
         APOE_TRY(launch_max_u32(ctx, d_sidx.p, hs[n], d_max.p));
         APOE_TRY(launch_max_u32(ctx, d_bidx.p, hb[n], d_max.p));
@@ -272,6 +272,7 @@ int apoe_corpus_create_without(apoe_ctx* ctx, uint32_t without, uint32_t n, uint
         APOE_REQUIRE(off16 < (1ull << DESC_OFF_BITS), "corpus of %llu bytes exceeds the record address range", (unsigned long long)off16 * 16);
         c->rec_bytes = off16 * 16;
         c->total_pairs = (uint64_t)hs[n] + hb[n];
+        c->pairs_s = hs[n];
         APOE_TRY(c->desc.alloc(n));
         if (codes) {
             // Nothing depends on the codes (about 4 % of the records): a corpus that would take more than a quarter of the free device memory with
@@ -307,6 +308,13 @@ int apoe_corpus_create_without(apoe_ctx* ctx, uint32_t without, uint32_t n, uint
             c->sketch.release();
         APOE_TRY(launch_pack(ctx, n, d_dense.p, d_soff.p, d_sidx.p, d_sval.p, d_boff.p, d_bidx.p, d_bval.p, c->desc.p, c->recs.p, c->dnorm.p,
                              c->sketch_meta.p, c->sketch.p, c->narrow, c->coded));
+        if (c->coded) { // what tells a search whether the codes pay
+            const uint32_t sample = std::min(n, 4096u);
+            float sums[3 * ROW_SCALE_PARTS];
+            APOE_TRY(launch_row_scale(ctx, n, sample, d_dense.p, d_soff.p, d_sval.p, d_boff.p, d_bval.p, reinterpret_cast<float*>(d_max.p + 1)));
+            APOE_TRY(copy_out(ctx, sums, d_max.p + 1, sizeof(sums)));
+            for (uint32_t i = 0; i < 3 * ROW_SCALE_PARTS; i++) c->mean_sq[i % 3] += (double)sums[i] / sample;
+        }
         APOE_HIP(hipStreamSynchronize(ctx->stream));
     }
     *out = c.release();

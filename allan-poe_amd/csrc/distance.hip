@@ -110,6 +110,34 @@ __global__ __launch_bounds__(256) void pack_kernel(uint32_t n, const float* __re
     }
 }
 
+// Squared norms of the three parts of every sampled row (row i * n / sample), summed per wave: a wave takes rows w, w + ROW_SCALE_PARTS, ...
+__global__ __launch_bounds__(256) void row_scale_kernel(uint32_t n, uint32_t sample, const float* __restrict__ dense, const uint32_t* __restrict__ s_off,
+                                                        const float* __restrict__ s_val, const uint32_t* __restrict__ b_off, const float* __restrict__ b_val, float* out) {
+    const uint32_t w = blockIdx.x * (256 / WAVE) + threadIdx.x / WAVE, lane = lane_id();
+    float sq[3] = {0.f, 0.f, 0.f};
+    for (uint32_t i = w; i < sample; i += ROW_SCALE_PARTS) {
+        const uint32_t doc = (uint32_t)((uint64_t)i * n / sample);
+        const float4* row = reinterpret_cast<const float4*>(dense + (size_t)doc * DIM);
+#pragma unroll
+        for (int k = 0; k < NV; k++) {
+            const float4 x = row[lane + WAVE * k];
+            sq[0] += x.x * x.x + x.y * x.y + x.z * x.z + x.w * x.w;
+        }
+        for (uint32_t j = s_off[doc] + lane; j < s_off[doc + 1]; j += WAVE) sq[1] = fmaf(s_val[j], s_val[j], sq[1]);
+        for (uint32_t j = b_off[doc] + lane; j < b_off[doc + 1]; j += WAVE) sq[2] = fmaf(b_val[j], b_val[j], sq[2]);
+    }
+    for (int p = 0; p < 3; p++) {
+        const float x = wave_sum_dpp(sq[p]);
+        if (lane == 0) out[w * 3 + p] = x;
+    }
+}
+int launch_row_scale(apoe_ctx* ctx, uint32_t n, uint32_t sample, const float* dense, const uint32_t* s_off, const float* s_val, const uint32_t* b_off, const float* b_val,
+                     float* out_dev) {
+    row_scale_kernel<<<ROW_SCALE_PARTS / (256 / WAVE), 256, 0, ctx->stream>>>(n, sample, dense, s_off, s_val, b_off, b_val, out_dev);
+    APOE_HIP(hipGetLastError());
+    return APOE_OK;
+}
+
 int launch_pack(apoe_ctx* ctx, uint32_t n, const float* dense, const uint32_t* s_off, const uint32_t* s_idx, const float* s_val,
                 const uint32_t* b_off, const uint32_t* b_idx, const float* b_val, const uint64_t* desc, char* recs, float* dnorm,
                 SketchMeta* sketch_meta, uint32_t* sketch, bool narrow, bool coded) {

@@ -1,6 +1,7 @@
 // Greedy beam search over the hybrid graph: one workgroup per query; the candidate pool, the
 // query's dense row, its sparse-term tables and the fresh-neighbour list in LDS; an exact
 // visited bitmap per workgroup in HBM.
+#include <cmath>
 #include <mutex>
 #include <type_traits>
 
@@ -1169,6 +1170,30 @@ static int launch_mode(apoe_ctx* ctx, int mode, int nw, const SearchArgs& a, uin
 
 // static_ws: null, or the device address of this GPU's search_scratch: then nothing is allocated, the grid is cut to
 // the bitmaps that fit, and a call without `stats` returns with the work still running on the context's stream.
+// Whether a search asks the codes. They pay where the dense part decides, so that pairs settle little and memory bounds a long batch; elsewhere pairs settle
+// what the looser bound leaves open, and their kernels, which take more vector instructions a row, are the slower ones. What decides is estimated from the
+// corpus: the dense part of a score reaches w_dense |q_d| |d_d|, the sparse part at most w |q_s| |d_s| a path, with the documents' mean squared norms (a query's
+// dense row is as long as a document's; its pairs are as long as a document's, but fewer). Time without codes / with codes, 10 000 queries on 1 M docs,
+// cands 64 ... 256, by the ratio of the two, on lists of near rows and on a built index:
+//   plain    i.i.d. 0.014: 0.97-1.05  0.03: 0.98-1.03  0.08: 0.96-1.03  0.17: 1.07-1.12  0.4: 1.10-1.11  1.5: 1.08   dense neighbours 0.09: 0.93-0.96  0.18: 1.00-1.07
+//            0.36: 1.10-1.13  2.2: 1.08-1.14
+//   half     0.014: 0.90-0.97  0.03: 0.87-0.95  0.08: 0.87-1.02  0.17: 1.01-1.08  1.5: 0.99-1.06;  0.09: 0.88-0.93  0.18: 0.99-1.05  0.36: 1.09-1.11
+//   keyword  0.014: 0.91-0.98  0.03: 0.86-0.99  0.08: 0.89-0.97  0.17: 0.96-1.07  1.5: 0.97-1.04;  0.09: 0.93-0.94  0.18: 1.00-1.04  0.36: 1.06-1.08  2.2: 1.07-1.08
+// The line lies at an eighth. A linking entity's bonus is a third part: where it exceeds the dense part, the pool holds linked documents, no sketch is asked and the
+// pairs of most others are read twice (bonus 40; dense part 8 and 16 with dense neighbours 0.91, 49: 1.07-1.09, 100 on i.i.d. rows 1.03-1.08). Pairs alone never
+// ask them (SPLADE, cands 256: 24.5 ms without, 25.8 with). The codes are kernels of their own: with both ways in one, spilled registers cost searches without codes 3 %.
+static bool codes_pay(const apoe_corpus* c, const apoe_queries* q, const apoe_search_params* p, uint32_t q_count, uint32_t paths, bool kg) {
+    if (!(paths & PATH_DENSE) || !(paths & (PATH_SPARSE | PATH_BM25))) return false;
+    auto part = [&](float w, double mean_sq, uint64_t pairs, uint64_t q_pairs) { // of a path with that many pairs in all documents and in the batch
+        return pairs ? fabs((double)w) * mean_sq * sqrt((double)q_pairs / q_count / ((double)pairs / c->n)) : 0.0;
+    };
+    const uint32_t q0 = p->q_begin, q1 = q0 + q_count;
+    const double dense = (double)p->w_dense * c->mean_sq[0];
+    const double sparse = (paths & PATH_SPARSE ? part(p->w_sparse, c->mean_sq[1], c->pairs_s, q->h_s_off[q1] - q->h_s_off[q0]) : 0.0) +
+                          (paths & PATH_BM25 ? part(p->w_bm25, c->mean_sq[2], c->total_pairs - c->pairs_s, q->h_b_off[q1] - q->h_b_off[q0]) : 0.0);
+    return dense >= sparse / 8 && (!kg || dense >= p->kg_weight);
+}
+
 int launch_search(apoe_ctx* ctx, const apoe_corpus* c, const apoe_queries* q, const apoe_graph* g, const apoe_kg* kg,
                   const apoe_search_params* p, uint32_t* out_ids_dev, float* out_dist_dev, apoe_search_stats* stats, char* static_ws) {
     APOE_REQUIRE(p->cands >= 1 && p->cands <= APOE_MAX_CANDS, "cands must be in 1..%d, got %u", APOE_MAX_CANDS, p->cands);
@@ -1221,12 +1246,7 @@ int launch_search(apoe_ctx* ctx, const apoe_corpus* c, const apoe_queries* q, co
         APOE_REQUIRE(c->n < (1u << 30), "keyword-filter search keeps two flag bits on a document id: %u documents are too many", c->n);
         a.paths = PATH_DENSE | PATH_SPARSE | PATH_BM25; // query.cu:2005-2007: always the three-path loop
     }
-    // The codes pay where the dense part decides, so that pairs settle little and memory bounds a long batch: 10 000 queries on 1 M docs with / without them,
-    // dense neighbours under (49, 1, 1) at cands 80 19.5 / 21.5 ms, i.i.d. under (1729, 6.28, 1) at cands 256 45.7 / 49.3. Under (1, 1, 1) it is the graph
-    // that tells (i.i.d. at cands 256: lists of near rows 36.0 / 38.4, a built index, whose hubs stay in the cache, 30.7 / 29.9, at cands 64 10.9 / 10.0),
-    // and pairs alone are bound by vector instructions, of which a coded row takes more (SPLADE, cands 256: 25.8 / 24.5). The line lies between the
-    // measured ratios of 1 and 49. The codes are kernels of their own: with both ways in one, spilled registers cost searches without codes 3 %.
-    a.coded = c->coded && !a.full_eval && p->w_dense >= 8.f * fmaxf(p->w_sparse, p->w_bm25) && (a.paths & PATH_DENSE) && (a.paths & (PATH_SPARSE | PATH_BM25)) ? 1u : 0u;
+    a.coded = c->coded && !a.full_eval && codes_pay(c, q, p, q_count, a.paths, use_kg) ? 1u : 0u;
     if (use_kg) {
         APOE_REQUIRE(kg->n_queries >= p->q_begin + q_count, "knowledge graph holds entities for %u queries, %u needed", kg->n_queries, p->q_begin + q_count);
         a.e2e_off = kg->e2e_off.p;

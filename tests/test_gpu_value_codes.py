@@ -81,3 +81,22 @@ def test_bytes_of_evaluations_that_the_codes_leave_open(gpu_ctx):
         assert sa.evaluations == sa.dense_rows == sb.evaluations == sb.dense_rows
         coded, rest = divmod(sa.algo_bytes - sb.algo_bytes, 3 * pairs + 1032)
         assert rest == 0 and 0 < coded < sa.evaluations, (coded, rest)
+
+
+def test_codes_are_asked_where_the_dense_part_decides(gpu_ctx):
+    """Under one set of weights: asked on a corpus whose dense parts weigh as much as its pairs, not on one whose values are ten times as
+    large, and not where the bonus of a linking entity exceeds the dense part. A corpus without codes reads other bytes if they are asked."""
+    import apoe
+    import apoe_synth as S
+    corpus, queries, rows, entry = world("plain", 3)
+    kg = apoe.KnowledgeGraph(gpu_ctx, *S.to_numpy(S.knowledge_graph(800, N, NQ, seed=23, device="cpu", mean_out=6.0)))
+    gq, gg = apoe.Queries(gpu_ctx, *queries), apoe.Graph(gpu_ctx, rows, entry)
+    for scale, more, asked in ((1, {}, True), (10, {}, False), (1, dict(kg=kg, kg_weight=100.0), True), (1, dict(kg=kg, kg_weight=2000.0), False)):
+        arrays = list(corpus)
+        arrays[3], arrays[6] = arrays[3] * np.float32(scale), arrays[6] * np.float32(scale)
+        read = []
+        for without in (0, apoe.WITHOUT_CODES):
+            gc = apoe.Corpus(gpu_ctx, *arrays, without=without)
+            read.append(apoe.search(gpu_ctx, gc, gq, gg, (49, 1, 1), 64, variant=4, **more)[2].algo_bytes)
+            gc.close()
+        assert (read[0] != read[1]) == asked, (scale, sorted(more))
