@@ -40,7 +40,7 @@ constexpr int JT_COLS = 128;
 // tile, so neither workgroup lacks work. Builds of ten steps against one workgroup of sixteen waves (wide pairs: of eight) with the
 // columns' pairs in registers: 100 000 docs K = 64 145.2 -> 113.3 ms, 30 011 docs K = 128 97.3 -> 76.7 ms, 20 000 docs wide 54.5 ->
 // 37.4 ms, 300 000 docs of the i.i.d. corpus 299 -> 254 ms. A corpus whose longest row does not fit the table of the smaller LDS takes one
-// workgroup of sixteen waves per CU (tile_shape).
+// workgroup of sixteen waves per CU, and so does one whose rows are long (tile_shape).
 constexpr int JT_PAIR_THREADS = 512, JT_SOLO_THREADS = 1024;
 constexpr int JT_STRIDE = JT_COLS + 1;
 constexpr int JT_STAGE_DIMS = 256; // the picker rows are staged at least this many dimensions at a time
@@ -884,7 +884,11 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
 // Table of a tile, and whether two workgroups share a CU (half of its LDS each). The table then takes as many slots as fit, up to
 // eight rows of the longest kind: an average group of eight rows of 180 terms has 1 000 distinct ones, 1 280 slots fit beside a
 // bitmap for a vocabulary of 32 768. A group that exceeds them is done in halves; a corpus with a single row that does
-// would lose that row, so it takes the whole LDS.
+// would lose that row, so it takes the whole LDS. So does a narrow corpus of whose average rows the smaller table holds fewer than four: its groups
+// are pairs and single rows, each a build and a probe of every column. Eight steps on 12 000 docs, K = 64, two workgroups / one, by rows that the
+// smaller table holds: vocabulary 32 768 (1 332 slots) 7.6 rows 8.8 / 11.6 ms, 4.2 11.5 / 13.3, 4.0 10.7 / 10.4, 3.9 16.3 / 14.6, 3.1 18.5 / 16.7,
+// 1.6 74.7 / 45.3; 65 536 (820 slots) 4.7 10.6 / 12.1, 4.1 12.2 / 12.1, 3.6 12.6 / 12.0, 3.1 17.6 / 13.3. Wide corpora, whose builds and probes
+// wait longer, gain from the second workgroup at any length (7.5 rows 16.0 / 20.8 ms, 1.6 198 / 235).
 struct TileShape {
     uint32_t index_bits, slot_cap, span, lds;
     bool pair;
@@ -897,7 +901,8 @@ static TileShape tile_shape(const apoe_ctx* ctx, const apoe_corpus* c) {
     const uint32_t half = (uint32_t)(ctx->lds_per_block / 2), floor_slots = std::max(longest, 256u);
     s.slot_cap = want;
     while (s.slot_cap > floor_slots && JoinLds(s.index_bits, s.slot_cap, c->narrow).total > half) s.slot_cap -= 64;
-    s.pair = s.slot_cap >= floor_slots && JoinLds(s.index_bits, s.slot_cap, c->narrow).total <= half;
+    s.pair = s.slot_cap >= floor_slots && JoinLds(s.index_bits, s.slot_cap, c->narrow).total <= half &&
+             (!c->narrow || (uint64_t)s.slot_cap * c->n >= 4 * c->total_pairs);
     if (!s.pair) s.slot_cap = std::min<uint32_t>(want, (uint32_t)APOE_JOIN_MAX_ROW_TERMS);
     s.lds = JoinLds(s.index_bits, s.slot_cap, c->narrow).total;
     return s;

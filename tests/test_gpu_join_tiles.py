@@ -95,3 +95,25 @@ def test_a_row_that_takes_the_whole_table(gpu_ctx, shift, terms):
     ids[:, 0] = row  # every document picks the long row, and it is a column wherever it is not
     step_equals_oracle(gpu_ctx, gc, O.HybridSet(*arrays), ids, K)
     gc.close()
+
+
+@pytest.mark.parametrize("vocab,terms", [(30000, 300), (30000, 340), (30000, 700), (60000, 190), (60000, 215)])
+def test_rows_of_many_terms(gpu_ctx, vocab, terms):
+    """Rows on both sides of the line between two workgroups per CU, whose table holds four of them and more, and one."""
+    import apoe
+    import apoe_synth as S
+    import oracle as O
+    n, K = 600, 64
+    rng = np.random.default_rng(terms)
+    dense, _, _, _, b_off, b_idx, b_val = S.to_numpy(S.corpus(n, seed=5, device="cpu"))
+    cnt = np.maximum(1, terms - np.diff(b_off.astype(np.int64)) + rng.integers(-20, 21, n))
+    off = np.concatenate([[0], np.cumsum(cnt)]).astype(np.uint32)
+    idx = np.concatenate([np.sort(rng.choice(vocab, c, replace=False)) for c in cnt]).astype(np.uint32)
+    idx[0] = 0
+    idx[off[1] - 1] = vocab - 1
+    arrays = (dense, off, idx, rng.uniform(0.1, 1.0, len(idx)).astype(np.float32), b_off, b_idx, b_val)
+    gc = apoe.Corpus(gpu_ctx, *arrays)
+    assert gc.pair_bytes() == 6
+    ids = np.stack([rng.choice(n, K, replace=False) for _ in range(n)]).astype(np.uint32)
+    step_equals_oracle(gpu_ctx, gc, O.HybridSet(*arrays), ids, K)
+    gc.close()
