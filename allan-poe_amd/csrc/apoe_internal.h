@@ -207,7 +207,8 @@ int launch_nnd_init(apoe_knn* g, uint64_t seed);
 int launch_nnd_iterate(apoe_knn* g, uint64_t* inserted);
 int launch_nnd_join_iterate(apoe_knn* g);
 int join_step_finish(apoe_knn* g, unsigned long long* unfit);
-int launch_gram_tiles(apoe_knn* g, const uint32_t* nodes, uint32_t node0, uint32_t n_nodes, float* gram, unsigned long long* unfit);
+int gram_tiles_pair(apoe_knn* g, const uint32_t* nodes, uint32_t n_nodes, bool* pair);
+int launch_gram_tiles(apoe_knn* g, const uint32_t* nodes, uint32_t node0, uint32_t n_nodes, bool pair, float* gram, unsigned long long* unfit);
 bool gram_tiles_fit(const apoe_knn* g);
 int launch_nnd_merge_reverse(apoe_knn* g);
 int launch_prune(apoe_knn* g, uint32_t degree);

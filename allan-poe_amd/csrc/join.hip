@@ -40,7 +40,7 @@ constexpr int JT_COLS = 128;
 // tile, so neither workgroup lacks work. Builds of ten steps against one workgroup of sixteen waves (wide pairs: of eight) with the
 // columns' pairs in registers: 100 000 docs K = 64 145.2 -> 113.3 ms, 30 011 docs K = 128 97.3 -> 76.7 ms, 20 000 docs wide 54.5 ->
 // 37.4 ms, 300 000 docs of the i.i.d. corpus 299 -> 254 ms. A corpus whose longest row does not fit the table of the smaller LDS takes one
-// workgroup of sixteen waves per CU, and so does one whose rows are long (tile_shape).
+// workgroup of sixteen waves per CU (tile_shape), and so does one whose rows are long (join_shape, gram_tiles_pair).
 constexpr int JT_PAIR_THREADS = 512, JT_SOLO_THREADS = 1024;
 constexpr int JT_STRIDE = JT_COLS + 1;
 constexpr int JT_STAGE_DIMS = 256; // the picker rows are staged at least this many dimensions at a time
@@ -881,19 +881,15 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
     }
 }
 
-// Table of a tile, and whether two workgroups share a CU (half of its LDS each). The table then takes as many slots as fit, up to
-// eight rows of the longest kind: an average group of eight rows of 180 terms has 1 000 distinct ones, 1 280 slots fit beside a
-// bitmap for a vocabulary of 32 768. A group that exceeds them is done in halves; a corpus with a single row that does
-// would lose that row, so it takes the whole LDS. So does a narrow corpus of whose average rows the smaller table holds fewer than four: its groups
-// are pairs and single rows, each a build and a probe of every column. Eight steps on 12 000 docs, K = 64, two workgroups / one, by rows that the
-// smaller table holds: vocabulary 32 768 (1 332 slots) 7.6 rows 8.8 / 11.6 ms, 4.2 11.5 / 13.3, 4.0 10.7 / 10.4, 3.9 16.3 / 14.6, 3.1 18.5 / 16.7,
-// 1.6 74.7 / 45.3; 65 536 (820 slots) 4.7 10.6 / 12.1, 4.1 12.2 / 12.1, 3.6 12.6 / 12.0, 3.1 17.6 / 13.3. Wide corpora, whose builds and probes
-// wait longer, gain from the second workgroup at any length (7.5 rows 16.0 / 20.8 ms, 1.6 198 / 235).
+// Table of a tile, and whether two workgroups share a CU (`pair`, where a row fits the table beside half of the LDS). The table then takes as many slots
+// as fit, up to eight rows of the longest kind: an average group of eight rows of 180 terms has 1 000 distinct ones, 1 332 slots fit beside a
+// bitmap for a vocabulary of 32 768. A group that exceeds them is done in halves; a corpus with a single row that does would lose that row, so it takes
+// the whole LDS.
 struct TileShape {
     uint32_t index_bits, slot_cap, span, lds;
     bool pair;
 };
-static TileShape tile_shape(const apoe_ctx* ctx, const apoe_corpus* c) {
+static TileShape tile_shape(const apoe_ctx* ctx, const apoe_corpus* c, bool pair) {
     TileShape s;
     s.span = next_pow2(std::max(c->max_term + 1, 1024u));
     s.index_bits = c->narrow ? 2 * s.span : 65536u;
@@ -901,11 +897,19 @@ static TileShape tile_shape(const apoe_ctx* ctx, const apoe_corpus* c) {
     const uint32_t half = (uint32_t)(ctx->lds_per_block / 2), floor_slots = std::max(longest, 256u);
     s.slot_cap = want;
     while (s.slot_cap > floor_slots && JoinLds(s.index_bits, s.slot_cap, c->narrow).total > half) s.slot_cap -= 64;
-    s.pair = s.slot_cap >= floor_slots && JoinLds(s.index_bits, s.slot_cap, c->narrow).total <= half &&
-             (!c->narrow || (uint64_t)s.slot_cap * c->n >= 4 * c->total_pairs);
+    s.pair = pair && s.slot_cap >= floor_slots && JoinLds(s.index_bits, s.slot_cap, c->narrow).total <= half;
     if (!s.pair) s.slot_cap = std::min<uint32_t>(want, (uint32_t)APOE_JOIN_MAX_ROW_TERMS);
     s.lds = JoinLds(s.index_bits, s.slot_cap, c->narrow).total;
     return s;
+}
+// Of the join: also one workgroup for a narrow corpus of whose average rows the smaller table holds fewer than four: its groups
+// are pairs and single rows, each a build and a probe of every column. Eight steps on 12 000 docs, K = 64, two workgroups / one, by rows that the
+// smaller table holds: vocabulary 32 768 (1 332 slots) 7.6 rows 8.8 / 11.6 ms, 4.2 11.5 / 13.3, 4.0 10.7 / 10.4, 3.9 16.3 / 14.6, 3.1 18.5 / 16.7,
+// 1.6 74.7 / 45.3; 65 536 (820 slots) 4.7 10.6 / 12.1, 4.1 12.2 / 12.1, 3.6 12.6 / 12.0, 3.1 17.6 / 13.3. Wide corpora, whose builds and probes
+// wait longer, gain from the second workgroup at any length (7.5 rows 16.0 / 20.8 ms, 1.6 198 / 235).
+static TileShape join_shape(const apoe_ctx* ctx, const apoe_corpus* c) {
+    const TileShape s = tile_shape(ctx, c, true);
+    return s.pair && c->narrow && (uint64_t)s.slot_cap * c->n < 4 * c->total_pairs ? tile_shape(ctx, c, false) : s;
 }
 
 // A persistent grid of tile workgroups.
@@ -949,7 +953,7 @@ int launch_nnd_join_iterate(apoe_knn* g) {
     const bool k128 = g->K == 128;
     const uint32_t halves = g->K / 64;
     if (!g->prop.p) APOE_TRY(join_alloc(g));
-    const TileShape shape = tile_shape(ctx, g->corpus);
+    const TileShape shape = join_shape(ctx, g->corpus);
     APOE_REQUIRE(shape.lds <= ctx->lds_per_block, "the local-join tile needs %u bytes of LDS, a workgroup may have %zu", shape.lds, ctx->lds_per_block);
 
     APOE_HIP(hipMemsetAsync(g->counter.p, 0, sizeof(unsigned long long), st)); // the inserted entries; the counts behind them run over the build
@@ -1005,14 +1009,79 @@ int launch_nnd_join_iterate(apoe_knn* g) {
     return APOE_OK;
 }
 
-// Gram matrices (upper triangles) of the lists of nodes[node0 .. node0 + n_nodes) into gram[n_nodes][128][128]. *unfit = rows
+// Whether two workgroups of the Gram tiles share a CU. Their tiles are full: a column is probed once for every eight rows, or for every four or two where the
+// distinct terms of eight exceed the table, and rows of one length may do either. So the terms of a few nodes' rows are counted: two workgroups where
+// their smaller table does not cost more than an eighth more probes than the whole LDS would. K = 128 prune of 12 000 docs, every node open, two workgroups / one:
+// rows of 179 terms, eight with 984 distinct ones (920 .. 1 032; tables of 1 332 and 2 304) 10.8 / 11.8 ms, 174 with 1 325 (1 305 .. 1 348) 14.4 / 13.3,
+// 252 with 1 365 16.9 / 14.3, 315 (four at a time in either) 18.8 / 19.7. Wide corpora gain at any length (29.8 / 60.5, 843 terms 498 / 967).
+constexpr uint32_t GRAM_SAMPLE = 64; // nodes
+__global__ __launch_bounds__(256) void gram_sample_kernel(GramTileArgs a, uint4* terms) { // terms[i] = distinct terms of the first one, two, four and eight rows of a node
+    extern __shared__ uint32_t bits[];
+    __shared__ uint32_t rows[RT_T], count, found[4];
+    const uint32_t u = a.nodes[(uint64_t)blockIdx.x * a.n_nodes / gridDim.x];
+    for (uint32_t w = threadIdx.x; w < a.index_bits / 32; w += 256) bits[w] = 0;
+    if (threadIdx.x < 4) found[threadIdx.x] = 0;
+    if (threadIdx.x == 0) {
+        uint32_t m = 0;
+        for (uint32_t i = 0; i < a.K && m < (uint32_t)RT_T; i++) {
+            const uint32_t v = a.ids[(size_t)u * a.K + i] & ~FLAG;
+            if (a.dist[(size_t)u * a.K + i] < INF_DIS && v < a.C.n && v != u) rows[m++] = v;
+        }
+        count = m;
+    }
+    __syncthreads();
+    for (uint32_t r = 0; r < count; r++) {
+        const uint64_t d = a.C.desc[rows[r]];
+        const Pairs sp = record_pairs(a.C, d);
+        uint32_t fresh = 0;
+        for (uint32_t j = threadIdx.x; j < sp.nnz; j += 256) {
+            const uint32_t x = sp.raw(j).x + (j >= sp.ns ? a.span : 0u), bit = 1u << (x & 31);
+            fresh += (atomicOr(&bits[x >> 5], bit) & bit) == 0;
+        }
+        if (fresh) atomicAdd(&found[r == 0 ? 0 : r < 2 ? 1 : r < 4 ? 2 : 3], fresh);
+        __syncthreads(); // a term belongs to the first row that holds it
+    }
+    if (threadIdx.x == 0) terms[blockIdx.x] = make_uint4(found[0], found[0] + found[1], found[0] + found[1] + found[2], found[0] + found[1] + found[2] + found[3]);
+}
+int gram_tiles_pair(apoe_knn* g, const uint32_t* nodes, uint32_t n_nodes, bool* pair) {
+    apoe_ctx* ctx = g->ctx;
+    const TileShape two = tile_shape(ctx, g->corpus, true), one = tile_shape(ctx, g->corpus, false);
+    *pair = two.pair;
+    if (!two.pair || !g->corpus->narrow) return APOE_OK;
+    if (!g->join_work.p) APOE_TRY(g->join_work.alloc(JOIN_COUNT_AT + JOIN_COUNT_PARTS * 8));
+    GramTileArgs a{};
+    a.C = g->corpus->view();
+    a.K = g->K;
+    a.n_nodes = n_nodes;
+    a.nodes = nodes;
+    a.ids = g->ids.p;
+    a.dist = g->dist.p;
+    a.index_bits = two.index_bits;
+    a.span = two.span;
+    const uint32_t sample = std::min(n_nodes, GRAM_SAMPLE);
+    static_assert(JOIN_COUNT_AT % 2 == 0 && JOIN_COUNT_PARTS * 8 >= 2 * (int)GRAM_SAMPLE, "the step's partial counters hold the sample");
+    uint4 *terms = reinterpret_cast<uint4*>(g->join_work.p + JOIN_COUNT_AT), h[GRAM_SAMPLE];
+    gram_sample_kernel<<<sample, 256, two.index_bits / 8, ctx->stream>>>(a, terms);
+    APOE_HIP(hipGetLastError());
+    APOE_HIP(hipMemcpyAsync(h, terms, sample * sizeof(uint4), hipMemcpyDeviceToHost, ctx->stream));
+    APOE_HIP(hipStreamSynchronize(ctx->stream));
+    auto probes = [&](uint32_t slots) { // of a column by eight rows, summed over the sample
+        uint32_t n = 0;
+        for (uint32_t i = 0; i < sample; i++) n += h[i].w <= slots ? 1 : h[i].z <= slots ? 2 : h[i].y <= slots ? 4 : 8;
+        return n;
+    };
+    *pair = 8 * probes(two.slot_cap) <= 9 * probes(one.slot_cap);
+    return APOE_OK;
+}
+
+// Gram matrices (upper triangles) of the lists of nodes[node0 .. node0 + n_nodes) (pair: gram_tiles_pair) into gram[n_nodes][128][128]. *unfit = rows
 // whose sparse terms did not fit the tile's table (their products lack the sparse part: the caller must not use the result).
-int launch_gram_tiles(apoe_knn* g, const uint32_t* nodes, uint32_t node0, uint32_t n_nodes, float* gram, unsigned long long* unfit) {
+int launch_gram_tiles(apoe_knn* g, const uint32_t* nodes, uint32_t node0, uint32_t n_nodes, bool pair, float* gram, unsigned long long* unfit) {
     apoe_ctx* ctx = g->ctx;
     hipStream_t st = ctx->stream;
     APOE_REQUIRE(g->K <= GT_MAX, "Gram tiles are built for lists of at most %u entries", GT_MAX);
     if (!g->join_work.p) APOE_TRY(g->join_work.alloc(JOIN_COUNT_AT + JOIN_COUNT_PARTS * 8));
-    const TileShape shape = tile_shape(ctx, g->corpus);
+    const TileShape shape = tile_shape(ctx, g->corpus, pair);
     APOE_REQUIRE(shape.lds <= ctx->lds_per_block, "a Gram tile needs %u bytes of LDS, a workgroup may have %zu", shape.lds, ctx->lds_per_block);
     fill_u64_kernel<<<1, 64, 0, st>>>(g->join_work.p, 8, 0ull);
     APOE_HIP(hipGetLastError());
@@ -1048,7 +1117,7 @@ int launch_gram_tiles(apoe_knn* g, const uint32_t* nodes, uint32_t node0, uint32
 // Whether launch_gram_tiles can serve this handle: lists of at most 128 entries, rows that fit a tile's table, LDS for a tile.
 bool gram_tiles_fit(const apoe_knn* g) {
     if (g->K > GT_MAX || g->corpus->max_nnz_s + g->corpus->max_nnz_b > (uint32_t)APOE_JOIN_MAX_ROW_TERMS) return false;
-    return tile_shape(g->ctx, g->corpus).lds <= g->ctx->lds_per_block;
+    return tile_shape(g->ctx, g->corpus, false).lds <= g->ctx->lds_per_block;
 }
 
 // How many rows did not fit the table in the last step (waits for it). Notes whether the lists have settled: less than a twelfth

@@ -1998,9 +1998,11 @@ int launch_prune(apoe_knn* g, uint32_t degree) {
             APOE_TRY(gram.alloc((size_t)batch * PS_MAX * PS_MAX));
             APOE_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&prune_select_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)SL.total));
             unsigned long long unfit = 0;
+            bool pair = false;
+            APOE_TRY(gram_tiles_pair(g, left.open_nodes, left.open, &pair));
             for (uint32_t node0 = 0; node0 < left.open && !unfit; node0 += batch) {
                 const uint32_t cnt = std::min(batch, left.open - node0);
-                APOE_TRY(launch_gram_tiles(g, left.open_nodes, node0, cnt, gram.p, &unfit));
+                APOE_TRY(launch_gram_tiles(g, left.open_nodes, node0, cnt, pair, gram.p, &unfit));
                 if (unfit) break;
                 prune_select_kernel<<<cnt, PS_THREADS, SL.total, ctx->stream>>>(g->corpus->view(), g->norms.p, g->K, g->ids.p, g->dist.p, degree, left.open_nodes, node0, gram.p,
                                                                               g->fwd.p, g->det.p, g->cnt.p, g->kw.p, uset_slots, map_slots, words);
