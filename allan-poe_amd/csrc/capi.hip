@@ -262,13 +262,18 @@ int apoe_corpus_create_without(apoe_ctx* ctx, uint32_t without, uint32_t n, uint
         c->max_term = max_term;
         std::vector<uint64_t> desc(n);
         const bool codes = c->narrow && !(without & APOE_WITHOUT_CODES);
-        uint64_t off16 = 0, with_codes = 0;
-        for (uint32_t i = 0; i < n; i++) {
-            const uint32_t ns = hs[i + 1] - hs[i], nb = hb[i + 1] - hb[i];
-            desc[i] = make_desc(codes ? with_codes : off16, ns, nb);
-            off16 += record_units(ns + nb, c->narrow, false);
-            with_codes += record_units(ns + nb, c->narrow, codes);
-        }
+        auto place = [&](bool coded) { // the records one behind the other; returns their 16-byte units
+            uint64_t at = 0;
+            for (uint32_t i = 0; i < n; i++) {
+                const uint32_t ns = hs[i + 1] - hs[i], nb = hb[i + 1] - hb[i];
+                desc[i] = make_desc(at, ns, nb);
+                at += record_units(ns + nb, c->narrow, coded);
+            }
+            return at;
+        };
+        uint64_t off16 = 0; // without codes
+        for (uint32_t i = 0; i < n; i++) off16 += record_units(hs[i + 1] - hs[i] + hb[i + 1] - hb[i], c->narrow, false);
+        const uint64_t with_codes = codes ? place(true) : 0;
         APOE_REQUIRE(off16 < (1ull << DESC_OFF_BITS), "corpus of %llu bytes exceeds the record address range", (unsigned long long)off16 * 16);
         c->rec_bytes = off16 * 16;
         c->total_pairs = (uint64_t)hs[n] + hb[n];
@@ -282,14 +287,7 @@ int apoe_corpus_create_without(apoe_ctx* ctx, uint32_t without, uint32_t n, uint
             c->coded = with_codes < (1ull << DESC_OFF_BITS) && with_codes * 16 <= free_now / 4 && c->recs.try_alloc(with_codes * 16 + ROW_LOAD_SLACK);
         }
         if (!c->coded) {
-            if (codes) {
-                off16 = 0;
-                for (uint32_t i = 0; i < n; i++) {
-                    const uint32_t ns = hs[i + 1] - hs[i], nb = hb[i + 1] - hb[i];
-                    desc[i] = make_desc(off16, ns, nb);
-                    off16 += record_units(ns + nb, true, false);
-                }
-            }
+            place(false);
             APOE_TRY(c->recs.alloc(c->rec_bytes + ROW_LOAD_SLACK)); // unclamped row loads may read past the last record
         }
         APOE_TRY(c->dnorm.alloc(n));
@@ -309,7 +307,7 @@ int apoe_corpus_create_without(apoe_ctx* ctx, uint32_t without, uint32_t n, uint
         APOE_TRY(launch_pack(ctx, n, d_dense.p, d_soff.p, d_sidx.p, d_sval.p, d_boff.p, d_bidx.p, d_bval.p, c->desc.p, c->recs.p, c->dnorm.p,
                              c->sketch_meta.p, c->sketch.p, c->narrow, c->coded));
         if (c->coded) { // what tells a search whether the codes pay
-            const uint32_t sample = std::min(n, 4096u);
+            const uint32_t sample = std::min(n, 4 * ROW_SCALE_PARTS);
             float sums[3 * ROW_SCALE_PARTS];
             APOE_TRY(launch_row_scale(ctx, n, sample, d_dense.p, d_soff.p, d_sval.p, d_boff.p, d_bval.p, reinterpret_cast<float*>(d_max.p + 1)));
             APOE_TRY(copy_out(ctx, sums, d_max.p + 1, sizeof(sums)));

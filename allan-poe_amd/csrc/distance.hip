@@ -34,14 +34,34 @@ __global__ __launch_bounds__(256) void pack_kernel(uint32_t n, const float* __re
         const float4* src = reinterpret_cast<const float4*>(dense + (size_t)doc * DIM);
         float4* dst = reinterpret_cast<float4*>(rec);
         static_assert(DIM / 4 == 256, "a thread per float4 of the dense row");
+        const uint32_t s0 = s_off[doc], ns = desc_nnz_s(d), b0 = b_off[doc], nb = desc_nnz_b(d), nnz = ns + nb;
         const float4 x = src[threadIdx.x];
+        // a pair per thread, requested with the dense row (narrow records; rows of more than 256 pairs read the rest below)
+        auto value = [&](uint32_t j) { return j < ns ? s_val[s0 + j] : b_val[b0 + (j - ns)]; };
+        auto term = [&](uint32_t j) { return j < ns ? s_idx[s0 + j] : b_idx[b0 + (j - ns)]; };
+        float v = 0.f;
+        uint32_t id = 0;
+        if (narrow && threadIdx.x < nnz) {
+            v = value(threadIdx.x);
+            id = term(threadIdx.x);
+        }
         dst[threadIdx.x] = x;
         const float sq = wave_sum_dpp(x.x * x.x + x.y * x.y + x.z * x.z + x.w * x.w);
         const float high = -wave_min_dpp(-max_abs4(x));
+        float largest[2] = {0.f, 0.f}; // magnitude per path; a value that is no number counts as infinite
+        if (coded) {
+            auto raise = [&](uint32_t j, float y) { float& to = largest[j < ns ? 0 : 1]; to = y == y ? fmaxf(to, fabsf(y)) : __builtin_inff(); };
+            if (threadIdx.x < nnz) raise(threadIdx.x, v);
+            for (uint32_t j = threadIdx.x + 256; j < nnz; j += 256) raise(j, value(j));
+            largest[0] = -wave_min_dpp(-largest[0]);
+            largest[1] = -wave_min_dpp(-largest[1]);
+        }
         __syncthreads();
         if (lane_id() == 0) {
             part[threadIdx.x / WAVE] = sq;
             top[threadIdx.x / WAVE] = high;
+            most[0][threadIdx.x / WAVE] = largest[0];
+            most[1][threadIdx.x / WAVE] = largest[1];
         }
         __syncthreads();
         const float norm = sqrtf(part[0] + part[1] + part[2] + part[3]);
@@ -57,47 +77,35 @@ __global__ __launch_bounds__(256) void pack_kernel(uint32_t n, const float* __re
             const float err = norm < __builtin_inff() && peak < 65504.f ? 1.0001f * sqrtf(rest[0] + rest[1] + rest[2] + rest[3]) : __builtin_inff();
             if (sketch) sketch_meta[doc] = SketchMeta{scale, err};
         }
-        const uint32_t s0 = s_off[doc], ns = desc_nnz_s(d), b0 = b_off[doc], nb = desc_nnz_b(d), nnz = ns + nb;
         if (narrow) {
             float* vals = reinterpret_cast<float*>(rec + DENSE_BYTES);
             uint16_t* keys = reinterpret_cast<uint16_t*>(rec + DENSE_BYTES + narrow_keys_offset(nnz));
-            for (uint32_t j = threadIdx.x; j < ns; j += blockDim.x) {
-                vals[j] = s_val[s0 + j];
-                keys[j] = (uint16_t)s_idx[s0 + j];
+            signed char* codes = reinterpret_cast<signed char*>(rec + DENSE_BYTES + codes_offset(nnz));
+            float per[2], step[2];
+#pragma unroll
+            for (int p = 0; p < 2; p++) {
+                const float m = fmaxf(fmaxf(most[p][0], most[p][1]), fmaxf(most[p][2], most[p][3]));
+                const bool usable = m > 1e-30f; // below, half a step of 2e-30 covers the value
+                per[p] = usable ? 127.f / m : 0.f;
+                step[p] = usable ? m / 127.f : m > 0.f ? 2e-30f : 0.f;
             }
-            for (uint32_t j = threadIdx.x; j < nb; j += blockDim.x) {
-                vals[ns + j] = b_val[b0 + j];
-                keys[ns + j] = (uint16_t)b_idx[b0 + j];
-            }
+            auto put = [&](uint32_t j, float y, uint32_t key) {
+                vals[j] = y;
+                keys[j] = (uint16_t)key;
+                if (coded) codes[j] = (signed char)sketch_code(y, j < ns ? per[0] : per[1]);
+            };
+            if (threadIdx.x < nnz) put(threadIdx.x, v, id);
+            for (uint32_t j = threadIdx.x + 256; j < nnz; j += 256) put(j, value(j), term(j));
             // fill the alignment gaps so that a record never holds stale bytes
-            for (uint32_t j = nnz + threadIdx.x; j < narrow_keys_offset(nnz) / 4; j += blockDim.x) vals[j] = 0.f;
+            for (uint32_t j = nnz + threadIdx.x; j < narrow_keys_offset(nnz) / 4; j += 256) vals[j] = 0.f;
             const uint32_t end = (uint32_t)(record_units(nnz, true, coded) * 16 - DENSE_BYTES);
             if (!coded) {
-                for (uint32_t j = nnz + threadIdx.x; j < (end - narrow_keys_offset(nnz)) / 2; j += blockDim.x) keys[j] = 0xFFFFu;
+                for (uint32_t j = nnz + threadIdx.x; j < (end - narrow_keys_offset(nnz)) / 2; j += 256) keys[j] = 0xFFFFu;
             } else {
-                float high[2] = {0.f, 0.f}; // largest magnitude per path; a value that is no number counts as infinite
-                auto raise = [](float& to, float v) { to = v == v ? fmaxf(to, fabsf(v)) : __builtin_inff(); };
-                for (uint32_t j = threadIdx.x; j < ns; j += blockDim.x) raise(high[0], s_val[s0 + j]);
-                for (uint32_t j = threadIdx.x; j < nb; j += blockDim.x) raise(high[1], b_val[b0 + j]);
-                for (int p = 0; p < 2; p++) {
-                    const float m = -wave_min_dpp(-high[p]);
-                    if (lane_id() == 0) most[p][threadIdx.x / WAVE] = m; // last read before the barriers at the next document's start
-                }
-                __syncthreads();
-                float per[2], step[2];
-                for (int p = 0; p < 2; p++) {
-                    const float m = fmaxf(fmaxf(most[p][0], most[p][1]), fmaxf(most[p][2], most[p][3]));
-                    const bool usable = m > 1e-30f; // below, half a step of 2e-30 covers the value
-                    per[p] = usable ? 127.f / m : 0.f;
-                    step[p] = usable ? m / 127.f : m > 0.f ? 2e-30f : 0.f;
-                }
-                signed char* codes = reinterpret_cast<signed char*>(rec + DENSE_BYTES + codes_offset(nnz));
-                for (uint32_t j = threadIdx.x; j < ns; j += blockDim.x) codes[j] = (signed char)sketch_code(s_val[s0 + j], per[0]);
-                for (uint32_t j = threadIdx.x; j < nb; j += blockDim.x) codes[ns + j] = (signed char)sketch_code(b_val[b0 + j], per[1]);
                 const uint32_t scales = code_scales_offset(nnz);
-                if (threadIdx.x < 2) reinterpret_cast<float*>(rec + DENSE_BYTES + scales)[threadIdx.x] = step[threadIdx.x];
+                if (threadIdx.x < 2) reinterpret_cast<float*>(rec + DENSE_BYTES + scales)[threadIdx.x] = threadIdx.x ? step[1] : step[0];
                 if (threadIdx.x < scales - codes_offset(nnz) - nnz) codes[nnz + threadIdx.x] = 0;
-                for (uint32_t j = scales + 8 + 4 * threadIdx.x; j < end; j += 4 * blockDim.x) *reinterpret_cast<uint32_t*>(rec + DENSE_BYTES + j) = ~0u;
+                for (uint32_t j = scales + 8 + 4 * threadIdx.x; j < end; j += 4 * 256) *reinterpret_cast<uint32_t*>(rec + DENSE_BYTES + j) = ~0u;
             }
         } else {
             uint2* sp = reinterpret_cast<uint2*>(rec + DENSE_BYTES);
