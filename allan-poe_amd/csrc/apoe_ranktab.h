@@ -410,42 +410,11 @@ __device__ __forceinline__ void ranktab_probe_rows(const RankTab& T, const RtRow
     }
 }
 
-// The wave totals of 2 streamed rows x 8 pivots from the per-lane accumulators of ranktab_probe_rows<., 2>. The two
-// halves of the pivots (0-3, 4-7) of each row are reduced inside every 16-lane row of the wave like four sums at once
-// (two exchange-and-add steps inside each quad leave lane l with pivot t(l) = 2 * (l & 1) + ((l >> 1) & 1) of its half,
-// then two rotations inside the 16 lanes); the four 16-lane rows of the wave then share out the four (streamed row,
-// half) combinations between them with three cross-row exchanges. Returns the total of streamed row *r_out, pivot *t_out.
-__device__ __forceinline__ float wave_sum_2x8(const float (&acc)[2][RT_T], int lane, uint32_t* t_out, uint32_t* r_out) {
-    float z[4]; // (row 0, low half), (row 0, high half), (row 1, low), (row 1, high)
-    const bool odd = lane & 1, hi = lane & 2;
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-        const float* a = &acc[k >> 1][4 * (k & 1)];
-        const float keep0 = odd ? a[2] : a[0], keep1 = odd ? a[3] : a[1];
-        const float give0 = odd ? a[0] : a[2], give1 = odd ? a[1] : a[3];
-        const float x0 = keep0 + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, give0), 0xB1, 0xF, 0xF, false));
-        const float x1 = keep1 + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, give1), 0xB1, 0xF, 0xF, false));
-        const float keep = hi ? x1 : x0, give = hi ? x0 : x1;
-        float y = keep + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, give), 0x4E, 0xF, 0xF, false));
-        y += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, y), 0x124, 0xF, 0xF, false)); // row_ror:4
-        y += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, y), 0x128, 0xF, 0xF, false)); // row_ror:8
-        z[k] = y;
-    }
-    const bool q0 = lane & 16, q1 = lane & 32;
-    const float keepA0 = q0 ? z[2] : z[0], giveA0 = q0 ? z[0] : z[2];
-    const float keepA1 = q0 ? z[3] : z[1], giveA1 = q0 ? z[1] : z[3];
-    const float xa = keepA0 + __shfl_xor(giveA0, 16, WAVE);
-    const float xb = keepA1 + __shfl_xor(giveA1, 16, WAVE);
-    const float keepB = q1 ? xb : xa, giveB = q1 ? xa : xb;
-    // 16-lane row q of the wave now holds combination k(q) = 2 * (q & 1) + (q >> 1): streamed row k >> 1, half k & 1
-    const uint32_t k = 2u * ((lane >> 4) & 1) + ((lane >> 5) & 1);
-    *r_out = k >> 1;
-    *t_out = 4u * (k & 1) + 2u * (lane & 1) + ((lane >> 1) & 1);
-    return keepB + __shfl_xor(giveB, 32, WAVE);
-}
-
-// The wave totals of one streamed row x 8 pivots from the per-lane accumulators of ranktab_probe_rows<., 1>: as
-// wave_sum_2x8 with two (low half, high half) instead of four combinations. Returns the total of pivot *t_out.
+// The wave totals of one streamed row x 8 pivots from the per-lane accumulators of ranktab_probe_rows<., 1>. The two
+// halves of the pivots (0-3, 4-7) are reduced inside every 16-lane row of the wave like four sums at once (two
+// exchange-and-add steps inside each quad leave lane l with pivot t(l) = 2 * (l & 1) + ((l >> 1) & 1) of its half, then
+// two rotations inside the 16 lanes); two cross-row exchanges then add up the rows of the wave, even ones the low half and
+// odd ones the high half. Returns the total of pivot *t_out.
 __device__ __forceinline__ float wave_sum_1x8(const float (&acc)[RT_T], int lane, uint32_t* t_out) {
     float z[2];
     const bool odd = lane & 1, hi = lane & 2;
