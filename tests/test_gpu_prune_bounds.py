@@ -42,6 +42,29 @@ def make(kind, wide):
     return tuple(a)
 
 
+def equal_but_for_ties(arrays, scale, ids, dist, got, want):
+    """All outputs of every node, but for nodes with a pair of neighbours whose product lies within the rounding of an fp32 sum of one
+    of their norms (1e-5 of what the parts of either can reach, as the kernels' own room); few nodes at most."""
+    import apoe
+    from scipy.sparse import csr_matrix
+    differ = np.flatnonzero(~np.logical_and.reduce([(g == w).reshape(len(ids), -1).all(axis=1) for g, w in zip(got, want)]))
+    dense, *pairs = arrays
+    for u in differ:
+        near = ids[u][(dist[u] < apoe.INF_DIS) & (ids[u] != u)]
+        d = dense[near].astype(np.float64) * scale
+        prod, reach = d @ d.T, np.outer(*2 * [np.linalg.norm(d, axis=1)])
+        with np.errstate(invalid="ignore"):
+            sq = 0.0
+            for off, idx, val in (pairs[:3], pairs[3:]):
+                m = csr_matrix((val.astype(np.float64), idx.astype(np.int64), off.astype(np.int64)), (len(dense), int(idx.max()) + 1))[near]
+                prod = prod + (m @ m.T).toarray()
+                sq = sq + np.asarray(m.multiply(m).sum(axis=1)).ravel()
+            reach = reach + np.sqrt(np.outer(sq, sq)) + 1.0
+            tie = np.abs(prod - np.diag(prod)) <= 1e-5 * reach
+        assert (tie & ~np.eye(len(near), dtype=bool)).any(), (u, [(g[u], w[u]) for g, w in zip(got, want)])
+    assert len(differ) <= 0.005 * len(ids), differ
+
+
 def check(gpu_ctx, kind, K, degree, wide, without=0):
     import apoe
     import oracle as O
@@ -59,10 +82,7 @@ def check(gpu_ctx, kind, K, degree, wide, without=0):
     knn.close()
     gc.close()
     c_fwd, c_det, c_cnt, c_kw = O.prune(C, 7.0, O.norms(C, 7.0), ids, dist, degree)
-    same = np.all(g_fwd == c_fwd, axis=1)
-    assert same.mean() >= 0.995, np.flatnonzero(~same)[:10]  # a product that rounds to either side of a norm
-    assert np.array_equal(g_det[same], c_det[same]) and np.array_equal(g_cnt[same], c_cnt[same])
-    assert np.all(g_kw == c_kw, axis=1)[same].mean() >= 0.995
+    equal_but_for_ties(arrays, 7.0, ids, dist, (g_fwd, g_det, g_cnt, g_kw), (c_fwd, c_det, c_cnt, c_kw))
     if kind == "near twins":
         assert np.any(c_cnt < min(degree, K - 1))  # the rule does reject here
 
