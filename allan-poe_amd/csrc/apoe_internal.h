@@ -177,7 +177,7 @@ struct apoe_knn {
     apoe::DevBuf<char> scan_tmp;
     // prune outputs
     apoe::DevBuf<uint32_t> fwd, det, cnt, kw;
-    apoe::DevBuf<uint32_t> open; // prune: which nodes the bounds left open [n], how many, and which
+    apoe::DevBuf<uint32_t> open; // prune: what a node leaves to another form [n], how many are left to either, and which [n]
 };
 
 namespace apoe {
