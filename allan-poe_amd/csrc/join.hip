@@ -235,15 +235,16 @@ __device__ __forceinline__ Pairs tile_pairs(const char* recs, const unsigned lon
 // eight rows in the rank table, every column probes it once per group. All threads of the workgroup call it after a barrier behind
 // those arrays; it ends with a barrier. `unfit` = counter of rows whose terms did not fit the table.
 // The pairs of a group's rows are requested while the group before it is probed, those of a wave's columns TILE_AHEAD columns ahead
-// (a tile has one group in most cases: with the columns held in registers for all groups a wave needs 96 of them and a CU holds
-// one workgroup only). A group of at most four pivots (an average tile of a 100 000-document build has five) reads one plane of
+// (a tile of the join has one group in most cases: with the columns held in registers for all groups a wave needs 96 of them and a CU holds
+// one workgroup only; HOLD does that for the full tiles of a Gram matrix where it is so: K = 128 prune of 12 000 docs, 360 terms a row 17.7 -> 16.5 ms). A group of at most four pivots (an average tile of a 100 000-document build has five) reads one plane of
 // the table; with the rows' lists looked up among the columns instead of sorted and searched, the tenth step of that build
 // went from 6.33 to 5.91 ms.
 // `meanwhile` runs once the first loads are on their way; it may use the table region and has to leave it behind a barrier.
-template <bool NARROW, int NT, typename Meanwhile>
+template <bool NARROW, int NT, bool HOLD, typename Meanwhile>
 __device__ __forceinline__ void tile_sparse(const char* recs, const RankTab& T, float* G, const unsigned long long* rowptr, const uint32_t* rownnz, uint32_t* scan, uint32_t R,
                                             uint32_t M, unsigned long long* unfit, int tid, int wave, int lane, Meanwhile meanwhile) {
-    constexpr int NW = NT / WAVE, TILE_AHEAD = NARROW ? 3 : 2;
+    constexpr int NW = NT / WAVE, TILE_AHEAD = HOLD ? JT_COLS / NW : NARROW ? 3 : 2;
+    constexpr int BATCH = HOLD && NW == 8 ? 2 : 1; // columns a wave probes together: with two waves per SIMD one at a time leaves waits uncovered
     static_assert(NW >= RT_T, "a wave per pivot of a group");
     auto row_pairs = [&](uint32_t i) { return tile_pairs<NARROW>(recs, rowptr, rownnz, i); };
     auto col_pairs = [&](uint32_t b) { return tile_pairs<NARROW>(recs, rowptr, rownnz, JT_ROWS + b); };
@@ -293,28 +294,39 @@ __device__ __forceinline__ void tile_sparse(const char* recs, const RankTab& T, 
             constexpr int NP = decltype(pivots)::value;
             for (uint32_t b0 = wave; b0 < M; b0 += TILE_AHEAD * NW) {
 #pragma unroll
-                for (int s = 0; s < TILE_AHEAD; s++) {
+                for (int s = 0; s < TILE_AHEAD; s += BATCH) {
                     const uint32_t b = b0 + s * NW;
-                    if (b < M) { // wave-uniform
-                        float acc[1][NP];
-                        RtRow<NARROW> rows[1] = {col[s]};
-                        const uint32_t shape[1] = {col_shape[s]};
-                        const uint32_t next = b + TILE_AHEAD * NW;
-                        if (next < M) col_load(s, next);
-                        else if (a1 < R) col_load(s, wave + s * NW); // the first of the slot again, for the next group
+                    if (b < M) { // wave-uniform; a second column that is not there has no pairs
+                        float acc[BATCH][NP];
+                        RtRow<NARROW> rows[BATCH];
+                        uint32_t shape[BATCH];
 #pragma unroll
-                        for (int t = 0; t < NP; t++) acc[0][t] = 0.f;
-                        ranktab_probe_rows<NARROW, 1, NP>(T, rows, shape, [&](int) { return col_pairs(b); }, n_ovf, acc, lane);
-                        uint32_t t;
-                        if constexpr (NP == 4) {
-                            const float z = wave_sum4_dpp(acc[0], lane, &t);
-                            if (lane < 4 && t < nt) G[(a0 + t) * JT_STRIDE + b] = z;
-                        } else {
-                            const float z = wave_sum_1x8(acc[0], lane, &t);
-                            if ((lane & 15) < 4 && lane < 32 && t < nt) G[(a0 + t) * JT_STRIDE + b] = z;
+                        for (int k = 0; k < BATCH; k++) {
+                            rows[k] = col[s + k];
+                            shape[k] = col_shape[s + k];
+                            if constexpr (HOLD) { // what follows from a row is worked out where it is used, not kept for all groups
+                                rows[k].touch();
+                                asm volatile("" : "+s"(shape[k]));
+                            }
+#pragma unroll
+                            for (int t = 0; t < NP; t++) acc[k][t] = 0.f;
+                        }
+                        if constexpr (!HOLD) {
+                            const uint32_t next = b + TILE_AHEAD * NW;
+                            if (next < M) col_load(s, next);
+                            else if (a1 < R) col_load(s, wave + s * NW); // the first of the slot again, for the next group
+                        }
+                        ranktab_probe_rows<NARROW, BATCH, NP>(T, rows, shape, [&](int k) { return col_pairs(b + k * NW); }, n_ovf, acc, lane);
+#pragma unroll
+                        for (int k = 0; k < BATCH; k++) {
+                            uint32_t t;
+                            float z;
+                            if constexpr (NP == 4) z = wave_sum4_dpp(acc[k], lane, &t);
+                            else z = wave_sum_1x8(acc[k], lane, &t);
+                            if ((lane & 15) < 4 && lane < (NP == 4 ? 4 : 32) && t < nt && b + k * NW < M) G[(a0 + t) * JT_STRIDE + b + k * NW] = z;
                         }
                     }
-                    __builtin_amdgcn_sched_barrier(0); // one column at a time: the scheduler must not pile up the reads of all of them
+                    __builtin_amdgcn_sched_barrier(0); // one batch at a time: the scheduler must not pile up the reads of all of them
                 }
             }
         };
@@ -619,7 +631,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
         // before entered a list (join_step_finish).
         const bool settled = a.sketch != nullptr;
         TileBound bound = {};
-        tile_sparse<NARROW, NT>(a.C.recs, T, G, rowptr, rownnz, scan, R, M, a.work + 3, tid, wave, lane, [&]() {
+        tile_sparse<NARROW, NT, false>(a.C.recs, T, G, rowptr, rownnz, scan, R, M, a.work + 3, tid, wave, lane, [&]() {
             if (settled)
                 tile_sketch<NT>(a.sketch_meta, a.sketch, a.C.dnorm, a.dense_mul, reinterpret_cast<uint4*>(smem + L.tab), row_id, col_id, S, bound, R, M, tid,
                                 wave, lane);
@@ -819,8 +831,8 @@ struct GramTileArgs {
     uint32_t index_bits, slot_cap, span;
 };
 
-template <bool NARROW, int NT>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void gram_tile_kernel(GramTileArgs a) {
+template <bool NARROW, int NT, bool HOLD>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(HOLD ? NT / 256 : 4, HOLD ? NT / 256 : 4))) void gram_tile_kernel(GramTileArgs a) {
     a.C.narrow = NARROW ? 1u : 0u;
     extern __shared__ __align__(16) char smem[];
     const JoinLds L(a.index_bits, a.slot_cap, NARROW);
@@ -870,7 +882,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
             gram_rows_gather(a.C, row_id, R, rowptr, rownnz, tid, NT);
             gram_rows_gather(a.C, col_id, M, rowptr + JT_ROWS, rownnz + JT_ROWS, tid, NT);
             __syncthreads();
-            tile_sparse<NARROW, NT>(a.C.recs, T, G, rowptr, rownnz, scan, R, M, a.work + 3, tid, wave, lane, [] {});
+            tile_sparse<NARROW, NT, HOLD>(a.C.recs, T, G, rowptr, rownnz, scan, R, M, a.work + 3, tid, wave, lane, [] {});
             tile_dense<NT>(a.C.recs, a.dense_mul, smem + L.tab, L.tab_bytes, G, rowptr, nullptr, R, M, R, M, tid, wave, lane);
             for (uint32_t p = tid; p < R * M; p += NT) {
                 const uint32_t r = p / M, c = p % M;
@@ -914,8 +926,7 @@ static TileShape join_shape(const apoe_ctx* ctx, const apoe_corpus* c) {
 
 // A persistent grid of tile workgroups.
 template <typename Args>
-static int launch_tiles(apoe_ctx* ctx, void (*kernel)(Args), const TileShape& shape, const Args& a) {
-    const int threads = shape.pair ? JT_PAIR_THREADS : JT_SOLO_THREADS;
+static int launch_tiles(apoe_ctx* ctx, void (*kernel)(Args), const TileShape& shape, int threads, const Args& a) {
     APOE_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)shape.lds));
     int per_cu = 1;
     APOE_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(kernel), threads, shape.lds));
@@ -999,8 +1010,8 @@ int launch_nnd_join_iterate(apoe_knn* g) {
         return k128 ? (narrow ? &join_tile_kernel<true, 128, NT> : &join_tile_kernel<false, 128, NT>)
                     : (narrow ? &join_tile_kernel<true, 64, NT> : &join_tile_kernel<false, 64, NT>);
     };
-    APOE_TRY(launch_tiles(ctx, shape.pair ? kernel_of(std::integral_constant<int, JT_PAIR_THREADS>{}) : kernel_of(std::integral_constant<int, JT_SOLO_THREADS>{}),
-                          shape, a));
+    if (shape.pair) APOE_TRY(launch_tiles(ctx, kernel_of(std::integral_constant<int, JT_PAIR_THREADS>{}), shape, JT_PAIR_THREADS, a));
+    else APOE_TRY(launch_tiles(ctx, kernel_of(std::integral_constant<int, JT_SOLO_THREADS>{}), shape, JT_SOLO_THREADS, a));
     if (k128) join_apply_kernel<128><<<(n + 3) / 4, 256, 0, st>>>(n, g->ids.p, g->dist.p, g->prop.p, g->rev.p, g->rev_cnt.p, g->join_work.p + JOIN_COUNT_AT);
     else join_apply_kernel<64><<<(n + 3) / 4, 256, 0, st>>>(n, g->ids.p, g->dist.p, g->prop.p, g->rev.p, g->rev_cnt.p, g->join_work.p + JOIN_COUNT_AT);
     APOE_HIP(hipGetLastError());
@@ -1010,44 +1021,71 @@ int launch_nnd_join_iterate(apoe_knn* g) {
 }
 
 // Whether two workgroups of the Gram tiles share a CU. Their tiles are full: a column is probed once for every eight rows, or for every four or two where the
-// distinct terms of eight exceed the table, and rows of one length may do either. So the terms of a few nodes' rows are counted: two workgroups where
-// their smaller table does not cost more than an eighth more probes than the whole LDS would. K = 128 prune of 12 000 docs, every node open, two workgroups / one:
-// rows of 179 terms, eight with 984 distinct ones (920 .. 1 032; tables of 1 332 and 2 304) 10.8 / 11.8 ms, 174 with 1 325 (1 305 .. 1 348) 14.4 / 13.3,
-// 252 with 1 365 16.9 / 14.3, 315 (four at a time in either) 18.8 / 19.7. Wide corpora gain at any length (29.8 / 60.5, 843 terms 498 / 967).
+// terms of eight exceed the table, and rows of one length may do either. So the terms of a few nodes' rows are counted; a probe costs a fifth more for every
+// overflow entry (wide pairs: a term whose bit another one of the group has). Narrow corpora take two workgroups where that does not cost more than an eighth more
+// with their smaller table than with the whole LDS. Wide ones, whose builds and probes wait longer, up to twice as much, or half more where rows exceed the
+// registers (their tails are read again by every probe). K = 128 prune of 12 000 docs, every node open, ms with two workgroups / one, by the terms a row and their vocabulary:
+//   narrow: 180 of the synthetic corpora 10.8 / 12.1; uniform 180 of 30 000 14.1 / 12.0, 260 of 2 000 17.4 / 13.5; 360 of 2 000 23.1 / 16.0; 860 of 30 000 200 / 106
+//   wide:   180 25.5 / 41.8; 180 of 30 000 35.6 / 85.4; 860 of 30 000 508 / 1027; few terms a bit: 180 of 2 000 17.0 / 20.1, 260 of 2 000 22.5 / 25.0, 360 of 2 000
+//           45.2 / 32.9, 460 of 3 000 66.1 / 61.0, 560 of 1 500 82.9 / 48.9
 constexpr uint32_t GRAM_SAMPLE = 64; // nodes
-__global__ __launch_bounds__(256) void gram_sample_kernel(GramTileArgs a, uint4* terms) { // terms[i] = distinct terms of the first one, two, four and eight rows of a node
-    extern __shared__ uint32_t bits[];
-    __shared__ uint32_t rows[RT_T], count, found[4];
+constexpr uint32_t GRAM_COUNTED = 3072; // terms: more than any table holds
+struct GramSample {
+    uint32_t terms[4], shared[4]; // distinct terms of the first one, two, four and eight rows of a node, and how many of them find their bit taken
+};
+template <bool NARROW>
+__global__ __launch_bounds__(256) void gram_sample_kernel(GramTileArgs a, GramSample* out) {
+    constexpr uint32_t SLOTS = 4096;
+    static_assert(GRAM_COUNTED + 256 < SLOTS, "a free slot is left whatever the threads insert at once");
+    __shared__ uint32_t keys[SLOTS], bits[NARROW ? 1 : 65536 / 32], rows[RT_T], rows_n, n_terms, n_shared;
     const uint32_t u = a.nodes[(uint64_t)blockIdx.x * a.n_nodes / gridDim.x];
-    for (uint32_t w = threadIdx.x; w < a.index_bits / 32; w += 256) bits[w] = 0;
-    if (threadIdx.x < 4) found[threadIdx.x] = 0;
+    RankTab T{};
+    T.index_bits = a.index_bits;
+    T.span = a.span;
+    for (uint32_t i = threadIdx.x; i < SLOTS; i += 256) keys[i] = EMPTY;
+    for (uint32_t i = threadIdx.x; i < (NARROW ? 0u : a.index_bits / 32); i += 256) bits[i] = 0;
     if (threadIdx.x == 0) {
         uint32_t m = 0;
         for (uint32_t i = 0; i < a.K && m < (uint32_t)RT_T; i++) {
             const uint32_t v = a.ids[(size_t)u * a.K + i] & ~FLAG;
             if (a.dist[(size_t)u * a.K + i] < INF_DIS && v < a.C.n && v != u) rows[m++] = v;
         }
-        count = m;
+        rows_n = m;
+        n_terms = n_shared = 0;
     }
     __syncthreads();
-    for (uint32_t r = 0; r < count; r++) {
-        const uint64_t d = a.C.desc[rows[r]];
-        const Pairs sp = record_pairs(a.C, d);
-        uint32_t fresh = 0;
-        for (uint32_t j = threadIdx.x; j < sp.nnz; j += 256) {
-            const uint32_t x = sp.raw(j).x + (j >= sp.ns ? a.span : 0u), bit = 1u << (x & 31);
-            fresh += (atomicOr(&bits[x >> 5], bit) & bit) == 0;
+    for (uint32_t r = 0; r < (uint32_t)RT_T; r++) {
+        if (r < rows_n) {
+            const uint64_t d = a.C.desc[rows[r]];
+            const Pairs sp = record_pairs(a.C, d);
+            for (uint32_t j = threadIdx.x; j < sp.nnz && __hip_atomic_load(&n_terms, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) < GRAM_COUNTED; j += 256) {
+                const uint32_t raw = sp.raw(j).x, idx = ranktab_index<NARROW>(T, raw, j >= sp.ns), key = NARROW ? idx : raw;
+                uint32_t h = term_hash(key, SLOTS - 1);
+                while (true) {
+                    const uint32_t old = atomicCAS(&keys[h], EMPTY, key);
+                    if (old == key) break;
+                    if (old == EMPTY) {
+                        atomicAdd(&n_terms, 1u);
+                        if (!NARROW && (atomicOr(&bits[idx >> 5], 1u << (idx & 31)) >> (idx & 31) & 1u)) atomicAdd(&n_shared, 1u);
+                        break;
+                    }
+                    h = (h + 1) & (SLOTS - 1);
+                }
+            }
         }
-        if (fresh) atomicAdd(&found[r == 0 ? 0 : r < 2 ? 1 : r < 4 ? 2 : 3], fresh);
-        __syncthreads(); // a term belongs to the first row that holds it
+        __syncthreads();
+        if (threadIdx.x == 0 && (r & (r + 1)) == 0) {
+            out[blockIdx.x].terms[__popc(r)] = n_terms;
+            out[blockIdx.x].shared[__popc(r)] = n_shared;
+        }
+        __syncthreads();
     }
-    if (threadIdx.x == 0) terms[blockIdx.x] = make_uint4(found[0], found[0] + found[1], found[0] + found[1] + found[2], found[0] + found[1] + found[2] + found[3]);
 }
 int gram_tiles_pair(apoe_knn* g, const uint32_t* nodes, uint32_t n_nodes, bool* pair) {
     apoe_ctx* ctx = g->ctx;
     const TileShape two = tile_shape(ctx, g->corpus, true), one = tile_shape(ctx, g->corpus, false);
     *pair = two.pair;
-    if (!two.pair || !g->corpus->narrow) return APOE_OK;
+    if (!two.pair) return APOE_OK;
     if (!g->join_work.p) APOE_TRY(g->join_work.alloc(JOIN_COUNT_AT + JOIN_COUNT_PARTS * 8));
     GramTileArgs a{};
     a.C = g->corpus->view();
@@ -1059,18 +1097,25 @@ int gram_tiles_pair(apoe_knn* g, const uint32_t* nodes, uint32_t n_nodes, bool* 
     a.index_bits = two.index_bits;
     a.span = two.span;
     const uint32_t sample = std::min(n_nodes, GRAM_SAMPLE);
-    static_assert(JOIN_COUNT_AT % 2 == 0 && JOIN_COUNT_PARTS * 8 >= 2 * (int)GRAM_SAMPLE, "the step's partial counters hold the sample");
-    uint4 *terms = reinterpret_cast<uint4*>(g->join_work.p + JOIN_COUNT_AT), h[GRAM_SAMPLE];
-    gram_sample_kernel<<<sample, 256, two.index_bits / 8, ctx->stream>>>(a, terms);
+    static_assert(JOIN_COUNT_PARTS * 8 * sizeof(unsigned long long) >= GRAM_SAMPLE * sizeof(GramSample), "the step's partial counters hold the sample");
+    GramSample *out = reinterpret_cast<GramSample*>(g->join_work.p + JOIN_COUNT_AT), h[GRAM_SAMPLE];
+    if (g->corpus->narrow) gram_sample_kernel<true><<<sample, 256, 0, ctx->stream>>>(a, out);
+    else gram_sample_kernel<false><<<sample, 256, 0, ctx->stream>>>(a, out);
     APOE_HIP(hipGetLastError());
-    APOE_HIP(hipMemcpyAsync(h, terms, sample * sizeof(uint4), hipMemcpyDeviceToHost, ctx->stream));
+    APOE_HIP(hipMemcpyAsync(h, out, sample * sizeof(GramSample), hipMemcpyDeviceToHost, ctx->stream));
     APOE_HIP(hipStreamSynchronize(ctx->stream));
-    auto probes = [&](uint32_t slots) { // of a column by eight rows, summed over the sample
-        uint32_t n = 0;
-        for (uint32_t i = 0; i < sample; i++) n += h[i].w <= slots ? 1 : h[i].z <= slots ? 2 : h[i].y <= slots ? 4 : 8;
-        return n;
+    auto cost = [&](uint32_t slots) { // of a column's probes by eight rows, in fifths of a probe, summed over the sample
+        uint64_t sum = 0;
+        for (uint32_t i = 0; i < sample; i++) {
+            int t = 3;
+            while (t > 0 && (h[i].terms[t] > slots || h[i].shared[t] > (uint32_t)RT_OVF)) t--;
+            sum += (8u >> t) * (5ull + h[i].shared[t]);
+        }
+        return sum;
     };
-    *pair = 8 * probes(two.slot_cap) <= 9 * probes(one.slot_cap);
+    const uint64_t c2 = cost(two.slot_cap), c1 = cost(one.slot_cap);
+    const bool window = g->corpus->total_pairs <= (uint64_t)RT_CHUNKS * WAVE * g->corpus->n;
+    *pair = g->corpus->narrow ? 8 * c2 <= 9 * c1 : window ? c2 <= 2 * c1 : 2 * c2 <= 3 * c1;
     return APOE_OK;
 }
 
@@ -1099,12 +1144,9 @@ int launch_gram_tiles(apoe_knn* g, const uint32_t* nodes, uint32_t node0, uint32
     a.index_bits = shape.index_bits;
     a.slot_cap = shape.slot_cap;
     a.span = shape.span;
-    auto kernel_of = [&](auto threads) {
-        constexpr int NT = decltype(threads)::value;
-        return g->corpus->narrow ? &gram_tile_kernel<true, NT> : &gram_tile_kernel<false, NT>;
-    };
-    APOE_TRY(launch_tiles(ctx, shape.pair ? kernel_of(std::integral_constant<int, JT_PAIR_THREADS>{}) : kernel_of(std::integral_constant<int, JT_SOLO_THREADS>{}),
-                          shape, a));
+    if (shape.pair) APOE_TRY(launch_tiles(ctx, g->corpus->narrow ? &gram_tile_kernel<true, JT_PAIR_THREADS, false> : &gram_tile_kernel<false, JT_PAIR_THREADS, false>, shape, JT_PAIR_THREADS, a));
+    else if (g->corpus->narrow) APOE_TRY(launch_tiles(ctx, &gram_tile_kernel<true, JT_SOLO_THREADS, true>, shape, JT_SOLO_THREADS, a));
+    else APOE_TRY(launch_tiles(ctx, &gram_tile_kernel<false, JT_PAIR_THREADS, true>, shape, JT_PAIR_THREADS, a));
     if (unfit) {
         unsigned long long h[4] = {0, 0, 0, 0};
         APOE_HIP(hipMemcpyAsync(h, g->join_work.p, sizeof(h), hipMemcpyDeviceToHost, st));

@@ -11,7 +11,7 @@ N = 1200
 def make(kind, wide):
     import apoe_synth as S
     rng = np.random.default_rng(5)
-    a = list(S.to_numpy((S.corpus if kind in ("pairs decide", "few shared") else S.latent_corpus)(N, seed=21, device="cpu")))
+    a = list(S.to_numpy((S.corpus if kind in ("pairs decide", "few shared", "few terms") else S.latent_corpus)(N, seed=21, device="cpu")))
     if kind == "near twins":  # copies of documents, a little longer or shorter: products within the sketch's error of a norm, and clear of it
         half = N // 2
         dense, s_off, s_idx, s_val, b_off, b_idx, b_val = a
@@ -30,6 +30,11 @@ def make(kind, wide):
         off = np.concatenate([[0], np.cumsum(cnt)]).astype(np.uint32)
         idx = np.concatenate([np.sort(rng.choice(30000, c, replace=False)) for c in cnt]).astype(np.uint32)
         a[1:4] = off, idx, rng.uniform(1.0, 8.0, len(idx)).astype(np.float32)
+    elif kind == "few terms":  # as "few shared", in the wide format too: eight rows share their terms with each other, and few terms a bit of the table
+        cnt = rng.integers(280, 320, N)
+        off = np.concatenate([[0], np.cumsum(cnt)]).astype(np.uint32)
+        idx = np.concatenate([np.sort(rng.choice(2000, c, replace=False)) for c in cnt]).astype(np.uint32)
+        a[1:4] = off, idx, rng.uniform(1.0, 4.0, len(idx)).astype(np.float32)
     elif kind == "odd rows":  # no dense part, no terms, far magnitudes
         a[0] = a[0] * rng.choice([0.0, 1e-3, 1.0, 1.0, 30.0], N).astype(np.float32)[:, None]
         keep = rng.random(N) < 0.8
@@ -89,6 +94,6 @@ def check(gpu_ctx, kind, K, degree, wide, without=0):
 
 @pytest.mark.parametrize("wide", [False, True])
 @pytest.mark.parametrize("K,degree", [(64, 32), (64, 64), (128, 48)])
-@pytest.mark.parametrize("kind", ["bounds settle", "pairs decide", "near twins", "rich rows", "few shared", "odd rows"])
+@pytest.mark.parametrize("kind", ["bounds settle", "pairs decide", "near twins", "rich rows", "few shared", "few terms", "odd rows"])
 def test_prune_matches_oracle(gpu_ctx, kind, K, degree, wide):
     check(gpu_ctx, kind, K, degree, wide)
