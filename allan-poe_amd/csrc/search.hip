@@ -1182,9 +1182,14 @@ static int launch_mode(apoe_ctx* ctx, int mode, int nw, const SearchArgs& a, uin
 //   keyword  0.014: 0.91-0.98  0.03: 0.86-0.99  0.08: 0.89-0.97  0.17: 0.96-1.07  1.5: 0.97-1.04;  0.09: 0.93-0.94  0.18: 1.00-1.04  0.36: 1.06-1.08  2.2: 1.07-1.08
 // The line lies at an eighth. A linking entity's bonus is a third part: where it exceeds the dense part, the pool holds linked documents, no sketch is asked and the
 // pairs of most others are read twice (bonus 40; dense part 8 and 16 with dense neighbours 0.91, 49: 1.07-1.09, 100 on i.i.d. rows 1.03-1.08). Pairs alone never
-// ask them (SPLADE, cands 256: 24.5 ms without, 25.8 with). The codes are kernels of their own: with both ways in one, spilled registers cost searches without codes 3 %.
-static bool codes_pay(const apoe_corpus* c, const apoe_queries* q, const apoe_search_params* p, uint32_t q_count, uint32_t paths, bool kg) {
+// ask them (SPLADE, cands 256: 24.5 ms without, 25.8 with). Rows longer than the loads of a batch (192 pairs) read their rest one chunk after the other: 10 000 queries
+// on 200 000 docs with dense neighbours, time without / with codes by the pairs of an average row, cands 16 ... 200: plain 180: 1.04-1.11, 240: 1.03-1.06,
+// 300-360: 0.99-1.02, 420-480: 0.98-1.01, 660: 0.95; half 180: 1.02-1.03, 240: 0.96-0.98, 300: 0.95-0.97; keyword 180: 0.99-1.02, 240: 0.95-0.97. The lines lie at
+// 192 and, for plain searches, 320 pairs. The codes are kernels of their own: with both ways in one, spilled registers cost searches without codes 3 %.
+static bool codes_pay(const apoe_corpus* c, const apoe_queries* q, const apoe_search_params* p, uint32_t q_count, uint32_t paths, bool kg, bool plain) {
     if (!(paths & PATH_DENSE) || !(paths & (PATH_SPARSE | PATH_BM25))) return false;
+    const uint64_t read = (paths & PATH_SPARSE ? c->pairs_s : 0) + (paths & PATH_BM25 ? c->total_pairs - c->pairs_s : 0);
+    if (read > (plain ? 320ull : 3ull * WAVE) * c->n) return false;
     auto part = [&](float w, double mean_sq, uint64_t pairs, uint64_t q_pairs) { // of a path with that many pairs in all documents and in the batch
         return pairs ? fabs((double)w) * mean_sq * sqrt((double)q_pairs / q_count / ((double)pairs / c->n)) : 0.0;
     };
@@ -1247,7 +1252,7 @@ int launch_search(apoe_ctx* ctx, const apoe_corpus* c, const apoe_queries* q, co
         APOE_REQUIRE(c->n < (1u << 30), "keyword-filter search keeps two flag bits on a document id: %u documents are too many", c->n);
         a.paths = PATH_DENSE | PATH_SPARSE | PATH_BM25; // query.cu:2005-2007: always the three-path loop
     }
-    a.coded = c->coded && !a.full_eval && codes_pay(c, q, p, q_count, a.paths, use_kg) ? 1u : 0u;
+    a.coded = c->coded && !a.full_eval && codes_pay(c, q, p, q_count, a.paths, use_kg, mode == MODE_PLAIN && !a.half) ? 1u : 0u;
     if (use_kg) {
         APOE_REQUIRE(kg->n_queries >= p->q_begin + q_count, "knowledge graph holds entities for %u queries, %u needed", kg->n_queries, p->q_begin + q_count);
         a.e2e_off = kg->e2e_off.p;

@@ -102,3 +102,25 @@ def test_codes_are_asked_where_the_dense_part_decides(gpu_ctx):
             read.append(apoe.search(gpu_ctx, gc, gq, gg, (49, 1, 1), 64, variant=4, **more)[2].algo_bytes)
             gc.close()
         assert (read[0] != read[1]) == asked, (scale, sorted(more))
+
+
+@pytest.mark.parametrize("pairs", [190, 194, 318, 322])
+def test_codes_are_asked_up_to_a_row_length(gpu_ctx, pairs):
+    """Rows of one length: to 192 pairs, what a batch of loads holds, in every search; to 320 in plain ones. Rows are those without codes either way."""
+    import apoe
+    rng = np.random.default_rng(pairs)
+    corpus, queries, rows, entry = world("plain", 3)
+    corpus = (corpus[0], *rows_of(rng, N, [pairs // 2], "plain"), *rows_of(rng, N, [pairs // 2], "plain"))
+    b_idx = queries[5].copy()
+    b_idx[queries[4][:-1]] |= np.uint32(0x80000000)
+    gq, gk, gg = apoe.Queries(gpu_ctx, *queries), apoe.Queries(gpu_ctx, *queries[:5], b_idx, queries[6]), apoe.Graph(gpu_ctx, rows, entry)
+    full, less = apoe.Corpus(gpu_ctx, *corpus), apoe.Corpus(gpu_ctx, *corpus, without=apoe.WITHOUT_CODES)
+    full.make_half_rows()
+    less.make_half_rows()
+    for query, variant, more, limit in ((gq, 4, {}, 320), (gq, 4 | 0x200, {}, 192), (gk, 4, dict(keyword_filter=True), 192)):
+        a, ad, sa = apoe.search(gpu_ctx, full, query, gg, (49, 1, 1), 64, variant=variant, **more)
+        b, bd, sb = apoe.search(gpu_ctx, less, query, gg, (49, 1, 1), 64, variant=variant, **more)
+        assert np.array_equal(a, b) and np.array_equal(ad, bd)
+        assert (sa.algo_bytes != sb.algo_bytes) == (pairs <= limit), (variant, sorted(more))
+    for x in (less, full, gg, gk, gq):
+        x.close()
