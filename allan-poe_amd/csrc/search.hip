@@ -329,15 +329,20 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
     extern __shared__ __align__(16) char smem[];
     const SearchLds L(a.slots_s, a.slots_b, a.ovf_cap, a.cands, MODE);
     // not volatile (barriers separate the waves' accesses): a volatile access through a generic pointer is a flat one, which waits for every
-    // load under way (one query 699 -> 663 us, 500 queries of pool 1000 8.27 -> 7.94 ms)
-    uint32_t* ctl = reinterpret_cast<uint32_t*>(smem + L.ctl);
+    // load under way (one query 699 -> 663 us, 500 queries of pool 1000 8.27 -> 7.94 ms). Knowledge-graph searches gain 1 to 5 % by that on eight and sixteen
+    // waves a query and lose up to 8 on four and two, most in small pools (700 queries, cands 16 / 64 / 256: 2.00 / 3.36 / 6.55 ms volatile, 2.15 / 3.54 / 6.67 not),
+    // so they keep it there.
+    constexpr bool FLAT = KG && NW <= 4;
+    using Word = std::conditional_t<FLAT, volatile uint32_t, uint32_t>;
+    using Scalar = std::conditional_t<FLAT, volatile float, float>;
+    Word* ctl = reinterpret_cast<Word*>(smem + L.ctl);
     float4* qd = reinterpret_cast<float4*>(smem + L.qd);
     float* part = reinterpret_cast<float*>(smem + L.part);
     QueryTabs T;
     T.b = reinterpret_cast<uint4*>(smem + L.tab);
     T.ovf = reinterpret_cast<uint2*>(smem + L.ovf);
     T.ovf_cap = a.ovf_cap;
-    T.n_ovf = &ctl[CTL_NOVF];
+    T.n_ovf = const_cast<uint32_t*>(&ctl[CTL_NOVF]);
     T.mask_s = a.slots_s - 1;
     T.mask_b = a.slots_b - 1;
     Pool P;
@@ -350,7 +355,7 @@ __global__ __launch_bounds__(NW* WAVE) __attribute__((amdgpu_waves_per_eu(MODE =
         reinterpret_cast<float4*>(part)[pos] = make_float4(__uint_as_float((uint32_t)desc), __uint_as_float((uint32_t)(desc >> 32)), dn, 0.f);
     };
     uint32_t* codes = a.codes + (size_t)blockIdx.x * (SKETCH_BYTES / 4);
-    float* qs = reinterpret_cast<float*>(smem + L.qs);
+    Scalar* qs = reinterpret_cast<Scalar*>(smem + L.qs);
     uint32_t* new_id = reinterpret_cast<uint32_t*>(smem + L.new_id);
     float* new_dist = reinterpret_cast<float*>(smem + L.new_dist);
     uint32_t* new_ent = reinterpret_cast<uint32_t*>(smem + L.new_ent);
