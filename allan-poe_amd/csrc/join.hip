@@ -308,22 +308,29 @@ __device__ __forceinline__ void tile_sparse(const char* recs, const RankTab& T, 
                                 rows[k].touch();
                                 asm volatile("" : "+s"(shape[k]));
                             }
-#pragma unroll
-                            for (int t = 0; t < NP; t++) acc[k][t] = 0.f;
                         }
                         if constexpr (!HOLD) {
                             const uint32_t next = b + TILE_AHEAD * NW;
                             if (next < M) col_load(s, next);
                             else if (a1 < R) col_load(s, wave + s * NW); // the first of the slot again, for the next group
                         }
+#pragma unroll
+                        for (int k = 0; k < BATCH; k++)
+#pragma unroll
+                            for (int t = 0; t < NP; t++) acc[k][t] = 0.f;
                         ranktab_probe_rows<NARROW, BATCH, NP>(T, rows, shape, [&](int k) { return col_pairs(b + k * NW); }, n_ovf, acc, lane);
 #pragma unroll
                         for (int k = 0; k < BATCH; k++) {
+                            const uint32_t at = b + k * NW;
+                            if (k > 0 && at >= M) continue;
                             uint32_t t;
-                            float z;
-                            if constexpr (NP == 4) z = wave_sum4_dpp(acc[k], lane, &t);
-                            else z = wave_sum_1x8(acc[k], lane, &t);
-                            if ((lane & 15) < 4 && lane < (NP == 4 ? 4 : 32) && t < nt && b + k * NW < M) G[(a0 + t) * JT_STRIDE + b + k * NW] = z;
+                            if constexpr (NP == 4) {
+                                const float z = wave_sum4_dpp(acc[k], lane, &t);
+                                if (lane < 4 && t < nt) G[(a0 + t) * JT_STRIDE + at] = z;
+                            } else {
+                                const float z = wave_sum_1x8(acc[k], lane, &t);
+                                if ((lane & 15) < 4 && lane < 32 && t < nt) G[(a0 + t) * JT_STRIDE + at] = z;
+                            }
                         }
                     }
                     __builtin_amdgcn_sched_barrier(0); // one batch at a time: the scheduler must not pile up the reads of all of them
