@@ -3,7 +3,7 @@ the products that do not involve them as they are, in each form of the prune."""
 import numpy as np
 import pytest
 
-from test_gpu_prune_bounds import equal_but_for_ties
+from test_gpu_prune_ties import equal_but_for_ties
 
 pytestmark = pytest.mark.gpu
 N = 1200

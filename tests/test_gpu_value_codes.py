@@ -44,7 +44,6 @@ def test_rows_are_those_of_a_walk_without_bounds(gpu_ctx, kind):
     gc, gq, gg = apoe.Corpus(gpu_ctx, *corpus), apoe.Queries(gpu_ctx, *queries), apoe.Graph(gpu_ctx, rows, entry)
     gk = apoe.Queries(gpu_ctx, *queries[:5], b_idx, queries[6])
     kg = apoe.KnowledgeGraph(gpu_ctx, *S.to_numpy(S.knowledge_graph(800, N, NQ, seed=23, device="cpu", mean_out=6.0)))
-    less = apoe.Corpus(gpu_ctx, *corpus, without=apoe.WITHOUT_CODES)
     gc.make_half_rows()
     for w3, cands, shape in (((8, 1, 1), 24, 4), ((49, 1, 1), 64, 1), ((24, 3, 0), 33, 1), ((16, 0, 2), 100, 4), ((1, 1, 1), 24, 4)):
         for query, more in ((gq, {}), (gk, dict(keyword_filter=True)), (gq, dict(kg=kg, kg_weight=5.0))):
@@ -52,12 +51,27 @@ def test_rows_are_those_of_a_walk_without_bounds(gpu_ctx, kind):
             b, bd, sb = apoe.search(gpu_ctx, gc, query, gg, w3, cands, variant=shape | 0x100, **more)
             assert np.array_equal(a, b) and np.array_equal(ad, bd, equal_nan=True), (w3, cands, sorted(more))
             assert sa.evaluations == sb.evaluations and sa.dense_rows <= sb.dense_rows
-            if kind == "plain":  # a corpus without codes reads other bytes where they are asked: the dense part reaches an eighth of the pairs' under all but equal weights
-                read = apoe.search(gpu_ctx, less, query, gg, w3, cands, variant=shape, **more)[2].algo_bytes
-                assert (sa.algo_bytes != read) == (w3[0] > 1), (w3, cands, sorted(more))
+            if kind == "plain" and w3 == (49, 1, 1):  # codes are in use: sketches and dense rows alone (1 032 and 4 096 bytes each) do not explain what was read
+                assert (sb.algo_bytes - sa.algo_bytes - 4096 * (sb.dense_rows - sa.dense_rows)) % 1032 != 0
         a, ad, _ = apoe.search(gpu_ctx, gc, gq, gg, w3, cands, variant=shape | 0x200)
         b, bd, _ = apoe.search(gpu_ctx, gc, gq, gg, w3, cands, variant=shape | 0x300)
         assert np.array_equal(a, b) and np.array_equal(ad, bd, equal_nan=True), (w3, cands, "half")
+
+
+def test_which_weights_ask_codes(gpu_ctx):
+    """A corpus without codes reads other bytes where they are asked: the dense part reaches an eighth of the pairs' under all but equal weights."""
+    import apoe
+    import apoe_synth as S
+    corpus, queries, rows, entry = world("plain", 3)
+    b_idx = queries[5].copy()
+    b_idx[queries[4][:-1]] |= np.uint32(0x80000000)
+    full, less = apoe.Corpus(gpu_ctx, *corpus), apoe.Corpus(gpu_ctx, *corpus, without=apoe.WITHOUT_CODES)
+    gq, gk, gg = apoe.Queries(gpu_ctx, *queries), apoe.Queries(gpu_ctx, *queries[:5], b_idx, queries[6]), apoe.Graph(gpu_ctx, rows, entry)
+    kg = apoe.KnowledgeGraph(gpu_ctx, *S.to_numpy(S.knowledge_graph(800, N, NQ, seed=23, device="cpu", mean_out=6.0)))
+    for w3, cands, shape in (((8, 1, 1), 24, 4), ((49, 1, 1), 64, 1), ((24, 3, 0), 33, 1), ((16, 0, 2), 100, 4), ((1, 1, 1), 24, 4)):
+        for query, more in ((gq, {}), (gk, dict(keyword_filter=True)), (gq, dict(kg=kg, kg_weight=5.0))):
+            read = [apoe.search(gpu_ctx, gc, query, gg, w3, cands, variant=shape, **more)[2].algo_bytes for gc in (full, less)]
+            assert (read[0] != read[1]) == (w3[0] > 1), (w3, cands, sorted(more))
 
 
 def test_bytes_of_evaluations_that_the_codes_leave_open(gpu_ctx):

@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 
 import test_gpu_join_tiles as tiles
-import test_gpu_prune_bounds as prune
+import test_gpu_prune_ties as prune
 import test_gpu_value_codes as values
 
 pytestmark = pytest.mark.gpu
